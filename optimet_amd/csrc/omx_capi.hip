@@ -143,7 +143,7 @@ struct omx_context {
   DBuf d_xyz, d_radius, d_eps, d_mu, d_eps_sh, d_kppp, d_kpar, d_gam, d_sph, d_ov, d_inc, d_incloc, d_Q, d_w,
       d_coef, d_S64, d_S32, d_V64, d_V32, d_x, d_xsh, d_xint, d_xintsh, d_K, d_K1, d_cross, d_cg, d_abscoef, d_abssh,
       d_absbes,
-      d_fpts, d_fout;
+      d_fpts, d_fout, d_fown, d_fpart;
   DBuf d_piv, d_perm, d_cand, d_cnt, d_map, d_status, d_wlu;
   hipStream_t aux = nullptr;
   hipEvent_t lu_ev[4] = {nullptr, nullptr, nullptr, nullptr};
@@ -2006,7 +2006,7 @@ void omx_destroy(omx_context *c) {
                   &c->d_wlu, &c->d_status, &c->d_basis, &c->d_basisZ, &c->d_w1, &c->d_w2, &c->d_r,
                   &c->d_part, &c->d_h, &c->d_nrm, &c->d_gpart, &c->d_piv2, &c->d_perm2,
                   &c->d_dinv, &c->d_dinv2, &c->d_F64, &c->d_F64sh, &c->d_abscoef, &c->d_abssh, &c->d_absbes,
-                  &c->d_fpts, &c->d_fout};
+                  &c->d_fpts, &c->d_fout, &c->d_fown, &c->d_fpart};
   for(DBuf *b : bufs) b->release(&c->total);
   auto &w = c->sw;
   DBuf *sbufs[] = {&w.S64, &w.S32, &w.V64, &w.V32, &w.F64, &w.F64sh, &w.eps, &w.eps_sh, &w.ov, &w.incloc, &w.Q,
@@ -2706,6 +2706,12 @@ int omx_fields(omx_context *c, int npts, const double *xyz, double *E, double *H
     const int cap = std::min(npts, chunk);
     c->d_fpts.ensure(sizeof(double) * 3 * cap, &c->total);
     c->d_fout.ensure(sizeof(cplx) * 12 * cap, &c->total);
+    c->d_fown.ensure(sizeof(int) * cap, &c->total);
+    // the last chunk is smaller than the others and may take more slices
+    const int tail = npts % chunk ? npts % chunk : cap;
+    const size_t pe = std::max((size_t)omx::fields_slices(c->P, cap, sh) * cap,
+                               (size_t)omx::fields_slices(c->P, tail, sh) * tail);
+    c->d_fpart.ensure(sizeof(cplx) * (sh ? 12 : 6) * pe, &c->total);
     for(int i0 = 0; i0 < npts; i0 += chunk) {
       const int n = std::min(chunk, npts - i0);
       cplx *o = c->d_fout.as<cplx>();
@@ -2715,7 +2721,7 @@ int omx_fields(omx_context *c, int npts, const double *xyz, double *E, double *H
                         c->d_eps_sh.as<cplx>(), c->d_gam.as<cplx>(), sh ? c->d_cg.as<double>() : nullptr,
                         c->d_inc.as<cplx>(), c->d_x.as<cplx>(), c->d_xint.as<cplx>(), c->d_xsh.as<cplx>(),
                         c->d_xintsh.as<cplx>(), c->d_fpts.as<double>(), o, o + 3 * (size_t)cap, o + 6 * (size_t)cap,
-                        o + 9 * (size_t)cap};
+                        o + 9 * (size_t)cap, c->d_fown.as<int>(), c->d_fpart.as<cplx>()};
       omx::run_fields(fa, c->st);
       HIPCHK(hipGetLastError());
       const size_t b = sizeof(cplx) * 3 * n, off = 6 * (size_t)i0;

@@ -100,7 +100,10 @@ struct FieldArgs {
   const cplx *x, *xint, *xsh, *xintsh;     // solution vectors (N each)
   const double *pts;                       // 3 npts
   cplx *E, *H, *Esh, *Hsh;                 // 3 npts each; Esh, Hsh unused without sh
+  int *owner;                              // workspace: npts
+  cplx *part;                              // workspace: fields_slices() x (sh ? 12 : 6) x npts
 };
+int fields_slices(int P, int npts, int sh);
 void run_fields(const FieldArgs &a, hipStream_t st);
 
 // nb > 1: a batch of nb systems in one launch (the batch fields of the args)
