@@ -180,19 +180,26 @@ struct omx_context {
     double rsum = 0, bytes = 0, ref_mb = 0;
     std::vector<int> rank;           // [i P + j]: r, -1 dense, 0 diagonal
     std::vector<const cplx *> where;  // [i P + j]: U (compressed) or the block (dense)
-    std::vector<DBuf> pools;          // factor pools, one per compression chunk
+    std::vector<DBuf> pools;          // factor pools, one per compression chunk (kept between builds)
     DBuf dense, desc, rowptr, acalist, t, part;
     bool built = false;
-    void release(size_t *T) {
-      for(auto &p : pools) p.release(T);
-      pools.clear();
-      DBuf *b[] = {&dense, &desc, &rowptr, &acalist, &t, &part};
-      for(DBuf *x : b) x->release(T);
+    // forgets the operator; its device buffers stay for the next one (a scan
+    // rebuilds it at every wavelength; freeing and mapping gigabytes again took
+    // 6 of 28 ms per solve of 300 spheres at nmax 5, and 140 of 173 ms in a
+    // process that had solved larger systems before)
+    void reset() {
       rank.clear();
       where.clear();
       built = false;
       bytes = ref_mb = rsum = 0;
       naca = ndense = rmax = 0;
+    }
+    void release(size_t *T) {
+      for(auto &p : pools) p.release(T);
+      pools.clear();
+      DBuf *b[] = {&dense, &desc, &rowptr, &acalist, &t, &part};
+      for(DBuf *x : b) x->release(T);
+      reset();
     }
   } aca[2];
   DBuf d_acaA, d_acaU, d_acaV, d_acaR, d_acaOff, d_plist;
@@ -402,10 +409,19 @@ float elapsed(omx_context *c, int a, int b) {
 constexpr double kAcaEps = 1e-3;            // PreconditionedMatrix.cpp:774
 constexpr double kAcaStagingBytes = 1.5e9;  // assembly + factor staging of one chunk
 
+// Gives back the compressed operators and their staging (another solver kind,
+// or omx_trim).
+void aca_release(omx_context *c) {
+  c->aca[0].release(&c->total);
+  c->aca[1].release(&c->total);
+  DBuf *b[] = {&c->d_acaA, &c->d_acaU, &c->d_acaV};
+  for(DBuf *x : b) x->release(&c->total);
+}
+
 void aca_build(omx_context *c, bool shf) {
   omx_context::AcaMat &m = c->aca[shf ? 1 : 0];
   size_t *T = &c->total;
-  m.release(T);
+  m.reset();
   const int P = c->P, nmax = c->nmax, n = 2 * c->nf;
   const size_t n2 = (size_t)n * n;
   hipStream_t st = c->st;
@@ -466,7 +482,8 @@ void aca_build(omx_context *c, bool shf) {
     c->d_plist.ensure(sizeof(int) * std::max((size_t)C, listn), T);
     std::vector<int> rk(C);
     std::vector<size_t> off(C);
-    for(int b0 = 0; b0 < m.naca; b0 += C) {
+    size_t chunk = 0;
+    for(int b0 = 0; b0 < m.naca; b0 += C, ++chunk) {
       const int nb = std::min(C, m.naca - b0);
       HIPCHK(hipMemcpyAsync(c->d_plist.p, al.data() + b0, sizeof(int) * nb, hipMemcpyHostToDevice, st));
       omx::PairArgs pa = base;
@@ -485,9 +502,11 @@ void aca_build(omx_context *c, bool shf) {
         off[b] = tot;
         tot += 2 * (size_t)n * rk[b];
       }
-      m.pools.emplace_back();
-      DBuf &pool = m.pools.back();
-      pool.ensure(sizeof(cplx) * tot, T);
+      if(m.pools.size() <= chunk) m.pools.emplace_back();
+      DBuf &pool = m.pools[chunk];
+      // an eighth to spare when it has to grow: ranks vary a little from one
+      // wavelength to the next
+      if(pool.bytes < sizeof(cplx) * tot) pool.ensure(sizeof(cplx) * (tot + tot / 8), T);
       HIPCHK(hipMemcpyAsync(c->d_acaOff.p, off.data(), sizeof(size_t) * nb, hipMemcpyHostToDevice, st));
       omx::run_aca_pack(c->d_acaU.as<cplx>(), c->d_acaV.as<cplx>(), n, nb, c->d_acaR.as<int>(), pool.as<cplx>(),
                         c->d_acaOff.as<size_t>(), st);
@@ -497,9 +516,6 @@ void aca_build(omx_context *c, bool shf) {
       }
       HIPCHK(hipStreamSynchronize(st));  // off, rk and the list buffer are reused
     }
-    // the staging is only needed while compressing
-    DBuf *stg[] = {&c->d_acaA, &c->d_acaU, &c->d_acaV};
-    for(DBuf *b : stg) b->release(T);
   }
   // descriptors, block row by block row
   std::vector<omx::AcaDesc> desc;
@@ -2255,8 +2271,7 @@ int omx_update(omx_context *c) {
       aca_build(c, false);
       if(c->sh) aca_build(c, true); else c->aca[1].release(&c->total);
     } else {
-      c->aca[0].release(&c->total);
-      c->aca[1].release(&c->total);
+      aca_release(c);
     }
     omx::PairArgs pa{P, nmax, omx::OV_T, c->waveK(), c->d_sph.as<double>(), c->d_ov.as<cplx>(),
                      c->d_coef.as<double>(), lda, c->d_S64.as<cplx>(), c->d_S32.as<float2>()};
@@ -3062,8 +3077,7 @@ int omx_trim(omx_context *c) {
                    &w.V32, &w.F64, &w.F64sh, &w.basis, &w.basisZ, &w.gpart, &c->d_basis, &c->d_basisZ,
                    &c->d_gpart};
     for(DBuf *b : big) b->release(&c->total);
-    c->aca[0].release(&c->total);
-    c->aca[1].release(&c->total);
+    aca_release(c);
     c->ws_in.release(&c->total);
     c->updated = c->solved = false;
     c->factored = c->factored_sh = false;
