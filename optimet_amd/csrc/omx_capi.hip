@@ -64,6 +64,12 @@ struct DBuf {
   template <typename T> T *as() const { return static_cast<T *>(p); }
 };
 
+// A part of a DBuf.
+struct DView {
+  void *p = nullptr;
+  template <typename T> T *as() const { return static_cast<T *>(p); }
+};
+
 // Normwise backward error accepted from a refinement that stopped above its
 // residual band: 1000 units of FP64 roundoff.
 const double kBackwardErrorBound = 1e3 * 1.1e-16;
@@ -140,7 +146,9 @@ struct omx_context {
   bool dirty32 = false, dirty32_sh = false;  // the FP32 matrix holds factors, not S (V)
   int cg_nmax = 0;
   // device buffers
-  DBuf d_xyz, d_radius, d_eps, d_mu, d_eps_sh, d_kppp, d_kpar, d_gam, d_sph, d_ov, d_inc, d_incloc, d_Q, d_w,
+  DBuf d_geo;  // the geometry's arrays, one after another (upload_geometry)
+  DView d_xyz, d_radius, d_eps, d_mu, d_eps_sh, d_kppp, d_kpar, d_gam;
+  DBuf d_sph, d_ov, d_inc, d_incloc, d_Q, d_w,
       d_coef, d_S64, d_S32, d_V64, d_V32, d_x, d_xsh, d_xint, d_xintsh, d_K, d_K1, d_cross, d_cg, d_abscoef, d_abssh,
       d_absbes,
       d_fpts, d_fout, d_fown, d_fpart;
@@ -159,6 +167,13 @@ struct omx_context {
   // pinned host staging of one Arnoldi step's projections and norm
   cplx *h_pin = nullptr;
   int h_pin_n = 0;
+  // pinned host staging of the geometry, and the event after its last copy
+  double *geo_pin = nullptr;
+  int geo_pin_n = 0;
+  hipEvent_t geo_ev = nullptr;
+  // omx_update's times (start, objects done, assembly done) and its joins
+  bool upd_timed = false;
+  hipEvent_t uev[3] = {nullptr, nullptr, nullptr}, ujoin[2] = {nullptr, nullptr};
   omx::LuWork lu{}, lu_sh{};
   bool profile = false;
   std::vector<hipEvent_t> pev;
@@ -311,19 +326,43 @@ void alloc_lu(omx_context *c, omx::LuWork &w, DBuf &piv, DBuf &perm, DBuf &dinv,
   w.gmax = gmax;
 }
 
+// The geometry's arrays on the device in one copy: mu, eps, eps_sh and the
+// susceptibilities (complex, P each), then the centres and radii.  The staging
+// is pinned, and rewritten only once the copy before has left it.
+constexpr int kGeoDoubles = 6 * 2 + 3 + 1;
+void upload_geometry(omx_context *c) {
+  const size_t P = c->P;
+  const int n = kGeoDoubles * c->P;
+  if(c->geo_pin_n < n) {
+    HIPCHK(hipEventSynchronize(c->geo_ev));
+    if(c->geo_pin) (void)hipHostFree(c->geo_pin);
+    c->geo_pin = nullptr;
+    c->geo_pin_n = 0;
+    HIPCHK(hipHostMalloc(reinterpret_cast<void **>(&c->geo_pin), sizeof(double) * n));
+    c->geo_pin_n = n;
+  }
+  HIPCHK(hipEventSynchronize(c->geo_ev));
+  DView *cv[] = {&c->d_mu, &c->d_eps, &c->d_eps_sh, &c->d_kppp, &c->d_kpar, &c->d_gam};
+  const std::vector<cplx> *src[] = {&c->mu, &c->eps, &c->eps_sh, &c->ksippp, &c->ksiparppar, &c->gamma};
+  double *h = c->geo_pin, *d = c->d_geo.as<double>();
+  for(int e = 0; e < 6; ++e) {
+    std::memcpy(h + 2 * P * e, src[e]->data(), sizeof(cplx) * P);
+    cv[e]->p = d + 2 * P * e;
+  }
+  std::memcpy(h + 12 * P, c->xyz.data(), sizeof(double) * 3 * P);
+  std::memcpy(h + 15 * P, c->radius.data(), sizeof(double) * P);
+  c->d_xyz.p = d + 12 * P;
+  c->d_radius.p = d + 15 * P;
+  HIPCHK(hipMemcpyAsync(d, h, sizeof(double) * n, hipMemcpyHostToDevice, c->st));
+  HIPCHK(hipEventRecord(c->geo_ev, c->st));
+}
+
 // (Re)allocates every size-dependent buffer.
 void alloc_all(omx_context *c) {
   const int P = c->P, nf = c->nf, N = c->N, Np = c->Np, S = c->nmax + 1;
   size_t *T = &c->total;
-  c->d_xyz.ensure(sizeof(double) * 3 * P, T);
-  c->d_radius.ensure(sizeof(double) * P, T);
-  c->d_eps.ensure(sizeof(cplx) * P, T);
-  c->d_mu.ensure(sizeof(cplx) * P, T);
-  c->d_eps_sh.ensure(sizeof(cplx) * P, T);
-  c->d_kppp.ensure(sizeof(cplx) * P, T);
-  c->d_kpar.ensure(sizeof(cplx) * P, T);
-  c->d_gam.ensure(sizeof(cplx) * P, T);
-  c->d_sph.ensure(sizeof(double) * 3 * P, T);
+  c->d_geo.ensure(sizeof(double) * kGeoDoubles * P, T);
+  c->d_sph.ensure(sizeof(double) * omx::kSphDoubles * P, T);
   c->d_ov.ensure(sizeof(cplx) * omx::OV_COUNT * P * 2 * S, T);
   c->d_inc.ensure(sizeof(cplx) * 2 * nf, T);
   c->d_incloc.ensure(sizeof(cplx) * N, T);
@@ -439,41 +478,47 @@ void aca_build(omx_context *c, bool shf) {
     ctr[3 * i + 1] = r * std::sin(th) * std::sin(ph);
     ctr[3 * i + 2] = r * std::cos(th);
   }
+  // unordered pairs i < j; blocks 2 b (i, j) and 2 b + 1 (j, i) of pair b
   std::vector<int> dl, al;
   for(int i = 0; i < P; ++i)
-    for(int j = 0; j < P; ++j) {
-      if(i == j) continue;
+    for(int j = i + 1; j < P; ++j) {
       const double d = std::sqrt(std::pow(ctr[3 * j] - ctr[3 * i], 2.0) + std::pow(ctr[3 * j + 1] - ctr[3 * i + 1], 2.0) +
                                  std::pow(ctr[3 * j + 2] - ctr[3 * i + 2], 2.0));
       if(d >= 2.0 * (c->radius[i] + c->radius[j])) {
         al.push_back(i * P + j);
       } else {
         dl.push_back(i * P + j);
-        m.rank[(size_t)i * P + j] = -1;
+        m.rank[(size_t)i * P + j] = m.rank[(size_t)j * P + i] = -1;
       }
     }
-  m.ndense = (int)dl.size();
-  m.naca = (int)al.size();
+  m.ndense = 2 * (int)dl.size();
+  m.naca = 2 * (int)al.size();
+  // block 2 b + h of a pair list as i P + j
+  auto block = [P](const std::vector<int> &l, size_t b) {
+    const int pid = l[b / 2];
+    return b & 1 ? (size_t)(pid % P) * P + pid / P : (size_t)pid;
+  };
   cplx k = c->waveK();
   if(shf) k = omx::mk(2.0 * k.x, 2.0 * k.y);  // PreconditionedMatrix.cpp:725
   omx::PairArgs base{P, nmax, shf ? omx::OV_TSH : omx::OV_T, k, c->d_sph.as<double>(), c->d_ov.as<cplx>(),
                      c->d_coef.as<double>(), (size_t)n, nullptr, nullptr};
-  base.zblk = n2;
+  base.zblk = n2;  // S_ij of pair b at 2 b n2, S_ji behind it
   const size_t listn = std::max(dl.size(), (size_t)1);
   if(m.ndense) {
-    m.dense.ensure(sizeof(cplx) * n2 * dl.size(), T);
+    m.dense.ensure(sizeof(cplx) * n2 * m.ndense, T);
     c->d_plist.ensure(sizeof(int) * listn, T);
     HIPCHK(hipMemcpyAsync(c->d_plist.p, dl.data(), sizeof(int) * dl.size(), hipMemcpyHostToDevice, st));
     omx::PairArgs pa = base;
     pa.S64 = m.dense.as<cplx>();
     pa.plist = c->d_plist.as<int>();
-    pa.nlist = m.ndense;
+    pa.nlist = (int)dl.size();
     omx::run_pairs(pa, st);
-    for(size_t b = 0; b < dl.size(); ++b) m.where[dl[b]] = m.dense.as<cplx>() + b * n2;
+    for(int b = 0; b < m.ndense; ++b) m.where[block(dl, b)] = m.dense.as<cplx>() + b * n2;
     HIPCHK(hipStreamSynchronize(st));  // dl and the list buffer are reused below
   }
   if(m.naca) {
-    const int C = (int)std::max<double>(1.0, std::min<double>(m.naca, kAcaStagingBytes / (48.0 * n2)));
+    // blocks of a chunk: whole pairs
+    const int C = 2 * (int)std::max<double>(1.0, std::min<double>(m.naca / 2, kAcaStagingBytes / (96.0 * n2)));
     c->d_acaA.ensure(sizeof(cplx) * n2 * C, T);
     c->d_acaU.ensure(sizeof(cplx) * n2 * C, T);
     c->d_acaV.ensure(sizeof(cplx) * n2 * C, T);
@@ -485,11 +530,11 @@ void aca_build(omx_context *c, bool shf) {
     size_t chunk = 0;
     for(int b0 = 0; b0 < m.naca; b0 += C, ++chunk) {
       const int nb = std::min(C, m.naca - b0);
-      HIPCHK(hipMemcpyAsync(c->d_plist.p, al.data() + b0, sizeof(int) * nb, hipMemcpyHostToDevice, st));
+      HIPCHK(hipMemcpyAsync(c->d_plist.p, al.data() + b0 / 2, sizeof(int) * (nb / 2), hipMemcpyHostToDevice, st));
       omx::PairArgs pa = base;
       pa.S64 = c->d_acaA.as<cplx>();
       pa.plist = c->d_plist.as<int>();
-      pa.nlist = nb;
+      pa.nlist = nb / 2;
       omx::run_pairs(pa, st);
       omx::AcaArgs aa{n, nb, kAcaEps, c->d_acaA.as<cplx>(), c->d_acaU.as<cplx>(), c->d_acaV.as<cplx>(),
                       c->d_acaR.as<int>()};
@@ -511,8 +556,8 @@ void aca_build(omx_context *c, bool shf) {
       omx::run_aca_pack(c->d_acaU.as<cplx>(), c->d_acaV.as<cplx>(), n, nb, c->d_acaR.as<int>(), pool.as<cplx>(),
                         c->d_acaOff.as<size_t>(), st);
       for(int b = 0; b < nb; ++b) {
-        m.rank[al[b0 + b]] = rk[b];
-        m.where[al[b0 + b]] = pool.as<cplx>() + off[b];
+        m.rank[block(al, b0 + b)] = rk[b];
+        m.where[block(al, b0 + b)] = pool.as<cplx>() + off[b];
       }
       HIPCHK(hipStreamSynchronize(st));  // off, rk and the list buffer are reused
     }
@@ -1651,31 +1696,35 @@ void sweep_chunk(omx_context *c, int nb, const double *lam, const cplx *eps, con
   oa.zov = ovs;
   omx::run_objects(oa, st, nb);
   omx::OriginArgs og{P, nmax, hk[0], c->d_sph.as<double>(), w.ov.as<cplx>(), c->d_coef.as<double>(),
-                     c->d_inc.as<cplx>(), w.incloc.as<cplx>(), w.Q.as<cplx>(), w.w.as<double>()};
+                     c->d_inc.as<cplx>(), w.incloc.as<cplx>(), w.Q.as<cplx>(), w.w.as<double>(), sh};
   og.kz = kz;
   og.zov = ovs;
   og.zvec = lda;
   og.zw = ws;
-  omx::run_origin(og, st, nb);
+  // beside the pairs, as in omx_update
+  HIPCHK(hipEventRecord(c->ujoin[0], st));
+  HIPCHK(hipStreamWaitEvent(c->st2, c->ujoin[0], 0));
+  omx::run_origin(og, c->st2, nb);
+  HIPCHK(hipEventRecord(c->ujoin[1], c->st2));
   omx::PairArgs pa{P, nmax, omx::OV_T, hk[0], c->d_sph.as<double>(), w.ov.as<cplx>(), c->d_coef.as<double>(), lda,
                    cS64, f64 ? nullptr : cS32};
   pa.kz = kz;
   pa.zov = ovs;
   pa.zS = n2;
+  if(sh) {  // V in the same launch
+    pa.tkind2 = omx::OV_TSH;
+    pa.kz2 = kz + nb;
+    pa.V64 = cV64;
+    pa.V32 = f64 ? nullptr : cV32;
+  }
   omx::run_pairs(pa, st, nb);
   omx::run_pad64(cS64, N, Np, lda, st, nb, n2);
   if(!f64) omx::run_pad32(cS32, N, Np, lda, st, nb, n2);
   if(sh) {
-    omx::PairArgs pv = pa;
-    pv.tkind = omx::OV_TSH;
-    pv.k = hk[nb];
-    pv.kz = kz + nb;
-    pv.S64 = cV64;
-    pv.S32 = f64 ? nullptr : cV32;
-    omx::run_pairs(pv, st, nb);
     omx::run_pad64(cV64, N, Np, lda, st, nb, n2);
     if(!f64) omx::run_pad32(cV32, N, Np, lda, st, nb, n2);
   }
+  HIPCHK(hipStreamWaitEvent(st, c->ujoin[1], 0));
   HIPCHK(hipGetLastError());
   auto status_scan = [&](std::vector<int> &flag, bool second) {
     std::vector<int> h(4 * nb);
@@ -1992,9 +2041,15 @@ int omx_create(omx_context **out, int device) {
       for(auto &e : c->lu_ev2) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
       for(auto &e : c->xev) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
       for(auto &e : c->ev) HIPCHK(hipEventCreate(&e));
-      c->d_coef.ensure(sizeof(double) * 6 * omx::kCoefStride, &c->total);
-      std::vector<double> h(6 * omx::kCoefStride, 0.0);
-      omx::fill_coef(h.data());
+      for(auto &e : c->uev) HIPCHK(hipEventCreate(&e));
+      for(hipEvent_t *e : {&c->geo_ev, &c->ujoin[0], &c->ujoin[1]})
+        HIPCHK(hipEventCreateWithFlags(e, hipEventDisableTiming));
+      c->d_coef.ensure(sizeof(double) * omx::CF_COUNT * omx::kCoefStride, &c->total);
+      static const std::vector<double> h = [] {
+        std::vector<double> v(omx::CF_COUNT * omx::kCoefStride, 0.0);
+        omx::fill_coef(v.data());
+        return v;
+      }();
       HIPCHK(hipMemcpy(c->d_coef.p, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice));
       omx::upload_factorials();
       c->scratch = scratch_address(device);
@@ -2015,8 +2070,7 @@ void omx_destroy(omx_context *c) {
   c->fg_sweep.reset();
   c->d_status2.release(&c->total);
   c->d_map2.release(&c->total);
-  DBuf *bufs[] = {&c->d_xyz, &c->d_radius, &c->d_eps, &c->d_mu, &c->d_eps_sh, &c->d_kppp, &c->d_kpar, &c->d_gam,
-                  &c->d_sph, &c->d_ov, &c->d_inc, &c->d_incloc, &c->d_Q, &c->d_w, &c->d_coef, &c->d_S64,
+  DBuf *bufs[] = {&c->d_geo, &c->d_sph, &c->d_ov, &c->d_inc, &c->d_incloc, &c->d_Q, &c->d_w, &c->d_coef, &c->d_S64,
                   &c->d_S32, &c->d_V64, &c->d_V32, &c->d_x, &c->d_xsh, &c->d_xint, &c->d_xintsh, &c->d_K,
                   &c->d_K1, &c->d_cross, &c->d_cg, &c->d_piv, &c->d_perm, &c->d_cand, &c->d_cnt, &c->d_map,
                   &c->d_wlu, &c->d_status, &c->d_basis, &c->d_basisZ, &c->d_w1, &c->d_w2, &c->d_r,
@@ -2045,7 +2099,8 @@ void omx_destroy(omx_context *c) {
     if(e) (void)hipEventDestroy(e);
   for(auto e : c->xev)
     if(e) (void)hipEventDestroy(e);
-
+  for(hipEvent_t e : {c->geo_ev, c->uev[0], c->uev[1], c->uev[2], c->ujoin[0], c->ujoin[1]})
+    if(e) (void)hipEventDestroy(e);
   for(auto e : c->pev2)
     if(e) (void)hipEventDestroy(e);
   if(c->aux2) (void)hipStreamDestroy(c->aux2);
@@ -2053,6 +2108,7 @@ void omx_destroy(omx_context *c) {
   if(c->aux) (void)hipStreamDestroy(c->aux);
   if(c->st) (void)hipStreamDestroy(c->st);
   if(c->h_pin) (void)hipHostFree(c->h_pin);
+  if(c->geo_pin) (void)hipHostFree(c->geo_pin);
   delete c;
 }
 
@@ -2244,56 +2300,55 @@ int omx_update(omx_context *c) {
       c->tuned_split = t.split;
     }
     const int P = c->P, nmax = c->nmax;
-    HIPCHK(hipEventRecord(c->ev[0], c->st));
-    HIPCHK(hipMemcpyAsync(c->d_xyz.p, c->xyz.data(), sizeof(double) * 3 * P, hipMemcpyHostToDevice, c->st));
-    HIPCHK(hipMemcpyAsync(c->d_radius.p, c->radius.data(), sizeof(double) * P, hipMemcpyHostToDevice, c->st));
-    HIPCHK(hipMemcpyAsync(c->d_eps.p, c->eps.data(), sizeof(cplx) * P, hipMemcpyHostToDevice, c->st));
-    HIPCHK(hipMemcpyAsync(c->d_mu.p, c->mu.data(), sizeof(cplx) * P, hipMemcpyHostToDevice, c->st));
-    HIPCHK(hipMemcpyAsync(c->d_eps_sh.p, c->eps_sh.data(), sizeof(cplx) * P, hipMemcpyHostToDevice, c->st));
-    HIPCHK(hipMemcpyAsync(c->d_kppp.p, c->ksippp.data(), sizeof(cplx) * P, hipMemcpyHostToDevice, c->st));
-    HIPCHK(hipMemcpyAsync(c->d_kpar.p, c->ksiparppar.data(), sizeof(cplx) * P, hipMemcpyHostToDevice, c->st));
-    HIPCHK(hipMemcpyAsync(c->d_gam.p, c->gamma.data(), sizeof(cplx) * P, hipMemcpyHostToDevice, c->st));
+    // The plane wave and the objects' origin couplings run on the second
+    // stream beside the pairs: they need the objects only, and one workgroup
+    // per object leaves the device to the pairs.  The call returns once all is
+    // enqueued; whatever reads its results follows on the context's stream.
+    hipStream_t st = c->st, st2 = c->st2;
+    HIPCHK(hipEventRecord(c->uev[0], st));
+    upload_geometry(c);
     const double omega = c->omega();
     const cplx bge = kEps0 * c->bg_eps_r, bgm = kMu0 * c->bg_mu_r;
     omx::ObjArgs oa{P, nmax, omega, bge, bgm, c->d_xyz.as<double>(), c->d_radius.as<double>(),
                     c->d_eps.as<cplx>(), c->d_mu.as<cplx>(), c->d_eps_sh.as<cplx>(), c->d_sph.as<double>(),
                     c->d_ov.as<cplx>()};
-    omx::run_objects(oa, c->st);
+    omx::run_objects(oa, st);
+    HIPCHK(hipEventRecord(c->uev[1], st));
+    HIPCHK(hipEventRecord(c->ujoin[0], st));
+    HIPCHK(hipStreamWaitEvent(st2, c->ujoin[0], 0));
     omx::IncArgs ia{nmax, c->theta, c->phi, c->eth, c->eph, c->d_inc.as<cplx>()};
-    omx::run_incident(ia, c->st);
-    HIPCHK(hipMemsetAsync(c->d_Q.p, 0, sizeof(cplx) * c->Np, c->st));
+    omx::run_incident(ia, st2);
+    HIPCHK(hipMemsetAsync(c->d_Q.p, 0, sizeof(cplx) * c->Np, st2));
     omx::OriginArgs og{P, nmax, c->waveK(), c->d_sph.as<double>(), c->d_ov.as<cplx>(), c->d_coef.as<double>(),
-                       c->d_inc.as<cplx>(), c->d_incloc.as<cplx>(), c->d_Q.as<cplx>(), c->d_w.as<double>()};
-    omx::run_origin(og, c->st);
-    HIPCHK(hipEventRecord(c->ev[1], c->st));
+                       c->d_inc.as<cplx>(), c->d_incloc.as<cplx>(), c->d_Q.as<cplx>(), c->d_w.as<double>(), c->sh};
+    omx::run_origin(og, st2);
+    HIPCHK(hipEventRecord(c->ujoin[1], st2));
     const size_t lda = (size_t)c->Np;
     if(c->kind == OMX_SOLVER_ACA_GMRES) {
       aca_build(c, false);
       if(c->sh) aca_build(c, true); else c->aca[1].release(&c->total);
     } else {
       aca_release(c);
+      omx::PairArgs pa{P, nmax, omx::OV_T, c->waveK(), c->d_sph.as<double>(), c->d_ov.as<cplx>(),
+                       c->d_coef.as<double>(), lda, c->d_S64.as<cplx>(), c->d_S32.as<float2>()};
+      if(c->sh) {  // V in the same launch
+        pa.tkind2 = omx::OV_TSH;
+        pa.k2 = omx::mk(2.0 * pa.k.x, 2.0 * pa.k.y);  // PreconditionedMatrix.cpp:592
+        pa.V64 = c->d_V64.as<cplx>();
+        pa.V32 = c->d_V32.as<float2>();
+      }
+      omx::run_pairs(pa, st);
+      if(c->d_S64.p) omx::run_pad64(c->d_S64.as<cplx>(), c->N, c->Np, lda, st);
+      if(c->d_S32.p) omx::run_pad32(c->d_S32.as<float2>(), c->N, c->Np, lda, st);
+      if(c->sh) {
+        if(c->d_V64.p) omx::run_pad64(c->d_V64.as<cplx>(), c->N, c->Np, lda, st);
+        if(c->d_V32.p) omx::run_pad32(c->d_V32.as<float2>(), c->N, c->Np, lda, st);
+      }
     }
-    omx::PairArgs pa{P, nmax, omx::OV_T, c->waveK(), c->d_sph.as<double>(), c->d_ov.as<cplx>(),
-                     c->d_coef.as<double>(), lda, c->d_S64.as<cplx>(), c->d_S32.as<float2>()};
-    if(c->kind != OMX_SOLVER_ACA_GMRES) omx::run_pairs(pa, c->st);
-    if(c->d_S64.p) omx::run_pad64(c->d_S64.as<cplx>(), c->N, c->Np, lda, c->st);
-    if(c->d_S32.p) omx::run_pad32(c->d_S32.as<float2>(), c->N, c->Np, lda, c->st);
-    if(c->sh && c->kind != OMX_SOLVER_ACA_GMRES) {
-      omx::PairArgs pv = pa;
-      pv.tkind = omx::OV_TSH;
-      cplx k = c->waveK();
-      pv.k = omx::mk(2.0 * k.x, 2.0 * k.y);  // PreconditionedMatrix.cpp:592
-      pv.S64 = c->d_V64.as<cplx>();
-      pv.S32 = c->d_V32.as<float2>();
-      omx::run_pairs(pv, c->st);
-      if(c->d_V64.p) omx::run_pad64(c->d_V64.as<cplx>(), c->N, c->Np, lda, c->st);
-      if(c->d_V32.p) omx::run_pad32(c->d_V32.as<float2>(), c->N, c->Np, lda, c->st);
-    }
+    HIPCHK(hipStreamWaitEvent(st, c->ujoin[1], 0));
     HIPCHK(hipGetLastError());
-    HIPCHK(hipEventRecord(c->ev[2], c->st));
-    HIPCHK(hipEventSynchronize(c->ev[2]));
-    c->stats.t_update_ms = elapsed(c, 0, 2);
-    c->stats.t_assemble_ms = elapsed(c, 1, 2);
+    HIPCHK(hipEventRecord(c->uev[2], st));
+    c->upd_timed = true;
     c->stats.N = c->N;
     c->stats.Np = c->Np;
     c->stats.device_bytes = c->total;
@@ -2531,6 +2586,7 @@ int omx_solve_group(omx_context *L, int n, omx_context *const *mem) {
     HIPCHK(hipMemsetAsync(L->d_status.p, 0, 16, st));
     // the members' matrices and right-hand sides, bordered by the identity
     cplx *S64 = w.S64.as<cplx>(), *V64 = sh ? w.V64.as<cplx>() : nullptr;
+    for(int z = 0; z < nb; ++z) HIPCHK(hipStreamWaitEvent(st, mem[z]->uev[2], 0));
     for(int z = 0; z < nb; ++z) {
       omx_context *m = mem[z];
       omx::pad_matrix64(S64 + z * n2, Np, m->d_S64.as<cplx>(), m->Np, st);
@@ -2756,6 +2812,11 @@ int omx_scattering_size(const omx_context *c) { return c ? c->N : 0; }
 int omx_get_stats(const omx_context *c, omx_stats *out) {
   if(!c || !out) return OMX_ERR_ARG;
   *out = c->stats;
+  if(c->upd_timed && hipEventSynchronize(c->uev[2]) == hipSuccess) {
+    float ms = 0;
+    if(hipEventElapsedTime(&ms, c->uev[0], c->uev[2]) == hipSuccess) out->t_update_ms = ms;
+    if(hipEventElapsedTime(&ms, c->uev[1], c->uev[2]) == hipSuccess) out->t_assemble_ms = ms;
+  }
   out->device_bytes = c->total;
   out->t_lu_gemm_ms = c->prof_gemm_ms;
   out->lu_gemm_flop = c->prof_flop;
@@ -2940,12 +3001,7 @@ int omx_solve_sweep(omx_context *c, int nl, const double *lambdas, const double 
     c->d_status.ensure(64, &c->total);
     const int P = c->P, N = c->N;
     // geometry and material constants on the device (as omx_update)
-    HIPCHK(hipMemcpyAsync(c->d_xyz.p, c->xyz.data(), sizeof(double) * 3 * P, hipMemcpyHostToDevice, c->st));
-    HIPCHK(hipMemcpyAsync(c->d_radius.p, c->radius.data(), sizeof(double) * P, hipMemcpyHostToDevice, c->st));
-    HIPCHK(hipMemcpyAsync(c->d_mu.p, c->mu.data(), sizeof(cplx) * P, hipMemcpyHostToDevice, c->st));
-    HIPCHK(hipMemcpyAsync(c->d_kppp.p, c->ksippp.data(), sizeof(cplx) * P, hipMemcpyHostToDevice, c->st));
-    HIPCHK(hipMemcpyAsync(c->d_kpar.p, c->ksiparppar.data(), sizeof(cplx) * P, hipMemcpyHostToDevice, c->st));
-    HIPCHK(hipMemcpyAsync(c->d_gam.p, c->gamma.data(), sizeof(cplx) * P, hipMemcpyHostToDevice, c->st));
+    upload_geometry(c);
     // batch size: at most 64 systems and half of the free device memory
     const bool f64 = c->kind == OMX_SOLVER_LU64;
     const double per = (double)c->Np * c->Np * ((c->sh ? 2 : 1) * (f64 ? 32.0 : 24.0));

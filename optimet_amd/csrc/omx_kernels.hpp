@@ -22,6 +22,22 @@ enum {
 
 constexpr int kCoefN = 2 * kMaxNmax + 2;
 constexpr int kCoefStride = (kCoefN + 1) * (kCoefN + 1);
+// Tables of square roots that do not depend on the pair, kCoefStride doubles
+// each (fill_coef): formed in the kernels they were half of the arithmetic of
+// an A / B coefficient and most of a workgroup's setup.
+enum {
+  CF_AP = 0, CF_AM, CF_BP, CF_BM,  // the recurrence's a+, a-, b+, b- (n, m)
+  CF_IAP, CF_IBP,                  // 1 / a+, 1 / b+
+  CF_A1, CF_A2,                    // sqrt((n-m)(n+m+1)), sqrt((n+m)(n-m+1))
+  CF_G0, CF_G1, CF_G2,             // sqrt((n-m)(n+m)), sqrt((n-m)(n-m-1)), sqrt((n+m)(n+m-1))
+  CF_LEGA, CF_LEGB,                // the Legendre recurrence of degree n, order m
+  CF_DEG,                          // by degree, at CF_NU, CF_MU, CF_LEGP + n
+  CF_COUNT
+};
+constexpr int CF_NU = 0, CF_MU = 64, CF_LEGP = 128;
+// Spherical coordinates of a centre as the assembly keeps them: r, sin and cos
+// of the polar angle, sin and cos of the azimuth.
+constexpr int kSphDoubles = 5;
 
 struct ObjArgs {
   int P, nmax;
@@ -29,7 +45,7 @@ struct ObjArgs {
   cplx bg_eps, bg_mu;                // absolute
   const double *xyz, *radius;
   const cplx *eps, *mu, *eps_sh;     // absolute
-  double *sph;                       // out: 3P spherical coordinates
+  double *sph;                       // out: kSphDoubles per centre
   cplx *ov;                          // out: per-object vectors
   // batches (blockIdx.z = system z): omega, eps, eps_sh and ov of system z at
   // omz[z], eps + z P, eps_sh + z P, ov + z zov (omz null: one system)
@@ -56,11 +72,18 @@ struct PairArgs {
   // batches (blockIdx.z = system z): wavenumber kz[z], ov + z zov, matrices + z zS
   const cplx *kz = nullptr;
   size_t zov = 0, zS = 0;
-  // pair list (plist non-null): nlist blocks, block b = pair plist[b] (i P + j)
-  // written to S64 / S32 + b zblk with leading dimension lda
+  // pair list (plist non-null): nlist unordered pairs, pair b = plist[b]
+  // (i P + j, i < j): S_ij written to S64 / S32 + 2 b zblk and S_ji to
+  // + (2 b + 1) zblk, with leading dimension lda
   const int *plist = nullptr;
   int nlist = 0;
   size_t zblk = 0;
+  // a second matrix in the same launch (either pointer non-null): V beside S
+  int tkind2 = 0;
+  cplx k2 = {0.0, 0.0};
+  const cplx *kz2 = nullptr;
+  cplx *V64 = nullptr;
+  float2 *V32 = nullptr;
 };
 
 struct OriginArgs {
@@ -72,7 +95,8 @@ struct OriginArgs {
   const cplx *inc;
   cplx *incloc;                      // out: N
   cplx *Q;                           // out: N
-  double *w;                         // out: [2][P][nf]
+  double *w;                         // out: [2][P][nf]; the second half (at 2k) with sh only
+  int sh;
   // batches (blockIdx.z = system z): wavenumber kz[z], ov + z zov,
   // incloc/Q + z zvec, w + z zw
   const cplx *kz = nullptr;
