@@ -936,35 +936,50 @@ void run_pad32(float2 *A, int N, int Np, size_t lda, hipStream_t st, int nb, siz
   hipLaunchKernelGGL(pad_kernel<float2>, dim3((unsigned)((n + 255) / 256), 1, nb), dim3(256), 0, st, A, N, Np, lda, zs);
 }
 
-// Coefficient tables (CF_*), at index n*n + n + m of each for n <= kCoefN.
-void fill_coef(double *h) {
-  auto at = [&](int kind, int i) -> double & { return h[kind * kCoefStride + i]; };
-  for(int n = 0; n <= kCoefN; ++n) {
-    for(int m = -n; m <= n; ++m) {
-      int i = n * n + n + m;
-      at(CF_AP, i) = a_plus(n, m);
-      at(CF_AM, i) = a_minus(n, m);
-      at(CF_BP, i) = b_plus(n, m);
-      at(CF_BM, i) = b_minus(n, m);
-      at(CF_IAP, i) = a_plus(n, m) != 0.0 ? 1.0 / a_plus(n, m) : 0.0;
-      at(CF_IBP, i) = b_plus(n, m) != 0.0 ? 1.0 / b_plus(n, m) : 0.0;
-      at(CF_A1, i) = sqrt((double)((n - m) * (n + m + 1)));
-      at(CF_A2, i) = sqrt((double)((n + m) * (n - m + 1)));
-      at(CF_G0, i) = sqrt((double)((n - m) * (n + m)));
-      at(CF_G1, i) = n > m ? sqrt((double)((n - m) * (n - m - 1))) : 0.0;
-      at(CF_G2, i) = n > -m ? sqrt((double)((n + m) * (n + m - 1))) : 0.0;
-      const int l = n, am = m;
-      if(am >= 0 && l == am + 1) at(CF_LEGA, i) = sqrt(2.0 * am + 3.0);
-      if(am >= 0 && l >= am + 2) {
-        at(CF_LEGA, i) = sqrt((4.0 * l * l - 1.0) / ((double)l * l - (double)am * am));
-        at(CF_LEGB, i) = sqrt(((l - 1.0) * (l - 1.0) - (double)am * am) / (4.0 * (l - 1.0) * (l - 1.0) - 1.0));
-      }
-    }
-    if(n == 0) continue;
-    at(CF_DEG, CF_NU + n) = 1.0 / sqrt((double)(n * (n + 1)));
-    at(CF_DEG, CF_MU + n) = sqrt((double)(2 * n + 1) / (double)((2 * n - 1) * n * (n + 1)));
-    at(CF_DEG, CF_LEGP + n) = -sqrt((2.0 * n + 1.0) / (2.0 * n));
+// Coefficient tables (CF_*), at index n*n + n + m of each for n <= kCoefN: one
+// thread per entry.
+__global__ void fill_coef_kernel(double *h) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if(i >= kCoefStride) return;
+  auto at = [&](int kind) -> double & { return h[kind * kCoefStride + i]; };
+  int n = (int)sqrt((double)i);
+  const int m = i - n * n - n;
+  const double ap = a_plus(n, m), bp = b_plus(n, m);
+  at(CF_AP) = ap;
+  at(CF_AM) = a_minus(n, m);
+  at(CF_BP) = bp;
+  at(CF_BM) = b_minus(n, m);
+  at(CF_IAP) = ap != 0.0 ? 1.0 / ap : 0.0;
+  at(CF_IBP) = bp != 0.0 ? 1.0 / bp : 0.0;
+  at(CF_A1) = sqrt((double)((n - m) * (n + m + 1)));
+  at(CF_A2) = sqrt((double)((n + m) * (n - m + 1)));
+  at(CF_G0) = sqrt((double)((n - m) * (n + m)));
+  at(CF_G1) = n > m ? sqrt((double)((n - m) * (n - m - 1))) : 0.0;
+  at(CF_G2) = n > -m ? sqrt((double)((n + m) * (n + m - 1))) : 0.0;
+  double la = 0.0, lb = 0.0;
+  const int l = n, am = m;
+  if(am >= 0 && l == am + 1) la = sqrt(2.0 * am + 3.0);
+  if(am >= 0 && l >= am + 2) {
+    la = sqrt((4.0 * l * l - 1.0) / ((double)l * l - (double)am * am));
+    lb = sqrt(((l - 1.0) * (l - 1.0) - (double)am * am) / (4.0 * (l - 1.0) * (l - 1.0) - 1.0));
   }
+  at(CF_LEGA) = la;
+  at(CF_LEGB) = lb;
+  // by degree: entry i of the table is CF_NU, CF_MU or CF_LEGP + d
+  const int d = i < CF_MU ? i - CF_NU : i < CF_LEGP ? i - CF_MU : i - CF_LEGP;
+  double v = 0.0;
+  if(d >= 1 && d <= kCoefN) {
+    if(i < CF_MU)
+      v = 1.0 / sqrt((double)(d * (d + 1)));
+    else if(i < CF_LEGP)
+      v = sqrt((double)(2 * d + 1) / (double)((2 * d - 1) * d * (d + 1)));
+    else
+      v = -sqrt((2.0 * d + 1.0) / (2.0 * d));
+  }
+  at(CF_DEG) = v;
+}
+void fill_coef(double *d, hipStream_t st) {
+  hipLaunchKernelGGL(fill_coef_kernel, dim3((kCoefStride + 255) / 256), dim3(256), 0, st, d);
 }
 
 }  // namespace omx

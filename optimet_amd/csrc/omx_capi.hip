@@ -152,7 +152,7 @@ struct omx_context {
       d_coef, d_S64, d_S32, d_V64, d_V32, d_x, d_xsh, d_xint, d_xintsh, d_K, d_K1, d_cross, d_cg, d_abscoef, d_abssh,
       d_absbes,
       d_fpts, d_fout, d_fown, d_fpart;
-  DBuf d_piv, d_perm, d_cand, d_cnt, d_map, d_status, d_wlu;
+  DBuf d_perm, d_cand, d_map, d_status, d_wlu;
   hipStream_t aux = nullptr;
   hipEvent_t lu_ev[4] = {nullptr, nullptr, nullptr, nullptr};
   // the second-harmonic system's own streams, events, status and maps, so
@@ -180,7 +180,7 @@ struct omx_context {
   omx::LuProf prof{};
   double prof_gemm_ms = 0, prof_panel_ms = 0, prof_flop = 0, prof_total_ms = 0;
   int prof_launches = 0;
-  DBuf d_piv2, d_perm2;
+  DBuf d_perm2;
   DBuf d_dinv, d_dinv2, d_F64, d_F64sh;  // diagonal-block inverses; FP64 factors (the FP64 matrices stay intact)
   // wavelength sweeps: per-system buffers of one batch ([system][...])
   struct Sweep {
@@ -281,16 +281,14 @@ cplx C(const double *p, int i) { return omx::mk(p[2 * i], p[2 * i + 1]); }
 bool use32(int kind) { return kind == OMX_SOLVER_LU32_IR || kind == OMX_SOLVER_GMRES32_IR; }
 bool is_lu(int kind) { return kind == OMX_SOLVER_LU64 || kind == OMX_SOLVER_LU32_IR; }
 
-void alloc_lu(omx_context *c, omx::LuWork &w, DBuf &piv, DBuf &perm, DBuf &dinv, bool second) {
+void alloc_lu(omx_context *c, omx::LuWork &w, DBuf &perm, DBuf &dinv, bool second) {
   const int Np = c->Np;
   const int gmax = (Np + omx::kPanelRows - 1) / omx::kPanelRows + 1;
-  piv.ensure(sizeof(int) * Np, &c->total);
   dinv.ensure(sizeof(cplx) * omx::dinv_elems(Np), &c->total);
   perm.ensure(sizeof(int) * Np, &c->total);
   // tournament scratch: one half per system, as S and V may be factored
   // at the same time
   c->d_cand.ensure(sizeof(int) * 4 * gmax * omx::kNB, &c->total);
-  c->d_cnt.ensure(sizeof(int) * 4 * gmax, &c->total);
   c->d_wlu.ensure(sizeof(cplx) * 6 * omx::kNB * omx::kNB, &c->total);
   if(!second) {
     c->d_map.ensure(sizeof(int) * (3 * ((size_t)Np + 2 * omx::kNB)), &c->total);
@@ -303,13 +301,10 @@ void alloc_lu(omx_context *c, omx::LuWork &w, DBuf &piv, DBuf &perm, DBuf &dinv,
   DBuf &status = second ? c->d_status2 : c->d_status;
   HIPCHK(hipMemsetAsync(status.p, 0, 64, c->st));
   w = omx::LuWork{};
-  w.piv = piv.as<int>();
   w.perm = perm.as<int>();
   const int half = second ? 1 : 0;
   w.cand[0] = c->d_cand.as<int>() + (2 * half) * gmax * omx::kNB;
   w.cand[1] = c->d_cand.as<int>() + (2 * half + 1) * gmax * omx::kNB;
-  w.cnt[0] = c->d_cnt.as<int>() + (2 * half) * gmax;
-  w.cnt[1] = c->d_cnt.as<int>() + (2 * half + 1) * gmax;
   w.mdst = map.as<int>();
   w.msrc = map.as<int>() + (Np + 2 * omx::kNB);
   w.mcnt = map.as<int>() + 2 * (Np + 2 * omx::kNB);
@@ -425,8 +420,8 @@ void alloc_matrices(omx_context *c) {
   } else {
     c->ws_in.release(T);
   }
-  alloc_lu(c, c->lu, c->d_piv, c->d_perm, c->d_dinv, false);
-  if(c->sh) alloc_lu(c, c->lu_sh, c->d_piv2, c->d_perm2, c->d_dinv2, true);
+  alloc_lu(c, c->lu, c->d_perm, c->d_dinv, false);
+  if(c->sh) alloc_lu(c, c->lu_sh, c->d_perm2, c->d_dinv2, true);
 }
 
 float elapsed(omx_context *c, int a, int b) {
@@ -1458,7 +1453,6 @@ omx::LuWork sweep_lu(omx_context *c, int nb, bool second) {
   const int Np = c->Np;
   omx::LuWork lw{};
   lw.perm = (second ? w.perm2 : w.perm).as<int>();
-  lw.piv = lw.perm;  // unused by block pivoting
   lw.dinv = (second ? w.dinv2 : w.dinv).p;
   const int ms = Np + 2 * omx::kNB;
   int *map = (second ? w.map2 : w.map).as<int>();
@@ -1973,11 +1967,9 @@ struct NoAllocLayout {
   static constexpr int Np = kNoAllocMaxN;
   static constexpr int gmax = Np / omx::kPanelRows + 1;
   static constexpr size_t status = 0;  // 16 ints
-  static constexpr size_t piv = status + align256(16 * sizeof(int));  // Np ints
-  static constexpr size_t perm = piv + align256(Np * sizeof(int));  // Np ints
+  static constexpr size_t perm = status + align256(16 * sizeof(int));  // Np ints
   static constexpr size_t cand = perm + align256(Np * sizeof(int));  // 2 x gmax x 64 ints
-  static constexpr size_t cnt = cand + align256(2 * gmax * omx::kNB * sizeof(int));  // 2 x gmax ints
-  static constexpr size_t map = cnt + align256(2 * gmax * sizeof(int));  // 3 x (Np + 128) ints
+  static constexpr size_t map = cand + align256(2 * gmax * omx::kNB * sizeof(int));  // 3 x (Np + 128) ints
   static constexpr size_t wlu = map + align256(3 * (Np + 2 * omx::kNB) * sizeof(int));  // 3 x 64 x 64 complex
   static constexpr size_t dinv = wlu + align256(3 * omx::kNB * omx::kNB * sizeof(cplx));  // 2 x 64 x Np complex
   static constexpr size_t rhs = dinv + align256(2 * omx::kNB * (size_t)Np * sizeof(cplx));  // Np complex
@@ -2045,12 +2037,7 @@ int omx_create(omx_context **out, int device) {
       for(hipEvent_t *e : {&c->geo_ev, &c->ujoin[0], &c->ujoin[1]})
         HIPCHK(hipEventCreateWithFlags(e, hipEventDisableTiming));
       c->d_coef.ensure(sizeof(double) * omx::CF_COUNT * omx::kCoefStride, &c->total);
-      static const std::vector<double> h = [] {
-        std::vector<double> v(omx::CF_COUNT * omx::kCoefStride, 0.0);
-        omx::fill_coef(v.data());
-        return v;
-      }();
-      HIPCHK(hipMemcpy(c->d_coef.p, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice));
+      omx::fill_coef(c->d_coef.as<double>(), c->st);
       omx::upload_factorials();
       c->scratch = scratch_address(device);
     } catch(...) {
@@ -2072,9 +2059,9 @@ void omx_destroy(omx_context *c) {
   c->d_map2.release(&c->total);
   DBuf *bufs[] = {&c->d_geo, &c->d_sph, &c->d_ov, &c->d_inc, &c->d_incloc, &c->d_Q, &c->d_w, &c->d_coef, &c->d_S64,
                   &c->d_S32, &c->d_V64, &c->d_V32, &c->d_x, &c->d_xsh, &c->d_xint, &c->d_xintsh, &c->d_K,
-                  &c->d_K1, &c->d_cross, &c->d_cg, &c->d_piv, &c->d_perm, &c->d_cand, &c->d_cnt, &c->d_map,
+                  &c->d_K1, &c->d_cross, &c->d_cg, &c->d_perm, &c->d_cand, &c->d_map,
                   &c->d_wlu, &c->d_status, &c->d_basis, &c->d_basisZ, &c->d_w1, &c->d_w2, &c->d_r,
-                  &c->d_part, &c->d_h, &c->d_nrm, &c->d_gpart, &c->d_piv2, &c->d_perm2,
+                  &c->d_part, &c->d_h, &c->d_nrm, &c->d_gpart, &c->d_perm2,
                   &c->d_dinv, &c->d_dinv2, &c->d_F64, &c->d_F64sh, &c->d_abscoef, &c->d_abssh, &c->d_absbes,
                   &c->d_fpts, &c->d_fout, &c->d_fown, &c->d_fpart};
   for(DBuf *b : bufs) b->release(&c->total);
@@ -3158,12 +3145,9 @@ int omx_dense_solve_noalloc(omx_context *c, int N, double *A, size_t lda, const 
     auto ip = [&](size_t off) { return reinterpret_cast<int *>(base + off); };
     omx::LuWork w{};
     w.status = ip(L::status);
-    w.piv = ip(L::piv);
     w.perm = ip(L::perm);
     w.cand[0] = ip(L::cand);
     w.cand[1] = ip(L::cand) + L::gmax * omx::kNB;
-    w.cnt[0] = ip(L::cnt);
-    w.cnt[1] = ip(L::cnt) + L::gmax;
     w.mdst = ip(L::map);
     w.msrc = ip(L::map) + (L::Np + 2 * omx::kNB);
     w.mcnt = ip(L::map) + 2 * (L::Np + 2 * omx::kNB);
@@ -3179,7 +3163,7 @@ int omx_dense_solve_noalloc(omx_context *c, int N, double *A, size_t lda, const 
     w.nb = 1;
     cplx *rb = reinterpret_cast<cplx *>(base + L::rhs), *xs = reinterpret_cast<cplx *>(base + L::x);
     // the array keeps the last call's contents: the status words start at zero
-    const int nz = (int)((L::piv - L::status) / sizeof(int));
+    const int nz = (int)((L::perm - L::status) / sizeof(int));
     hipLaunchKernelGGL(zero_ints_kernel, dim3((nz + 255) / 256), dim3(256), 0, st, ip(L::status), nz);
     hipLaunchKernelGGL(stage_rhs_kernel, dim3((Np + 255) / 256), dim3(256), 0, st, reinterpret_cast<const cplx *>(b),
                        rb, N, Np);

@@ -139,7 +139,7 @@ void run_cross(const CrossArgs &a, hipStream_t st);
 // identity padding of nb matrices zs elements apart
 void run_pad64(cplx *A, int N, int Np, size_t lda, hipStream_t st, int nb = 1, size_t zs = 0);
 void run_pad32(float2 *A, int N, int Np, size_t lda, hipStream_t st, int nb = 1, size_t zs = 0);
-void fill_coef(double *host);
+void fill_coef(double *dev, hipStream_t st);  // CF_COUNT x kCoefStride
 
 // ---------------------------------------------------------------- ACA
 struct AcaArgs {
@@ -174,7 +174,7 @@ void aca_matvec(const AcaOp &op, const cplx *x, cplx *y, hipStream_t st);
 
 // ---------------------------------------------------------------- LU
 constexpr int kNB = 64;        // LU block size (panel width, padding granule)
-constexpr int kPanelRows = 128; // rows of the panel held by one workgroup
+constexpr int kPanelRows = 192; // fewest rows of the panel held by one workgroup (tournament)
 
 // Distances between the systems of a batch (element counts of each buffer);
 // all zero for a single system.  A batch runs with blockIdx.z = system.
@@ -190,10 +190,8 @@ struct BatchStrides {
 
 struct LuWork {
   // device scratch of one factorization
-  int *piv;             // Np: LAPACK-style swap sequence
   int *perm;            // Np: final row permutation (row i of P A is row perm[i] of A)
   int *cand[2];         // tournament candidates, ping-pong, [Gmax][NB]
-  int *cnt[2];          // candidates per set, [Gmax]
   int *mdst, *msrc;     // gather maps: tournament 2 NB entries at the start; block
   int *mcnt;            // pivoting NB entries per panel (panel k at k NB, count mcnt[k])
   int *status;          // [0]: singular pivot column+1, [1]: wait timeout

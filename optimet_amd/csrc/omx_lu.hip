@@ -7,11 +7,10 @@
 //                  diagonal block, in one workgroup, which also inverts L11
 //                  and U11; the solver recovers full accuracy by iterative
 //                  refinement and refactors with the tournament if that fails
-//   partial        tournament pivoting (TSLU): register-resident partial-
-//                  pivoting LUs of 128-row chunks nominate candidate rows, a
-//                  binary tree of merges picks the NB pivot rows (tslu_leaf,
-//                  tslu_merge), tslu_finish turns them into a gather map and
-//                  panel_inv writes the block's factors and inverses
+//   partial        tournament pivoting (TSLU, tslu_panel): register-resident
+//                  partial-pivoting LUs of row chunks nominate candidate
+//                  rows, a tree of merges picks the NB pivot rows, and its root
+//                  writes the gather map, the block's factors and inverses
 // Shared by both:
 //   laswp_map      the panel's row interchanges on the other columns, as one
 //                  parallel gather/scatter
@@ -164,289 +163,6 @@ __global__ void iota_kernel(int *p, int n, int sp) {
 }
 
 // ------------------------------------------------------------------ panel
-// Tournament pivoting (TSLU, Grigori, Demmel and Xiang 2011): the panel's
-// pivot rows are chosen by a reduction tree of local partial-pivoting LUs
-// instead of one device-wide search per column.
-
-template <typename T, int NB>
-struct SelShared {
-  CxOf<T> rowb[2][2][NB];  // [parity][0: old row c, 1: pivot row][column]
-  CxOf<T> lcol[128];
-  int rid[128];
-  int sel[NB];
-  double wv[2];
-  int wi[2];
-};
-
-// Partial-pivoting LU of an R x 64 block (R <= 128) held in registers: thread
-// t owns row r = t & 127, columns h*32 .. h*32+31 with h = t >> 7.  Rows carry
-// global ids in s.rid; s.sel receives the ids of the pivot rows in order.
-template <typename T>
-__device__ __forceinline__ void reg_select(CxOf<T> (&v)[32], SelShared<T, 64> &s, int R) {
-  using C = CxOf<T>;
-  const int t = threadIdx.x, r = t & 127, h = t >> 7, lane = t & 63, w = t >> 6;
-  const C zero{};
-  const int nc = min(R, 64);
-  // two halves of 32 columns; inside a half the column index is a
-  // compile-time constant, so v[] stays in registers
-#pragma unroll 1
-  for(int hc = 0; hc < 2; ++hc) {
-#pragma unroll
-    for(int jc = 0; jc < 32; ++jc) {
-      const int c = hc * 32 + jc, par = jc & 1;
-      if(c < nc) {
-        if(h == hc) {
-          const bool ok = r >= c && r < R;
-          double val = ok ? mag2(v[jc]) : -1.0;
-          int idx = ok ? r : INT_MAX;
-#pragma unroll
-          for(int off = 32; off > 0; off >>= 1) {
-            double ov = __shfl_xor(val, off, 64);
-            int oi = __shfl_xor(idx, off, 64);
-            if(ov > val || (ov == val && oi < idx)) val = ov, idx = oi;
-          }
-          if(lane == 0) {
-            s.wv[w - 2 * hc] = val;
-            s.wi[w - 2 * hc] = idx;
-          }
-        }
-        __syncthreads();
-        const int b = (s.wv[1] > s.wv[0] || (s.wv[1] == s.wv[0] && s.wi[1] < s.wi[0])) ? s.wi[1] : s.wi[0];
-        if(r == b) {
-#pragma unroll
-          for(int j = 0; j < 32; ++j) s.rowb[par][1][h * 32 + j] = v[j];
-        }
-        if(r == c) {
-#pragma unroll
-          for(int j = 0; j < 32; ++j) s.rowb[par][0][h * 32 + j] = v[j];
-        }
-        if(t == 0) {
-          const int id = s.rid[b];
-          s.rid[b] = s.rid[c];
-          s.rid[c] = id;
-          s.sel[c] = id;
-        }
-        __syncthreads();
-        if(b != c) {
-          if(r == c) {
-#pragma unroll
-            for(int j = 0; j < 32; ++j) v[j] = s.rowb[par][1][h * 32 + j];
-          } else if(r == b) {
-#pragma unroll
-            for(int j = 0; j < 32; ++j) v[j] = s.rowb[par][0][h * 32 + j];
-          }
-        }
-        const C pv = s.rowb[par][1][c];
-        const C ip = mag2(pv) > 0.0 ? crecip(pv) : zero;
-        C l = zero;
-        if(h == hc && r > c && r < R) {
-          l = cm(v[jc], ip);
-          v[jc] = l;
-          s.lcol[r] = l;
-        }
-        __syncthreads();
-        if(r > c && r < R) {
-          if(h != hc) l = s.lcol[r];
-          if(h == hc) {
-#pragma unroll
-            for(int j = jc + 1; j < 32; ++j) v[j] = csub(v[j], cm(l, s.rowb[par][1][h * 32 + j]));
-          } else if(h > hc) {
-#pragma unroll
-            for(int j = 0; j < 32; ++j) v[j] = csub(v[j], cm(l, s.rowb[par][1][h * 32 + j]));
-          }
-        }
-      }
-    }
-  }
-}
-
-// Root output: the LU factors of the selected rows (top 64 rows after the
-// local pivoting), column-major 64 x 64.
-template <typename T>
-__device__ __forceinline__ void emit_factors(const CxOf<T> (&v)[32], T *wlu) {
-  const int t = threadIdx.x, r = t & 127, h = t >> 7;
-  if(r < 64) {
-#pragma unroll
-    for(int j = 0; j < 32; ++j) {
-      T o;
-      o.x = v[j].x;
-      o.y = v[j].y;
-      wlu[(h * 32 + j) * 64 + r] = o;
-    }
-  }
-}
-
-// Leaves: workgroup g factors panel rows [j0 + 128 g, ...) and nominates its
-// pivot rows; with a single leaf it is also the root.
-template <typename T>
-__global__ __launch_bounds__(256) void tslu_leaf(const T *A, size_t lda, int Np, int j0, int *cand, int *cnt,
-                                                 T *wlu) {
-  __shared__ SelShared<T, 64> s;
-  const int g = blockIdx.x, t = threadIdx.x, r = t & 127, h = t >> 7;
-  const int r0 = j0 + g * 128, nr = min(128, Np - r0);
-  CxOf<T> v[32];
-#pragma unroll
-  for(int j = 0; j < 32; ++j) {
-    T a = r < nr ? A[(size_t)(j0 + h * 32 + j) * lda + r0 + r] : T{};
-    v[j] = CxOf<T>{a.x, a.y};
-  }
-  if(h == 0) s.rid[r] = r0 + r;
-  __syncthreads();
-  reg_select<T>(v, s, nr);
-  __syncthreads();
-  const int k = min(nr, 64);
-  if(t < k) cand[g * 64 + t] = s.sel[t];
-  if(t == 0) cnt[g] = k;
-  if(gridDim.x == 1) emit_factors<T>(v, wlu);
-}
-
-// One tree level: workgroup g plays candidate sets 2g and 2g+1.
-template <typename T>
-__global__ __launch_bounds__(256) void tslu_merge(const T *A, size_t lda, int j0, int gin, const int *cin,
-                                                  const int *nin, int *cout, int *nout, T *wlu) {
-  __shared__ SelShared<T, 64> s;
-  const int g = blockIdx.x, t = threadIdx.x, r = t & 127, h = t >> 7;
-  const int a = 2 * g, b = 2 * g + 1;
-  const int na = nin[a], nb = b < gin ? nin[b] : 0;
-  const int R = na + nb;
-  if(h == 0 && r < R) s.rid[r] = r < na ? cin[a * 64 + r] : cin[b * 64 + (r - na)];
-  __syncthreads();
-  CxOf<T> v[32];
-  const int id = r < R ? s.rid[r] : 0;
-#pragma unroll
-  for(int j = 0; j < 32; ++j) {
-    T a = r < R ? A[(size_t)(j0 + h * 32 + j) * lda + id] : T{};
-    v[j] = CxOf<T>{a.x, a.y};
-  }
-  reg_select<T>(v, s, R);
-  __syncthreads();
-  const int k = min(R, 64);
-  if(t < k) cout[g * 64 + t] = s.sel[t];
-  if(t == 0) nout[g] = k;
-  if(gridDim.x == 1) emit_factors<T>(v, wlu);
-}
-
-// One wave: turns the winners sel[0..nsel) into the LAPACK swap sequence
-// piv[j0..j0+nsel) and into a gather map (position dst[i] receives the row
-// that was at src[i]); also applies the map to the running permutation.
-__global__ __launch_bounds__(64) void tslu_finish(const int *sel, const int *nsel_p, int j0, int *piv, int *mdst,
-                                                 int *msrc, int *mcnt, int *perm) {
-  const int l = threadIdx.x;  // 64 lanes; NB == 64
-  __shared__ int top[64];
-  const int nsel = *nsel_p;
-  top[l] = j0 + l;
-  int opos = -1, ocont = -1;  // lane s: outside slot s
-  int nout = 0;
-  __syncthreads();
-  for(int jj = 0; jj < nsel; ++jj) {
-    const int X = sel[jj];
-    // current position of row X
-    unsigned long long mt = __ballot(top[l] == X);
-    unsigned long long mo = __ballot(l < nout && ocont == X);
-    int pos;
-    if(mt) pos = j0 + __ffsll((long long)mt) - 1;
-    else if(mo) pos = __shfl(opos, __ffsll((long long)mo) - 1, 64);
-    else pos = X;
-    const int cur = top[jj];
-    if(l == 0) piv[j0 + jj] = pos;
-    if(pos != j0 + jj) {
-      if(pos >= j0 && pos < j0 + 64) {
-        if(l == 0) {
-          top[pos - j0] = cur;
-          top[jj] = X;
-        }
-      } else {
-        unsigned long long mp = __ballot(l < nout && opos == pos);
-        int slot = mp ? __ffsll((long long)mp) - 1 : nout;
-        if(l == slot) {
-          opos = pos;
-          ocont = cur;
-        }
-        if(!mp) ++nout;
-        if(l == 0) top[jj] = X;
-      }
-    }
-    __syncthreads();
-  }
-  // gather map: top positions, then outside slots; identity entries dropped
-  const int t0 = top[l];
-  const bool mv0 = t0 != j0 + l;
-  const bool mv1 = l < nout;
-  int v0 = mv0 ? perm[t0] : 0, v1 = mv1 ? perm[ocont] : 0;
-  unsigned long long b0 = __ballot(mv0), b1 = __ballot(mv1);
-  const int n0 = __popcll(b0);
-  const unsigned long long below = (l == 0) ? 0ull : (~0ull >> (64 - l));
-  __syncthreads();
-  if(mv0) {
-    int i = __popcll(b0 & below);
-    mdst[i] = j0 + l;
-    msrc[i] = t0;
-    perm[j0 + l] = v0;
-  }
-  if(mv1) {
-    int i = n0 + __popcll(b1 & below);
-    mdst[i] = opos;
-    msrc[i] = ocont;
-    perm[opos] = v1;
-  }
-  if(l == 0) *mcnt = n0 + __popcll(b1);
-}
-
-// Writes the selected block's factors into A and inverts L11 (unit lower)
-// and U11 (thread j builds column j of each inverse, one after the other).  wlu holds [factors | Linv | Uinv], each 64 x 64 column-major.
-template <typename T>
-__global__ __launch_bounds__(256) void panel_inv(T *A, size_t lda, int j0, const T *wlu, T *dinv, int *status) {
-  __shared__ T F[64 * 65];
-  __shared__ T X[64 * 64];   // row-major: X[i * 64 + j]; L11^{-1}, then U11^{-1}
-  const int t = threadIdx.x;
-  for(int idx = t; idx < 64 * 64; idx += 256) {
-    int c = idx / 64, r = idx % 64;
-    T v = wlu[idx];
-    F[c * 65 + r] = v;
-    A[(size_t)(j0 + c) * lda + j0 + r] = v;
-  }
-  __syncthreads();
-  const T zero{};
-  if(t < 64) {  // column j of L11^{-1} (unit lower)
-    const int j = t;
-    for(int i = 0; i < 64; ++i) {
-      T x = (i == j) ? T{1, 0} : zero;
-      if(i > j)
-        for(int k = j; k < i; ++k) x = csub(x, cm(F[k * 65 + i], X[k * 64 + j]));
-      X[i * 64 + j] = (i < j) ? zero : x;
-    }
-  }
-  __syncthreads();
-  for(int idx = t; idx < 64 * 64; idx += 256) {
-    int c = idx / 64, r = idx % 64;
-    dinv[idx] = X[r * 64 + c];
-  }
-  __syncthreads();
-  if(t < 64) {  // column j of U11^{-1}
-    const int j = t;
-    for(int i = 63; i >= 0; --i) {
-      T y = zero;
-      if(i <= j) {
-        y = (i == j) ? T{1, 0} : zero;
-        for(int k = i + 1; k <= j; ++k) y = csub(y, cm(F[k * 65 + i], X[k * 64 + j]));
-        const T d = F[i * 65 + i];
-        if(!(mag2(d) > 0.0)) {
-          atomicCAS(&status[0], 0, j0 + i + 1);
-          y = zero;
-        } else {
-          y = cm(y, crecip(d));
-        }
-      }
-      X[i * 64 + j] = y;
-    }
-  }
-  __syncthreads();
-  for(int idx = t; idx < 64 * 64; idx += 256) {
-    int c = idx / 64, r = idx % 64;
-    dinv[4096 + idx] = X[r * 64 + c];
-  }
-}
-
 // Maximum of an unsigned key over the 64 lanes of a wave, returned to every
 // lane: row shifts build each 16-lane row's maximum in its lane 15, two row
 // broadcasts combine the rows into lane 63.
@@ -459,6 +175,265 @@ __device__ inline unsigned wave_max_u32(unsigned x) {
   x = max(x, (unsigned)__builtin_amdgcn_update_dpp((int)x, (int)x, 0x143, 0xC, 0xF, false));  // row_bcast:31
   return (unsigned)__builtin_amdgcn_readlane((int)x, 63);
 }
+
+// [L11^{-1} | U11^{-1}] of the factored block F (column-major, 65 apart) into
+// dinv, by a workgroup of 8 waves: lane = row i; waves 0-3 hold columns 16 w ..
+// 16 w + 15 of L11^{-1}, waves 4-7 those of U11^{-1}; row k is broadcast within
+// the wave by lane reads, so the waves run without barriers.
+template <typename T> __device__ __forceinline__ void invert_block(const CxOf<T> *F, T *dinv) {
+  using C = CxOf<T>;
+  const int t = threadIdx.x, lane = t & 63, q = t >> 6;
+  const C zero{}, one{1, 0};
+  const int i = lane, w = q & 3;
+  C x[16];
+#pragma unroll
+  for(int m = 0; m < 16; ++m) x[m] = csel(16 * w + m == i, one, zero);
+  if(q < 4) {
+    // L11^{-1} (unit lower): for k: row i -= L[i][k] row k, i > k.  Column
+    // 16 w + m starts as e_{16 w + m} and its rows above 16 w + m stay zero,
+    // so the steps k < 16 w leave this wave's columns as they are: skipped
+    C fn = F[(16 * w) * 65 + i];  // column k of L, read one step ahead
+#pragma unroll 1
+    for(int k = 16 * w; k < 63; ++k) {
+      const int ks = __builtin_amdgcn_readfirstlane(k);
+      const C lik = csel(i > ks, fn, zero);
+      fn = F[(ks + 1) * 65 + i];
+#pragma unroll
+      for(int m = 0; m < 16; ++m) x[m] = cfms(x[m], lik, rdl(x[m], ks));
+    }
+  } else {
+    // U11^{-1} = (D^{-1} U11)^{-1} D^{-1} with D = diag(U11): a unit-upper
+    // sweep (row i -= (U[i][k] / U[i][i]) row k, i < k, k = 63..0), then
+    // column j scaled by 1 / U[j][j].  Rows below 16 w + 15 of this wave's
+    // columns stay zero, so the sweep starts at k = 16 w + 15
+    const C di = F[i * 65 + i];
+    const C rinv = csel(mag2(di) > 0.0, crecip(di), zero);
+    C fn = F[(16 * w + 15) * 65 + i];  // column k of U, read one step ahead
+#pragma unroll 1
+    for(int k = 16 * w + 15; k > 0; --k) {
+      const int ks = __builtin_amdgcn_readfirstlane(k);
+      const C uik = csel(i < ks, cm(fn, rinv), zero);
+      fn = F[(ks - 1) * 65 + i];
+#pragma unroll
+      for(int m = 0; m < 16; ++m) x[m] = cfms(x[m], uik, rdl(x[m], ks));
+    }
+#pragma unroll
+    for(int m = 0; m < 16; ++m) x[m] = cm(x[m], rdl(rinv, 16 * w + m));
+  }
+  T *out = dinv + (q < 4 ? 0 : 4096);
+#pragma unroll
+  for(int m = 0; m < 16; ++m) {
+    T o;
+    o.x = x[m].x;
+    o.y = x[m].y;
+    out[(16 * w + m) * 64 + i] = o;
+  }
+}
+
+// The unsigned word that orders non-negative values: all of a float, the
+// upper half of a double (11 bits of exponent, 20 of mantissa).
+__device__ inline unsigned order_key(float m) { return __float_as_uint(m); }
+__device__ inline unsigned order_key(double m) { return (unsigned)__double2hiint(m); }
+
+// Tournament pivoting (TSLU, Grigori, Demmel and Xiang 2011): the panel's pivot
+// rows are chosen by a tree of local partial-pivoting LUs of up to 64 RPL rows,
+// each in one workgroup of 8 waves: the leaves nominate 64 rows of their chunk,
+// a merge takes the candidates of RPL sets, and the last one (the root, which
+// may be a leaf) also writes the selected rows' factors (wlu, column-major 64 x
+// 64), their inverses, the gather map that brings the rows to the top
+// (mdst <- msrc, at most 128 entries) and the permutation.
+//
+// As diag_lu: a wave holds 8 columns, here of RPL rows per lane; a panel of 8
+// columns' owner runs its pivot steps without barriers (the largest
+// max(|re|, |im|) of the rows left, to 20 bits of mantissa, the first row on
+// ties) and publishes the multipliers; after one barrier the later columns'
+// waves apply its 8 rank-1 updates.  A pivot row sits in one of RPL register
+// slots: the step branches on the slot, uniform in the wave.
+//
+// Bound: the chain of 64 pivot steps, per level of the tree.  With 128 rows per
+// workgroup in 256 threads, three barriers a column and a tree of fan-in two,
+// plus the inverses by one thread a column in a kernel of its own, the panels of
+// an FP64 system of 1500 took 1.0 ms each; now 0.25 ms (100 us a level), and the
+// solve 7.75 ms against 26.5.
+template <typename T, int RPL>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(1, 2))) void tslu_panel(
+    const T *A, size_t lda, int Np, int j0, int gin, const int *cin, int *cout, T *wlu, T *dinv, int *mdst, int *msrc,
+    int *mcnt, int *perm, int *status) {
+  using C = CxOf<T>;
+  constexpr int ROWS = 64 * RPL, LM = 2 * 8 * ROWS, FB = 64 * 65;
+  // the multipliers of two panels of 8 columns ([parity][step][row]), and after
+  // the last of them the factored block
+  __shared__ C buf[LM > FB ? LM : FB];
+  __shared__ int rid[ROWS], pidx[64], pb[2][8], outpos[64], wtop[64];
+  const int t = threadIdx.x, lane = t & 63, q = t >> 6, g = blockIdx.x;
+  const bool root = gridDim.x == 1;
+  const C zero{};
+  const int r0 = j0 + g * ROWS;
+  const int R = cin ? 64 * min(RPL, gin - RPL * g) : min(ROWS, Np - r0);
+  if(t < R) rid[t] = cin ? cin[g * ROWS + t] : r0 + t;
+  __syncthreads();
+  const int pq = 2 * (q & 3) + (q >> 2);  // as diag_lu
+  C v[RPL][8];
+  bool used[RPL];
+  int mypos[RPL];
+#pragma unroll
+  for(int s = 0; s < RPL; ++s) {
+    const int idx = lane + 64 * s;
+    used[s] = idx >= R;
+    mypos[s] = -1;
+    const T *row = A + (size_t)(j0 + 8 * pq) * lda + (idx < R ? rid[idx] : j0);
+#pragma unroll
+    for(int j = 0; j < 8; ++j) {
+      const T a = row[(size_t)j * lda];
+      v[s][j] = idx < R ? C{a.x, a.y} : zero;
+    }
+  }
+  // columns from .. 7 of the row in slot sl of lane b (both uniform)
+  auto pivot_row = [&](int sl, int b, C(&pr)[8], int from) {
+#pragma unroll
+    for(int s = 0; s < RPL; ++s)
+      if(sl == s) {
+#pragma unroll
+        for(int j = 0; j < 8; ++j)
+          if(j >= from) pr[j] = rdl(v[s][j], b);
+      }
+  };
+#pragma unroll 1
+  for(int pc = 0; pc < 8; ++pc) {
+    const int par = pc & 1;
+    C *lm = buf + par * 8 * ROWS;
+    if(pq == pc) {
+#pragma unroll
+      for(int jj = 0; jj < 8; ++jj) {
+        const int c = 8 * pc + jj;
+        unsigned key[RPL], kx = 0;
+#pragma unroll
+        for(int s = 0; s < RPL; ++s) {
+          const auto ax = fabs(v[s][jj].x), ay = fabs(v[s][jj].y);  // -0 orders as 0
+          key[s] = used[s] ? 0u : order_key(ax > ay ? ax : ay);
+          kx = max(kx, key[s]);
+        }
+        const unsigned M = wave_max_u32(kx);
+        int sl = 0, b = 0;
+#pragma unroll
+        for(int s = RPL - 1; s >= 0; --s) {
+          const unsigned long long m = __ballot(!used[s] && key[s] == M);
+          if(m) {
+            sl = s;
+            b = __ffsll((long long)m) - 1;
+          }
+        }
+        sl = __builtin_amdgcn_readfirstlane(sl);
+        b = __builtin_amdgcn_readfirstlane(b);
+        C pr[8];
+        pivot_row(sl, b, pr, jj);
+        const bool sing = !(mag2(pr[jj]) > 0.0);
+        if(root && sing && lane == b) atomicCAS(&status[0], 0, j0 + c + 1);
+        const C ip = csel(sing, zero, crecip(pr[jj]));
+        if(lane == 0) {
+          pb[par][jj] = 64 * sl + b;
+          pidx[c] = 64 * sl + b;
+        }
+#pragma unroll
+        for(int s = 0; s < RPL; ++s) {
+          if(s == sl && lane == b) {
+            used[s] = true;
+            mypos[s] = c;
+          }
+          const C l = csel(used[s], zero, cm(v[s][jj], ip));
+          v[s][jj] = csel(used[s], v[s][jj], l);
+          lm[jj * ROWS + 64 * s + lane] = l;
+#pragma unroll
+          for(int j = jj + 1; j < 8; ++j) v[s][j] = cfms(v[s][j], l, pr[j]);
+        }
+      }
+    }
+    __syncthreads();  // one barrier per panel: the buffers alternate
+    if(pq != pc) {
+#pragma unroll 1
+      for(int jj = 0; jj < 8; ++jj) {
+        const int e = __builtin_amdgcn_readfirstlane(pb[par][jj]), sl = e >> 6, b = e & 63;
+#pragma unroll
+        for(int s = 0; s < RPL; ++s)
+          if(s == sl && lane == b) {
+            used[s] = true;
+            mypos[s] = 8 * pc + jj;
+          }
+        if(pq > pc) {
+          C pr[8];
+          pivot_row(sl, b, pr, 0);
+#pragma unroll
+          for(int s = 0; s < RPL; ++s) {
+            const C l = lm[jj * ROWS + 64 * s + lane];
+#pragma unroll
+            for(int j = 0; j < 8; ++j) v[s][j] = cfms(v[s][j], l, pr[j]);
+          }
+        }
+      }
+    }
+  }
+  __syncthreads();
+  if(!root) {
+    if(t < 64) cout[g * 64 + t] = rid[pidx[t]];
+    return;
+  }
+  // the selected rows' factors in pivoted order
+#pragma unroll
+  for(int s = 0; s < RPL; ++s)
+    if(mypos[s] >= 0) {
+#pragma unroll
+      for(int j = 0; j < 8; ++j) {
+        const int col = 8 * pq + j;
+        buf[col * 65 + mypos[s]] = v[s][j];
+        T o;
+        o.x = v[s][j].x;
+        o.y = v[s][j].y;
+        wlu[col * 64 + mypos[s]] = o;
+      }
+    }
+  if(t < 64) wtop[t] = 0;
+  __syncthreads();
+  if(q == 0) {
+    // winner lane goes to row j0 + lane; the top rows that did not win take the
+    // places of the winners from further down, in order
+    const int X = rid[pidx[lane]];
+    const bool in_top = X < j0 + 64;
+    if(in_top) wtop[X - j0] = 1;
+    const unsigned long long below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
+    const unsigned long long om = __ballot(!in_top);
+    if(!in_top) outpos[__popcll(om & below)] = X;
+    __builtin_amdgcn_wave_barrier();
+    __threadfence_block();
+    const bool gone = wtop[lane] == 0;  // row j0 + lane is displaced
+    const unsigned long long gm = __ballot(gone), mm = __ballot(X != j0 + lane);
+    const int v0 = perm[X], v1 = perm[j0 + lane];
+    // every lane's reads have returned before the first write
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    const int n0 = __popcll(mm);
+    if(X != j0 + lane) {
+      const int i = __popcll(mm & below);
+      mdst[i] = j0 + lane;
+      msrc[i] = X;
+      perm[j0 + lane] = v0;
+    }
+    if(gone) {
+      const int i = __popcll(gm & below), dst = outpos[i];
+      mdst[n0 + i] = dst;
+      msrc[n0 + i] = j0 + lane;
+      perm[dst] = v1;
+    }
+    if(lane == 0) *mcnt = n0 + __popcll(gm);
+  }
+  invert_block<T>(buf, dinv);
+}
+
+// Rows per lane of tslu_panel, and so the tree's fan-in: as many as the
+// register file holds (four FP64 rows of 8 columns need three times the
+// scratch; FP64 solves with 3 / 2 rows: N = 1500 7.9 / 8.5 ms, N = 4000 28.9 /
+// 30.8 ms).
+template <typename T> struct TsluCfg {
+  static constexpr int RPL = sizeof(T) == 16 ? 3 : 4;
+};
 
 // Diagonal-block pivoting: LU with partial pivoting restricted to the 64 x 64
 // diagonal block of the panel (rows are chosen among the block's rows; the
@@ -597,53 +572,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
     __builtin_amdgcn_wave_barrier();
     perm[j0 + lane] = old;
   }
-  // Inversions: lane = row i; waves 0-3 hold columns 16 w .. 16 w + 15 of
-  // L11^{-1}, waves 4-7 those of U11^{-1}; row k is broadcast within the wave
-  // by lane reads, so the waves run without barriers.
-  const int i = lane, w = q & 3;
-  C x[16];
-#pragma unroll
-  for(int m = 0; m < 16; ++m) x[m] = csel(16 * w + m == i, one, zero);
-  if(q < 4) {
-    // L11^{-1} (unit lower): for k: row i -= L[i][k] row k, i > k.  Column
-    // 16 w + m starts as e_{16 w + m} and its rows above 16 w + m stay zero,
-    // so the steps k < 16 w leave this wave's columns as they are: skipped
-    C fn = F[(16 * w) * 65 + i];  // column k of L, read one step ahead
-#pragma unroll 1
-    for(int k = 16 * w; k < 63; ++k) {
-      const int ks = __builtin_amdgcn_readfirstlane(k);
-      const C lik = csel(i > ks, fn, zero);
-      fn = F[(ks + 1) * 65 + i];
-#pragma unroll
-      for(int m = 0; m < 16; ++m) x[m] = cfms(x[m], lik, rdl(x[m], ks));
-    }
-  } else {
-    // U11^{-1} = (D^{-1} U11)^{-1} D^{-1} with D = diag(U11): a unit-upper
-    // sweep (row i -= (U[i][k] / U[i][i]) row k, i < k, k = 63..0), then
-    // column j scaled by 1 / U[j][j].  Rows below 16 w + 15 of this wave's
-    // columns stay zero, so the sweep starts at k = 16 w + 15
-    const C di = F[i * 65 + i];
-    const C rinv = csel(mag2(di) > 0.0, crecip(di), zero);
-    C fn = F[(16 * w + 15) * 65 + i];  // column k of U, read one step ahead
-#pragma unroll 1
-    for(int k = 16 * w + 15; k > 0; --k) {
-      const int ks = __builtin_amdgcn_readfirstlane(k);
-      const C uik = csel(i < ks, cm(fn, rinv), zero);
-      fn = F[(ks - 1) * 65 + i];
-#pragma unroll
-      for(int m = 0; m < 16; ++m) x[m] = cfms(x[m], uik, rdl(x[m], ks));
-    }
-#pragma unroll
-    for(int m = 0; m < 16; ++m) x[m] = cm(x[m], rdl(rinv, 16 * w + m));
-  }
-  T *out = dinv + (q < 4 ? 0 : 4096);
-#pragma unroll
-  for(int m = 0; m < 16; ++m) {
-    T o;
-    o.x = x[m].x;
-    o.y = x[m].y;
-    out[(16 * w + m) * 64 + i] = o;
-  }
+  invert_block<T>(F, dinv);
 }
 
 // In-place block product with a 64 x 64 factor M (column-major):
@@ -652,15 +581,14 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
 // with off = first + 64 blockIdx.x.  K is staged through LDS in chunks of
 // 16 (a small LDS footprint lets these workgroups start beside the bulk
 // update's); the block is overwritten only after all of it has been read.
+constexpr int kBlkBK = 16, kBlkPad = 16;
+template <typename T> using BlkPlanes = typename CT<T>::R[2][kBlkBK][64 + kBlkPad];  // [plane][k][m or n]
 template <typename T, bool LEFT>
-__global__ __launch_bounds__(256) void blk_mul(T *A, size_t lda, int j0, int first, const T *M, BatchStrides bs) {
-  A += blockIdx.z * bs.a;
-  M += blockIdx.z * bs.inv;
+__device__ __forceinline__ void blk_mul_body(T *A, size_t lda, int j0, int first, const T *M, BlkPlanes<T> &As,
+                                             BlkPlanes<T> &Bs) {
   using R = typename CT<T>::R;
   using V4 = typename CT<T>::V4;
-  constexpr int BK = 16, PAD = 16;
-  __shared__ R As[2][BK][64 + PAD];  // [plane][k][m]
-  __shared__ R Bs[2][BK][64 + PAD];  // [plane][k][n]
+  constexpr int BK = kBlkBK;
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6, wm = wv & 1, wn = wv >> 1;
   const int off = first + blockIdx.x * 64;
   V4 cr[2][2], ci[2][2];
@@ -749,16 +677,32 @@ __global__ __launch_bounds__(256) void blk_mul(T *A, size_t lda, int j0, int fir
       }
     }
 }
+template <typename T, bool LEFT>
+__global__ __launch_bounds__(256) void blk_mul(T *A, size_t lda, int j0, int first, const T *M, BatchStrides bs) {
+  __shared__ BlkPlanes<T> As, Bs;
+  blk_mul_body<T, LEFT>(A + blockIdx.z * bs.a, lda, j0, first, M + blockIdx.z * bs.inv, As, Bs);
+}
+// Both products of a panel in one launch: U12 (blockIdx.y = 0) and L21, with the
+// inverses [L11^{-1} | U11^{-1}] at M.
+template <typename T>
+__global__ __launch_bounds__(256) void blk_mul_both(T *A, size_t lda, int j0, int first, const T *M) {
+  __shared__ BlkPlanes<T> As, Bs;
+  if(blockIdx.y == 0)
+    blk_mul_body<T, true>(A, lda, j0, first, M, As, Bs);
+  else
+    blk_mul_body<T, false>(A, lda, j0, first, M + kNB * kNB, As, Bs);
+}
 
 // ------------------------------------------------------------------ swaps
 // Applies a gather map (rows mdst[i] <- msrc[i], i < *mcnt <= 128) to the
 // columns c0 .. cend-1, leaving out skip0 .. skip0 + NB - 1 when skip0 >= 0:
 // each workgroup handles 8 columns, reads all moved entries into registers,
-// then writes them back.
+// then writes them back.  With wlu (the tournament), the columns j0 .. j0 + NB -
+// 1 then take the factored block from it.
 template <typename T>
 __global__ __launch_bounds__(256) void laswp_map(T *A, size_t lda, int c0, int cend, const int *__restrict__ mdst,
                                                  const int *__restrict__ msrc, const int *__restrict__ mcnt,
-                                                 int skip0, BatchStrides bs) {
+                                                 int skip0, BatchStrides bs, const T *__restrict__ wlu, int j0) {
   A += blockIdx.z * bs.a;
   mdst += (size_t)blockIdx.z * bs.map;
   msrc += (size_t)blockIdx.z * bs.map;
@@ -785,14 +729,23 @@ __global__ __launch_bounds__(256) void laswp_map(T *A, size_t lda, int c0, int c
     for(int k = 0; k < 4; ++k)
       if(d[k] >= 0) a[d[k]] = v[k];
   }
+  if(wlu && col >= j0 && col < j0 + kNB) {
+    // the moves into the block's rows came from this column's 32 lanes, half a
+    // wave: in order before these stores
+    T *a = A + (size_t)col * lda + j0;
+    const T *w = wlu + (col - j0) * kNB;
+    __builtin_amdgcn_wave_barrier();
+    a[li] = w[li];
+    a[li + 32] = w[li + 32];
+  }
 }
 template <typename T>
 void laswp(T *A, size_t lda, int c0, int cend, const int *mdst, const int *msrc, const int *mcnt, int skip0,
-           hipStream_t st, int nb = 1, BatchStrides bs = BatchStrides{}) {
+           hipStream_t st, int nb = 1, BatchStrides bs = BatchStrides{}, const T *wlu = nullptr, int j0 = 0) {
   const int n = cend - c0 - (skip0 >= 0 ? kNB : 0);
   if(n > 0)
     hipLaunchKernelGGL((laswp_map<T>), dim3((n + 7) / 8, 1, nb), dim3(256), 0, st, A, lda, c0, cend, mdst, msrc, mcnt,
-                       skip0, bs);
+                       skip0, bs, wlu, j0);
 }
 
 // Deferred interchanges of block pivoting: panel k = blockIdx.y (>= 1)
@@ -1398,35 +1351,29 @@ int lu_factor(T *A, int Np, size_t lda, LuWork &w, hipStream_t st, LuProf *prof)
   auto pivoting = [&](int j0) {
     (void)hipEventRecord(w.ev_next, st);
     (void)hipStreamWaitEvent(sb, w.ev_next, 0);
-    const int G = (Np - j0 + kPanelRows - 1) / kPanelRows;
-    hipLaunchKernelGGL((tslu_leaf<T>), dim3(G), dim3(256), 0, sb, A, lda, Np, j0, w.cand[0], w.cnt[0], wlu);
-    int gin = G, buf = 0;
-    while(gin > 1) {
-      const int gout = (gin + 1) / 2;
-      hipLaunchKernelGGL((tslu_merge<T>), dim3(gout), dim3(256), 0, sb, A, lda, j0, gin, w.cand[buf], w.cnt[buf],
-                         w.cand[buf ^ 1], w.cnt[buf ^ 1], wlu);
+    constexpr int RPL = TsluCfg<T>::RPL;
+    static_assert(64 * RPL >= kPanelRows, "the candidate lists are sized for workgroups of kPanelRows rows");
+    int gin = 0, buf = 0;
+    for(int g = (Np - j0 + 64 * RPL - 1) / (64 * RPL);; g = (g + RPL - 1) / RPL) {
+      hipLaunchKernelGGL((tslu_panel<T, RPL>), dim3(g), dim3(512), 0, sb, A, lda, Np, j0, gin,
+                         gin ? w.cand[buf] : nullptr, w.cand[buf ^ 1], wlu, dk(j0), w.mdst, w.msrc, w.mcnt, w.perm,
+                         w.status);
+      if(g == 1) break;
+      gin = g;
       buf ^= 1;
-      gin = gout;
     }
-    hipLaunchKernelGGL(tslu_finish, dim3(1), dim3(64), 0, sb, w.cand[buf], w.cnt[buf], j0, w.piv, w.mdst, w.msrc,
-                       w.mcnt, w.perm);
     (void)hipEventRecord(w.ev_piv, sb);
   };
-  // interchanges on every column and the block's factors and inverses
+  // interchanges on every column, and the factored block
   auto swaps = [&](int j0) {
     (void)hipStreamWaitEvent(st, w.ev_piv, 0);
-    laswp<T>(A, lda, 0, Np, w.mdst, w.msrc, w.mcnt, -1, st);
-    hipLaunchKernelGGL((panel_inv<T>), dim3(1), dim3(256), 0, st, A, lda, j0, wlu, dk(j0), w.status);
+    laswp<T>(A, lda, 0, Np, w.mdst, w.msrc, w.mcnt, -1, st, 1, BatchStrides{}, wlu, j0);
   };
   // L21 and U12 of panel j0
   auto solves = [&](int j0) {
     const int rest = Np - j0 - kNB;
-    if(rest > 0) {
-      hipLaunchKernelGGL((blk_mul<T, true>), dim3(rest / 64), dim3(256), 0, st, A, lda, j0, j0 + kNB, dk(j0),
-                         BatchStrides{});
-      hipLaunchKernelGGL((blk_mul<T, false>), dim3(rest / 64), dim3(256), 0, st, A, lda, j0, j0 + kNB,
-                         dk(j0) + kNB * kNB, BatchStrides{});
-    }
+    if(rest > 0)
+      hipLaunchKernelGGL((blk_mul_both<T>), dim3(rest / 64, 2), dim3(256), 0, st, A, lda, j0, j0 + kNB, dk(j0));
   };
   if((Np + kPanelRows - 1) / kPanelRows > w.gmax) return -2;
   pivoting(0);
