@@ -70,6 +70,47 @@ struct DView {
   template <typename T> T *as() const { return static_cast<T *>(p); }
 };
 
+// Device state of the iterations of nb systems (omx_krylov.hip), the pinned words
+// that tell the host how each step ended (a ring of kTicks), and their events.
+struct KryWs {
+  static constexpr int kTicks = 4;
+  DBuf c, sc, fl, part, pnrm;
+  int *pin = nullptr;    // [kTicks][nb][2], then the final scalars, flags and two status words
+  size_t pin_bytes = 0;
+  hipEvent_t ev[kTicks] = {};
+  static size_t tick_ints(int nb) { return 2 * (size_t)nb; }
+  void ensure(int n, int m, int nb, size_t *T) {
+    const size_t blk = omx::kry_blocks(n);
+    c.ensure(sizeof(cplx) * omx::kry_cplx(m) * nb, T);
+    sc.ensure(sizeof(double) * omx::KS_COUNT * nb, T);
+    fl.ensure(sizeof(int) * omx::KF_COUNT * nb, T);
+    part.ensure(sizeof(cplx) * 2 * nb * blk * (m + 2), T);
+    pnrm.ensure(sizeof(double) * 2 * nb * blk, T);
+    const size_t b =
+        sizeof(double) * omx::KS_COUNT * nb + sizeof(int) * (omx::KF_COUNT * nb + kTicks * tick_ints(nb) + 2);
+    if(pin_bytes < b) {
+      if(pin) (void)hipHostFree(pin);
+      pin = nullptr;
+      pin_bytes = 0;
+      HIPCHK(hipHostMalloc(reinterpret_cast<void **>(&pin), b));
+      pin_bytes = b;
+    }
+    for(hipEvent_t &e : ev)
+      if(!e) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  }
+  void release(size_t *T) {
+    DBuf *b[] = {&c, &sc, &fl, &part, &pnrm};
+    for(DBuf *x : b) x->release(T);
+    if(pin) (void)hipHostFree(pin);
+    pin = nullptr;
+    pin_bytes = 0;
+    for(hipEvent_t &e : ev) {
+      if(e) (void)hipEventDestroy(e);
+      e = nullptr;
+    }
+  }
+};
+
 // Normwise backward error accepted from a refinement that stopped above its
 // residual band: 1000 units of FP64 roundoff.
 const double kBackwardErrorBound = 1e3 * 1.1e-16;
@@ -163,13 +204,14 @@ struct omx_context {
   DBuf d_status2, d_map2;
   std::vector<hipEvent_t> pev2;
   omx::LuProf prof2{};
-  DBuf d_basis, d_basisZ, d_w1, d_w2, d_r, d_part, d_h, d_nrm, d_gpart;
-  // pinned host staging of one Arnoldi step's projections and norm
-  cplx *h_pin = nullptr;
-  int h_pin_n = 0;
+  DBuf d_basis, d_basisZ, d_w1, d_w2, d_r, d_nrm, d_gpart;
+  KryWs kry;
   // pinned host staging of the geometry, and the event after its last copy
   double *geo_pin = nullptr;
   int geo_pin_n = 0;
+  // pinned staging of the solution vectors
+  char *out_pin = nullptr;
+  size_t out_pin_bytes = 0;
   hipEvent_t geo_ev = nullptr;
   // omx_update's times (start, objects done, assembly done) and its joins
   bool upd_timed = false;
@@ -186,8 +228,8 @@ struct omx_context {
   struct Sweep {
     DBuf S64, S32, V64, V32, F64, F64sh, eps, eps_sh, ov, incloc, Q, w, x, xint, xsh, xintsh, K, K1, cross, abscoef,
         abssh, absbes;
-    DBuf perm, perm2, dinv, dinv2, map, status, basis, basisZ, r, w1, w2, gpart, part, hd, nrm, sc,
-        act, kz, omz, sys, map2, status2;
+    DBuf perm, perm2, dinv, dinv2, map, status, basis, basisZ, r, w1, w2, gpart, kz, omz, map2, status2;
+    KryWs kry;
   } sw;
   // ACA-compressed operators S (0) and V (1) of OMX_SOLVER_ACA_GMRES
   struct AcaMat {
@@ -218,17 +260,14 @@ struct omx_context {
     }
   } aca[2];
   DBuf d_acaA, d_acaU, d_acaV, d_acaR, d_acaOff, d_plist;
-  // the inner GMRES of OMX_SOLVER_GMRES32_IR: its own basis, vectors and pinned staging
+  // the inner GMRES of OMX_SOLVER_GMRES32_IR: its own basis and vectors
   struct GmresWs {
-    DBuf basis, r, w1, w2, h, part, nrm, gpart;
-    cplx *h_pin = nullptr;
-    int h_pin_n = 0;
+    DBuf basis, r, w1, gpart;
+    KryWs kry;
     void release(size_t *T) {
-      DBuf *b[] = {&basis, &r, &w1, &w2, &h, &part, &nrm, &gpart};
+      DBuf *b[] = {&basis, &r, &w1, &gpart};
       for(DBuf *x : b) x->release(T);
-      if(h_pin) (void)hipHostFree(h_pin);
-      h_pin = nullptr;
-      h_pin_n = 0;
+      kry.release(T);
     }
   } ws_in;
   // Captured factorisations (omx_set_graphs): executable graphs of S's
@@ -326,6 +365,10 @@ void alloc_lu(omx_context *c, omx::LuWork &w, DBuf &perm, DBuf &dinv, bool secon
 // is pinned, and rewritten only once the copy before has left it.
 constexpr int kGeoDoubles = 6 * 2 + 3 + 1;
 void upload_geometry(omx_context *c) {
+  if(!c->d_coef.p) {  // the assembly's coefficient tables, once per context
+    c->d_coef.ensure(sizeof(double) * omx::CF_COUNT * omx::kCoefStride, &c->total);
+    omx::fill_coef(c->d_coef.as<double>(), c->st);
+  }
   const size_t P = c->P;
   const int n = kGeoDoubles * c->P;
   if(c->geo_pin_n < n) {
@@ -377,8 +420,6 @@ void alloc_all(omx_context *c) {
   c->d_w1.ensure(sizeof(cplx) * Np, T);
   c->d_w2.ensure(sizeof(cplx) * Np, T);
   c->d_gpart.ensure(sizeof(cplx) * Np * omx::kGemvSplitMax, T);
-  c->d_part.ensure(sizeof(cplx) * 128 * (c->restart + 2), T);
-  c->d_h.ensure(sizeof(cplx) * 2 * (c->restart + 2), T);
   c->d_nrm.ensure(sizeof(double) * 256, T);
 }
 
@@ -412,10 +453,6 @@ void alloc_matrices(omx_context *c) {
     w.basis.ensure(sizeof(cplx) * Np * (kInnerSteps + 1), T);
     w.r.ensure(sizeof(cplx) * Np, T);
     w.w1.ensure(sizeof(cplx) * Np, T);
-    w.w2.ensure(sizeof(cplx) * Np, T);
-    w.h.ensure(sizeof(cplx) * 2 * (kInnerSteps + 2), T);
-    w.part.ensure(sizeof(cplx) * 128 * (kInnerSteps + 2), T);
-    w.nrm.ensure(sizeof(double) * 256, T);
     w.gpart.ensure(sizeof(cplx) * Np * omx::kGemvSplitMax, T);
   } else {
     c->ws_in.release(T);
@@ -609,177 +646,175 @@ void aca_apply(omx_context *c, bool shf, const cplx *x, cplx *y, hipStream_t st)
   omx::aca_matvec(op, x, y, st);
 }
 
+// The error that a factorisation's status words tell of, if any.
+void throw_status(const int *s) {
+  if(s[1]) throw OmxError(OMX_ERR_DEVICE, "device wait timed out (code " + std::to_string(s[1]) + ")");
+  if(s[0]) throw OmxError(OMX_ERR_SINGULAR, "zero pivot at column " + std::to_string(s[0] - 1));
+}
+
 // ------------------------------------------------------------------ GMRES
-// Right-preconditioned restarted GMRES in FP64 with classical Gram-Schmidt
-// (two passes).  prec(in, out) applies M^{-1} (identity when null).  The
-// Arnoldi process follows Gmres_Zcomp (PreconditionedMatrix.cpp:892-985):
-// Givens rotations on the Hessenberg column, convergence on |g_{j+1}|.
-struct Gmres {
+// Right-preconditioned restarted GMRES in FP64 with classical Gram-Schmidt (two
+// passes), in flexible form: the preconditioned vectors M^{-1} v_j are kept, so
+// the end of a cycle needs no further preconditioner application.  nb systems
+// run in lockstep, each with its own Hessenberg matrix and stopping state; one
+// that has converged drops out of the products and solves.  The algebra runs on
+// the device (omx_krylov.hip); the host only learns, a step later, which systems
+// go on.
+struct Krylov {
   omx_context *c;
-  const cplx *A;  // FP64 operator
-  std::function<void(const cplx *, cplx *)> prec;
-  int N;
-  hipStream_t s;  // the stream every step runs on
-  // an operator given as a product (set: used instead of A), and its bytes
-  // read per product
+  int n, nb;
+  hipStream_t s;
+  KryWs &ws;
+  cplx *V, *Z;            // bases; Z of the preconditioned vectors (V itself without one)
+  cplx *r, *w, *gpart;
+  // the operator: FP64 matrices A (sA apart), or their complex-FP32 copy, or a
+  // product given as a function
+  const cplx *A = nullptr;
+  size_t sA = 0;
+  const float2 *A32 = nullptr;
   std::function<void(const cplx *, cplx *)> op = nullptr;
   double op_bytes = 0.0;
-  // a workspace of its own (null: the context's); one_cycle: x starts at 0
-  // (the caller zeroes it) and a single cycle runs, with no residual product
-  // before or after it (a fixed-cost preconditioner)
-  omx_context::GmresWs *ws = nullptr;
-  bool one_cycle = false;
-  double nrm(const cplx *x) {
-    DBuf &dn = ws ? ws->nrm : c->d_nrm;
-    omx::nrm2sq(x, N, dn.as<double>() + 1, dn.as<double>(), s);
-    double v;
-    HIPCHK(hipMemcpyAsync(&v, dn.p, sizeof(double), hipMemcpyDeviceToHost, s));
-    HIPCHK(hipStreamSynchronize(s));
-    return std::sqrt(v);
-  }
-  void matvec(const cplx *x, cplx *y) {
-    if(c->profile) HIPCHK(hipEventRecord(c->ev[6], s));
-    if(op) {
-      op(x, y);
-      c->mv_bytes += op_bytes;
-    } else {
-      omx::gemv64(A, (size_t)c->Np, N, x, y, c->d_gpart.as<cplx>(), s);
-      c->mv_bytes += 16.0 * c->Np * (double)c->Np;
-    }
-    ++c->mv_calls;
-    if(c->profile) {
+  // out = M^{-1} in for the systems whose flag is set (identity when null)
+  std::function<void(const cplx *in, cplx *out, const int *live)> prec = nullptr;
+  bool x_zero = false;     // x starts at 0: no product before the first cycle
+  bool one_cycle = false;  // and no residual after it (a fixed-cost preconditioner)
+  bool batch = false;      // the batched sweeps' stopping rules
+  bool lazy = false;       // never enqueue a step that may turn out not to be needed
+  const int *status = nullptr;  // the factorisation's status words, looked at once the first step is known
+  std::vector<double> res;
+  std::vector<int> its;
+  int bits = 0;            // binary digits between the residual and its goal, as last known
+
+  // Enqueues A x into gpart (returns the column parts) or w (returns 0).
+  int product(const cplx *x, const int *flag, int live) {
+    const bool prof = c->profile;
+    if(prof) HIPCHK(hipEventRecord(c->ev[6], s));
+    int ns = 0;
+    if(op)
+      op(x, w);
+    else if(A32)
+      ns = omx::gemv_partial(A32, (size_t)c->Np, n, x, gpart, s, flag);
+    else
+      ns = omx::gemv_partial(A, (size_t)c->Np, n, x, gpart, s, nb, sA, (size_t)n, flag, std::max(1, live));
+    if(prof) {
       HIPCHK(hipEventRecord(c->ev[7], s));
       HIPCHK(hipEventSynchronize(c->ev[7]));
       float ms = 0;
       HIPCHK(hipEventElapsedTime(&ms, c->ev[6], c->ev[7]));
       c->mv_ms += ms;
     }
+    return ns;
   }
-  // Solves A x = b; x holds the initial guess.  Returns iterations; *res the
-  // final true relative residual.
-  int solve(const cplx *b, cplx *x, double tol, int maxit, int m, double *res) {
-    // flexible form: the preconditioned vectors M^{-1} v_j are kept (Zb), so
-    // the end of a cycle needs no further preconditioner application
-    cplx *V = (ws ? ws->basis : c->d_basis).as<cplx>(), *Zb = c->d_basisZ.as<cplx>();
-    cplx *r = (ws ? ws->r : c->d_r).as<cplx>(), *w = (ws ? ws->w1 : c->d_w1).as<cplx>();
-    cplx *z = (ws ? ws->w2 : c->d_w2).as<cplx>();
-    cplx *hd = (ws ? ws->h : c->d_h).as<cplx>(), *part = (ws ? ws->part : c->d_part).as<cplx>();
-    DBuf &dnrm = ws ? ws->nrm : c->d_nrm;
-    cplx *&h_pin = ws ? ws->h_pin : c->h_pin;
-    int &h_pin_n = ws ? ws->h_pin_n : c->h_pin_n;
-    const size_t ld = (size_t)c->Np;
-    double bn = nrm(b);
-    if(bn == 0.0) {
-      omx::vaxpby(x, omx::mk(0.0), x, omx::mk(0.0), N, s);
-      *res = 0.0;
-      return 0;
+  void count(int live) {
+    if(live < 1) return;
+    ++c->mv_calls;
+    c->mv_bytes += (op ? op_bytes : (A32 ? 8.0 : 16.0) * n * (double)n) * live;
+  }
+  // Solves A x = b; x holds the initial guesses.  res: the final relative
+  // residuals, its: the iterations.  (A one-cycle solve leaves both unread.)
+  void solve(const cplx *b, cplx *x, double tol, int maxit, int m) {
+    ws.ensure(n, m, nb, &c->total);
+    const bool never = lazy || c->profile || op != nullptr;
+    omx::KryState st{n,
+                     m,
+                     nb,
+                     0,
+                     tol,
+                     maxit,
+                     ws.c.as<cplx>(),
+                     ws.sc.as<double>(),
+                     ws.fl.as<int>(),
+                     ws.part.as<cplx>(),
+                     ws.pnrm.as<double>(),
+                     V,
+                     prec ? Z : V,
+                     (size_t)n * nb,
+                     (size_t)n,
+                     r,
+                     w,
+                     (size_t)n};
+    const int *live = st.fl + omx::KF_LIVE, *active = st.fl + omx::KF_ACTIVE;
+    int tick = -1, known = -1;  // the last event recorded, and the last one waited for
+    auto slot = [&](int t) { return ws.pin + (size_t)(t % KryWs::kTicks) * KryWs::tick_ints(nb); };
+    auto mark = [&] {
+      ++tick;
+      HIPCHK(hipEventRecord(ws.ev[tick % KryWs::kTicks], s));
+    };
+    // waits for the next event: the systems that go on, and the digits left
+    int nlive = nb, last_bits = 0, restart = 0;
+    double left = 0.0;  // steps to the goal after the last known one, by its gain
+    double *hs = reinterpret_cast<double *>(ws.pin + KryWs::kTicks * KryWs::tick_ints(nb));
+    int *hf = reinterpret_cast<int *>(hs + omx::KS_COUNT * nb), *hst = hf + omx::KF_COUNT * nb;
+    if(status) HIPCHK(hipMemcpyAsync(hst, status, 2 * sizeof(int), hipMemcpyDeviceToHost, s));
+    auto wait = [&] {
+      const int before = nlive;
+      ++known;
+      HIPCHK(hipEventSynchronize(ws.ev[known % KryWs::kTicks]));
+      if(status && known == 0) throw_status(hst);
+      const int *h = slot(known);
+      nlive = bits = 0;
+      for(int z = 0; z < nb; ++z)
+        if(h[2 * z]) {
+          ++nlive;
+          bits = std::max(bits, h[2 * z + 1]);
+        }
+      const int gain = last_bits - bits;
+      left = known != restart && gain > 0 ? (double)bits / gain : 0.0;
+      last_bits = bits;
+      if(known != restart) count(before);
+    };
+    int ns = 0;
+    if(!x_zero && !one_cycle) {
+      ns = product(x, nullptr, nb);
+      if(op) ns = -1;
+      count(nb);
     }
-    if(h_pin_n < 2 * (m + 2) + 1) {
-      if(h_pin) (void)hipHostFree(h_pin);
-      h_pin = nullptr;
-      h_pin_n = 0;
-      HIPCHK(hipHostMalloc(reinterpret_cast<void **>(&h_pin), sizeof(cplx) * (2 * (m + 2) + 1)));
-      h_pin_n = 2 * (m + 2) + 1;
-    }
-    cplx *hpin = h_pin;
-    int it = 0, stall = 0;
-    double prev = 0.0;
-    bool tiny_step = false;
-    std::vector<std::complex<double>> H((size_t)(m + 1) * m), g(m + 1), cs(m), sn(m);
-    int cycles = 0;
-    while(true) {
-      if(one_cycle && cycles == 1) break;
-      if(one_cycle) {  // x = 0: r = b
-        omx::vcopy(r, b, N, s);
-      } else {
-        matvec(x, r);
-        omx::vsub(r, b, r, N, s);
-      }
-      ++cycles;
-      double beta = one_cycle ? bn : nrm(r);
-      *res = beta / bn;
-      if(*res <= tol || it >= maxit || tiny_step) break;
-      // stagnation at the FP64 floor: a restart cycle without halving once the
-      // residual is within the acceptance band (<= 1e3 tol), two once it is
-      // down to 1e-10 (further up a slow phase of the restarted iteration is
-      // waited out, up to maxit)
-      if(prev > 0.0 && beta > 0.5 * prev && *res < 1e-10) {
-        if(++stall >= 2 || *res <= 1e3 * tol) break;
-      } else {
-        stall = 0;
-      }
-      prev = beta;
-      omx::vaxpby(V, omx::mk(1.0 / beta), r, omx::mk(0.0), N, s);
-      std::fill(g.begin(), g.end(), 0.0);
-      g[0] = beta;
-      int j = 0;
-      for(; j < m && it < maxit; ++j, ++it) {
-        const cplx *vj = V + (size_t)j * ld;
+    omx::kry_restart(st, b, x, gpart, ns, (size_t)std::max(0, ns) * n, true, batch, slot(tick + 1), s);
+    mark();
+    if(never) wait();
+    while(known < tick || nlive > 0) {
+      bool over = false;
+      for(int j = 0; j < m && !over; ++j) {
+        st.j = j;
+        const cplx *vj = V + (size_t)j * st.ldk, *pj = vj;
         if(prec) {
-          prec(vj, Zb + (size_t)j * ld);
-          matvec(Zb + (size_t)j * ld, w);
-        } else {
-          matvec(vj, w);
+          cplx *zj = Z + (size_t)j * st.ldk;
+          prec(vj, zj, live);
+          pj = zj;
         }
-        // two Gram-Schmidt passes and the norm, copied to pinned memory with
-        // one wait for all three
-        for(int pass = 0; pass < 2; ++pass) {
-          cplx *hp = hd + (size_t)pass * (m + 2);
-          omx::dotc_multi(V, ld, j + 1, w, N, part, hp, s);
-          omx::axpy_multi(V, ld, j + 1, hp, w, N, s);
-          HIPCHK(hipMemcpyAsync(hpin + (size_t)pass * (m + 2), hp, sizeof(cplx) * (j + 1), hipMemcpyDeviceToHost, s));
-        }
-        omx::nrm2sq(w, N, dnrm.as<double>() + 1, dnrm.as<double>(), s);
-        HIPCHK(hipMemcpyAsync(hpin + 2 * (m + 2), dnrm.p, sizeof(double), hipMemcpyDeviceToHost, s));
-        HIPCHK(hipStreamSynchronize(s));
-        const cplx *h1 = hpin, *h2 = hpin + (m + 2);
-        double hn = std::sqrt(reinterpret_cast<const double *>(hpin + 2 * (m + 2))[0]);
-        for(int i = 0; i <= j; ++i)
-          H[(size_t)j * (m + 1) + i] = std::complex<double>(h1[i].x + h2[i].x, h1[i].y + h2[i].y);
-        H[(size_t)j * (m + 1) + j + 1] = hn;
-        if(hn > 0.0) omx::vaxpby(V + (size_t)(j + 1) * ld, omx::mk(1.0 / hn), w, omx::mk(0.0), N, s);
-        auto *hc = &H[(size_t)j * (m + 1)];
-        for(int i = 0; i < j; ++i) {
-          std::complex<double> t = cs[i] * hc[i] + sn[i] * hc[i + 1];
-          hc[i + 1] = -std::conj(sn[i]) * hc[i] + cs[i] * hc[i + 1];
-          hc[i] = t;
-        }
-        double den = std::sqrt(std::norm(hc[j]) + std::norm(hc[j + 1]));
-        if(den == 0.0) {
-          cs[j] = 1.0;
-          sn[j] = 0.0;
-        } else {
-          std::complex<double> ph = std::abs(hc[j]) > 0 ? hc[j] / std::abs(hc[j]) : 1.0;
-          cs[j] = std::abs(hc[j]) / den;
-          sn[j] = ph * std::conj(hc[j + 1]) / den;
-        }
-        hc[j] = cs[j] * hc[j] + sn[j] * hc[j + 1];
-        hc[j + 1] = 0.0;
-        g[j + 1] = -std::conj(sn[j]) * g[j];
-        g[j] = cs[j] * g[j];
-        if(std::abs(g[j + 1]) <= 0.5 * tol * bn || hn == 0.0) {
-          ++j;
-          ++it;
-          break;
+        ns = product(pj, live, nlive);
+        omx::kry_step(st, gpart, ns, (size_t)ns * n, slot(tick + 1), s);
+        mark();
+        // Go on at once when the steps enqueued since the last known one are
+        // surely not enough (its gain repeated, and one to spare); otherwise
+        // wait for the outcomes, oldest first
+        while(known < tick && !over) {
+          const int open = tick - known;
+          if(!never && j + 1 < m && left > open + 0.5 && open < KryWs::kTicks - 1) break;
+          wait();
+          over = nlive == 0;
         }
       }
-      // y = H^{-1} g (upper triangular j x j), x += M^{-1} V y
-      std::vector<std::complex<double>> y(j);
-      for(int i = j - 1; i >= 0; --i) {
-        std::complex<double> s = g[i];
-        for(int k = i + 1; k < j; ++k) s -= H[(size_t)k * (m + 1) + i] * y[k];
-        y[i] = s / H[(size_t)i * (m + 1) + i];
-      }
-      std::vector<cplx> yh(j);
-      for(int i = 0; i < j; ++i) yh[i] = omx::mk(y[i].real(), y[i].imag());
-      HIPCHK(hipMemcpyAsync(hd, yh.data(), sizeof(cplx) * j, hipMemcpyHostToDevice, s));
-      omx::gemv_multi(prec ? Zb : V, ld, j, hd, z, N, s);
-      const cplx *dx = z;
-      omx::vaxpby(x, omx::mk(1.0), dx, omx::mk(1.0), N, s);
-      // a correction below the FP64 resolution of x ends the refinement
-      if(!one_cycle && nrm(dx) <= 1e-16 * nrm(x)) tiny_step = true;
+      while(known < tick) wait();
+      omx::kry_end_cycle(st, x, !one_cycle, batch, s);
+      if(one_cycle) return;
+      ns = product(x, active, nb);
+      if(op) ns = -1;
+      count(nb);
+      omx::kry_restart(st, b, x, gpart, ns, (size_t)std::max(0, ns) * n, false, batch, slot(tick + 1), s);
+      mark();
+      restart = tick;
+      wait();
     }
-    return it;
+    HIPCHK(hipMemcpyAsync(hs, st.sc, sizeof(double) * omx::KS_COUNT * nb, hipMemcpyDeviceToHost, s));
+    HIPCHK(hipMemcpyAsync(hf, st.fl, sizeof(int) * omx::KF_COUNT * nb, hipMemcpyDeviceToHost, s));
+    HIPCHK(hipStreamSynchronize(s));
+    res.resize(nb);
+    its.resize(nb);
+    for(int z = 0; z < nb; ++z) {
+      res[z] = hs[omx::KS_COUNT * z + omx::KS_RES];
+      its[z] = hf[omx::KF_COUNT * z + omx::KF_ITS];
+    }
   }
 };
 
@@ -790,8 +825,7 @@ void check_status(omx_context *c, bool shf = false) {
   hipStream_t st = sys_stream(c, shf);
   HIPCHK(hipMemcpyAsync(s, (shf ? c->d_status2 : c->d_status).p, sizeof(s), hipMemcpyDeviceToHost, st));
   HIPCHK(hipStreamSynchronize(st));
-  if(s[1]) throw OmxError(OMX_ERR_DEVICE, "device wait timed out (code " + std::to_string(s[1]) + ")");
-  if(s[0]) throw OmxError(OMX_ERR_SINGULAR, "zero pivot at column " + std::to_string(s[0] - 1));
+  throw_status(s);
 }
 
 omx::LuProf *prof_begin(omx_context *c, bool shf) {
@@ -1004,10 +1038,16 @@ void factor_graphed(omx_context *c, bool with_v, int mark) {
 // residual's floor is u ||A|| ||x|| / ||b||, far above u when x is large).  The
 // bound is a constant: it does not grow with tol, so a caller's loose tol
 // never lets an FP32-quality answer through.
-bool backward_stable(omx_context *c, Gmres &gm, const cplx *A64, const cplx *rhs, const cplx *x, double res,
-                     hipStream_t st) {
+bool backward_stable(omx_context *c, const cplx *A64, const cplx *rhs, const cplx *x, double res, hipStream_t st) {
   const size_t Np = (size_t)c->Np;
-  const double bn = gm.nrm(rhs), xn = gm.nrm(x);
+  auto nrm = [&](const cplx *v) {
+    omx::nrm2sq(v, c->Np, c->d_nrm.as<double>() + 1, c->d_nrm.as<double>(), st);
+    double e = 0.0;
+    HIPCHK(hipMemcpyAsync(&e, c->d_nrm.p, sizeof(double), hipMemcpyDeviceToHost, st));
+    HIPCHK(hipStreamSynchronize(st));
+    return std::sqrt(e);
+  };
+  const double bn = nrm(rhs), xn = nrm(x);
   double a2 = 0.0;
   const size_t n2 = Np * Np, chunk = (size_t)1 << 28;
   for(size_t off = 0; off < n2; off += chunk) {
@@ -1031,30 +1071,39 @@ void solve_system(omx_context *c, bool shf, const cplx *rhs, cplx *x, int *iters
   const size_t lda = (size_t)Np;
   hipStream_t st = sys_stream(c, shf);
   DBuf &status = shf ? c->d_status2 : c->d_status;
-  Gmres gm{c, A64, nullptr, Np, st};
+  Krylov gm{c,          Np,
+            1,          st,
+            c->kry,     c->d_basis.as<cplx>(),
+            c->d_basisZ.as<cplx>(), c->d_r.as<cplx>(),
+            c->d_w1.as<cplx>(),     c->d_gpart.as<cplx>()};
+  gm.A = A64;
+  auto run = [&](cplx *xx, int maxit) {
+    gm.solve(rhs, xx, c->tol, maxit, c->restart);
+    *iters = gm.its[0];
+    *res = gm.res[0];
+  };
   if(c->kind == OMX_SOLVER_ACA_GMRES) {  // Gmres_Zcomp on the compressed operator
     gm.op = [c, shf, st](const cplx *in, cplx *out) { aca_apply(c, shf, in, out, st); };
     gm.op_bytes = c->aca[shf ? 1 : 0].bytes;
   }
   // mixed Krylov: the preconditioner is one GMRES cycle on the FP32 copy
-  Gmres inner{c, nullptr, nullptr, Np, st};
+  auto &wi = c->ws_in;
+  Krylov inner{c,      Np,
+               1,      st,
+               wi.kry, wi.basis.as<cplx>(),
+               nullptr, wi.r.as<cplx>(),
+               wi.w1.as<cplx>(), wi.gpart.as<cplx>()};
   if(c->kind == OMX_SOLVER_GMRES32_IR) {
     float2 *A32w = (shf ? c->d_V32 : c->d_S32).as<float2>();
     bool &dirty = shf ? c->dirty32_sh : c->dirty32;
     if(dirty) omx::demote(A32w, A64, (size_t)Np * lda, st);  // an earlier factorisation overwrote it
     dirty = false;
-    const float2 *A32c = A32w;
-    cplx *gpart = c->ws_in.gpart.as<cplx>();
-    inner.op = [A32c, lda, Np, gpart, st](const cplx *in, cplx *out) {
-      omx::gemv32(A32c, lda, Np, in, out, gpart, st);
-    };
-    inner.op_bytes = 8.0 * Np * (double)Np;
-    inner.ws = &c->ws_in;
+    inner.A32 = A32w;
     inner.one_cycle = true;
-    gm.prec = [&inner, Np, st](const cplx *in, cplx *out) {
+    gm.lazy = true;  // its preconditioner is a solve of its own
+    gm.prec = [&inner, Np, st](const cplx *in, cplx *out, const int *) {
       HIPCHK(hipMemsetAsync(out, 0, sizeof(cplx) * Np, st));
-      double r = 0.0;
-      inner.solve(in, out, kInnerTol, kInnerSteps, kInnerSteps, &r);
+      inner.solve(in, out, kInnerTol, kInnerSteps, kInnerSteps);
     };
   }
   if(!is_lu(c->kind)) {
@@ -1064,9 +1113,11 @@ void solve_system(omx_context *c, bool shf, const cplx *rhs, cplx *x, int *iters
       HIPCHK(hipMemsetAsync(x, 0, sizeof(cplx) * Np, st));
       const int maxit =
           try_first ? std::min(c->maxit, c->auto_budget > 0 ? c->auto_budget : auto_krylov_steps(c->N)) : c->maxit;
-      *iters = gm.solve(rhs, x, c->tol, maxit, c->restart, res);
+      gm.x_zero = true;
+      run(x, maxit);
+      gm.x_zero = false;
       check_status(c, shf);
-      if(!(*res <= 1e3 * c->tol) && (c->kind == OMX_SOLVER_ACA_GMRES || !backward_stable(c, gm, A64, rhs, x, *res, st)))
+      if(!(*res <= 1e3 * c->tol) && (c->kind == OMX_SOLVER_ACA_GMRES || !backward_stable(c, A64, rhs, x, *res, st)))
         throw OmxError(OMX_ERR_NOCONV, "GMRES stopped at relative residual " + std::to_string(*res));
       return;
     } catch(OmxError &e) {
@@ -1080,8 +1131,10 @@ void solve_system(omx_context *c, bool shf, const cplx *rhs, cplx *x, int *iters
     omx::zero_ints(status.as<int>(), 4, st);
     HIPCHK(hipMemsetAsync(x, 0, sizeof(cplx) * Np, st));
     const int maxit = std::min(c->maxit, c->auto_budget > 0 ? c->auto_budget : auto_gmres64_steps(c->N));
-    *iters = gm.solve(rhs, x, c->tol, maxit, c->restart, res);
-    if(*res <= 1e3 * c->tol || backward_stable(c, gm, A64, rhs, x, *res, st)) return;
+    gm.x_zero = true;
+    run(x, maxit);
+    gm.x_zero = false;
+    if(*res <= 1e3 * c->tol || backward_stable(c, A64, rhs, x, *res, st)) return;
     ++c->fallbacks;
   }
   const bool f64 = c->kind == OMX_SOLVER_LU64;
@@ -1094,25 +1147,30 @@ void solve_system(omx_context *c, bool shf, const cplx *rhs, cplx *x, int *iters
     const bool last = pv == OMX_PIVOT_PARTIAL;
     try {
       if(!fact || lu.pivot != pv) factor_enqueue(c, shf, pv);
-      check_status(c, shf);  // zero pivots of this factorisation
+      gm.status = status.as<int>();  // zero pivots of this factorisation
       if(f64) {
-        gm.prec = [F64, &lu, Np, lda, st](const cplx *in, cplx *out) {
+        gm.prec = [F64, &lu, Np, lda, st](const cplx *in, cplx *out, const int *live) {
+          lu.live = live;
           omx::lu_solve<double2>(reinterpret_cast<const double2 *>(F64), Np, lda, lu, in, out, st);
+          lu.live = nullptr;
         };
         omx::lu_solve<double2>(reinterpret_cast<const double2 *>(F64), Np, lda, lu, rhs, x, st);
         if(pv == OMX_PIVOT_PARTIAL) {  // plain FP64 LU with partial pivoting
+          gm.status = nullptr;
           check_status(c, shf);
           *iters = 0;
           *res = -1.0;
           return;
         }
       } else {
-        gm.prec = [A32, &lu, Np, lda, st](const cplx *in, cplx *out) {
+        gm.prec = [A32, &lu, Np, lda, st](const cplx *in, cplx *out, const int *live) {
+          lu.live = live;
           omx::lu_solve<float2>(A32, Np, lda, lu, in, out, st);
+          lu.live = nullptr;
         };
         omx::lu_solve<float2>(A32, Np, lda, lu, rhs, x, st);  // x0 = M^{-1} b
       }
-      *iters = gm.solve(rhs, x, c->tol, c->maxit, c->restart, res);
+      run(x, c->maxit);
       check_status(c, shf);
       // the target may sit below the FP64 residual floor of an ill-conditioned
       // system; a stagnated refinement within 1000x of it is accepted, and so
@@ -1121,7 +1179,7 @@ void solve_system(omx_context *c, bool shf, const cplx *rhs, cplx *x, int *iters
       // floor is u ||A|| ||x|| / ||b||, far above u when x is large).  That
       // bound is a constant: it does not grow with tol, so a caller's loose
       // tol never lets an FP32-quality answer through.
-      if(!(*res <= 1e3 * c->tol) && !backward_stable(c, gm, A64, rhs, x, *res, st))
+      if(!(*res <= 1e3 * c->tol) && !backward_stable(c, A64, rhs, x, *res, st))
         throw OmxError(OMX_ERR_NOCONV, "refinement stopped at relative residual " + std::to_string(*res) +
                                            ", backward error above " + std::to_string(kBackwardErrorBound));
       return;
@@ -1132,238 +1190,6 @@ void solve_system(omx_context *c, bool shf, const cplx *rhs, cplx *x, int *iters
     }
   }
 }
-
-// ------------------------------------------------------------------ batches
-// Restarted GMRES for nb systems in lockstep (the Gmres above, with every
-// vector operation batched): each system keeps its own Hessenberg matrix,
-// rotations, residual and stopping state; a system that has converged (or
-// stalled) in a cycle has its further basis vectors scaled to zero and its
-// solution left alone.  prec(in, out) applies the batched preconditioner.
-struct GmresB {
-  omx_context *c;
-  const cplx *A;  // FP64 operators, sA apart
-  size_t sA;
-  int Np, nb;
-  std::function<void(const cplx *, cplx *)> prec;
-  omx_context::Sweep &w;
-  omx::LuWork *lw = nullptr;  // the preconditioner's factorisation: its solves may take a subset
-  size_t sv() const { return (size_t)Np; }
-  // The systems with mask[z] set: their count, and (when some are left out)
-  // their indices in w.sys, so the matrix-sized work runs on those only.
-  // Converged systems thus drop out of the lockstep batch's products and
-  // triangular solves; their vectors are left as they are and ignored.
-  int subset(const std::vector<int> &mask, const int **sys) {
-    std::vector<int> idx;
-    for(int z = 0; z < nb; ++z)
-      if(mask[z]) idx.push_back(z);
-    *sys = nullptr;
-    if((int)idx.size() == nb || idx.empty()) return (int)idx.size();
-    HIPCHK(hipMemcpyAsync(w.sys.p, idx.data(), sizeof(int) * idx.size(), hipMemcpyHostToDevice, c->st));
-    *sys = w.sys.as<int>();
-    return (int)idx.size();
-  }
-  void precond(const cplx *in, cplx *out, const std::vector<int> &mask) {
-    if(!lw) {
-      prec(in, out);
-      return;
-    }
-    const int *sys;
-    const int n = subset(mask, &sys);
-    if(n == 0) return;
-    lw->sys = sys;
-    lw->nsys = n;
-    prec(in, out);
-    lw->sys = nullptr;
-    lw->nsys = 0;
-  }
-  std::vector<double> nrms(const cplx *x) {
-    omx::nrm2sq_b(x, sv(), Np, nb, w.nrm.as<double>() + nb, w.nrm.as<double>(), c->st);
-    std::vector<double> v(nb);
-    HIPCHK(hipMemcpyAsync(v.data(), w.nrm.p, sizeof(double) * nb, hipMemcpyDeviceToHost, c->st));
-    HIPCHK(hipStreamSynchronize(c->st));
-    for(double &e : v) e = std::sqrt(e);
-    return v;
-  }
-  void matvec(const cplx *x, cplx *y, const std::vector<int> &mask) {
-    const int *sys;
-    const int n = subset(mask, &sys);
-    if(n == 0) return;
-    if(c->profile) HIPCHK(hipEventRecord(c->ev[4], c->st));
-    omx::gemv64(A, (size_t)Np, Np, x, y, w.gpart.as<cplx>(), c->st, nb, sA, sv(), sys, n);
-    ++c->mv_calls;
-    c->mv_bytes += 16.0 * Np * (double)Np * n;
-    if(c->profile) {
-      HIPCHK(hipEventRecord(c->ev[5], c->st));
-      HIPCHK(hipEventSynchronize(c->ev[5]));
-      float ms = 0;
-      HIPCHK(hipEventElapsedTime(&ms, c->ev[4], c->ev[5]));
-      c->mv_ms += ms;
-    }
-  }
-  // per-system scalars a[z], b[z] in device memory
-  void scale(cplx *y, size_t sy, const std::vector<cplx> &a, const cplx *x, size_t sx, const std::vector<cplx> &b,
-             const int *act) {
-    cplx *sc = w.sc.as<cplx>();
-    std::vector<cplx> h(2 * nb);
-    for(int z = 0; z < nb; ++z) {
-      h[z] = a[z];
-      h[nb + z] = b[z];
-    }
-    HIPCHK(hipMemcpyAsync(sc, h.data(), sizeof(cplx) * 2 * nb, hipMemcpyHostToDevice, c->st));
-    omx::vaxpby_b(y, sy, sc, x, sx, sc + nb, Np, nb, act, c->st);
-  }
-  // Solves A_z x_z = b_z (x holds the initial guesses); res[z] the final
-  // relative residual, its[z] the iterations spent on system z.
-  void solve(const cplx *b, cplx *x, double tol, int maxit, int m, std::vector<double> &res, std::vector<int> &its) {
-    // basis vector k of system z at V + (k nb + z) Np: the systems' k-th
-    // vectors are contiguous, as the batched preconditioner expects
-    cplx *V = w.basis.as<cplx>(), *Zb = w.basisZ.as<cplx>();  // Zb: M^{-1} V (flexible form)
-    const size_t sV = (size_t)Np, ld = (size_t)Np * nb;
-    cplx *r = w.r.as<cplx>(), *wv = w.w1.as<cplx>();
-    cplx *hd = w.hd.as<cplx>(), *part = w.part.as<cplx>();
-    const int sh = m + 2;
-    int *act_d = w.act.as<int>();
-    res.assign(nb, 0.0);
-    its.assign(nb, 0);
-    const std::vector<double> bn = nrms(b);
-    std::vector<int> active(nb), stall(nb, 0);
-    std::vector<double> prev(nb, 0.0);
-    for(int z = 0; z < nb; ++z) active[z] = bn[z] > 0.0;
-    const cplx zero = omx::mk(0.0), one = omx::mk(1.0);
-    {  // zero right-hand side: zero solution
-      std::vector<cplx> a(nb, zero), bb(nb);
-      bool any = false;
-      for(int z = 0; z < nb; ++z) {
-        bb[z] = active[z] ? one : zero;
-        any |= !active[z];
-      }
-      if(any) scale(x, sv(), a, x, sv(), bb, nullptr);
-    }
-    using Z = std::complex<double>;
-    std::vector<Z> H((size_t)nb * (m + 1) * m), g((size_t)nb * (m + 1)), cs((size_t)nb * m), sn((size_t)nb * m);
-    std::vector<int> jz(nb);
-    int it = 0;
-    while(true) {
-      matvec(x, r, active);
-      omx::vsub_b(r, b, r, Np, nb, sv(), c->st);
-      const std::vector<double> beta = nrms(r);
-      bool any = false;
-      for(int z = 0; z < nb; ++z) {
-        if(!active[z]) continue;
-        res[z] = beta[z] / bn[z];
-        if(res[z] <= tol || its[z] >= maxit || !(res[z] == res[z])) {
-          active[z] = 0;
-          continue;
-        }
-        if(prev[z] > 0.0 && beta[z] > 0.5 * prev[z]) {
-          // within the acceptance band one cycle without halving is the
-          // FP64 floor; further up, two
-          if(++stall[z] >= 2 || res[z] <= 1e3 * tol) {
-            active[z] = 0;
-            continue;
-          }
-        } else {
-          stall[z] = 0;
-        }
-        prev[z] = beta[z];
-        any = true;
-      }
-      if(!any || it >= maxit) break;
-      std::vector<int> live(active);  // systems still building this cycle's basis
-      {
-        std::vector<cplx> a(nb, zero), bb(nb, zero);
-        for(int z = 0; z < nb; ++z) a[z] = live[z] ? omx::mk(1.0 / beta[z]) : zero;
-        scale(V, sV, a, r, sv(), bb, nullptr);  // V_0 of every system
-      }
-      for(int z = 0; z < nb; ++z) {
-        std::fill(g.begin() + (size_t)z * (m + 1), g.begin() + (size_t)(z + 1) * (m + 1), Z(0.0));
-        g[(size_t)z * (m + 1)] = beta[z];
-        jz[z] = 0;
-      }
-      for(int j = 0; j < m && it < maxit; ++j, ++it) {
-        const cplx *vj = V + (size_t)j * ld;
-        cplx *zj = Zb + (size_t)j * ld;
-        precond(vj, zj, live);
-        matvec(zj, wv, live);
-        std::vector<cplx> h1((size_t)nb * sh), h2((size_t)nb * sh);
-        for(int pass = 0; pass < 2; ++pass) {
-          omx::dotc_multi_b(V, ld, sV, j + 1, wv, sv(), Np, nb, part, hd, sh, c->st);
-          omx::axpy_multi_b(V, ld, sV, j + 1, hd, sh, wv, sv(), Np, nb, c->st);
-          HIPCHK(hipMemcpyAsync(pass ? h2.data() : h1.data(), hd, sizeof(cplx) * nb * sh, hipMemcpyDeviceToHost,
-                                c->st));
-        }
-        const std::vector<double> hn = nrms(wv);
-        {
-          std::vector<cplx> a(nb, zero), bb(nb, zero);
-          for(int z = 0; z < nb; ++z) a[z] = (live[z] && hn[z] > 0.0) ? omx::mk(1.0 / hn[z]) : zero;
-          scale(V + (size_t)(j + 1) * ld, sV, a, wv, sv(), bb, nullptr);
-        }
-        bool any_live = false;
-        for(int z = 0; z < nb; ++z) {
-          if(!live[z]) continue;
-          Z *hc = &H[((size_t)z * m + j) * (m + 1)];
-          for(int i = 0; i <= j; ++i)
-            hc[i] = Z(h1[(size_t)z * sh + i].x + h2[(size_t)z * sh + i].x, h1[(size_t)z * sh + i].y + h2[(size_t)z * sh + i].y);
-          hc[j + 1] = hn[z];
-          Z *csz = &cs[(size_t)z * m], *snz = &sn[(size_t)z * m], *gz = &g[(size_t)z * (m + 1)];
-          for(int i = 0; i < j; ++i) {
-            Z t = csz[i] * hc[i] + snz[i] * hc[i + 1];
-            hc[i + 1] = -std::conj(snz[i]) * hc[i] + csz[i] * hc[i + 1];
-            hc[i] = t;
-          }
-          const double den = std::sqrt(std::norm(hc[j]) + std::norm(hc[j + 1]));
-          if(den == 0.0) {
-            csz[j] = 1.0;
-            snz[j] = 0.0;
-          } else {
-            const Z ph = std::abs(hc[j]) > 0 ? hc[j] / std::abs(hc[j]) : Z(1.0);
-            csz[j] = std::abs(hc[j]) / den;
-            snz[j] = ph * std::conj(hc[j + 1]) / den;
-          }
-          hc[j] = csz[j] * hc[j] + snz[j] * hc[j + 1];
-          hc[j + 1] = 0.0;
-          gz[j + 1] = -std::conj(snz[j]) * gz[j];
-          gz[j] = csz[j] * gz[j];
-          jz[z] = j + 1;
-          ++its[z];
-          if(std::abs(gz[j + 1]) <= 0.5 * tol * bn[z] || hn[z] == 0.0 || its[z] >= maxit)
-            live[z] = 0;  // its later basis vectors are zero
-          else
-            any_live = true;
-        }
-        if(!any_live) {
-          ++it;
-          break;
-        }
-      }
-      // y_z = H_z^{-1} g_z, x_z += Z_z y_z (= M^{-1} V_z y_z)
-      int jmax = 0;
-      std::vector<cplx> yh((size_t)nb * sh, zero);
-      for(int z = 0; z < nb; ++z) {
-        if(!active[z]) continue;
-        const int jj = jz[z];
-        jmax = std::max(jmax, jj);
-        std::vector<Z> y(jj);
-        for(int i = jj - 1; i >= 0; --i) {
-          Z sacc = g[(size_t)z * (m + 1) + i];
-          for(int k = i + 1; k < jj; ++k) sacc -= H[((size_t)z * m + k) * (m + 1) + i] * y[k];
-          y[i] = sacc / H[((size_t)z * m + i) * (m + 1) + i];
-        }
-        for(int i = 0; i < jj; ++i) yh[(size_t)z * sh + i] = omx::mk(y[i].real(), y[i].imag());
-      }
-      if(jmax == 0) break;
-      HIPCHK(hipMemcpyAsync(hd, yh.data(), sizeof(cplx) * nb * sh, hipMemcpyHostToDevice, c->st));
-      omx::gemv_multi_b(Zb, ld, sV, jmax, hd, sh, wv, sv(), Np, nb, c->st);
-      std::vector<int> act_h(active);
-      HIPCHK(hipMemcpyAsync(act_d, act_h.data(), sizeof(int) * nb, hipMemcpyHostToDevice, c->st));
-      scale(x, sv(), std::vector<cplx>(nb, one), wv, sv(), std::vector<cplx>(nb, one), act_d);
-      // a correction below the FP64 resolution of x ends that system's refinement
-      const std::vector<double> dn = nrms(wv), xn = nrms(x);
-      for(int z = 0; z < nb; ++z)
-        if(active[z] && dn[z] <= 1e-16 * xn[z]) active[z] = 0;
-    }
-  }
-};
 
 // Buffers of a batch of nb systems of order Np (mixed: FP32 copies too).
 // Enqueues V's factorisation from a host thread of its own: the enqueueing
@@ -1431,7 +1257,6 @@ void sweep_alloc(omx_context *c, int nb, bool f64, bool sh) {
   for(DBuf *b : {&w.dinv, &w.dinv2}) b->ensure(sizeof(cplx) * omx::dinv_elems(Np) * nb, T);
   w.map.ensure(sizeof(int) * 3 * (Np + 2 * omx::kNB) * nb, T);
   w.status.ensure(sizeof(int) * 4 * nb, T);
-  w.sys.ensure(sizeof(int) * nb, T);
   if(sh) {  // V's factorisation runs beside S's: maps and status words of its own
     w.map2.ensure(sizeof(int) * 3 * (Np + 2 * omx::kNB) * nb, T);
     w.status2.ensure(sizeof(int) * 4 * nb, T);
@@ -1439,11 +1264,6 @@ void sweep_alloc(omx_context *c, int nb, bool f64, bool sh) {
   w.basis.ensure(sizeof(cplx) * Np * (m + 1) * nb, T);
   w.basisZ.ensure(sizeof(cplx) * Np * (m + 1) * nb, T);
   w.gpart.ensure(sizeof(cplx) * Np * omx::kGemvSplitMax * nb, T);
-  w.part.ensure(sizeof(cplx) * 128 * (m + 2) * nb, T);
-  w.hd.ensure(sizeof(cplx) * (m + 2) * nb, T);
-  w.nrm.ensure(sizeof(double) * 160 * nb, T);
-  w.sc.ensure(sizeof(cplx) * 2 * nb, T);
-  w.act.ensure(sizeof(int) * nb, T);
   w.kz.ensure(sizeof(cplx) * 2 * nb, T);
   w.omz.ensure(sizeof(double) * nb, T);
 }
@@ -1480,6 +1300,21 @@ omx::LuWork sweep_lu(omx_context *c, int nb, bool second) {
   lw.bs.cnt = ms;
   lw.bs.status = 4;
   return lw;
+}
+
+// The lockstep iteration of a batch on the FP64 matrices A (Np^2 apart), in the
+// sweep's buffers: basis vector k of system z at V + (k nb + z) Np.
+Krylov sweep_krylov(omx_context *c, int nb, const cplx *A) {
+  auto &w = c->sw;
+  Krylov gm{c,     c->Np,
+            nb,    c->st,
+            w.kry, w.basis.as<cplx>(),
+            w.basisZ.as<cplx>(), w.r.as<cplx>(),
+            w.w1.as<cplx>(),     w.gpart.as<cplx>()};
+  gm.A = A;
+  gm.sA = (size_t)c->Np * c->Np;
+  gm.batch = true;
+  return gm;
 }
 
 // ------------------------------------------------------------------ autotuner
@@ -1657,10 +1492,6 @@ void sweep_chunk(omx_context *c, int nb, const double *lam, const cplx *eps, con
   HIPCHK(hipMemcpyAsync(w.eps_sh.p, eps_sh, sizeof(cplx) * P * nb, hipMemcpyHostToDevice, st));
   HIPCHK(hipMemsetAsync(w.status.p, 0, w.status.bytes, st));
   if(sh) HIPCHK(hipMemsetAsync(w.status2.p, 0, w.status2.bytes, st));
-  // the lockstep refinement leaves the vectors of systems that dropped out
-  // as they are: start them finite
-  HIPCHK(hipMemsetAsync(w.basisZ.p, 0, w.basisZ.bytes, st));
-  HIPCHK(hipMemsetAsync(w.w1.p, 0, w.w1.bytes, st));
   HIPCHK(hipMemsetAsync(w.Q.p, 0, w.Q.bytes, st));
   HIPCHK(hipMemsetAsync(c->d_status.p, 0, 16, st));
   const cplx bge = kEps0 * c->bg_eps_r, bgm = kMu0 * c->bg_mu_r;
@@ -1824,30 +1655,26 @@ void sweep_chunk(omx_context *c, int nb, const double *lam, const cplx *eps, con
   auto refine = [&](bool second, omx::LuWork &lw, void *F, const cplx *rhs, cplx *x, bool from_x = false) {
     status_scan(bad, second);
     cplx *A64 = second ? cV64 : cS64;
-    omx::LuWork *lwp = &lw;
-    GmresB gm{c, A64, n2, Np, nb, nullptr, w};
-    gm.lw = lwp;
-    if(f64)
-      gm.prec = [c, F, lwp, Np, lda](const cplx *in, cplx *out) {
-        omx::lu_solve<double2>(static_cast<const double2 *>(F), Np, lda, *lwp, in, out, c->st);
-      };
-    else
-      gm.prec = [c, F, lwp, Np, lda](const cplx *in, cplx *out) {
-        omx::lu_solve<float2>(static_cast<const float2 *>(F), Np, lda, *lwp, in, out, c->st);
-      };
-    if(!from_x) gm.prec(rhs, x);  // else: start from the iterate x holds
-    std::vector<double> res;
-    std::vector<int> its;
+    Krylov gm = sweep_krylov(c, nb, A64);
+    gm.prec = [c, F, &lw, Np, lda, f64](const cplx *in, cplx *out, const int *live) {
+      lw.live = live;
+      if(f64)
+        omx::lu_solve<double2>(static_cast<const double2 *>(F), Np, lda, lw, in, out, c->st);
+      else
+        omx::lu_solve<float2>(static_cast<const float2 *>(F), Np, lda, lw, in, out, c->st);
+      lw.live = nullptr;
+    };
+    if(!from_x) gm.prec(rhs, x, nullptr);  // else: start from the iterate x holds
     // the batch runs in lockstep until its slowest system stops: a system
     // still short of the target after four restart cycles is left to the
     // one-at-a-time path (partial pivoting) instead of holding the batch
     const int bmax = nb > 1 ? std::min(c->maxit, 4 * c->restart) : c->maxit;
-    gm.solve(rhs, x, c->tol, bmax, c->restart, res, its);
+    gm.solve(rhs, x, c->tol, bmax, c->restart);
     status_scan(bad, second);
     for(int z = 0; z < nb; ++z) {
-      if(!(res[z] <= 1e3 * c->tol)) bad[z] = 1;
-      iters[2 * z + (second ? 1 : 0)] = its[z];
-      resid[2 * z + (second ? 1 : 0)] = res[z];
+      if(!(gm.res[z] <= 1e3 * c->tol)) bad[z] = 1;
+      iters[2 * z + (second ? 1 : 0)] = gm.its[z];
+      resid[2 * z + (second ? 1 : 0)] = gm.res[z];
     }
   };
   if(krylov_s) {
@@ -1855,19 +1682,17 @@ void sweep_chunk(omx_context *c, int nb, const double *lam, const cplx *eps, con
     // single-system budget (S's solve runs beside V's factorisation); a
     // system short of the target is left to the one-at-a-time path
     status_scan(bad, false);
-    GmresB gm{c, cS64, n2, Np, nb, nullptr, w};
+    Krylov gm = sweep_krylov(c, nb, cS64);
     cplx *Sx = w.x.as<cplx>();
-    gm.prec = [c, Np, nb](const cplx *in, cplx *out) { omx::vcopy(out, in, Np * nb, c->st); };
+    gm.x_zero = true;
     HIPCHK(hipMemsetAsync(Sx, 0, sizeof(cplx) * lda * nb, st));
-    std::vector<double> res;
-    std::vector<int> its;
     const int budget = std::min(c->maxit, c->auto_budget > 0 ? c->auto_budget : 2 * auto_gmres64_steps(c->N));
-    gm.solve(w.Q.as<cplx>(), Sx, c->tol, budget, c->restart, res, its);
+    gm.solve(w.Q.as<cplx>(), Sx, c->tol, budget, c->restart);
     bool short_any = false;
     for(int z = 0; z < nb; ++z) {
-      short_any |= !(res[z] <= 1e3 * c->tol);
-      iters[2 * z] = its[z];
-      resid[2 * z] = res[z];
+      short_any |= !(gm.res[z] <= 1e3 * c->tol);
+      iters[2 * z] = gm.its[z];
+      resid[2 * z] = gm.res[z];
     }
     if(short_any) {
       // S factored for the batch after all; every system refined from its
@@ -2036,8 +1861,6 @@ int omx_create(omx_context **out, int device) {
       for(auto &e : c->uev) HIPCHK(hipEventCreate(&e));
       for(hipEvent_t *e : {&c->geo_ev, &c->ujoin[0], &c->ujoin[1]})
         HIPCHK(hipEventCreateWithFlags(e, hipEventDisableTiming));
-      c->d_coef.ensure(sizeof(double) * omx::CF_COUNT * omx::kCoefStride, &c->total);
-      omx::fill_coef(c->d_coef.as<double>(), c->st);
       omx::upload_factorials();
       c->scratch = scratch_address(device);
     } catch(...) {
@@ -2061,7 +1884,7 @@ void omx_destroy(omx_context *c) {
                   &c->d_S32, &c->d_V64, &c->d_V32, &c->d_x, &c->d_xsh, &c->d_xint, &c->d_xintsh, &c->d_K,
                   &c->d_K1, &c->d_cross, &c->d_cg, &c->d_perm, &c->d_cand, &c->d_map,
                   &c->d_wlu, &c->d_status, &c->d_basis, &c->d_basisZ, &c->d_w1, &c->d_w2, &c->d_r,
-                  &c->d_part, &c->d_h, &c->d_nrm, &c->d_gpart, &c->d_perm2,
+                  &c->d_nrm, &c->d_gpart, &c->d_perm2,
                   &c->d_dinv, &c->d_dinv2, &c->d_F64, &c->d_F64sh, &c->d_abscoef, &c->d_abssh, &c->d_absbes,
                   &c->d_fpts, &c->d_fout, &c->d_fown, &c->d_fpart};
   for(DBuf *b : bufs) b->release(&c->total);
@@ -2069,11 +1892,13 @@ void omx_destroy(omx_context *c) {
   DBuf *sbufs[] = {&w.S64, &w.S32, &w.V64, &w.V32, &w.F64, &w.F64sh, &w.eps, &w.eps_sh, &w.ov, &w.incloc, &w.Q,
                    &w.w, &w.x, &w.xint, &w.xsh, &w.xintsh, &w.K, &w.K1, &w.cross, &w.perm, &w.perm2,
                    &w.dinv, &w.dinv2, &w.map, &w.status, &w.basis, &w.basisZ, &w.r, &w.w1, &w.w2, &w.gpart,
-                   &w.part, &w.hd, &w.nrm, &w.sc, &w.act, &w.abscoef, &w.abssh, &w.absbes, &w.kz, &w.omz};
+                   &w.abscoef, &w.abssh, &w.absbes, &w.kz, &w.omz};
   for(DBuf *b : sbufs) b->release(&c->total);
   c->aca[0].release(&c->total);
   c->aca[1].release(&c->total);
   c->ws_in.release(&c->total);
+  c->kry.release(&c->total);
+  w.kry.release(&c->total);
   DBuf *abufs[] = {&c->d_acaA, &c->d_acaU, &c->d_acaV, &c->d_acaR, &c->d_acaOff, &c->d_plist};
   for(DBuf *b : abufs) b->release(&c->total);
   for(auto &e : c->ev)
@@ -2094,8 +1919,8 @@ void omx_destroy(omx_context *c) {
   if(c->st2) (void)hipStreamDestroy(c->st2);
   if(c->aux) (void)hipStreamDestroy(c->aux);
   if(c->st) (void)hipStreamDestroy(c->st);
-  if(c->h_pin) (void)hipHostFree(c->h_pin);
   if(c->geo_pin) (void)hipHostFree(c->geo_pin);
+  if(c->out_pin) (void)hipHostFree(c->out_pin);
   delete c;
 }
 
@@ -2367,6 +2192,27 @@ void sh_source(omx_context *c, hipStream_t st) {
   omx::run_shsrc(sa, st);
 }
 
+// The solution vectors to the caller's arrays (null: left out), after all of the
+// context's work on its first stream: through pinned staging, so that the
+// copies take one wait between them.
+void read_vectors(omx_context *c, double *x_sca, double *x_int, double *x_sca_sh, double *x_int_sh) {
+  double *dst[] = {x_sca, x_int, c->sh ? x_sca_sh : nullptr, c->sh ? x_int_sh : nullptr};
+  const DBuf *src[] = {&c->d_x, &c->d_xint, &c->d_xsh, &c->d_xintsh};
+  const size_t b = sizeof(cplx) * c->N;
+  if(c->out_pin_bytes < 4 * b) {
+    if(c->out_pin) (void)hipHostFree(c->out_pin);
+    c->out_pin = nullptr;
+    c->out_pin_bytes = 0;
+    HIPCHK(hipHostMalloc(reinterpret_cast<void **>(&c->out_pin), 4 * b));
+    c->out_pin_bytes = 4 * b;
+  }
+  for(int e = 0; e < 4; ++e)
+    if(dst[e]) HIPCHK(hipMemcpyAsync(c->out_pin + e * b, src[e]->p, b, hipMemcpyDeviceToHost, c->st));
+  HIPCHK(hipStreamSynchronize(c->st));
+  for(int e = 0; e < 4; ++e)
+    if(dst[e]) std::memcpy(dst[e], c->out_pin + e * b, b);
+}
+
 int omx_solve(omx_context *c, double *x_sca, double *x_int, double *x_sca_sh, double *x_int_sh) {
   return guard([&] {
     if(!c || !c->updated) throw OmxError(OMX_ERR_STATE, "omx_update must precede omx_solve");
@@ -2446,8 +2292,6 @@ int omx_solve(omx_context *c, double *x_sca, double *x_int, double *x_sca_sh, do
     // X_int = X_sca (.) Iaux (Solver.cpp:57-77)
     omx::vmul_ov(c->d_xint.as<cplx>(), c->d_x.as<cplx>(), c->d_ov.as<cplx>(), omx::OV_IAUX, P, nmax, nullptr, N, c->st);
     HIPCHK(hipEventRecord(c->ev[2], c->st));
-    HIPCHK(hipEventSynchronize(c->ev[2]));
-    ts += elapsed(c, 0, 2);
     if(c->sh) {
       ensure_cg(c, c->st);
       HIPCHK(hipEventRecord(c->ev[3], c->st));
@@ -2465,24 +2309,17 @@ int omx_solve(omx_context *c, double *x_sca, double *x_int, double *x_sca_sh, do
       HIPCHK(hipEventRecord(c->xev[2], c->st2));
       HIPCHK(hipStreamWaitEvent(c->st, c->xev[2], 0));
       HIPCHK(hipEventRecord(c->ev[5], c->st));
-      HIPCHK(hipEventSynchronize(c->ev[5]));
+    }
+    HIPCHK(hipGetLastError());
+    read_vectors(c, x_sca, x_int, x_sca_sh, x_int_sh);
+    ts += elapsed(c, 0, 2);
+    if(c->sh) {
       tsh = elapsed(c, 3, 4);
       ts += elapsed(c, 4, 5);
     }
-    HIPCHK(hipGetLastError());
     c->stats.t_factor_ms = tf;
     c->stats.t_solve_ms = ts;
     c->stats.t_sh_source_ms = tsh;
-    auto cp = [&](double *dst, const DBuf &b) {
-      if(dst) HIPCHK(hipMemcpyAsync(dst, b.p, sizeof(cplx) * N, hipMemcpyDeviceToHost, c->st));
-    };
-    cp(x_sca, c->d_x);
-    cp(x_int, c->d_xint);
-    if(c->sh) {
-      cp(x_sca_sh, c->d_xsh);
-      cp(x_int_sh, c->d_xintsh);
-    }
-    HIPCHK(hipStreamSynchronize(c->st));
     c->solved = true;
   });
 }
@@ -2507,15 +2344,9 @@ void group_alloc(omx_context *L, int nb, bool f64, bool sh) {
   for(DBuf *b : {&w.dinv, &w.dinv2}) b->ensure(sizeof(cplx) * omx::dinv_elems(Np) * nb, T);
   for(DBuf *b : {&w.map, &w.map2}) b->ensure(sizeof(int) * 3 * (Np + 2 * omx::kNB) * nb, T);
   for(DBuf *b : {&w.status, &w.status2}) b->ensure(sizeof(int) * 4 * nb, T);
-  w.sys.ensure(sizeof(int) * nb, T);
   w.basis.ensure(sizeof(cplx) * Np * (m + 1) * nb, T);
   w.basisZ.ensure(sizeof(cplx) * Np * (m + 1) * nb, T);
   w.gpart.ensure(sizeof(cplx) * Np * omx::kGemvSplitMax * nb, T);
-  w.part.ensure(sizeof(cplx) * 128 * (m + 2) * nb, T);
-  w.hd.ensure(sizeof(cplx) * (m + 2) * nb, T);
-  w.nrm.ensure(sizeof(double) * 160 * nb, T);
-  w.sc.ensure(sizeof(cplx) * 2 * nb, T);
-  w.act.ensure(sizeof(int) * nb, T);
   L->d_status.ensure(64, T);
 }
 
@@ -2569,7 +2400,7 @@ int omx_solve_group(omx_context *L, int n, omx_context *const *mem) {
     const TuneChoice tune = L->autotune ? sweep_tune(L, nb, f64) : TuneChoice{L->lu32_gemm == OMX_GEMM_BF16X3, 0};
     auto &w = L->sw;
     hipStream_t st = L->st;
-    for(DBuf *b : {&w.status, &w.status2, &w.basisZ, &w.w1}) HIPCHK(hipMemsetAsync(b->p, 0, b->bytes, st));
+    for(DBuf *b : {&w.status, &w.status2}) HIPCHK(hipMemsetAsync(b->p, 0, b->bytes, st));
     HIPCHK(hipMemsetAsync(L->d_status.p, 0, 16, st));
     // the members' matrices and right-hand sides, bordered by the identity
     cplx *S64 = w.S64.as<cplx>(), *V64 = sh ? w.V64.as<cplx>() : nullptr;
@@ -2621,27 +2452,23 @@ int omx_solve_group(omx_context *L, int n, omx_context *const *mem) {
     };
     auto refine = [&](bool second, omx::LuWork &lw, void *F, const cplx *A64, const cplx *rhs, cplx *x) {
       status_scan(second);
-      omx::LuWork *lwp = &lw;
-      GmresB gm{L, A64, n2, Np, nb, nullptr, w};
-      gm.lw = lwp;
-      if(f64)
-        gm.prec = [L, F, lwp, Np, lda](const cplx *in, cplx *out) {
-          omx::lu_solve<double2>(static_cast<const double2 *>(F), Np, lda, *lwp, in, out, L->st);
-        };
-      else
-        gm.prec = [L, F, lwp, Np, lda](const cplx *in, cplx *out) {
-          omx::lu_solve<float2>(static_cast<const float2 *>(F), Np, lda, *lwp, in, out, L->st);
-        };
-      gm.prec(rhs, x);
-      std::vector<double> res;
-      std::vector<int> its;
+      Krylov gm = sweep_krylov(L, nb, A64);
+      gm.prec = [L, F, &lw, Np, lda, f64](const cplx *in, cplx *out, const int *live) {
+        lw.live = live;
+        if(f64)
+          omx::lu_solve<double2>(static_cast<const double2 *>(F), Np, lda, lw, in, out, L->st);
+        else
+          omx::lu_solve<float2>(static_cast<const float2 *>(F), Np, lda, lw, in, out, L->st);
+        lw.live = nullptr;
+      };
+      gm.prec(rhs, x, nullptr);
       const int bmax = nb > 1 ? std::min(L->maxit, 4 * L->restart) : L->maxit;
-      gm.solve(rhs, x, L->tol, bmax, L->restart, res, its);
+      gm.solve(rhs, x, L->tol, bmax, L->restart);
       status_scan(second);
       for(int z = 0; z < nb; ++z) {
-        if(!(res[z] <= 1e3 * L->tol)) bad[z] = 1;
-        iters[2 * z + (second ? 1 : 0)] = its[z];
-        resid[2 * z + (second ? 1 : 0)] = res[z];
+        if(!(gm.res[z] <= 1e3 * L->tol)) bad[z] = 1;
+        iters[2 * z + (second ? 1 : 0)] = gm.its[z];
+        resid[2 * z + (second ? 1 : 0)] = gm.res[z];
       }
     };
     // fundamental: S x = Q for every member, then each member's x and x_int
@@ -2697,16 +2524,7 @@ int omx_read_solution(omx_context *c, double *x_sca, double *x_int, double *x_sc
   return guard([&] {
     if(!c || !c->solved) throw OmxError(OMX_ERR_STATE, "no solution: omx_solve or omx_solve_group first");
     HIPCHK(hipSetDevice(c->device));
-    auto cp = [&](double *dst, const DBuf &b) {
-      if(dst) HIPCHK(hipMemcpyAsync(dst, b.p, sizeof(cplx) * c->N, hipMemcpyDeviceToHost, c->st));
-    };
-    cp(x_sca, c->d_x);
-    cp(x_int, c->d_xint);
-    if(c->sh) {
-      cp(x_sca_sh, c->d_xsh);
-      cp(x_int_sh, c->d_xintsh);
-    }
-    HIPCHK(hipStreamSynchronize(c->st));
+    read_vectors(c, x_sca, x_int, x_sca_sh, x_int_sh);
   });
 }
 
@@ -2941,8 +2759,6 @@ int omx_dense_solve(omx_context *c, int N, const double *A, const double *b, dou
     ctx.d_w1.ensure(sizeof(cplx) * Np, &ctx.total);
     ctx.d_w2.ensure(sizeof(cplx) * Np, &ctx.total);
     ctx.d_gpart.ensure(sizeof(cplx) * Np * omx::kGemvSplitMax, &ctx.total);
-    ctx.d_part.ensure(sizeof(cplx) * 128 * (ctx.restart + 2), &ctx.total);
-    ctx.d_h.ensure(sizeof(cplx) * 2 * (ctx.restart + 2), &ctx.total);
     ctx.d_nrm.ensure(sizeof(double) * 256, &ctx.total);
     alloc_matrices(&ctx);
     HIPCHK(hipMemsetAsync(ctx.d_Q.p, 0, sizeof(cplx) * Np, ctx.st));

@@ -203,8 +203,7 @@ struct LuWork {
   int pivot;            // kPivotBlock or kPivotPartial
   int nb = 1;           // systems in the batch (block pivoting only when > 1)
   BatchStrides bs;      // their strides; the pointers above are system 0's
-  const int *sys = nullptr;  // lu_solve on a subset: its nsys systems' indices (null: all nb)
-  int nsys = 0;
+  const int *live = nullptr;  // lu_solve: systems whose flag (KF_COUNT ints apart) is 0 are left out (null: none)
   int trsv = 0;              // triangular-solve variant (kTrsvVariants; 0: the default)
   bool split = true;             // FP32 factors: bulk updates on the split-bf16 MFMA
   hipEvent_t ev_mark = nullptr;  // when set: recorded on the bulk stream once the
@@ -247,15 +246,50 @@ template <typename T>
 void lu_solve(const T *A, int Np, size_t lda, LuWork &w, const cplx *b, cplx *x, hipStream_t st);
 
 // ---------------------------------------------------------------- iterative
-// (sys non-null: only the nsys systems it lists)
-void gemv64(const cplx *A, size_t lda, int N, const cplx *x, cplx *y, cplx *part, hipStream_t st, int nb = 1,
-            size_t sA = 0, size_t sv = 0, const int *sys = nullptr, int nsys = 0);
-// y = A x with A the complex-FP32 copy (FP64 vectors and sums); part as gemv64's
-void gemv32(const float2 *A, size_t lda, int N, const cplx *x, cplx *y, cplx *part, hipStream_t st);
+// Partial sums of y = A x for nb systems (matrices sA, vectors sv apart), or of
+// its complex-FP32 copy (FP64 vectors and sums): part[z][k][N], k < the returned
+// number of column parts (<= kGemvSplitMax), chosen for `live` working systems.
+// Systems whose flag (KF_COUNT ints apart; null: all) is 0 are left out.
+int gemv_partial(const cplx *A, size_t lda, int N, const cplx *x, cplx *part, hipStream_t st, int nb = 1,
+                 size_t sA = 0, size_t sv = 0, const int *flag = nullptr, int live = 1);
+int gemv_partial(const float2 *A, size_t lda, int N, const cplx *x, cplx *part, hipStream_t st,
+                 const int *flag = nullptr);
 constexpr int kGemvSplitMax = 32;
 
-// level-1 helpers (omx_iter.hip); reductions return through small device arrays
-void vcopy(cplx *y, const cplx *x, int n, hipStream_t st);
+// GMRES with its small algebra on the device (omx_krylov.hip), nb systems in
+// lockstep: the state of each, and the vectors they share.
+enum { KF_LIVE = 0, KF_ACTIVE, KF_J, KF_ITS, KF_STALL, KF_TINY, KF_COUNT = 8 };  // flags, ints
+enum { KS_BN = 0, KS_PREV, KS_RES, KS_COUNT = 4 };                              // scalars, doubles
+struct KryState {
+  int n, m, nb, j;     // order, restart length (<= 256), systems, step of the cycle
+  double tol;
+  int maxit;
+  cplx *c;             // [nb][kry_cplx(m)]: Hessenberg columns, g, rotations, y, h
+  double *sc;          // [nb][KS_COUNT]
+  int *fl;             // [nb][KF_COUNT]
+  cplx *part;          // [2][nb][kry_blocks(n)][m + 2]
+  double *pnrm;        // [2][nb][kry_blocks(n)]
+  cplx *V;             // basis: vector k of system z at V + k ldk + z sz
+  const cplx *Z;       // preconditioned basis, laid out alike (V itself without one)
+  size_t ldk, sz;
+  cplx *r, *w;         // residual and work vector, system z at + z sv (as b and x)
+  size_t sv;
+};
+__host__ __device__ inline size_t kry_cplx(int m) {
+  return (size_t)m * (m + 1) + (m + 1) + 3 * (size_t)m + (m + 2);
+}
+int kry_blocks(int n);
+// Arnoldi step s.j after its product: partial sums gpart + z sg + k n, k < ns, or
+// the product itself in s.w (ns 0).  host (pinned, [nb][2]): the system goes on,
+// and the binary digits that its residual has to fall to the goal.
+void kry_step(const KryState &s, const cplx *gpart, int ns, size_t sg, int *host, hipStream_t st);
+void kry_end_cycle(const KryState &s, cplx *x, bool tiny, bool batch, hipStream_t st);
+// b - A x and the restart's decisions; ns as above, 0: no product (x = 0), -1:
+// the product is in s.w
+void kry_restart(const KryState &s, const cplx *b, cplx *x, const cplx *gpart, int ns, size_t sg, bool first,
+                 bool batch, int *host, hipStream_t st);
+
+// level-1 helpers (omx_iter.hip)
 void demote(float2 *y, const cplx *x, size_t n, hipStream_t st);                 // y = (c64) x
 // p[0..n) = 0 by a kernel (a memset node must not go into a captured graph)
 void zero_ints(int *p, int n, hipStream_t st);
@@ -264,28 +298,8 @@ void zero_ints(int *p, int n, hipStream_t st);
 void pad_matrix64(cplx *dst, int Nd, const cplx *src, int Ns, hipStream_t st);
 void pad_matrix32(float2 *dst, int Nd, const cplx *src, int Ns, hipStream_t st);
 void pad_vector(cplx *dst, int Nd, const cplx *src, int Ns, hipStream_t st);
-void vaxpby(cplx *y, cplx a, const cplx *x, cplx b, int n, hipStream_t st);   // y = a x + b y
-void vsub(cplx *z, const cplx *x, const cplx *y, int n, hipStream_t st);      // z = x - y
 void vmul_ov(cplx *y, const cplx *x, const cplx *ov, int kind, int P, int nmax, const cplx *sub, int n,
              hipStream_t st);                                                  // y = x (.) ov[kind] - sub
-void dotc_multi(const cplx *V, size_t ldv, int nv, const cplx *w, int n, cplx *part, cplx *out,
-                hipStream_t st);                                               // out[k] = V_k^H w
-void axpy_multi(const cplx *V, size_t ldv, int nv, const cplx *h, cplx *w, int n, hipStream_t st); // w -= V h
-void gemv_multi(const cplx *V, size_t ldv, int nv, const cplx *h, cplx *z, int n, hipStream_t st); // z = V h
 void nrm2sq(const cplx *x, int n, double *part, double *out, hipStream_t st);
-// the same for nb systems side by side (vectors sv, sy, sx apart, bases sV apart,
-// per-system scalars a[z], b[z], coefficient vectors sh apart, outputs so apart);
-// act (may be null) skips the systems whose flag is 0
-void vaxpby_b(cplx *y, size_t sy, const cplx *a, const cplx *x, size_t sx, const cplx *b, int n, int nb,
-              const int *act, hipStream_t st);
-void vsub_b(cplx *z, const cplx *x, const cplx *y, int n, int nb, size_t sv, hipStream_t st);
-int red_blocks_b(int n, int nb);  // partial sums per system of the reductions below
-void dotc_multi_b(const cplx *V, size_t ldv, size_t sV, int nv, const cplx *w, size_t sv, int n, int nb, cplx *part,
-                  cplx *out, int so, hipStream_t st);
-void axpy_multi_b(const cplx *V, size_t ldv, size_t sV, int nv, const cplx *h, int sh, cplx *w, size_t sv, int n,
-                  int nb, hipStream_t st);
-void gemv_multi_b(const cplx *V, size_t ldv, size_t sV, int nv, const cplx *h, int sh, cplx *z, size_t sv, int n,
-                  int nb, hipStream_t st);
-void nrm2sq_b(const cplx *x, size_t sv, int n, int nb, double *part, double *out, hipStream_t st);
 
 }  // namespace omx

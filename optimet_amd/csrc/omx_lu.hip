@@ -1429,8 +1429,9 @@ __device__ inline double with_tag(double v, unsigned tg) {
 }
 // The permuted right-hand side, with the tag bits cleared: a word the
 // triangular solves have not yet published can never carry their tag.
-__global__ void gather_kernel(const cplx *b, const int *perm, cplx *y, int Np, BatchStrides bs, const int *sys) {
-  const size_t z = sys ? sys[blockIdx.z] : blockIdx.z;
+__global__ void gather_kernel(const cplx *b, const int *perm, cplx *y, int Np, BatchStrides bs, const int *live) {
+  const size_t z = blockIdx.z;
+  if(live && !live[z * KF_COUNT]) return;
   b += z * bs.vec;
   y += z * bs.vec;
   perm += z * bs.perm;
@@ -1465,10 +1466,11 @@ __global__ void gather_kernel(const cplx *b, const int *perm, cplx *y, int Np, B
 template <typename T, bool LOWER, int SB, int PRE>
 __global__ __launch_bounds__(256) void trsv_kernel(const T *__restrict__ A, size_t lda, int Np,
                                                    const T *__restrict__ dinv, cplx *x,
-                                                   int *status, BatchStrides bs, const int *sys) {
+                                                   int *status, BatchStrides bs, const int *live) {
   constexpr int NB = kNB;
   constexpr int NI = SB * (SB - 1) / 2;
-  const size_t zs = sys ? sys[blockIdx.z] : blockIdx.z;  // the system (a subset may be listed)
+  const size_t zs = blockIdx.z;
+  if(live && !live[zs * KF_COUNT]) return;  // the whole system: no workgroup waits for it
   A += zs * bs.a;
   dinv += zs * bs.inv;
   x += zs * bs.vec;
@@ -1695,16 +1697,15 @@ static void trsv_pair(const T *A, int Np, size_t lda, LuWork &w, cplx *x, int nz
   const T *dinv = reinterpret_cast<const T *>(w.dinv);
   const int nblk = Np / kNB, nsb = (nblk + SB - 1) / SB;
   hipLaunchKernelGGL((trsv_kernel<T, true, SB, PRE>), dim3(nsb, 1, nz), dim3(256), 0, st, A, lda, Np, dinv, x,
-                     w.status, w.bs, w.sys);
+                     w.status, w.bs, w.live);
   hipLaunchKernelGGL((trsv_kernel<T, false, SB, PRE>), dim3(nsb, 1, nz), dim3(256), 0, st, A, lda, Np, dinv, x,
-                     w.status, w.bs, w.sys);
+                     w.status, w.bs, w.live);
 }
 
 template <typename T>
 void lu_solve(const T *A, int Np, size_t lda, LuWork &w, const cplx *b, cplx *x, hipStream_t st) {
-  const int nz = w.sys ? w.nsys : w.nb;
-  if(nz < 1) return;
-  hipLaunchKernelGGL(gather_kernel, dim3((Np + 255) / 256, 1, nz), dim3(256), 0, st, b, w.perm, x, Np, w.bs, w.sys);
+  const int nz = w.nb;
+  hipLaunchKernelGGL(gather_kernel, dim3((Np + 255) / 256, 1, nz), dim3(256), 0, st, b, w.perm, x, Np, w.bs, w.live);
   switch(w.trsv) {
   case 1: trsv_pair<T, 1>(A, Np, lda, w, x, nz, st); break;
   case 2: trsv_pair<T, 2>(A, Np, lda, w, x, nz, st); break;
@@ -1732,8 +1733,9 @@ constexpr int kGemvSplit = 32;
 template <typename T>
 __global__ __launch_bounds__(256) void gemv_part_kernel(const T *__restrict__ A, size_t lda, int N,
                                                         const cplx *__restrict__ x, cplx *part, int chunk, size_t sA,
-                                                        size_t sv, const int *sys) {
-  const size_t zs = sys ? sys[blockIdx.z] : blockIdx.z;
+                                                        size_t sv, const int *flag) {
+  const size_t zs = blockIdx.z;
+  if(flag && !flag[zs * KF_COUNT]) return;
   A += zs * sA;
   x += zs * sv;
   part += (size_t)blockIdx.z * gridDim.y * N;
@@ -1760,17 +1762,6 @@ __global__ __launch_bounds__(256) void gemv_part_kernel(const T *__restrict__ A,
   }
   if(r < N) part[(size_t)blockIdx.y * N + r] = acc;
 }
-__global__ void gemv_reduce_kernel(const cplx *part, int ns, int N, cplx *y, size_t sv, const int *sys) {
-  part += (size_t)blockIdx.z * ns * N;
-  y += (sys ? sys[blockIdx.z] : blockIdx.z) * sv;
-  int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if(r >= N) return;
-  cplx s = mk(0.0);
-  for(int k = 0; k < ns; ++k) s = s + part[(size_t)k * N + r];
-  y[r] = s;
-}
-// y = A x for nb systems (matrices sA, vectors sv apart); part holds
-// kGemvSplit N partial vectors per system
 // Column parts of a batched product: the fewest (the longest runs of
 // columns, the fewest partial vectors) that still give 1280 workgroups, about
 // five per CU.  Measured on 3840 x 3840 systems: 6.75 TB/s with 8 parts for 64
@@ -1783,22 +1774,18 @@ inline int gemv_parts(int N, int nz) {
     if(rb * nz * s >= 1280) return s;
   return kGemvSplit;
 }
-void gemv64(const cplx *A, size_t lda, int N, const cplx *x, cplx *y, cplx *part, hipStream_t st, int nb, size_t sA,
-            size_t sv, const int *sys, int nsys) {
-  const int nz = sys ? nsys : nb;
-  if(nz < 1) return;
-  const int ns = gemv_parts(N, nz);  // <= kGemvSplit: part holds kGemvSplit N vectors per system
-  int chunk = (N + ns - 1) / ns;
-  hipLaunchKernelGGL(gemv_part_kernel<cplx>, dim3((N + 255) / 256, ns, nz), dim3(256), 0, st, A, lda, N, x, part,
-                     chunk, sA, sv, sys);
-  hipLaunchKernelGGL(gemv_reduce_kernel, dim3((N + 255) / 256, 1, nz), dim3(256), 0, st, part, ns, N, y, sv, sys);
+int gemv_partial(const cplx *A, size_t lda, int N, const cplx *x, cplx *part, hipStream_t st, int nb, size_t sA,
+                 size_t sv, const int *flag, int live) {
+  const int ns = gemv_parts(N, live), chunk = (N + ns - 1) / ns;  // ns <= kGemvSplitMax
+  hipLaunchKernelGGL(gemv_part_kernel<cplx>, dim3((N + 255) / 256, ns, nb), dim3(256), 0, st, A, lda, N, x, part,
+                     chunk, sA, sv, flag);
+  return ns;
 }
-void gemv32(const float2 *A, size_t lda, int N, const cplx *x, cplx *y, cplx *part, hipStream_t st) {
-  int chunk = (N + kGemvSplit - 1) / kGemvSplit;
+int gemv_partial(const float2 *A, size_t lda, int N, const cplx *x, cplx *part, hipStream_t st, const int *flag) {
+  const int chunk = (N + kGemvSplit - 1) / kGemvSplit;
   hipLaunchKernelGGL(gemv_part_kernel<float2>, dim3((N + 255) / 256, kGemvSplit, 1), dim3(256), 0, st, A, lda, N, x,
-                     part, chunk, (size_t)0, (size_t)0, (const int *)nullptr);
-  hipLaunchKernelGGL(gemv_reduce_kernel, dim3((N + 255) / 256, 1, 1), dim3(256), 0, st, part, kGemvSplit, N, y,
-                     (size_t)0, (const int *)nullptr);
+                     part, chunk, (size_t)0, (size_t)0, flag);
+  return kGemvSplit;
 }
 
 }  // namespace omx
