@@ -79,6 +79,9 @@ template <typename T> __device__ inline T csub(T a, T b) {
   return r;
 }
 template <typename T> __device__ inline double mag2(T a) { return (double)a.x * a.x + (double)a.y * a.y; }
+// Whether a pivot counts as one (an FP64 square that underflows does not)
+__device__ inline bool nonzero(Cx<double> a) { return mag2(a) > 0.0; }
+__device__ inline bool nonzero(Cx<float> a) { return fabsf(a.x) + fabsf(a.y) > 0.0f; }
 // Reciprocal: the hardware estimate refined by Newton's iteration
 // r <- r + r (1 - d r), which doubles the number of correct bits per step:
 // one step after the single-precision estimate (within 1 ulp), two after the
@@ -171,62 +174,162 @@ __device__ inline unsigned wave_max_u32(unsigned x) {
   x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xF, 0xF, true));  // row_shr:2
   x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xF, 0xF, true));  // row_shr:4
   x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xF, 0xF, true));  // row_shr:8
-  x = max(x, (unsigned)__builtin_amdgcn_update_dpp((int)x, (int)x, 0x142, 0xA, 0xF, false));  // row_bcast:15
-  x = max(x, (unsigned)__builtin_amdgcn_update_dpp((int)x, (int)x, 0x143, 0xC, 0xF, false));  // row_bcast:31
+  x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xA, 0xF, false));  // row_bcast:15
+  x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xC, 0xF, false));  // row_bcast:31
   return (unsigned)__builtin_amdgcn_readlane((int)x, 63);
 }
 
-// [L11^{-1} | U11^{-1}] of the factored block F (column-major, 65 apart) into
-// dinv, by a workgroup of 8 waves: lane = row i; waves 0-3 hold columns 16 w ..
-// 16 w + 15 of L11^{-1}, waves 4-7 those of U11^{-1}; row k is broadcast within
-// the wave by lane reads, so the waves run without barriers.
-template <typename T> __device__ __forceinline__ void invert_block(const CxOf<T> *F, T *dinv) {
-  using C = CxOf<T>;
-  const int t = threadIdx.x, lane = t & 63, q = t >> 6;
-  const C zero{}, one{1, 0};
-  const int i = lane, w = q & 3;
-  C x[16];
-#pragma unroll
-  for(int m = 0; m < 16; ++m) x[m] = csel(16 * w + m == i, one, zero);
-  if(q < 4) {
-    // L11^{-1} (unit lower): for k: row i -= L[i][k] row k, i > k.  Column
-    // 16 w + m starts as e_{16 w + m} and its rows above 16 w + m stay zero,
-    // so the steps k < 16 w leave this wave's columns as they are: skipped
-    C fn = F[(16 * w) * 65 + i];  // column k of L, read one step ahead
-#pragma unroll 1
-    for(int k = 16 * w; k < 63; ++k) {
-      const int ks = __builtin_amdgcn_readfirstlane(k);
-      const C lik = csel(i > ks, fn, zero);
-      fn = F[(ks + 1) * 65 + i];
-#pragma unroll
-      for(int m = 0; m < 16; ++m) x[m] = cfms(x[m], lik, rdl(x[m], ks));
-    }
-  } else {
-    // U11^{-1} = (D^{-1} U11)^{-1} D^{-1} with D = diag(U11): a unit-upper
-    // sweep (row i -= (U[i][k] / U[i][i]) row k, i < k, k = 63..0), then
-    // column j scaled by 1 / U[j][j].  Rows below 16 w + 15 of this wave's
-    // columns stay zero, so the sweep starts at k = 16 w + 15
-    const C di = F[i * 65 + i];
-    const C rinv = csel(mag2(di) > 0.0, crecip(di), zero);
-    C fn = F[(16 * w + 15) * 65 + i];  // column k of U, read one step ahead
-#pragma unroll 1
-    for(int k = 16 * w + 15; k > 0; --k) {
-      const int ks = __builtin_amdgcn_readfirstlane(k);
-      const C uik = csel(i < ks, cm(fn, rinv), zero);
-      fn = F[(ks - 1) * 65 + i];
-#pragma unroll
-      for(int m = 0; m < 16; ++m) x[m] = cfms(x[m], uik, rdl(x[m], ks));
-    }
-#pragma unroll
-    for(int m = 0; m < 16; ++m) x[m] = cm(x[m], rdl(rinv, 16 * w + m));
+// Value of lane K of each row of 16 lanes (DPP row_newbcast), to the whole row.
+template <int K> __device__ inline float row_bcast(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + K, 0xF, 0xF, false));
+}
+template <int K> __device__ inline double row_bcast(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), 0x150 + K, 0xF, 0xF, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), 0x150 + K, 0xF, 0xF, false);
+  return __hiloint2double(hi, lo);
+}
+template <int K, typename R> __device__ inline Cx<R> row_bcast(Cx<R> v) {
+  return Cx<R>{row_bcast<K>(v.x), row_bcast<K>(v.y)};
+}
+// f(integral_constant<0>) ... f(integral_constant<N - 1>)
+template <int N, int I = 0, typename F> __device__ __forceinline__ void each(F &&f) {
+  if constexpr(I < N) {
+    f(std::integral_constant<int, I>{});
+    each<N, I + 1>(f);
   }
-  T *out = dinv + (q < 4 ? 0 : 4096);
+}
+
+// [L11^{-1} | U11^{-1}] of the factored block F (column-major, 65 apart, rinv the
+// reciprocals of its diagonal, 0 for a zero) into dinv, by a workgroup of 8 waves, in place of F: the 16 x 16 diagonal blocks by
+// substitution (waves 0-3 those of L11, waves 4-7 of U11; a row of 16 lanes
+// holds all rows of 4 columns, so row k reaches them by DPP), then the blocks off
+// the diagonal by X21 = -L22^{-1} (L21 L11^{-1}) and X12 = -U11^{-1} (U12
+// U22^{-1}) on the matrix cores, 16 and then 32 wide.
+//
+// Bound: the serial chain.  A substitution over all 64 rows, lane = row, with
+// row k broadcast by lane reads, took 64 steps of 16 complex updates: 22 us
+// (FP64) of the panel's 65 us; these 15 steps and 4 products take 9 us (FP64; 7 FP32).
+template <typename T> __device__ __forceinline__ void invert_block(CxOf<T> *F, const CxOf<T> *rinv, T *dinv) {
+  using C = CxOf<T>;
+  using R = typename CT<T>::R;
+  using V4 = typename CT<T>::V4;
+  const int t = threadIdx.x, lane = t & 63, q = __builtin_amdgcn_readfirstlane(t >> 6), li = lane & 15, g = lane >> 4;
+  const C zero{}, one{1, 0};
+  const bool low = q < 4;  // this wave works on L11, else on U11
+  {
+    const int o = 16 * (q & 3);
+    C x[4], f[16];
+#pragma unroll
+    for(int k = 0; k < 16; ++k) f[k] = F[(o + k) * 65 + o + li];  // row li of the block
+#pragma unroll
+    for(int m = 0; m < 4; ++m) x[m] = csel(4 * g + m == li, one, zero);
+    if(low) {
+      // unit lower: for k: row i -= L[i][k] row k, i > k
+      each<15>([&](auto ic) {
+        constexpr int k = decltype(ic)::value;
+        const C lik = csel(li > k, f[k], zero);
+#pragma unroll
+        for(int m = 0; m < 4; ++m) x[m] = cfms(x[m], lik, row_bcast<k>(x[m]));
+      });
+#pragma unroll
+      for(int m = 0; m < 4; ++m)
+        if(li > 4 * g + m) F[(o + 4 * g + m) * 65 + o + li] = x[m];
+    } else {
+      // U^{-1} = (D^{-1} U)^{-1} D^{-1} with D = diag(U): a unit-upper sweep
+      // (row i -= (U[i][k] / U[i][i]) row k, i < k, k = 15..1), then column j
+      // scaled by 1 / U[j][j]
+      const C ri = rinv[o + li];
+      each<15>([&](auto ic) {
+        constexpr int k = 15 - decltype(ic)::value;
+        const C uik = csel(li < k, cm(f[k], ri), zero);
+#pragma unroll
+        for(int m = 0; m < 4; ++m) x[m] = cfms(x[m], uik, row_bcast<k>(x[m]));
+      });
+#pragma unroll
+      for(int m = 0; m < 4; ++m)
+        if(li <= 4 * g + m) F[(o + 4 * g + m) * 65 + o + li] = cm(x[m], rinv[o + 4 * g + m]);
+    }
+  }
+  // element (i, k) of the triangular factor's inverse, both within its diagonal block
+  auto tri = [&](bool lo, int i, int k) {
+    const C v = F[k * 65 + i];
+    return lo ? csel(i > k, v, csel(i == k, one, zero)) : csel(i <= k, v, zero);
+  };
+  // D += S a b over steps k = k0 .. k0 + 3 + 4 (n - 1), a(k) of row li, b(s, k) of column li
+  auto mac = [](V4 &dr, V4 &di, C a, C b) {
+    dr = CT<T>::mfma(a.x, b.x, dr);
+    di = CT<T>::mfma(a.x, b.y, di);
+    dr = CT<T>::mfma(-a.y, b.y, dr);
+    di = CT<T>::mfma(a.y, b.x, di);
+  };
+  __syncthreads();
+  if(q < 2 || q > 5) {
+    // pairs of 16: waves 0, 1 of L11, waves 6, 7 of U11 (each on a SIMD, and so a
+    // matrix core, of its own).  The first product's
+    // accumulators are the second's right operand as they stand: register v
+    // holds row(lane, v), and any order of k will do
+    const int p = q & 1, r0 = 32 * p + (low ? 16 : 0), c0 = 32 * p + (low ? 0 : 16);
+    V4 tr = {0, 0, 0, 0}, ti = {0, 0, 0, 0}, xr = {0, 0, 0, 0}, xi = {0, 0, 0, 0};
+    C l[4], m[4], r[4];
+#pragma unroll
+    for(int s = 0; s < 4; ++s) {
+      m[s] = F[(c0 + 4 * s + g) * 65 + r0 + li];
+      r[s] = tri(low, c0 + 4 * s + g, c0 + li);
+      l[s] = tri(low, r0 + li, r0 + CT<T>::row(lane, s));
+    }
+#pragma unroll
+    for(int s = 0; s < 4; ++s) mac(tr, ti, m[s], r[s]);
+#pragma unroll
+    for(int s = 0; s < 4; ++s) mac(xr, xi, C{-l[s].x, -l[s].y}, C{tr[s], ti[s]});
+    // the block written here is read by this wave alone
+#pragma unroll
+    for(int v = 0; v < 4; ++v) F[(c0 + li) * 65 + r0 + CT<T>::row(lane, v)] = C{xr[v], xi[v]};
+  }
+  __syncthreads();
+  {
+    // the pair of 32: a wave one 16 x 16 tile (rows 16 a, columns 16 b) of the
+    // two products, the first one's result passed on in F; of the triangles'
+    // zero blocks one half of the steps is left out
+    const int a = q & 1, b = (q >> 1) & 1, r0 = low ? 32 : 0, c0 = low ? 0 : 32;
+    V4 tr = {0, 0, 0, 0}, ti = {0, 0, 0, 0}, xr = {0, 0, 0, 0}, xi = {0, 0, 0, 0};
+    C m[8], r[8];
+#pragma unroll
+    for(int s = 0; s < 8; ++s) {
+      m[s] = F[(c0 + 4 * s + g) * 65 + r0 + 16 * a + li];
+      r[s] = tri(low, c0 + 4 * s + g, c0 + 16 * b + li);
+    }
+    if(!low || b == 0)
+#pragma unroll
+      for(int s = 0; s < 4; ++s) mac(tr, ti, m[s], r[s]);
+    if(low || b == 1)
+#pragma unroll
+      for(int s = 4; s < 8; ++s) mac(tr, ti, m[s], r[s]);
+    __syncthreads();
+#pragma unroll
+    for(int v = 0; v < 4; ++v) F[(c0 + 16 * b + li) * 65 + r0 + 16 * a + CT<T>::row(lane, v)] = C{tr[v], ti[v]};
+#pragma unroll
+    for(int s = 0; s < 8; ++s) m[s] = tri(low, r0 + 16 * a + li, r0 + 4 * s + g);
+    __syncthreads();
+#pragma unroll
+    for(int s = 0; s < 8; ++s) r[s] = F[(c0 + 16 * b + li) * 65 + r0 + 4 * s + g];
+    if(low || a == 0)
+#pragma unroll
+      for(int s = 0; s < 4; ++s) mac(xr, xi, C{-m[s].x, -m[s].y}, r[s]);
+    if(!low || a == 1)
+#pragma unroll
+      for(int s = 4; s < 8; ++s) mac(xr, xi, C{-m[s].x, -m[s].y}, r[s]);
+    __syncthreads();
+#pragma unroll
+    for(int v = 0; v < 4; ++v) F[(c0 + 16 * b + li) * 65 + r0 + 16 * a + CT<T>::row(lane, v)] = C{xr[v], xi[v]};
+  }
+  __syncthreads();
 #pragma unroll
   for(int m = 0; m < 16; ++m) {
+    const C v = tri(low, lane, 16 * (q & 3) + m);
     T o;
-    o.x = x[m].x;
-    o.y = x[m].y;
-    out[(16 * w + m) * 64 + i] = o;
+    o.x = v.x;
+    o.y = v.y;
+    dinv[(low ? 0 : 4096) + (16 * (q & 3) + m) * 64 + lane] = o;
   }
 }
 
@@ -265,6 +368,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
   // the last of them the factored block
   __shared__ C buf[LM > FB ? LM : FB];
   __shared__ int rid[ROWS], pidx[64], pb[2][8], outpos[64], wtop[64];
+  __shared__ C rinv[64];
   const int t = threadIdx.x, lane = t & 63, q = t >> 6, g = blockIdx.x;
   const bool root = gridDim.x == 1;
   const C zero{};
@@ -333,6 +437,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
         if(lane == 0) {
           pb[par][jj] = 64 * sl + b;
           pidx[c] = 64 * sl + b;
+          rinv[c] = ip;
         }
 #pragma unroll
         for(int s = 0; s < RPL; ++s) {
@@ -424,7 +529,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
     }
     if(lane == 0) *mcnt = n0 + __popcll(gm);
   }
-  invert_block<T>(buf, dinv);
+  invert_block<T>(buf, rinv, dinv);
 }
 
 // Rows per lane of tslu_panel, and so the tree's fan-in: as many as the
@@ -438,16 +543,21 @@ template <typename T> struct TsluCfg {
 // Diagonal-block pivoting: LU with partial pivoting restricted to the 64 x 64
 // diagonal block of the panel (rows are chosen among the block's rows; the
 // interchanges are applied to whole rows), then the inverses of L11 and U11.
-// One workgroup of 8 waves.  Elimination: each wave holds one panel of 8
-// columns of every row in registers, lane = row; rows are not moved (the
-// pivot order is recorded instead).  The panel's owner runs its 8 pivot steps
-// alone (pivot by a DPP maximum of a 32-bit key: max(|re|, |im|) as a float
-// with the row in the low bits) and publishes the multipliers and pivot rows;
-// after one barrier per panel the waves of later panels apply its 8 rank-1
-// updates, each with the pivot row read from its own lane b.  Inversion: waves 0-3 build L11^{-1}, waves 4-7 U11^{-1}
-// (lane = row, 16 columns per wave, row k broadcast by lane reads).  Writes
-// the factored block into A, the inverses into dinv ([L11^{-1} | U11^{-1}],
+// One workgroup of 8 waves.  Elimination: wave q holds columns 8 q .. 8 q + 7 of
+// every row in registers, lane = row; rows are not moved (the pivot order is
+// recorded instead).  The waves run without barriers: the owner of a column
+// chooses the pivot (DPP maximum of a 32-bit key: max(|re|, |im|) as a float with
+// the row in the low bits), leaves the multipliers in LDS and counts the step as
+// published; the waves of later columns follow the count, so the next owner has
+// applied all but the last steps when its own begin.  Every lane takes the
+// reciprocal of its own entry while the maximum is on its way.  Writes the
+// factored block into A, the inverses into dinv ([L11^{-1} | U11^{-1}],
 // column-major), the block's row map (mdst <- msrc) and the permutation.
+//
+// Bound: the chain of 64 pivot steps (maximum, multiplier, the next column's
+// update) at 2.4 GHz.  With a barrier a panel of 8 columns, the reciprocal after
+// the maximum and inverses by substitution: 65 us FP64, 47 us FP32; now 35 and
+// 26, of which the elimination takes 21 and 17.
 template <typename T>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(1, 2))) void diag_lu(T *A, size_t lda, int j0, T *dinv, int *mdst, int *msrc, int *mcnt,
                                                int *perm, int *status, BatchStrides bs) {
@@ -462,103 +572,83 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
     perm += (size_t)z * bs.perm;
     status += (size_t)z * bs.status;
   }
-  __shared__ int pb[2][8];  // a panel's pivot rows
-  __shared__ int prow[64];
-  __shared__ C F[64 * 65];  // factored block in pivoted order, column-major [c * 65 + r]
-  // A panel's multipliers, one column per pivot step (0 on rows already
-  // chosen), in two alternating buffers.  They live in F's storage: F is
-  // written only after the last panel's barrier, when no wave reads them any
-  // more, and the kernel's LDS stays small enough to start beside the bulk
-  // update's workgroups.
-  C(*lm)[8][64] = reinterpret_cast<C(*)[8][64]>(F);
-  const int t = threadIdx.x, lane = t & 63, q = t >> 6;
-  const C zero{}, one{1, 0};
-  {
-    // Wave q holds the columns of panel pq (8 columns); panels are taken in
-    // order 0..7, and the two waves of a SIMD (q and q + 4) hold consecutive
-    // panels, so every second panel's owner has its SIMD to itself.
-    const int pq = 2 * (q & 3) + (q >> 2);
-    C v[8];
+  // step c, once published: 1 + its row, + 128 for a zero pivot; the pivots'
+  // reciprocals (in both, 64 more slots take what the other lanes write: a store
+  // without a branch); the step of each row
+  __shared__ int step[128], pos[64];
+  __shared__ C rinv[128];
+  // factored block in pivoted order, column-major [c * 65 + r]; before, the
+  // multipliers of step c at [c * 64 + row] (0 on rows already chosen).  One
+  // storage: the kernel's LDS stays small enough to start beside the bulk
+  // update's workgroups
+  __shared__ C F[64 * 65];
+  const int t = threadIdx.x, lane = t & 63, q = __builtin_amdgcn_readfirstlane(t >> 6);
+  const C zero{};
+  C v[8];
 #pragma unroll
-    for(int j = 0; j < 8; ++j) {
-      T a = A[(size_t)(j0 + 8 * pq + j) * lda + j0 + lane];
-      v[j] = C{a.x, a.y};
-    }
-    bool used = false;
-    int mypos = 0;
-#pragma unroll 1
-    for(int pc = 0; pc < 8; ++pc) {
-      const int par = pc & 1;
-      if(pq == pc) {
-        // the owner's 8 pivot steps, without barriers: the pivot is the
-        // largest max(|re|, |im|) among the rows not chosen yet (a DPP maximum
-        // of a 32-bit key with the row in the low bits); the multipliers
-        // replace the column below the pivot and update the panel's later
-        // columns, and are published for the other waves
-#pragma unroll
-        for(int jj = 0; jj < 8; ++jj) {
-          const int c = 8 * pc + jj;
-          const float mx = (float)fmax(fabs((double)v[jj].x), fabs((double)v[jj].y));
-          const unsigned key = used ? 0u : ((__float_as_uint(mx) & ~0x7Fu) | (unsigned)(127 - lane));
-          const int b = __builtin_amdgcn_readfirstlane(127 - (int)(wave_max_u32(key) & 127));
-          const C pv = rdl(v[jj], b);
-          const bool sing = !(mag2(pv) > 0.0);
-          if(sing && lane == b) atomicCAS(&status[0], 0, j0 + c + 1);
-          const C ip = csel(sing, zero, crecip(pv));
-          if(lane == b) {
-            used = true;
-            mypos = c;
-          }
-          const C l = csel(used, zero, cm(v[jj], ip));
-          v[jj] = csel(used, v[jj], l);
-          lm[par][jj][lane] = l;
-          if(lane == 0) {
-            pb[par][jj] = b;
-            prow[c] = b;
-          }
-#pragma unroll
-          for(int j = jj + 1; j < 8; ++j) v[j] = cfms(v[j], l, rdl(v[j], b));
-        }
-      }
-      // one barrier per panel; the buffers alternate, so the next owner's
-      // writes cannot reach a panel that a slower wave still reads
-      __syncthreads();
-      if(pq != pc) {
-        int bb[8];
-#pragma unroll
-        for(int jj = 0; jj < 8; ++jj) {
-          bb[jj] = __builtin_amdgcn_readfirstlane(pb[par][jj]);
-          if(lane == bb[jj]) {
-            used = true;
-            mypos = 8 * pc + jj;
-          }
-        }
-        if(pq > pc) {
-          // the panel's 8 rank-1 updates, in the order of its pivot steps
-#pragma unroll
-          for(int jj = 0; jj < 8; ++jj) {
-            const C l = lm[par][jj][lane];
-#pragma unroll
-            for(int j = 0; j < 8; ++j) v[j] = cfms(v[j], l, rdl(v[j], bb[jj]));
-          }
-        }
-      }
-    }
-    // factored block in pivoted order
-#pragma unroll
-    for(int j = 0; j < 8; ++j) {
-      const int col = 8 * pq + j;
-      F[col * 65 + mypos] = v[j];
-      T o;
-      o.x = v[j].x;
-      o.y = v[j].y;
-      A[(size_t)(j0 + col) * lda + j0 + mypos] = o;
-    }
+  for(int j = 0; j < 8; ++j) {
+    T a = A[(size_t)(j0 + 8 * q + j) * lda + j0 + lane];
+    v[j] = C{a.x, a.y};
   }
+  if(t < 64) step[t] = 0;
   __syncthreads();
-  // row map and running permutation (wave 0)
-  if(q == 0) {
-    const int src = prow[lane];
+  // The steps of the earlier owners, each published before it is read; owners
+  // wait for earlier ones only, so every wait ends
+  bool used = false;
+#pragma unroll 1
+  for(int c = 0; c < 8 * q; ++c) {
+    int e;
+    do
+      e = __builtin_amdgcn_readfirstlane(__hip_atomic_load(&step[c], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP));
+    while(e == 0);
+    const int b = (e & 127) - 1;
+    const C l = F[c * 64 + lane];
+    used = used || lane == b;
+#pragma unroll
+    for(int j = 0; j < 8; ++j) v[j] = cfms(v[j], l, rdl(v[j], b));
+  }
+  __builtin_amdgcn_s_setprio(3);
+#pragma unroll
+  for(int jj = 0; jj < 8; ++jj) {
+    const int c = 8 * q + jj;
+    const float mx = (float)fmax(fabs((double)v[jj].x), fabs((double)v[jj].y));
+    const unsigned key = used ? 0u : ((__float_as_uint(mx) & ~0x7Fu) | (unsigned)(127 - lane));
+    const bool sing = !nonzero(v[jj]);
+    const C ir = csel(sing, zero, crecip(v[jj]));
+    const int e = (sing ? 129 : 1) + lane;
+    const int b = 127 - (int)(wave_max_u32(key) & 127);
+    used = used || lane == b;
+    const C ip = rdl(ir, b);
+    const C l = csel(used, zero, cm(v[jj], ip));
+    v[jj] = csel(used, v[jj], l);
+    F[c * 64 + lane] = l;
+#pragma unroll
+    for(int j = jj + 1; j < 8; ++j) v[j] = cfms(v[j], l, rdl(v[j], b));
+    // published after the multipliers: a wave's LDS stores are done in order
+    const int slot = lane == b ? c : 64 + lane;
+    rinv[slot] = ir;
+    asm volatile("" ::: "memory");
+    __hip_atomic_store(&step[slot], e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  }
+  __builtin_amdgcn_s_setprio(0);
+  __syncthreads();  // all steps published and all multipliers read
+  const int own = step[lane], src = (own & 127) - 1;  // the row of step `lane`
+  if(q == 0) pos[src] = lane;
+  __syncthreads();
+  const int mypos = pos[lane];
+#pragma unroll
+  for(int j = 0; j < 8; ++j) {
+    const int col = 8 * q + j;
+    F[col * 65 + mypos] = v[j];
+    T o;
+    o.x = v[j].x;
+    o.y = v[j].y;
+    A[(size_t)(j0 + col) * lda + j0 + mypos] = o;
+  }
+  // the first zero pivot, row map and running permutation (the last wave)
+  if(q == 7) {
+    const unsigned long long zm = __ballot(own > 128);
+    if(zm && lane == 0) atomicCAS(&status[0], 0, j0 + __ffsll((long long)zm));
     const bool mv = src != lane;
     const int old = perm[j0 + src];
     const unsigned long long bm = __ballot(mv);
@@ -572,7 +662,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
     __builtin_amdgcn_wave_barrier();
     perm[j0 + lane] = old;
   }
-  invert_block<T>(F, dinv);
+  __syncthreads();
+  invert_block<T>(F, rinv, dinv);
 }
 
 // In-place block product with a 64 x 64 factor M (column-major):
