@@ -192,8 +192,8 @@ struct LuWork {
   // device scratch of one factorization
   int *perm;            // Np: final row permutation (row i of P A is row perm[i] of A)
   int *cand[2];         // tournament candidates, ping-pong, [Gmax][NB]
-  int *mdst, *msrc;     // gather maps: tournament 2 NB entries at the start; block
-  int *mcnt;            // pivoting NB entries per panel (panel k at k NB, count mcnt[k])
+  int *mdst, *msrc;     // gather maps: tournament rows mdst <- msrc, mcnt of 2 NB entries at
+  int *mcnt;            // the start; block pivoting row i <- msrc[i]
   int *status;          // [0]: singular pivot column+1, [1]: wait timeout
   void *wlu;            // NB x NB complex: the tournament's selected-block factors
   void *dinv;           // per panel [L11^{-1} | U11^{-1}], 2 NB^2 elements of T, column-major

@@ -12,10 +12,11 @@
 //                  rows, a tree of merges picks the NB pivot rows, and its root
 //                  writes the gather map, the block's factors and inverses
 // Shared by both:
-//   laswp_map      the panel's row interchanges on the other columns, as one
-//                  parallel gather/scatter
-//   blk_mul        the two panel triangular solves as in-place MFMA block
-//                  products: U12 = L11^{-1} A12, L21 = A21 U11^{-1}
+//   panel_mul      the two panel triangular solves as in-place MFMA products
+//                  with the inverses: U12 = L11^{-1} A12, L21 = A21 U11^{-1};
+//                  block pivoting applies its interchanges here
+//   laswp_map      the tournament's row interchanges on the other columns, as
+//                  one parallel gather/scatter
 //   gemm_tile      A22 -= L21 U12 as complex products on the matrix cores:
 //                  v_mfma_f64_16x16x4f64 (FP64) or v_mfma_f32_16x16x4f32
 //                  (FP32), four real MFMAs per complex tile product, planar
@@ -552,23 +553,21 @@ template <typename T> struct TsluCfg {
 // applied all but the last steps when its own begin.  Every lane takes the
 // reciprocal of its own entry while the maximum is on its way.  Writes the
 // factored block into A, the inverses into dinv ([L11^{-1} | U11^{-1}],
-// column-major), the block's row map (mdst <- msrc) and the permutation.
+// column-major), the block's row map (row j0 + i <- msrc[i]) and the permutation.
 //
 // Bound: the chain of 64 pivot steps (maximum, multiplier, the next column's
 // update) at 2.4 GHz.  With a barrier a panel of 8 columns, the reciprocal after
 // the maximum and inverses by substitution: 65 us FP64, 47 us FP32; now 35 and
 // 26, of which the elimination takes 21 and 17.
 template <typename T>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(1, 2))) void diag_lu(T *A, size_t lda, int j0, T *dinv, int *mdst, int *msrc, int *mcnt,
-                                               int *perm, int *status, BatchStrides bs) {
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(1, 2))) void diag_lu(T *A, size_t lda, int j0, T *dinv, int *msrc, int *perm,
+                                               int *status, BatchStrides bs) {
   using C = CxOf<T>;
   {
     const int z = blockIdx.z;
     A += z * bs.a;
     dinv += z * bs.inv;
-    mdst += (size_t)z * bs.map;
     msrc += (size_t)z * bs.map;
-    mcnt += (size_t)z * bs.cnt;
     perm += (size_t)z * bs.perm;
     status += (size_t)z * bs.status;
   }
@@ -649,16 +648,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
   if(q == 7) {
     const unsigned long long zm = __ballot(own > 128);
     if(zm && lane == 0) atomicCAS(&status[0], 0, j0 + __ffsll((long long)zm));
-    const bool mv = src != lane;
     const int old = perm[j0 + src];
-    const unsigned long long bm = __ballot(mv);
-    const unsigned long long below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    if(mv) {
-      const int i = __popcll(bm & below);
-      mdst[i] = j0 + lane;
-      msrc[i] = j0 + src;
-    }
-    if(lane == 0) *mcnt = __popcll(bm);
+    msrc[lane] = j0 + src;
     __builtin_amdgcn_wave_barrier();
     perm[j0 + lane] = old;
   }
@@ -666,122 +657,184 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
   invert_block<T>(F, rinv, dinv);
 }
 
-// In-place block product with a 64 x 64 factor M (column-major):
-//   LEFT:  A[j0 + i, off + n] = sum_k M(i, k) A[j0 + k, off + n]
-//   RIGHT: A[off + m, j0 + n] = sum_k A[off + m, j0 + k] M(k, n)
-// with off = first + 64 blockIdx.x.  K is staged through LDS in chunks of
-// 16 (a small LDS footprint lets these workgroups start beside the bulk
-// update's); the block is overwritten only after all of it has been read.
-constexpr int kBlkBK = 16, kBlkPad = 16;
-template <typename T> using BlkPlanes = typename CT<T>::R[2][kBlkBK][64 + kBlkPad];  // [plane][k][m or n]
-template <typename T, bool LEFT>
-__device__ __forceinline__ void blk_mul_body(T *A, size_t lda, int j0, int first, const T *M, BlkPlanes<T> &As,
-                                             BlkPlanes<T> &Bs) {
-  using R = typename CT<T>::R;
+// ------------------------------------------------------------------ panel products
+// The products with a panel's 64 x 64 inverses, in place, a strip of 16 NT rows or
+// columns per workgroup of 4 waves:
+//   blockIdx.x < nright   L21 = A21 U11^{-1} on rows first_r ..
+//   then                  U12 = L11^{-1} (P A12) on columns first_c .., the block's
+//                         interchanges applied as the strip is read (ms, null: none)
+// PAIR: the second panel of a pair.  L21 as above; a strip of the columns goes
+// through both panels: U12 of p0, block row p1 -= L(p1, p0) U12, U12 of p1.
+//
+// The strip is staged in LDS; wave w takes 16 of the block's 64 rows (columns),
+// its part of the 64 x 64 operands in registers straight from memory, all loads
+// of the chain first.  Either product is written so that the accumulators'
+// lanes run along the columns of A.
+//
+// Bound: launch and load latency while the strips are fewer than the chip's
+// workgroups, the matrix cores above.  These were 64-wide blocks (few workgroups,
+// each 16 us FP64 and 9 us FP32) with the interchanges and the update of block
+// row p1 in launches of their own: five launches a pair that are now one.
+template <typename T, int NT, bool PAIR>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void panel_mul(
+    T *A, size_t lda, int p0, int p1, int nright, int first_r, int first_c, const T *d0, const T *d1, const int *ms0,
+    const int *ms1, BatchStrides bs) {
+  using C = CxOf<T>;
   using V4 = typename CT<T>::V4;
-  constexpr int BK = kBlkBK;
-  const int t = threadIdx.x, lane = t & 63, wv = t >> 6, wm = wv & 1, wn = wv >> 1;
-  const int off = first + blockIdx.x * 64;
-  V4 cr[2][2], ci[2][2];
+  constexpr int W = 16 * NT, LD = 65;
+  A += blockIdx.z * bs.a;
+  d0 += blockIdx.z * bs.inv;
+  if(PAIR) d1 += blockIdx.z * bs.inv;
+  __shared__ C S0[W * LD], S1[PAIR ? W * LD : 1];
+  const int t = threadIdx.x, lane = t & 63, li = lane & 15, g = lane >> 4;
+  // the waves' shares of a triangular product differ: spread them over the SIMDs
+  const int tw = __builtin_amdgcn_readfirstlane(t >> 6), w = (tw + blockIdx.x) & 3;
+  auto ld = [](const T *p) {
+    const T v = *p;
+    return C{v.x, v.y};
+  };
+  auto st = [](T *p, decltype(T{}.x) x, decltype(T{}.x) y) {
+    T v;
+    v.x = x;
+    v.y = y;
+    *p = v;
+  };
+  // x += over k of a(row li, k) b(k, column li), k = 4 s + g in step s
+  auto mac = [](V4 &xr, V4 &xi, C a, C b) {
+    xr = CT<T>::mfma(a.x, b.x, xr);
+    xi = CT<T>::mfma(a.x, b.y, xi);
+    xr = CT<T>::mfma(-a.y, b.y, xr);
+    xi = CT<T>::mfma(a.y, b.x, xi);
+  };
+  if((int)blockIdx.x < nright) {
+    const int off = first_r + W * blockIdx.x, j0 = PAIR ? p1 : p0;
+    const T *M = (PAIR ? d1 : d0) + kNB * kNB;
+    C m[16], v[4 * NT];
 #pragma unroll
-  for(int a = 0; a < 2; ++a)
-#pragma unroll
-    for(int b = 0; b < 2; ++b) {
-      cr[a][b] = V4{0, 0, 0, 0};
-      ci[a][b] = V4{0, 0, 0, 0};
+    for(int i = 0; i < 4 * NT; ++i) {
+      const int e = t + 256 * i, r = e % W, k = e / W;
+      v[i] = ld(A + (size_t)(j0 + k) * lda + off + r);
     }
-  // both operands in registers first (one round of load latency), then
-  // staged through LDS chunk by chunk
-  R ar_[4][4], ai_[4][4], br_[4][4], bi_[4][4];
 #pragma unroll
-  for(int ch = 0; ch < 4; ++ch)
+    for(int s = 0; s < 16; ++s) m[s] = ld(M + (16 * w + li) * kNB + 4 * s + g);
 #pragma unroll
-    for(int it = 0; it < 4; ++it) {
-      const int idx = t + 256 * it, kc = ch * BK;
-      // left operand (m = idx % 64, k = idx / 64), right operand (k = idx % 16, n = idx / 16)
-      const int m = idx & 63, ka = idx >> 6, kb = idx & 15, n = idx >> 4;
-      T av, bv;
-      if(LEFT) {
-        av = M[(kc + ka) * 64 + m];                              // M(m, k)
-        bv = A[(size_t)(off + n) * lda + j0 + kc + kb];          // block(k, n)
-      } else {
-        av = A[(size_t)(j0 + kc + ka) * lda + off + m];          // block(m, k)
-        bv = M[n * 64 + kc + kb];                                // M(k, n)
-      }
-      ar_[ch][it] = av.x;
-      ai_[ch][it] = av.y;
-      br_[ch][it] = bv.x;
-      bi_[ch][it] = bv.y;
-    }
-#pragma unroll
-  for(int ch = 0; ch < 4; ++ch) {
-    __syncthreads();
-#pragma unroll
-    for(int it = 0; it < 4; ++it) {
-      const int idx = t + 256 * it;
-      const int m = idx & 63, ka = idx >> 6, kb = idx & 15, n = idx >> 4;
-      As[0][ka][m] = ar_[ch][it];
-      As[1][ka][m] = ai_[ch][it];
-      Bs[0][kb][n] = br_[ch][it];
-      Bs[1][kb][n] = bi_[ch][it];
+    for(int i = 0; i < 4 * NT; ++i) {
+      const int e = t + 256 * i, r = e % W, k = e / W;
+      S0[r * LD + k] = v[i];
     }
     __syncthreads();
+    V4 xr[NT], xi[NT];
 #pragma unroll
-    for(int ks = 0; ks < BK / 4; ++ks) {
-      const int kr = ks * 4 + (lane >> 4), li = lane & 15;
-      R ar[2], ai[2], nai[2], br[2], bi[2];
+    for(int n = 0; n < NT; ++n) xr[n] = xi[n] = V4{0, 0, 0, 0};
 #pragma unroll
-      for(int a = 0; a < 2; ++a) {
-        ar[a] = As[0][kr][wm * 32 + a * 16 + li];
-        ai[a] = As[1][kr][wm * 32 + a * 16 + li];
-        nai[a] = -ai[a];
-        br[a] = Bs[0][kr][wn * 32 + a * 16 + li];
-        bi[a] = Bs[1][kr][wn * 32 + a * 16 + li];
-      }
+    for(int c = 0; c < 4; ++c)
+      if(c <= w)  // U11^{-1} is zero below the diagonal
 #pragma unroll
-      for(int a = 0; a < 2; ++a)
+        for(int s = 4 * c; s < 4 * c + 4; ++s)
 #pragma unroll
-        for(int b = 0; b < 2; ++b) {
-          cr[a][b] = CT<T>::mfma(ar[a], br[b], cr[a][b]);
-          ci[a][b] = CT<T>::mfma(ar[a], bi[b], ci[a][b]);
-          cr[a][b] = CT<T>::mfma(nai[a], bi[b], cr[a][b]);
-          ci[a][b] = CT<T>::mfma(ai[a], br[b], ci[a][b]);
-        }
-    }
+          for(int n = 0; n < NT; ++n) mac(xr[n], xi[n], m[s], S0[(16 * n + li) * LD + 4 * s + g]);
+#pragma unroll
+    for(int n = 0; n < NT; ++n)
+#pragma unroll
+      for(int v = 0; v < 4; ++v)
+        st(A + (size_t)(j0 + 16 * w + CT<T>::row(lane, v)) * lda + off + 16 * n + li, xr[n][v], xi[n][v]);
+    return;
   }
-  __syncthreads();  // every workgroup thread has read the block before it is overwritten
+  const int off = first_c + W * ((int)blockIdx.x - nright);
+  C m0[16], m1[PAIR ? 16 : 1], m2[PAIR ? 16 : 1], v[4 * NT];
+  // lane k takes row k of the interchanged block
+  const int s0 = ms0 ? ms0[(size_t)blockIdx.z * bs.map + lane] : p0 + lane;
+  const int s1 = PAIR ? ms1[(size_t)blockIdx.z * bs.map + lane] - p1 : 0;
 #pragma unroll
-  for(int a = 0; a < 2; ++a)
+  for(int s = 0; s < 16; ++s) m0[s] = ld(d0 + (4 * s + g) * kNB + 16 * w + li);
 #pragma unroll
-    for(int b = 0; b < 2; ++b) {
-      const int n = wn * 32 + b * 16 + (lane & 15);
+  for(int i = 0; i < 4 * NT; ++i) v[i] = ld(A + (size_t)(off + 4 * i + tw) * lda + s0);
+  V4 cr[NT], ci[NT];
+  if constexpr(PAIR) {
 #pragma unroll
-      for(int v = 0; v < 4; ++v) {
-        const int m = wm * 32 + a * 16 + CT<T>::row(lane, v);
-        T o;
-        o.x = cr[a][b][v];
-        o.y = ci[a][b][v];
-        if(LEFT)
-          A[(size_t)(off + n) * lda + j0 + m] = o;
-        else
-          A[(size_t)(j0 + n) * lda + off + m] = o;
+    for(int n = 0; n < NT; ++n)
+#pragma unroll
+      for(int k = 0; k < 4; ++k) {
+        const C x = ld(A + (size_t)(off + 16 * n + CT<T>::row(lane, k)) * lda + p1 + 16 * w + li);
+        cr[n][k] = x.x;
+        ci[n][k] = x.y;
       }
+#pragma unroll
+    for(int s = 0; s < 16; ++s) {
+      const C x = ld(A + (size_t)(p0 + 4 * s + g) * lda + p1 + 16 * w + li);
+      m1[s] = C{-x.x, -x.y};
     }
+#pragma unroll
+    for(int s = 0; s < 16; ++s) m2[s] = ld(d1 + (4 * s + g) * kNB + 16 * w + li);
+  }
+#pragma unroll
+  for(int i = 0; i < 4 * NT; ++i) S0[(4 * i + tw) * LD + lane] = v[i];
+  __syncthreads();
+  V4 xr[NT], xi[NT];
+  auto left = [&](const C *S, const C(&m)[16]) {
+#pragma unroll
+    for(int n = 0; n < NT; ++n) xr[n] = xi[n] = V4{0, 0, 0, 0};
+#pragma unroll
+    for(int c = 0; c < 4; ++c)
+      if(c <= w)  // L11^{-1} is zero above the diagonal
+#pragma unroll
+        for(int s = 4 * c; s < 4 * c + 4; ++s)
+#pragma unroll
+          for(int n = 0; n < NT; ++n) mac(xr[n], xi[n], S[(16 * n + li) * LD + 4 * s + g], m[s]);
+  };
+  auto store = [&](int j0) {
+#pragma unroll
+    for(int n = 0; n < NT; ++n)
+#pragma unroll
+      for(int k = 0; k < 4; ++k)
+        st(A + (size_t)(off + 16 * n + CT<T>::row(lane, k)) * lda + j0 + 16 * w + li, xr[n][k], xi[n][k]);
+  };
+  left(S0, m0);
+  store(p0);
+  if constexpr(PAIR) {
+#pragma unroll
+    for(int n = 0; n < NT; ++n)
+#pragma unroll
+      for(int k = 0; k < 4; ++k) S1[(16 * n + CT<T>::row(lane, k)) * LD + 16 * w + li] = C{xr[n][k], xi[n][k]};
+    __syncthreads();
+#pragma unroll
+    for(int s = 0; s < 16; ++s)
+#pragma unroll
+      for(int n = 0; n < NT; ++n) mac(cr[n], ci[n], S1[(16 * n + li) * LD + 4 * s + g], m1[s]);
+    // S0 was read out before the last barrier
+#pragma unroll
+    for(int n = 0; n < NT; ++n)
+#pragma unroll
+      for(int k = 0; k < 4; ++k) S0[(16 * n + CT<T>::row(lane, k)) * LD + 16 * w + li] = C{cr[n][k], ci[n][k]};
+    __syncthreads();
+    // p1's interchanges on the strip: a wave 4 NT of its columns
+    C y[4 * NT];
+#pragma unroll
+    for(int i = 0; i < 4 * NT; ++i) y[i] = S0[(4 * i + tw) * LD + s1];
+    // S1's readers are past the barrier
+#pragma unroll
+    for(int i = 0; i < 4 * NT; ++i) S1[(4 * i + tw) * LD + lane] = y[i];
+    __syncthreads();
+    left(S1, m2);
+    store(p1);
+  }
 }
-template <typename T, bool LEFT>
-__global__ __launch_bounds__(256) void blk_mul(T *A, size_t lda, int j0, int first, const T *M, BatchStrides bs) {
-  __shared__ BlkPlanes<T> As, Bs;
-  blk_mul_body<T, LEFT>(A + blockIdx.z * bs.a, lda, j0, first, M + blockIdx.z * bs.inv, As, Bs);
-}
-// Both products of a panel in one launch: U12 (blockIdx.y = 0) and L21, with the
-// inverses [L11^{-1} | U11^{-1}] at M.
-template <typename T>
-__global__ __launch_bounds__(256) void blk_mul_both(T *A, size_t lda, int j0, int first, const T *M) {
-  __shared__ BlkPlanes<T> As, Bs;
-  if(blockIdx.y == 0)
-    blk_mul_body<T, true>(A, lda, j0, first, M, As, Bs);
+constexpr long kWideStrips = 512;
+// Strip width: 16 while that fills the chip no more than twice, else 32 (the
+// 64 x 64 operands are then read half as often).
+template <typename T, bool PAIR>
+void panel_products(T *A, size_t lda, int p0, int p1, int rows, int first_r, int cols, int first_c, const T *d0,
+                    const T *d1, const int *ms0, const int *ms1, hipStream_t st, int nb, BatchStrides bs) {
+  if(rows + cols <= 0) return;
+  const bool wide = (long)(rows + cols) / 16 * nb > kWideStrips;
+  const int w = wide ? 32 : 16;
+  const dim3 grid(rows / w + cols / w, 1, nb);
+  if(wide)
+    hipLaunchKernelGGL((panel_mul<T, 2, PAIR>), grid, dim3(256), 0, st, A, lda, p0, p1, rows / w, first_r, first_c, d0,
+                       d1, ms0, ms1, bs);
   else
-    blk_mul_body<T, false>(A, lda, j0, first, M + kNB * kNB, As, Bs);
+    hipLaunchKernelGGL((panel_mul<T, 1, PAIR>), grid, dim3(256), 0, st, A, lda, p0, p1, rows / w, first_r, first_c, d0,
+                       d1, ms0, ms1, bs);
 }
 
 // ------------------------------------------------------------------ swaps
@@ -840,39 +893,21 @@ void laswp(T *A, size_t lda, int c0, int cend, const int *mdst, const int *msrc,
 }
 
 // Deferred interchanges of block pivoting: panel k = blockIdx.y (>= 1)
-// applies its map (NB entries at k NB) to the columns left of it.
+// applies its map (NB rows at k NB) to the columns left of it.
 template <typename T>
-__global__ __launch_bounds__(256) void laswp_left(T *A, size_t lda, const int *__restrict__ mdst,
-                                                  const int *__restrict__ msrc, const int *__restrict__ mcnt,
-                                                  BatchStrides bs) {
+__global__ __launch_bounds__(256) void laswp_left(T *A, size_t lda, const int *__restrict__ msrc, BatchStrides bs) {
   A += blockIdx.z * bs.a;
-  mdst += (size_t)blockIdx.z * bs.map;
   msrc += (size_t)blockIdx.z * bs.map;
-  mcnt += (size_t)blockIdx.z * bs.cnt;
   const int k = blockIdx.y + 1;
   const int cl = threadIdx.x / 32, li = threadIdx.x % 32;
-  const int col = blockIdx.x * 8 + cl;
+  T *a = A + (size_t)(blockIdx.x * 8 + cl) * lda;
   if(blockIdx.x * 8 >= k * kNB) return;  // whole workgroup past the panel
-  const int m = mcnt[k];
-  const int *md = mdst + k * kNB, *ms = msrc + k * kNB;
   T v[2];
-  int d[2];
-  if(col < k * kNB) {
-    const T *a = A + (size_t)col * lda;
 #pragma unroll
-    for(int q = 0; q < 2; ++q) {
-      const int i = li + 32 * q;
-      d[q] = i < m ? md[i] : -1;
-      if(i < m) v[q] = a[ms[i]];
-    }
-  }
+  for(int q = 0; q < 2; ++q) v[q] = a[msrc[k * kNB + li + 32 * q]];
   __syncthreads();
-  if(col < k * kNB) {
-    T *a = A + (size_t)col * lda;
 #pragma unroll
-    for(int q = 0; q < 2; ++q)
-      if(d[q] >= 0) a[d[q]] = v[q];
-  }
+  for(int q = 0; q < 2; ++q) a[k * kNB + li + 32 * q] = v[q];
 }
 
 // ------------------------------------------------------------------ gemm
@@ -1333,10 +1368,10 @@ void bulk_update(T *A, size_t lda, int row0, int col0, int k0, int M, int N, hip
 //
 // Block pivoting (interchanges stay inside a panel's 64 rows), two streams:
 // sb (panel work) runs pair s+1 while st (bulk updates) finishes pair s.
-//   sb  diag_lu p0; swaps on p1's columns; L21(p0); U12(p0) on p1's columns;
-//       p1's columns -= L21(p0) U12(p0); diag_lu p1; L21(p1)
-//   sb  after st's bulk update of pair s-1: swaps of p0 on the far columns,
-//       U12(p0), block row p1 -= L(p1, p0) U12(p0), swaps of p1, U12(p1)
+//   sb  diag_lu p0; L21(p0) and U12(p0) on p1's columns; p1's columns -=
+//       L21(p0) U12(p0); diag_lu p1
+//   sb  after st's bulk update of pair s-1: L21(p1); on the far columns U12(p0),
+//       block row p1 -= L(p1, p0) U12(p0), U12(p1) (one launch)
 //   st  A22 -= [L21(p0) L21(p1)] [U12(p0); U12(p1)]: the next pair's
 //       columns first (sb starts on them), then the rest
 // Interchanges on the columns left of each panel are applied once at the end
@@ -1368,12 +1403,6 @@ int lu_factor(T *A, int Np, size_t lda, LuWork &w, hipStream_t st, LuProf *prof)
     prof->gemm_launches = 0;
   }
   if(block) {
-    auto map = [&](int j0, int **d, int **s_, int **c) {
-      const int k = j0 / kNB;
-      *d = w.mdst + k * kNB;
-      *s_ = w.msrc + k * kNB;
-      *c = w.mcnt + k;
-    };
     (void)hipEventRecord(w.ev_next, st);
     (void)hipEventRecord(w.ev_bulk, st);
     for(int J = 0, pi = 0; J < Np; J += 2 * kNB, ++pi) {
@@ -1382,34 +1411,26 @@ int lu_factor(T *A, int Np, size_t lda, LuWork &w, hipStream_t st, LuProf *prof)
       const int rest0 = Np - p0 - kNB, restf = Np - far;
       const bool rec = prof && pi < prof->cap;
       hipEvent_t *pe = rec ? prof->ev + 4 * pi : nullptr;
-      int *d0, *s0, *c0, *d1, *s1, *c1;
-      map(p0, &d0, &s0, &c0);
-      map(p1, &d1, &s1, &c1);
+      const int *m0 = w.msrc + p0, *m1 = w.msrc + p1;
       (void)hipStreamWaitEvent(sb, w.ev_next, 0);
       if(rec) (void)hipEventRecord(pe[0], sb);
-      hipLaunchKernelGGL((diag_lu<T>), dim3(1, 1, nb), dim3(512), 0, sb, A, lda, p0, dk(p0), d0, s0, c0, w.perm,
+      hipLaunchKernelGGL((diag_lu<T>), dim3(1, 1, nb), dim3(512), 0, sb, A, lda, p0, dk(p0), w.msrc + p0, w.perm,
                          w.status, bs);
-      if(rest0 > 0)
-        hipLaunchKernelGGL((blk_mul<T, false>), dim3(rest0 / 64, 1, nb), dim3(256), 0, sb, A, lda, p0, p1,
-                           dk(p0) + kNB * kNB, bs);
       if(two) {
-        laswp<T>(A, lda, p1, p1 + kNB, d0, s0, c0, -1, sb, nb, bs);
-        hipLaunchKernelGGL((blk_mul<T, true>), dim3(1, 1, nb), dim3(256), 0, sb, A, lda, p0, p1, dk(p0), bs);
+        panel_products<T, false>(A, lda, p0, p1, rest0, p1, kNB, p1, dk(p0), nullptr, m0, nullptr, sb, nb, bs);
         trailing_update<T, kNB, ThinTile>(A, lda, p1, p1, p0, Np - p1, kNB, sb, nb, bs.a);
-        hipLaunchKernelGGL((diag_lu<T>), dim3(1, 1, nb), dim3(512), 0, sb, A, lda, p1, dk(p1), d1, s1, c1, w.perm,
+        hipLaunchKernelGGL((diag_lu<T>), dim3(1, 1, nb), dim3(512), 0, sb, A, lda, p1, dk(p1), w.msrc + p1, w.perm,
                            w.status, bs);
-        if(restf > 0)
-          hipLaunchKernelGGL((blk_mul<T, false>), dim3(restf / 64, 1, nb), dim3(256), 0, sb, A, lda, p1, far,
-                             dk(p1) + kNB * kNB, bs);
       }
+      // L21 of p1 goes with the far columns' strips, unless they wait for a bulk
+      // update that it can run beside
+      const bool apart = (long)restf / 16 * nb > kWideStrips;
+      if(two && restf > 0 && apart)
+        panel_products<T, true>(A, lda, p0, p1, restf, far, 0, far, dk(p0), dk(p1), m0, m1, sb, nb, bs);
       if(rec) (void)hipEventRecord(pe[1], sb);
       if(two && restf > 0) {
         (void)hipStreamWaitEvent(sb, w.ev_bulk, 0);
-        laswp<T>(A, lda, far, Np, d0, s0, c0, -1, sb, nb, bs);
-        hipLaunchKernelGGL((blk_mul<T, true>), dim3(restf / 64, 1, nb), dim3(256), 0, sb, A, lda, p0, far, dk(p0), bs);
-        trailing_update<T, kNB, ThinTile>(A, lda, p1, far, p0, kNB, restf, sb, nb, bs.a);
-        laswp<T>(A, lda, far, Np, d1, s1, c1, -1, sb, nb, bs);
-        hipLaunchKernelGGL((blk_mul<T, true>), dim3(restf / 64, 1, nb), dim3(256), 0, sb, A, lda, p1, far, dk(p1), bs);
+        panel_products<T, true>(A, lda, p0, p1, apart ? 0 : restf, far, restf, far, dk(p0), dk(p1), m0, m1, sb, nb, bs);
       }
       (void)hipEventRecord(w.ev_pan, sb);
       (void)hipStreamWaitEvent(st, w.ev_pan, 0);
@@ -1433,8 +1454,8 @@ int lu_factor(T *A, int Np, size_t lda, LuWork &w, hipStream_t st, LuProf *prof)
     }
     if(w.ev_mark && Np < w.mark_col) mark(w, st);
     if(Np > kNB)
-      hipLaunchKernelGGL((laswp_left<T>), dim3((Np - kNB) / 8, Np / kNB - 1, nb), dim3(256), 0, st, A, lda, w.mdst,
-                         w.msrc, w.mcnt, bs);
+      hipLaunchKernelGGL((laswp_left<T>), dim3((Np - kNB) / 8, Np / kNB - 1, nb), dim3(256), 0, st, A, lda,
+                         w.msrc, bs);
     return 0;
   }
 
@@ -1463,8 +1484,7 @@ int lu_factor(T *A, int Np, size_t lda, LuWork &w, hipStream_t st, LuProf *prof)
   // L21 and U12 of panel j0
   auto solves = [&](int j0) {
     const int rest = Np - j0 - kNB;
-    if(rest > 0)
-      hipLaunchKernelGGL((blk_mul_both<T>), dim3(rest / 64, 2), dim3(256), 0, st, A, lda, j0, j0 + kNB, dk(j0));
+    panel_products<T, false>(A, lda, j0, 0, rest, j0 + kNB, rest, j0 + kNB, dk(j0), nullptr, nullptr, nullptr, st, 1, bs);
   };
   if((Np + kPanelRows - 1) / kPanelRows > w.gmax) return -2;
   pivoting(0);
