@@ -1103,9 +1103,8 @@ void trailing_update(T *A, size_t lda, int row0, int col0, int k0, int M, int N,
 // 128-byte runs.
 //
 // LDS holds the three split planes of a K chunk as 16-byte units (4 complex k
-// of one row of A or one column of B); the global loads of chunk c + 2 are in
-// flight while chunk c is multiplied, and C's tile is fetched during the last
-// chunk.  Workgroups are numbered so that each XCD takes a contiguous range of
+// of one row of A or one column of B); the global loads of chunk c + 1 are in
+// flight while chunk c is multiplied.  Workgroups are numbered so that each XCD takes a contiguous range of
 // tiles, walked in groups of GM tile rows (operands reused from its L2).
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -1118,49 +1117,52 @@ __device__ inline f32x16 mfma_bf16_32(u32x4 a, u32x4 b, f32x16 c) {
 
 // f[0..7] -> three words of 8 bf16 each (x1, x2, x3 of every value)
 __device__ inline void split_bf16x3(const float *f, u32x4 &h, u32x4 &m, u32x4 &l) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  auto pack = [](float a, float b) {  // one conversion for both
+    const f32x2 v = {a, b};
+    return __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2));
+  };
+  auto rest = [](float x, unsigned half) { return x - __uint_as_float(half); };
 #pragma unroll
   for(int d = 0; d < 4; ++d) {
-    unsigned hh[2], mm[2], ll[2];
-#pragma unroll
-    for(int e = 0; e < 2; ++e) {
-      const float x = f[2 * d + e];
-      const __bf16 b1 = (__bf16)x;
-      const float r1 = x - (float)b1;
-      const __bf16 b2 = (__bf16)r1;
-      const float r2 = r1 - (float)b2;
-      const __bf16 b3 = (__bf16)r2;
-      hh[e] = __builtin_bit_cast(unsigned short, b1);
-      mm[e] = __builtin_bit_cast(unsigned short, b2);
-      ll[e] = __builtin_bit_cast(unsigned short, b3);
-    }
-    h[d] = hh[0] | (hh[1] << 16);
-    m[d] = mm[0] | (mm[1] << 16);
-    l[d] = ll[0] | (ll[1] << 16);
+    const float x = f[2 * d], y = f[2 * d + 1];
+    h[d] = pack(x, y);
+    const float x1 = rest(x, h[d] << 16), y1 = rest(y, h[d] & 0xffff0000u);
+    m[d] = pack(x1, y1);
+    l[d] = pack(rest(x1, m[d] << 16), rest(y1, m[d] & 0xffff0000u));
   }
 }
 
-// DB: the split planes double-buffered in LDS, so that each wave splits and
-// stores chunk c + 1 while its products of chunk c run (one barrier per
-// chunk); the products and their order are those of the single buffer.
-template <int TM, int TN, int KD, int WGM, int WGN, int BK, int GM, bool DB = false, bool NTC = false>
-__global__ __launch_bounds__(64 * WGM * WGN) void gemm_split(float2 *A, size_t lda, int row0, int col0, int k0, int M,
-                                                            int N, size_t sA) {
+// A wave of the 4 holds 64 x 64 of the tile in 128 accumulator registers, so that
+// an operand read from LDS feeds two instructions, and the planes of one chunk
+// take 48 KB: two workgroups share a CU, the one's loads, splitting and C tile
+// beside the other's products.
+//
+// Bound: the matrix cores.  Per K = 128 at M = N = 9984 a pass costs 416 us (245
+// TFLOP/s complex, six times that in bf16) and 200 us for C and the ends: 165
+// TFLOP/s with K = 128, 198 with K = 256.  Eight waves of 32 x 64 in one
+// workgroup per CU, double-buffered, C fetched during the last chunk: 154 and
+// 185.  The products and their order, and so the bits, are the same.
+template <int TM, int TN, int KD, int WGM, int WGN, int BK, int GM>
+__global__ __launch_bounds__(64 * WGM * WGN, 2) void gemm_split(float2 *A, size_t lda, int row0, int col0, int k0,
+                                                               int M, int N, size_t sA) {
   A += blockIdx.z * sA;
   constexpr int NT = 64 * WGM * WGN;
   constexpr int WM = TM / WGM, WN = TN / WGN, FM = WM / 32, FN = WN / 32;
-  constexpr int KG = BK / 4, NC = KD / BK, NBUF = DB ? 2 : 1;
+  constexpr int KG = BK / 4, NC = KD / BK;
   constexpr int UA = TM * KG / NT, UB = TN * KG / NT;
   static_assert(UA * NT == TM * KG && UB * NT == TN * KG, "tile not divisible");
   static_assert(FM >= 1 && FN >= 1 && BK % 8 == 0 && KD % BK == 0, "tile shape");
-  __shared__ u32x4 Ys[NBUF][3][KG][TM];
-  __shared__ u32x4 Xs[NBUF][3][KG][TN];
+  __shared__ u32x4 Ys[3][KG][TM];
+  __shared__ u32x4 Xs[3][KG][TN];
   const int gx = (M + TM - 1) / TM, gy = (N + TN - 1) / TN, T = gx * gy;
   int L = blockIdx.x;
   const int full = T / 8 * 8;
   if(L < full) L = (L % 8) * (full / 8) + L / 8;
   const int per = GM * gy, g0 = (L / per) * GM, gsz = min(gx - g0, GM), r = L % per;
   const int bm = (g0 + r % gsz) * TM, bn = (r / gsz) * TN;
-  const int t = threadIdx.x, lane = t & 63, wv = t >> 6, wm = wv % WGM, wn = wv / WGM;
+  const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6), wm = wv % WGM, wn = wv / WGM;
   f32x16 accR[FM][FN], accI[FM][FN];
 #pragma unroll
   for(int a = 0; a < FM; ++a)
@@ -1169,109 +1171,66 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_split(float2 *A, size_t l
       accR[a][b] = f32x16{};
       accI[a][b] = f32x16{};
     }
-  float ga[2][UA][8], gb[2][UB][8];
-  auto gload = [&](int kc, int sl) {
+  // rows and columns past the end read the last one: their products are not stored
+  const float2 *pa[UA], *pb[UB];
 #pragma unroll
-    for(int i = 0; i < UA; ++i) {
-      const int u = t + NT * i, m = u % TM, kg = u / TM;
-#pragma unroll
-      for(int j = 0; j < 4; ++j) {
-        ga[sl][i][2 * j] = 0;
-        ga[sl][i][2 * j + 1] = 0;
-        if(bm + m < M) {
-          const float2 v = A[(size_t)(k0 + kc + 4 * kg + j) * lda + row0 + bm + m];
-          ga[sl][i][2 * j] = v.x;
-          ga[sl][i][2 * j + 1] = v.y;
-        }
-      }
-    }
-#pragma unroll
-    for(int i = 0; i < UB; ++i) {
-      const int u = t + NT * i, kg = u % KG, n = u / KG;
-#pragma unroll
-      for(int j = 0; j < 8; ++j) gb[sl][i][j] = 0;
-      if(bn + n < N) {
-        const float4 *p = reinterpret_cast<const float4 *>(A + (size_t)(col0 + bn + n) * lda + k0 + kc + 4 * kg);
-        const float4 p0 = p[0], p1 = p[1];
-        gb[sl][i][0] = p0.x;
-        gb[sl][i][1] = p0.y;
-        gb[sl][i][2] = p0.z;
-        gb[sl][i][3] = p0.w;
-        gb[sl][i][4] = p1.x;
-        gb[sl][i][5] = p1.y;
-        gb[sl][i][6] = p1.z;
-        gb[sl][i][7] = p1.w;
-      }
-    }
-  };
-  // C's tile: lane l, register v of block (a, b) holds D[n][m] with
-  // m = 32 a + l % 32, n = 32 b + 8 (v / 4) + 4 (l / 32) + v % 4; M and N are
-  // multiples of 32, so each 32 x 32 block is wholly in or out of range
-  float vr[FM][FN][16], vi[FM][FN][16];
-  auto cload = [&]() {
-#pragma unroll
-    for(int a = 0; a < FM; ++a)
-#pragma unroll
-      for(int b = 0; b < FN; ++b) {
-        const int mb = bm + wm * WM + 32 * a, nb = bn + wn * WN + 32 * b;
-        const bool ok = mb < M && nb < N;
-#pragma unroll
-        for(int v = 0; v < 16; ++v) {
-          vr[a][b][v] = 0;
-          vi[a][b][v] = 0;
-          if(ok) {
-            const int n = nb + 8 * (v / 4) + 4 * (lane >> 5) + (v % 4), m = mb + (lane & 31);
-            const float2 *cp = A + (size_t)(col0 + n) * lda + row0 + m;
-            const float2 c = NTC ? ld_stream(cp) : *cp;
-            vr[a][b][v] = c.x;
-            vi[a][b][v] = c.y;
-          }
-        }
-      }
-  };
-  // chunk c's operands from register slot sl, split into LDS buffer buf
-  auto split_store = [&](int sl, int buf) {
-#pragma unroll
-    for(int i = 0; i < UA; ++i) {
-      const int u = t + NT * i, m = u % TM, kg = u / TM;
-      u32x4 h, md, lo;
-      split_bf16x3(ga[sl][i], h, md, lo);
-      Ys[buf][0][kg][m] = h;
-      Ys[buf][1][kg][m] = md;
-      Ys[buf][2][kg][m] = lo;
-    }
-#pragma unroll
-    for(int i = 0; i < UB; ++i) {
-      const int u = t + NT * i, kg = u % KG, n = u / KG;
-      u32x4 h, md, lo;
-      split_bf16x3(gb[sl][i], h, md, lo);
-      Xs[buf][0][kg][n] = h;
-      Xs[buf][1][kg][n] = md;
-      Xs[buf][2][kg][n] = lo;
-    }
-  };
-  gload(0, 0);
-  if(NC > 1) gload(BK, 1);
-  if constexpr(DB) {
-    split_store(0, 0);
-    __syncthreads();
-    if(NC > 2) gload(2 * BK, 0);
+  for(int i = 0; i < UA; ++i) {
+    const int u = t + NT * i, m = u % TM, kg = u / TM;
+    pa[i] = A + (size_t)(k0 + 4 * kg) * lda + row0 + min(bm + m, M - 1);
   }
 #pragma unroll
-  for(int c = 0; c < NC; ++c) {
-    const int sl = c & 1, buf = DB ? (c & 1) : 0;
-    if constexpr(DB) {
-      // chunk c + 1 into the other buffer (read by every wave before the
-      // barrier that closed the previous chunk), then its slot refilled
-      if(c + 1 < NC) split_store((c + 1) & 1, buf ^ 1);
-      if(c + 3 < NC) gload((c + 3) * BK, (c + 1) & 1);
-    } else {
-      __syncthreads();  // the previous chunk has been read out of LDS
-      split_store(sl, 0);
-      __syncthreads();
-      if(c + 2 < NC) gload((c + 2) * BK, sl);
+  for(int i = 0; i < UB; ++i) {
+    const int u = t + NT * i, kg = u % KG, n = u / KG;
+    pb[i] = A + (size_t)(col0 + min(bn + n, N - 1)) * lda + k0 + 4 * kg;
+  }
+  float ga[UA][8], gb[UB][8];
+  auto gload = [&](int kc) {
+#pragma unroll
+    for(int i = 0; i < UA; ++i)
+#pragma unroll
+      for(int j = 0; j < 4; ++j) {
+        const float2 v = pa[i][(size_t)(kc + j) * lda];
+        ga[i][2 * j] = v.x;
+        ga[i][2 * j + 1] = v.y;
+      }
+#pragma unroll
+    for(int i = 0; i < UB; ++i) {
+      const float4 *p = reinterpret_cast<const float4 *>(pb[i] + kc);
+      const float4 p0 = p[0], p1 = p[1];
+      gb[i][0] = p0.x;
+      gb[i][1] = p0.y;
+      gb[i][2] = p0.z;
+      gb[i][3] = p0.w;
+      gb[i][4] = p1.x;
+      gb[i][5] = p1.y;
+      gb[i][6] = p1.z;
+      gb[i][7] = p1.w;
     }
-    if(c + 1 == NC) cload();
+  };
+  gload(0);
+#pragma unroll 1
+  for(int c = 0; c < NC; ++c) {
+    __syncthreads();  // the previous chunk has been read out of LDS
+#pragma unroll
+    for(int i = 0; i < UA; ++i) {
+      const int u = t + NT * i, m = u % TM, kg = u / TM;
+      u32x4 h, md, lo;
+      split_bf16x3(ga[i], h, md, lo);
+      Ys[0][kg][m] = h;
+      Ys[1][kg][m] = md;
+      Ys[2][kg][m] = lo;
+    }
+#pragma unroll
+    for(int i = 0; i < UB; ++i) {
+      const int u = t + NT * i, kg = u % KG, n = u / KG;
+      u32x4 h, md, lo;
+      split_bf16x3(gb[i], h, md, lo);
+      Xs[0][kg][n] = h;
+      Xs[1][kg][n] = md;
+      Xs[2][kg][n] = lo;
+    }
+    __syncthreads();
+    if(c + 1 < NC) gload((c + 1) * BK);
 #pragma unroll
     for(int ks = 0; ks < BK / 8; ++ks) {
       // lane l feeds rows/columns l % 32 at k' = 16 ks + 8 (l / 32) .. + 7
@@ -1280,10 +1239,10 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_split(float2 *A, size_t l
 #pragma unroll
       for(int s = 0; s < 3; ++s) {
 #pragma unroll
-        for(int b = 0; b < FN; ++b) x[s][b] = Xs[buf][s][kg][wn * WN + 32 * b + li];
+        for(int b = 0; b < FN; ++b) x[s][b] = Xs[s][kg][wn * WN + 32 * b + li];
 #pragma unroll
         for(int a = 0; a < FM; ++a) {
-          const u32x4 y = Ys[buf][s][kg][wm * WM + 32 * a + li];
+          const u32x4 y = Ys[s][kg][wm * WM + 32 * a + li];
 #pragma unroll
           for(int d = 0; d < 4; ++d) {
             yr[s][a][d] = y[d] ^ 0x80000000u;
@@ -1303,63 +1262,59 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_split(float2 *A, size_t l
             accI[a][b] = mfma_bf16_32(x[SX[p]][b], yi[SY[p]][a], accI[a][b]);
           }
     }
-    if constexpr(DB) __syncthreads();  // chunk c read out; chunk c + 1 stored
   }
+  // C's tile: lane l, register v of block (a, b) holds D[n][m] with
+  // m = 32 a + l % 32, n = 32 b + 8 (v / 4) + 4 (l / 32) + v % 4; M and N are
+  // multiples of 32, so each 32 x 32 block is wholly in or out of range.  Read
+  // and written with the nontemporal hint (2 % at M = N = 9984)
 #pragma unroll
-  for(int a = 0; a < FM; ++a)
+  for(int b = 0; b < FN; ++b)
 #pragma unroll
-    for(int b = 0; b < FN; ++b) {
+    for(int a = 0; a < FM; ++a) {
       const int mb = bm + wm * WM + 32 * a, nb = bn + wn * WN + 32 * b;
       if(mb >= M || nb >= N) continue;
+      float2 *cp = A + (size_t)(col0 + nb + 4 * (lane >> 5)) * lda + row0 + mb + (lane & 31);
+      float2 c[16];
+#pragma unroll
+      for(int v = 0; v < 16; ++v) c[v] = ld_stream(cp + (size_t)(8 * (v / 4) + (v % 4)) * lda);
 #pragma unroll
       for(int v = 0; v < 16; ++v) {
-        const int n = nb + 8 * (v / 4) + 4 * (lane >> 5) + (v % 4), m = mb + (lane & 31);
-        float2 c;
-        c.x = vr[a][b][v] - accR[a][b][v];
-        c.y = vi[a][b][v] - accI[a][b][v];
-        if constexpr(NTC)
-          st_stream(A + (size_t)(col0 + n) * lda + row0 + m, c);
-        else
-          A[(size_t)(col0 + n) * lda + row0 + m] = c;
+        c[v].x -= accR[a][b][v];
+        c[v].y -= accI[a][b][v];
+        st_stream(cp + (size_t)(8 * (v / 4) + (v % 4)) * lda, c[v]);
       }
     }
 }
 
-// Tile of the split-bf16 update (fastest of a sweep at M = N = 10112,
-// K = 128: 145 TFLOP/s complex, against 87 for gemm_tile<float2> on the same
-// random data).
+// Tile of the split-bf16 update (fastest of a sweep at M = N = 9984 and at 16
+// systems of 2304; 128 x 64 with 2 or 4 waves, chunks of 8 double-buffered and 8
+// waves are within 8 % or slower).
 struct SplitTile {
-  static constexpr int TM = 128, TN = 128, WGM = 4, WGN = 2, BK = 16, GM = 8;
-  // double-buffered split planes: bit-identical, 149 against 125 TFLOP/s at
-  // M = N = 10112 (one matrix), 156 against 154 for 64 systems of 3712
-  static constexpr bool DB = true;
-  // C's tile read and written with the nontemporal hint: bit-identical, 5510
-  // against 5644 us for 64 systems of 3840 (2.4%), 1-5% at one matrix of 10240
-  static constexpr bool NTC = true;
+  static constexpr int TM = 128, TN = 128, WGM = 2, WGN = 2, BK = 16, GM = 8;
 };
 
-// The bulk update with K = 2 NB: split-bf16 for FP32 factors when `split`,
-// gemm_tile otherwise.  M and N are multiples of 64.
-template <typename T>
+// The bulk update with K = KD (2 NB or 4 NB): split-bf16 for FP32 factors when
+// `split`, gemm_tile otherwise.  M and N are multiples of 64.
+template <typename T, int KD = 2 * kNB>
 void bulk_update(T *A, size_t lda, int row0, int col0, int k0, int M, int N, hipStream_t st, int nb, size_t sA,
                  bool split) {
   if(M <= 0 || N <= 0) return;
   if(N <= 2 * kNB) {
     // the next pair's columns (on the panel chain's critical path): small
     // tiles over many workgroups finish sooner than a few large split tiles
-    trailing_update<T, 2 * kNB, ThinTile>(A, lda, row0, col0, k0, M, N, st, nb, sA);
+    trailing_update<T, KD, ThinTile>(A, lda, row0, col0, k0, M, N, st, nb, sA);
     return;
   }
   if constexpr(std::is_same<T, float2>::value) {
     if(split) {
       using U = SplitTile;
       const int tiles = ((M + U::TM - 1) / U::TM) * ((N + U::TN - 1) / U::TN);
-      hipLaunchKernelGGL((gemm_split<U::TM, U::TN, 2 * kNB, U::WGM, U::WGN, U::BK, U::GM, U::DB, U::NTC>), dim3(tiles, 1, nb),
+      hipLaunchKernelGGL((gemm_split<U::TM, U::TN, KD, U::WGM, U::WGN, U::BK, U::GM>), dim3(tiles, 1, nb),
                          dim3(64 * U::WGM * U::WGN), 0, st, A, lda, row0, col0, k0, M, N, sA);
       return;
     }
   }
-  trailing_update<T, 2 * kNB>(A, lda, row0, col0, k0, M, N, st, nb, sA);
+  trailing_update<T, KD>(A, lda, row0, col0, k0, M, N, st, nb, sA);
 }
 
 // ------------------------------------------------------------------ driver
