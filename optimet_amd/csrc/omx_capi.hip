@@ -959,6 +959,7 @@ void capture_at_mark(void *arg) {
   HIPCHK(hipStreamEndCapture(c->st2, &cm->gv));
   HIPCHK(hipStreamBeginCapture(c->st, hipStreamCaptureModeThreadLocal));
   HIPCHK(hipEventRecord(c->lu.ev_next, c->st));
+  HIPCHK(hipEventRecord(c->lu.ev_piv, c->st));
   HIPCHK(hipEventRecord(c->lu.ev_bulk, c->st));
 }
 

@@ -1293,15 +1293,17 @@ struct SplitTile {
   static constexpr int TM = 128, TN = 128, WGM = 2, WGN = 2, BK = 16, GM = 8;
 };
 
+constexpr long kThinRows = 16384;  // columns that fill the chip with split tiles of 128 rows, half of it busy
 // The bulk update with K = KD (2 NB or 4 NB): split-bf16 for FP32 factors when
 // `split`, gemm_tile otherwise.  M and N are multiples of 64.
 template <typename T, int KD = 2 * kNB>
 void bulk_update(T *A, size_t lda, int row0, int col0, int k0, int M, int N, hipStream_t st, int nb, size_t sA,
                  bool split) {
   if(M <= 0 || N <= 0) return;
-  if(N <= 2 * kNB) {
-    // the next pair's columns (on the panel chain's critical path): small
-    // tiles over many workgroups finish sooner than a few large split tiles
+  if(N <= 2 * kNB || (M <= 2 * kNB && (long)N * nb <= kThinRows)) {
+    // the next pair's columns or a second pair's block rows (on the panel chain's
+    // critical path): small tiles over many workgroups finish sooner than a few
+    // large split tiles (128 rows by 1800 columns: 9 us against 29)
     trailing_update<T, KD, ThinTile>(A, lda, row0, col0, k0, M, N, st, nb, sA);
     return;
   }
@@ -1318,17 +1320,21 @@ void bulk_update(T *A, size_t lda, int row0, int col0, int k0, int M, int N, hip
 }
 
 // ------------------------------------------------------------------ driver
-// Panels of NB columns are taken in pairs (p0 = J, p1 = J + NB) so that the
-// bulk of the trailing update runs with K = 2 NB.
+// Panels of NB columns are taken in pairs (p0 = J, p1 = J + NB), and pairs in
+// groups of one or two, so that the bulk of the trailing update runs with K = 2 NB
+// or 4 NB.
 //
 // Block pivoting (interchanges stay inside a panel's 64 rows), two streams:
-// sb (panel work) runs pair s+1 while st (bulk updates) finishes pair s.
+// sb (panel work) runs group s+1 while st (bulk updates) finishes group s.
 //   sb  diag_lu p0; L21(p0) and U12(p0) on p1's columns; p1's columns -=
 //       L21(p0) U12(p0); diag_lu p1
-//   sb  after st's bulk update of pair s-1: L21(p1); on the far columns U12(p0),
-//       block row p1 -= L(p1, p0) U12(p0), U12(p1) (one launch)
-//   st  A22 -= [L21(p0) L21(p1)] [U12(p0); U12(p1)]: the next pair's
-//       columns first (sb starts on them), then the rest
+//   sb  (groups of two) L21(p1) and U12 of both on the second pair's columns;
+//       these columns' update with K = 2 NB; the second pair as the first
+//   sb  after st's bulk update of group s-1, on the far columns: U12(p0), block
+//       row p1 -= L(p1, p0) U12(p0), U12(p1) (one launch); (groups of two) the
+//       second pair's block rows' update with K = 2 NB, then their U12
+//   st  A22 -= [L21 ..] [U12; ..]: the next group's columns first, pair by pair
+//       (sb starts on them), then the rest
 // Interchanges on the columns left of each panel are applied once at the end
 // (panels touch disjoint rows, so their order does not matter).
 //
@@ -1358,54 +1364,98 @@ int lu_factor(T *A, int Np, size_t lda, LuWork &w, hipStream_t st, LuProf *prof)
     prof->gemm_launches = 0;
   }
   if(block) {
-    (void)hipEventRecord(w.ev_next, st);
-    (void)hipEventRecord(w.ev_bulk, st);
-    for(int J = 0, pi = 0; J < Np; J += 2 * kNB, ++pi) {
-      const int p0 = J, p1 = J + kNB, far = J + 2 * kNB;
-      const bool two = p1 < Np;
-      const int rest0 = Np - p0 - kNB, restf = Np - far;
-      const bool rec = prof && pi < prof->cap;
-      hipEvent_t *pe = rec ? prof->ev + 4 * pi : nullptr;
-      const int *m0 = w.msrc + p0, *m1 = w.msrc + p1;
-      (void)hipStreamWaitEvent(sb, w.ev_next, 0);
-      if(rec) (void)hipEventRecord(pe[0], sb);
+    // G panels a group: quads (two pairs), whose bulk update has K = 4 NB, where
+    // that update is the split-bf16 one, which C's traffic holds back at K = 2 NB;
+    // pairs where gemm_tile does it, which the matrix cores bound at either K and
+    // whose quads only lengthen the panel chain.  Mixed solves with quads / pairs:
+    // N = 2720 4.63 / 4.70 ms, 10240 42.9 / 44.9 ms, 16 wavelengths of 2560 226 / 233
+    // ms; FP64, N = 2208 4.48 / 4.10 ms
+    constexpr bool f32 = std::is_same<T, float2>::value;
+    const int G = f32 && w.split ? 4 : 2;
+    // a pair's panels (the second if two); its columns are up to date
+    auto pair = [&](int p0, bool two) {
+      const int p1 = p0 + kNB;
       hipLaunchKernelGGL((diag_lu<T>), dim3(1, 1, nb), dim3(512), 0, sb, A, lda, p0, dk(p0), w.msrc + p0, w.perm,
                          w.status, bs);
-      if(two) {
-        panel_products<T, false>(A, lda, p0, p1, rest0, p1, kNB, p1, dk(p0), nullptr, m0, nullptr, sb, nb, bs);
-        trailing_update<T, kNB, ThinTile>(A, lda, p1, p1, p0, Np - p1, kNB, sb, nb, bs.a);
-        hipLaunchKernelGGL((diag_lu<T>), dim3(1, 1, nb), dim3(512), 0, sb, A, lda, p1, dk(p1), w.msrc + p1, w.perm,
-                           w.status, bs);
+      if(!two) return;
+      panel_products<T, false>(A, lda, p0, p1, Np - p1, p1, kNB, p1, dk(p0), nullptr, w.msrc + p0, nullptr, sb, nb, bs);
+      trailing_update<T, kNB, ThinTile>(A, lda, p1, p1, p0, Np - p1, kNB, sb, nb, bs.a);
+      hipLaunchKernelGGL((diag_lu<T>), dim3(1, 1, nb), dim3(512), 0, sb, A, lda, p1, dk(p1), w.msrc + p1, w.perm,
+                         w.status, bs);
+    };
+    // L21 of a pair's second panel on rows >= p0 + 2 NB (when l21); U12 of both on
+    // cols columns from c0
+    auto through = [&](int p0, bool l21, int cols, int c0) {
+      const int p1 = p0 + kNB, below = p1 + kNB;
+      panel_products<T, true>(A, lda, p0, p1, l21 ? Np - below : 0, below, cols, c0, dk(p0), dk(p1), w.msrc + p0,
+                              w.msrc + p1, sb, nb, bs);
+    };
+    // ev_next, ev_piv: the next group's first and second pair are up to date
+    (void)hipEventRecord(w.ev_next, st);
+    (void)hipEventRecord(w.ev_piv, st);
+    (void)hipEventRecord(w.ev_bulk, st);
+    for(int J = 0, pi = 0; J < Np; J += G * kNB, ++pi) {
+      const int np = std::min(G, (Np - J) / kNB);  // panels of this group
+      const int q = J + 2 * kNB, far = J + np * kNB, restf = Np - far;
+      const bool rec = prof && pi < prof->cap;
+      hipEvent_t *pe = rec ? prof->ev + 4 * pi : nullptr;
+      (void)hipStreamWaitEvent(sb, w.ev_next, 0);
+      if(rec) (void)hipEventRecord(pe[0], sb);
+      pair(J, np > 1);
+      if(np > 2) {
+        // the second pair's columns: through the first, then its update
+        (void)hipStreamWaitEvent(sb, w.ev_piv, 0);
+        through(J, true, (np - 2) * kNB, q);
+        bulk_update<T>(A, lda, q, q, J, Np - q, (np - 2) * kNB, sb, nb, bs.a, w.split);
+        pair(q, np > 3);
       }
-      // L21 of p1 goes with the far columns' strips, unless they wait for a bulk
-      // update that it can run beside
-      const bool apart = (long)restf / 16 * nb > kWideStrips;
-      if(two && restf > 0 && apart)
-        panel_products<T, true>(A, lda, p0, p1, restf, far, 0, far, dk(p0), dk(p1), m0, m1, sb, nb, bs);
+      // L21 of the last panel goes with the far columns' strips, unless they wait
+      // for a bulk update that it can run beside
+      const int last = far - 2 * kNB;  // the group's last pair
+      const bool apart = restf > 0 && (long)restf / 16 * nb > kWideStrips;
+      if(apart) through(last, true, 0, far);
       if(rec) (void)hipEventRecord(pe[1], sb);
-      if(two && restf > 0) {
+      if(restf > 0) {
         (void)hipStreamWaitEvent(sb, w.ev_bulk, 0);
-        panel_products<T, true>(A, lda, p0, p1, apart ? 0 : restf, far, restf, far, dk(p0), dk(p1), m0, m1, sb, nb, bs);
+        if(G == 4) {
+          through(J, false, restf, far);
+          bulk_update<T>(A, lda, q, far, J, 2 * kNB, restf, sb, nb, bs.a, w.split);
+        }
+        through(last, !apart, restf, far);
       }
       (void)hipEventRecord(w.ev_pan, sb);
       (void)hipStreamWaitEvent(st, w.ev_pan, 0);
       if(rec) (void)hipEventRecord(pe[2], st);
-      if(two && restf > 0) {
-        const int nn = restf < 2 * kNB ? restf : 2 * kNB;
-        bulk_update<T>(A, lda, far, far, p0, restf, nn, st, nb, bs.a, w.split);
+      if(restf > 0) {
+        auto bulk = [&](int c0, int n) {
+          if constexpr(f32)
+            if(G == 4) return bulk_update<T, 4 * kNB>(A, lda, far, c0, J, restf, n, st, nb, bs.a, w.split);
+          bulk_update<T>(A, lda, far, c0, J, restf, n, st, nb, bs.a, w.split);
+        };
+        // the next group's first pair, its second, and the rest
+        int c0 = far;
+        const int n1 = std::min(2 * kNB, Np - c0);
+        bulk(c0, n1);
         (void)hipEventRecord(w.ev_next, st);
-        bulk_update<T>(A, lda, far, far + nn, p0, restf, restf - nn, st, nb, bs.a, w.split);
+        c0 += n1;
+        if(G == 4) {
+          const int n2 = std::min(2 * kNB, Np - c0);
+          bulk(c0, n2);
+          (void)hipEventRecord(w.ev_piv, st);
+          c0 += n2;
+        }
+        bulk(c0, Np - c0);
         (void)hipEventRecord(w.ev_bulk, st);
         if(rec) {
-          prof->gemm_flop += 8.0 * (double)restf * restf * (2 * kNB) * nb;
-          prof->gemm_launches += restf > nn ? 2 : 1;
+          prof->gemm_flop += 8.0 * (double)restf * restf * (G * kNB) * nb;
+          prof->gemm_launches += (restf > n1 ? 2 : 1) + (G == 4 && Np - far > 4 * kNB ? 1 : 0);
         }
       }
       if(rec) {
         (void)hipEventRecord(pe[3], st);
         prof->used = pi + 1;
       }
-      if(w.ev_mark && far >= w.mark_col && far - 2 * kNB < w.mark_col) mark(w, st);
+      if(w.ev_mark && far >= w.mark_col && J < w.mark_col) mark(w, st);
     }
     if(w.ev_mark && Np < w.mark_col) mark(w, st);
     if(Np > kNB)
