@@ -98,21 +98,45 @@ __device__ inline void sum_parts(const cplx *part, int ld, int nblk, int nv, cpl
   }
   __syncthreads();
 }
-// Partial sums of V_k^H w over the block's rows, k < nv, into out[k].
-__device__ inline void dots(const cplx *V, size_t ldk, int nv, cplx w, int r, int n, cplx *out, cplx (*red)[4]) {
-  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
-  for(int k0 = 0; k0 < nv; k0 += kRows) {
-    const int nk = min(kRows, nv - k0);
-    __syncthreads();
-#pragma unroll 4
-    for(int k = 0; k < nk; ++k) {
-      cplx s = mk(0.0);
-      if(r < n) s = conj(V[(size_t)(k0 + k) * ldk + r]) * w;
-      s = wave_red(s);
-      if(lane == 0) red[k][wv] = s;
+__device__ inline cplx shfl_xor(cplx v, int o) { return cplx{__shfl_xor(v.x, o, 64), __shfl_xor(v.y, o, 64)}; }
+// (sum of a) + (sum of b) + ((sum of c) + (sum of d)) over the wave, each sum by
+// halves (lanes 32 apart, 16 apart, ..), to every lane: the first two halvings
+// take two and four of the sums at once, in the lanes the others leave.
+__device__ inline cplx wave_red4(cplx a, cplx b, cplx c, cplx d) {
+  const bool hi = threadIdx.x & 32, hj = threadIdx.x & 16;
+  auto pick = [](bool p, cplx x, cplx y) { return cplx{p ? x.x : y.x, p ? x.y : y.y}; };
+  const cplx u = pick(hi, b, a) + shfl_xor(pick(hi, a, b), 32);
+  const cplx v = pick(hi, d, c) + shfl_xor(pick(hi, c, d), 32);
+  cplx s = pick(hj, v, u) + shfl_xor(pick(hj, u, v), 16);
+#pragma unroll
+  for(int o = 8; o > 0; o >>= 1) s = s + shfl_xor(s, o);
+  s = s + shfl_xor(s, 32);
+  return s + shfl_xor(s, 16);
+}
+
+// Partial sums of V_k^H w over the block's rows, k < nv, into out[k]: a wave takes
+// every fourth k over all 256 rows, one reduction each (with 64 rows a wave, and
+// so four reductions for every k, the step's two passes took 28 us instead of 16
+// at N = 2720, j = 35; the same sums).
+__device__ inline void dots(const cplx *V, size_t ldk, int nv, cplx w, int n, cplx *out, cplx (&ws)[kRows]) {
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6, r0 = blockIdx.x * kRows + lane;
+  __syncthreads();
+  ws[t] = w;
+  __syncthreads();
+  cplx x[4];
+#pragma unroll
+  for(int i = 0; i < 4; ++i) x[i] = ws[lane + 64 * i];
+#pragma unroll 2
+  for(int k = wv; k < nv; k += 4) {
+    const cplx *v = V + (size_t)k * ldk + r0;
+    cplx e[4];
+#pragma unroll
+    for(int i = 0; i < 4; ++i) {
+      e[i] = mk(0.0);
+      if(r0 + 64 * i < n) e[i] = conj(v[64 * i]) * x[i];
     }
-    __syncthreads();
-    if(t < nk) out[k0 + t] = (red[t][0] + red[t][1]) + (red[t][2] + red[t][3]);
+    const cplx s = wave_red4(e[0], e[1], e[2], e[3]);
+    if(lane == 0) out[k] = s;
   }
 }
 
@@ -120,7 +144,7 @@ __global__ __launch_bounds__(kRows) void kry_dots(KryState s, const cplx *gpart,
   const int z = blockIdx.y, j = s.j, r = blockIdx.x * kRows + threadIdx.x;
   const Sys q(s, z);
   if(!q.fl[KF_LIVE]) return;
-  __shared__ cplx red[kRows][4];
+  __shared__ cplx ws[kRows];
   cplx w = mk(0.0);
   cplx *W = s.w + z * s.sv;
   if(r < s.n) {
@@ -132,26 +156,26 @@ __global__ __launch_bounds__(kRows) void kry_dots(KryState s, const cplx *gpart,
       w = W[r];
     }
   }
-  dots(s.V + z * s.sz, s.ldk, j + 1, w, r, s.n, part_of(s, 0, z) + (size_t)blockIdx.x * (s.m + 2), red);
+  dots(s.V + z * s.sz, s.ldk, j + 1, w, s.n, part_of(s, 0, z) + (size_t)blockIdx.x * (s.m + 2), ws);
 }
 
 __global__ __launch_bounds__(kRows) void kry_orth(KryState s) {
   const int z = blockIdx.y, j = s.j, t = threadIdx.x, r = blockIdx.x * kRows + t;
   const Sys q(s, z);
   if(!q.fl[KF_LIVE]) return;
-  __shared__ cplx red[kRows][4], hs[260];
-  sum_parts(part_of(s, 0, z), s.m + 2, gridDim.x, j + 1, hs, &red[0][0]);
+  __shared__ cplx ws[kRows], hs[260];
+  sum_parts(part_of(s, 0, z), s.m + 2, gridDim.x, j + 1, hs, ws);
   if(blockIdx.x == 0)
     for(int k = t; k <= j; k += kRows) q.h[k] = hs[k];
   const cplx *V = s.V + z * s.sz;
   cplx w = mk(0.0);
   if(r < s.n) {
     w = s.w[z * s.sv + r];
-#pragma unroll 4
+#pragma unroll 8
     for(int k = 0; k <= j; ++k) w = w - V[(size_t)k * s.ldk + r] * hs[k];
     s.w[z * s.sv + r] = w;
   }
-  dots(V, s.ldk, j + 1, w, r, s.n, part_of(s, 1, z) + (size_t)blockIdx.x * (s.m + 2), red);
+  dots(V, s.ldk, j + 1, w, s.n, part_of(s, 1, z) + (size_t)blockIdx.x * (s.m + 2), ws);
 }
 
 __global__ __launch_bounds__(kRows) void kry_orth2(KryState s) {
@@ -167,7 +191,7 @@ __global__ __launch_bounds__(kRows) void kry_orth2(KryState s) {
   double e = 0.0;
   if(r < s.n) {
     cplx w = s.w[z * s.sv + r];
-#pragma unroll 4
+#pragma unroll 8
     for(int k = 0; k <= j; ++k) w = w - V[(size_t)k * s.ldk + r] * hs[k];
     s.w[z * s.sv + r] = w;
     e = norm2(w);
