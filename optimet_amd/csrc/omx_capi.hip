@@ -122,6 +122,7 @@ const double kBackwardErrorBound = 1e3 * 1.1e-16;
 constexpr int kInnerSteps = 30;
 constexpr double kInnerTol = 1e-6;
 
+constexpr int kMarkN = 9216;  // see omx_solve
 // OMX_SOLVER_AUTO: systems of order N >= kAutoKrylovN start with the mixed
 // Krylov, within a budget of outer steps whose matvecs cost what the mixed LU
 // would (8/3 N^3 flop at about 140 TFLOP/s against an 8 N^2-byte product at
@@ -175,8 +176,9 @@ struct omx_context {
   // (OMX_SH_OVERLAP overrides; 0 starts both together)
   double sh_overlap = 0.5;
   // OMX_SOLVER_AUTO with S by GMRES: fraction of V's columns factored before
-  // S's GMRES starts (OMX_KRYLOV_MARK overrides; 0 starts both together)
-  double krylov_mark = 0.5;
+  // S's GMRES starts (OMX_KRYLOV_MARK overrides; 0 starts both together), from
+  // N = kMarkN on by default
+  double krylov_mark = -1.0;
   int lu32_gemm = OMX_GEMM_BF16X3;
   int fallbacks = 0;
   double tol = 1e-16;
@@ -2259,12 +2261,16 @@ int omx_solve(omx_context *c, double *x_sca, double *x_int, double *x_sca_sh, do
         c->lu.ev_mark = nullptr;
         c->lu.on_mark = nullptr;
       } else if(c->krylov_s && !c->factored) {
-        // S's GMRES starts once V's factorisation has passed krylov_mark of
-        // its columns: the first columns carry most of the bulk-update work,
-        // which the GMRES products would only slow down, and the panel-bound
-        // rest leaves the device room for them
+        // From kMarkN on, S's GMRES starts once V's factorisation has passed
+        // krylov_mark of its columns: the first columns carry most of the
+        // bulk-update work, which the GMRES products would only slow down, and
+        // the panel-bound rest leaves the device room for them.  Below, the whole
+        // factorisation is panel-bound and both start together.  Solves with 0 /
+        // 0.25 / 0.5: N = 1280 2.89 / 3.29 / 3.57 ms, 2720 5.05 / 5.71 / 6.08, 5120
+        // 11.4 / 11.7 / 12.6, 7200 21.0 / 22.6 / 24.0, 10240 42.1 / 41.6 / 43.0
         HIPCHK(hipEventRecord(c->xev[0], c->st));
-        const int kmark = (int)(c->krylov_mark * c->Np);
+        const double frac = c->krylov_mark >= 0.0 ? c->krylov_mark : c->N >= kMarkN ? 0.25 : 0.0;
+        const int kmark = (int)(frac * c->Np);
         if(kmark > 0) {
           c->lu_sh.ev_mark = c->xev[3];
           c->lu_sh.mark_col = kmark;
