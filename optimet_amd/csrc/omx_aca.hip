@@ -32,133 +32,136 @@ __device__ inline void wave_argmax(double &v, int &i) {
   }
 }
 
-// Workgroup argmax of v over threads (v < 0: not a candidate); every thread
-// returns the winning index, or -1 when no candidate has a non-zero modulus.
-__device__ inline int block_argmax(double v, double (*wv)[3], int *wi, int *out) {
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-  int i = t;
-  wave_argmax(v, i);
-  if(lane == 0) {
-    wv[w][0] = v;
-    wi[w] = i;
-  }
-  __syncthreads();
-  if(t == 0) {
-    double bv = wv[0][0];
-    int bi = wi[0];
-    for(int k = 1; k < (int)(blockDim.x >> 6); ++k)
-      if(wv[k][0] > bv || (wv[k][0] == bv && wi[k] < bi)) {
-        bv = wv[k][0];
-        bi = wi[k];
-      }
-    *out = bv > 0.0 ? bi : -1;
-  }
-  __syncthreads();
-  return *out;
-}
-
 }  // namespace
 
-// One workgroup (256 threads, thread t owns row / column t; n <= 256) per
-// block.  Step k: the residual row I_k against the k terms so far, its
+// One wave per block; lane l owns rows / columns l + 64 g, g < R (n <= 64 R <=
+// 256).  Step k: the residual row I_k against the k terms so far, its
 // largest unused entry J_k, v_k = row / pivot, the residual column J_k -> u_k,
 // the reference's norm estimate (the cross terms over p <= k-2 and the first
 // k entries, unconjugated, :826-843) and its stopping test for k >= 1, then
 // I_{k+1} = largest unused entry of u_k.  A residual row or column with no
 // non-zero candidate ends the iteration with the terms so far (they reproduce
 // the block exactly).
-__global__ __launch_bounds__(256) void aca_kernel(AcaArgs a) {
-  const int b = blockIdx.x, t = threadIdx.x, n = a.n;
-  const int lane = t & 63, w = t >> 6;
+//
+// Bound: the latency of a step's dependent reads, so by the blocks in flight.
+// With 256 threads a block, most of them idle at n = 70, and eight barriers a
+// step: 7.9 ms for the 90 000 blocks of 300 spheres; now 4.4 ms.
+template <int R> __global__ __launch_bounds__(64, R < 3 ? 4 : 2) void aca_kernel(AcaArgs a) {
+  const int b = blockIdx.x, lane = threadIdx.x, n = a.n;
   const cplx *A = a.A + (size_t)b * n * n;
   cplx *U = a.U + (size_t)b * n * n, *V = a.V + (size_t)b * n * n;
-  __shared__ cplx coef[256], uk[256], vk[256];
-  __shared__ unsigned char usedR[256], usedC[256];
-  __shared__ double wv[4][3];
-  __shared__ int wi[4];
-  __shared__ int s_idx, s_stop;
-  __shared__ cplx s_piv;
-  usedR[t] = 0;
-  usedC[t] = 0;
-  double norma = 0.0;  // thread 0's running estimate
+  __shared__ cplx coef[64 * R], uk[64 * R], vk[64 * R];
+  bool usedR[R], usedC[R];
+#pragma unroll
+  for(int g = 0; g < R; ++g) usedR[g] = usedC[g] = lane + 64 * g >= n;
+  // index of the largest |x| not used (the first on ties), -1 when all are zero
+  auto argmax = [&](const cplx(&x)[R], const bool(&used)[R]) {
+    double v = -1.0;
+    int i = lane;
+#pragma unroll
+    for(int g = 0; g < R; ++g) {
+      const double m = used[g] ? -1.0 : cabs(x[g]);
+      if(m > v) {
+        v = m;
+        i = lane + 64 * g;
+      }
+    }
+    wave_argmax(v, i);
+    return v > 0.0 ? i : -1;
+  };
+  double norma = 0.0;
   int ik = 0, r = 0;
-  __syncthreads();
   for(int k = 0; k < n; ++k) {
-    if(t == 0) usedR[ik] = 1;
-    if(t < k) coef[t] = U[(size_t)t * n + ik];  // U(I_k, p)
+#pragma unroll
+    for(int g = 0; g < R; ++g) usedR[g] = usedR[g] || lane + 64 * g == ik;
+    for(int p = lane; p < k; p += 64) coef[p] = U[(size_t)p * n + ik];  // U(I_k, p)
     __syncthreads();
-    cplx rv = mk(0.0);
-    if(t < n) {
-      cplx s = mk(0.0);
-      for(int p = 0; p < k; ++p) s = s + coef[p] * V[(size_t)p * n + t];
-      rv = A[(size_t)t * n + ik] - s;
+    cplx rv[R], u[R];
+#pragma unroll
+    for(int g = 0; g < R; ++g) {
+      const int t = lane + 64 * g;
+      rv[g] = mk(0.0);
+      if(t < n) {
+        const cplx e = A[(size_t)t * n + ik];
+        cplx s = mk(0.0);
+#pragma unroll 4
+        for(int p = 0; p < k; ++p) s = s + coef[p] * V[(size_t)p * n + t];
+        rv[g] = e - s;
+      }
     }
-    const int jk = block_argmax((t < n && !usedC[t]) ? cabs(rv) : -1.0, wv, wi, &s_idx);
+    const int jk = argmax(rv, usedC);
     if(jk < 0) break;
-    if(t == jk) {
-      s_piv = rv;
-      usedC[jk] = 1;
+    cplx piv = mk(0.0);
+#pragma unroll
+    for(int g = 0; g < R; ++g) {
+      if(jk >> 6 == g) piv = cplx{__shfl(rv[g].x, jk & 63, 64), __shfl(rv[g].y, jk & 63, 64)};
+      usedC[g] = usedC[g] || lane + 64 * g == jk;
     }
+    double sv[R], su[R];
     __syncthreads();
-    cplx v = mk(0.0);
-    if(t < n) {
-      v = rv / s_piv;
-      V[(size_t)k * n + t] = v;
-      vk[t] = v;
-    }
-    if(t < k) coef[t] = V[(size_t)t * n + jk];  // V(p, J_k)
-    __syncthreads();
-    cplx u = mk(0.0);
-    if(t < n) {
-      cplx s = mk(0.0);
-      for(int p = 0; p < k; ++p) s = s + coef[p] * U[(size_t)p * n + t];
-      u = A[(size_t)jk * n + t] - s;
-      U[(size_t)k * n + t] = u;
-      uk[t] = u;
-    }
-    __syncthreads();
-    double cross = 0.0;
-    if(t < k - 1) {  // p = t
-      cplx p1 = mk(0.0), p2 = mk(0.0);
-      for(int q = 0; q < k; ++q) {
-        p1 = p1 + U[(size_t)t * n + q] * uk[q];
-        p2 = p2 + V[(size_t)t * n + q] * vk[q];
+#pragma unroll
+    for(int g = 0; g < R; ++g) {
+      const int t = lane + 64 * g;
+      cplx v = mk(0.0);
+      if(t < n) {
+        v = rv[g] / piv;
+        V[(size_t)k * n + t] = v;
+        vk[t] = v;
       }
-      cross = cabs(p1) * cabs(p2);
+      sv[g] = norm2(v);
     }
-    double su = wave_sum(norm2(u)), sv = wave_sum(norm2(v));
-    cross = wave_sum(cross);
-    if(lane == 0) {
-      wv[w][0] = su;
-      wv[w][1] = sv;
-      wv[w][2] = cross;
+    for(int p = lane; p < k; p += 64) coef[p] = V[(size_t)p * n + jk];  // V(p, J_k)
+    __syncthreads();
+#pragma unroll
+    for(int g = 0; g < R; ++g) {
+      const int t = lane + 64 * g;
+      u[g] = mk(0.0);
+      if(t < n) {
+        const cplx e = A[(size_t)jk * n + t];
+        cplx s = mk(0.0);
+#pragma unroll 4
+        for(int p = 0; p < k; ++p) s = s + coef[p] * U[(size_t)p * n + t];
+        u[g] = e - s;
+        U[(size_t)k * n + t] = u[g];
+        uk[t] = u[g];
+      }
+      su[g] = norm2(u[g]);
     }
     __syncthreads();
-    if(t == 0) {
-      double SU = 0.0, SV = 0.0, CR = 0.0;
-      for(int q = 0; q < 4; ++q) {
-        SU += wv[q][0];
-        SV += wv[q][1];
-        CR += wv[q][2];
+    double SU = 0.0, SV = 0.0, CR = 0.0;
+#pragma unroll
+    for(int g = 0; g < R; ++g) {
+      const int t = lane + 64 * g;
+      double cross = 0.0;
+      if(t < k - 1) {  // p = t
+        cplx p1 = mk(0.0), p2 = mk(0.0);
+#pragma unroll 4
+        for(int q = 0; q < k; ++q) {
+          p1 = p1 + U[(size_t)t * n + q] * uk[q];
+          p2 = p2 + V[(size_t)t * n + q] * vk[q];
+        }
+        cross = cabs(p1) * cabs(p2);
       }
-      const double cn = sqrt(SU), rn = sqrt(SV);
-      int stop = 0;
-      if(k == 0) {
-        norma = cn * cn * (rn * rn);
-      } else {
-        norma = norma + cn * cn * (rn * rn) + 2.0 * CR;
-        stop = a.eps * sqrt(norma) >= cn * rn;
-      }
-      s_stop = stop;
+      SU += wave_sum(su[g]);
+      SV += wave_sum(sv[g]);
+      if(64 * g < k - 1) CR += wave_sum(cross);
     }
-    __syncthreads();
+    const double cn = sqrt(SU), rn = sqrt(SV);
+    bool stop = false;
+    if(k == 0) {
+      norma = cn * cn * (rn * rn);
+    } else {
+      norma = norma + cn * cn * (rn * rn) + 2.0 * CR;
+      stop = a.eps * sqrt(norma) >= cn * rn;
+    }
     r = k + 1;
-    if(s_stop) break;
-    const int in = block_argmax((t < n && !usedR[t]) ? cabs(u) : -1.0, wv, wi, &s_idx);
+    if(stop) break;
+    const int in = argmax(u, usedR);
     if(in < 0) break;
     ik = in;
+    __syncthreads();
   }
-  if(t == 0) a.rank[b] = r;
+  if(lane == 0) a.rank[b] = r;
 }
 
 __global__ void aca_pack_kernel(const cplx *U, const cplx *V, int n, const int *rank, cplx *pool, const size_t *off) {
@@ -172,37 +175,109 @@ __global__ void aca_pack_kernel(const cplx *U, const cplx *V, int n, const int *
   }
 }
 
-__global__ __launch_bounds__(256) void aca_vt_kernel(AcaOp op, const cplx *x) {
-  const AcaDesc d = op.desc[op.acalist[blockIdx.x]];
-  const int n = op.n, r = d.rank, t = threadIdx.x, lane = t & 63, w = t >> 6;
-  __shared__ cplx xs[256];
-  if(t < n) xs[t] = x[(size_t)d.j * n + t];
-  __syncthreads();
+// A wave per compressed block: four rows of V at a time, 16 lanes each, x_j in NI
+// registers a lane (n <= 16 NI).  With a row per wave and all 64 lanes on it (n =
+// 70: a second pass of 6) the reductions bound it: 282 us a product for the 0.92
+// GB of V of 300 spheres, now 178 us (5.2 TB/s; a loop over blocks in six
+// workgroups a CU, each with the next descriptor on its way: 201).
+template <int NI> __global__ __launch_bounds__(256) void aca_vt_kernel(AcaOp op, const cplx *x) {
+  const int e = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if(e >= op.naca) return;
+  const AcaDesc d = op.desc[op.acalist[e]];
+  const int n = op.n, r = d.rank, lane = threadIdx.x & 63, g = lane >> 4, li = lane & 15;
+  cplx xs[NI];
+#pragma unroll
+  for(int i = 0; i < NI; ++i) {
+    xs[i] = mk(0.0);
+    if(li + 16 * i < n) xs[i] = x[(size_t)d.j * n + li + 16 * i];
+  }
   const cplx *Vb = d.M + (size_t)n * r;
-  for(int p = w; p < r; p += 4) {
-    cplx s = mk(0.0);
-    for(int c = lane; c < n; c += 64) s = s + Vb[(size_t)p * n + c] * xs[c];
-    s.x = wave_sum(s.x);
-    s.y = wave_sum(s.y);
-    if(lane == 0) op.t[d.toff + p] = s;
+  // H fours of rows at once, their loads first
+  constexpr int H = NI < 10 ? 2 : 1;
+  for(int p0 = 0; p0 < r; p0 += 4 * H) {
+    cplx v[H][NI];
+#pragma unroll
+    for(int h = 0; h < H; ++h)
+#pragma unroll
+      for(int i = 0; i < NI; ++i) {
+        const int p = p0 + 4 * h + g;
+        v[h][i] = mk(0.0);
+        if(p < r && li + 16 * i < n) v[h][i] = Vb[(size_t)p * n + li + 16 * i];
+      }
+#pragma unroll
+    for(int h = 0; h < H; ++h) {
+      const int p = p0 + 4 * h + g;
+      cplx s = mk(0.0);
+#pragma unroll
+      for(int i = 0; i < NI; ++i) s = s + v[h][i] * xs[i];
+#pragma unroll
+      for(int o = 8; o > 0; o >>= 1) {
+        s.x += __shfl_xor(s.x, o, 64);
+        s.y += __shfl_xor(s.y, o, 64);
+      }
+      if(p < r && li == 0) op.t[d.toff + p] = s;
+    }
   }
 }
 
-__global__ __launch_bounds__(256) void aca_rows_kernel(AcaOp op, const cplx *x) {
-  const int g = blockIdx.x, i = blockIdx.y, q = threadIdx.x, n = op.n;
-  __shared__ cplx vs[256];
-  cplx acc = mk(0.0);
-  for(int e = op.rowptr[i] + g; e < op.rowptr[i + 1]; e += op.G) {
-    const AcaDesc d = op.desc[e];
+// The group's blocks of a block row, dealt to the four waves: four columns at a
+// time, 16 lanes each, the rows' sums in NI registers a lane throughout; the
+// column groups' and the waves' sums meet at the end.  With a thread a row (n =
+// 70: a second wave of 6) and the right operand staged between barriers for every
+// block: 184 us a product, now 177 us (5.3 TB/s).
+template <int NI> __global__ __launch_bounds__(256) void aca_rows_kernel(AcaOp op, const cplx *x) {
+  const int gr = blockIdx.x, i0 = blockIdx.y, n = op.n, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int g = lane >> 4, li = lane & 15;
+  __shared__ cplx sum[3][16 * NI];
+  cplx acc[NI];
+#pragma unroll
+  for(int i = 0; i < NI; ++i) acc[i] = mk(0.0);
+  const int end = op.rowptr[i0 + 1], step = op.G * 4;
+  int e = op.rowptr[i0] + gr + op.G * w;
+  AcaDesc nx{};
+  if(e < end) nx = op.desc[e];
+  for(; e < end; e += step) {
+    const AcaDesc d = nx;
+    if(e + step < end) nx = op.desc[e + step];
     const int m = d.rank < 0 ? n : d.rank;
     const cplx *src = d.rank < 0 ? x + (size_t)d.j * n : op.t + d.toff;
-    __syncthreads();
-    if(q < m) vs[q] = src[q];
-    __syncthreads();
-    if(q < n)
-      for(int c = 0; c < m; ++c) acc = acc + d.M[(size_t)c * n + q] * vs[c];
+    constexpr int H = NI < 10 ? 2 : 1;
+    for(int c0 = 0; c0 < m; c0 += 4 * H) {
+      cplx v[H][NI], b[H];
+#pragma unroll
+      for(int h = 0; h < H; ++h) {
+        const int c = c0 + 4 * h + g;
+        b[h] = mk(0.0);
+        if(c < m) b[h] = src[c];
+#pragma unroll
+        for(int i = 0; i < NI; ++i) {
+          v[h][i] = mk(0.0);
+          if(c < m && li + 16 * i < n) v[h][i] = d.M[(size_t)c * n + li + 16 * i];
+        }
+      }
+#pragma unroll
+      for(int h = 0; h < H; ++h)
+#pragma unroll
+        for(int i = 0; i < NI; ++i) acc[i] = acc[i] + v[h][i] * b[h];
+    }
   }
-  if(q < n) op.part[((size_t)g * op.P + i) * n + q] = acc;
+#pragma unroll
+  for(int i = 0; i < NI; ++i) {
+#pragma unroll
+    for(int o = 32; o >= 16; o >>= 1) {
+      acc[i].x += __shfl_xor(acc[i].x, o, 64);
+      acc[i].y += __shfl_xor(acc[i].y, o, 64);
+    }
+    if(w > 0 && g == 0) sum[w - 1][li + 16 * i] = acc[i];
+  }
+  __syncthreads();
+  if(w == 0 && g == 0)
+#pragma unroll
+    for(int i = 0; i < NI; ++i)
+      if(li + 16 * i < n) {
+        const int q = li + 16 * i;
+        op.part[((size_t)gr * op.P + i0) * n + q] = ((acc[i] + sum[0][q]) + sum[1][q]) + sum[2][q];
+      }
 }
 
 __global__ void aca_sum_kernel(AcaOp op, const cplx *x, cplx *y) {
@@ -217,7 +292,12 @@ __global__ void aca_sum_kernel(AcaOp op, const cplx *x, cplx *y) {
 }
 
 void run_aca(const AcaArgs &a, hipStream_t st) {
-  hipLaunchKernelGGL(aca_kernel, dim3(a.nblk), dim3(256), 0, st, a);
+  switch((a.n + 63) / 64) {
+  case 1: hipLaunchKernelGGL(aca_kernel<1>, dim3(a.nblk), dim3(64), 0, st, a); break;
+  case 2: hipLaunchKernelGGL(aca_kernel<2>, dim3(a.nblk), dim3(64), 0, st, a); break;
+  case 3: hipLaunchKernelGGL(aca_kernel<3>, dim3(a.nblk), dim3(64), 0, st, a); break;
+  default: hipLaunchKernelGGL(aca_kernel<4>, dim3(a.nblk), dim3(64), 0, st, a); break;
+  }
 }
 
 void run_aca_pack(const cplx *U, const cplx *V, int n, int nblk, const int *rank, cplx *pool, const size_t *off,
@@ -225,10 +305,18 @@ void run_aca_pack(const cplx *U, const cplx *V, int n, int nblk, const int *rank
   hipLaunchKernelGGL(aca_pack_kernel, dim3(nblk), dim3(256), 0, st, U, V, n, rank, pool, off);
 }
 
+// The kernels of the smallest NI with n <= 16 NI, of the register counts that
+// n = 2 nmax (nmax + 2) = 6 16 30 48 70 96 126 160 198 240 come to.
+template <int NI> void run_products(const AcaOp &op, const cplx *x, hipStream_t st) {
+  constexpr int next = NI < 3 ? NI + 1 : NI == 3 ? 5 : NI == 5 ? 6 : NI < 10 ? NI + 2 : NI == 10 ? 13 : 16;
+  if constexpr(NI < 16)
+    if(op.n > 16 * NI) return run_products<next>(op, x, st);
+  if(op.naca > 0) hipLaunchKernelGGL(aca_vt_kernel<NI>, dim3((op.naca + 3) / 4), dim3(256), 0, st, op, x);
+  if(op.G > 0) hipLaunchKernelGGL(aca_rows_kernel<NI>, dim3(op.G, op.P), dim3(256), 0, st, op, x);
+}
+
 void aca_matvec(const AcaOp &op, const cplx *x, cplx *y, hipStream_t st) {
-  if(op.naca > 0) hipLaunchKernelGGL(aca_vt_kernel, dim3(op.naca), dim3(256), 0, st, op, x);
-  const int bd = ((op.n + 63) / 64) * 64;
-  if(op.G > 0) hipLaunchKernelGGL(aca_rows_kernel, dim3(op.G, op.P), dim3(bd), 0, st, op, x);
+  run_products<1>(op, x, st);
   hipLaunchKernelGGL(aca_sum_kernel, dim3((op.Np + 255) / 256), dim3(256), 0, st, op, x, y);
 }
 

@@ -624,7 +624,8 @@ void aca_build(omx_context *c, bool shf) {
     }
   }
   rowptr[P] = (int)desc.size();
-  m.G = P > 1 ? std::max(1, std::min(P - 1, (2048 + P - 1) / P)) : 0;
+  // one round of the chip, six workgroups a CU
+  m.G = P > 1 ? std::max(1, std::min((P + 2) / 4, 1536 / P)) : 0;
   m.desc.ensure(sizeof(omx::AcaDesc) * std::max<size_t>(desc.size(), 1), T);
   m.rowptr.ensure(sizeof(int) * (P + 1), T);
   m.acalist.ensure(sizeof(int) * std::max<size_t>(acalist.size(), 1), T);
