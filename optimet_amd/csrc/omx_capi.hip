@@ -421,7 +421,7 @@ void alloc_all(omx_context *c) {
   c->d_r.ensure(sizeof(cplx) * Np, T);
   c->d_w1.ensure(sizeof(cplx) * Np, T);
   c->d_w2.ensure(sizeof(cplx) * Np, T);
-  c->d_gpart.ensure(sizeof(cplx) * Np * omx::kGemvSplitMax, T);
+  c->d_gpart.ensure(sizeof(cplx) * Np * omx::gemv_part_rows(1), T);
   c->d_nrm.ensure(sizeof(double) * 256, T);
 }
 
@@ -455,7 +455,7 @@ void alloc_matrices(omx_context *c) {
     w.basis.ensure(sizeof(cplx) * Np * (kInnerSteps + 1), T);
     w.r.ensure(sizeof(cplx) * Np, T);
     w.w1.ensure(sizeof(cplx) * Np, T);
-    w.gpart.ensure(sizeof(cplx) * Np * omx::kGemvSplitMax, T);
+    w.gpart.ensure(sizeof(cplx) * Np * omx::gemv_part_rows(1), T);
   } else {
     c->ws_in.release(T);
   }
@@ -1267,7 +1267,7 @@ void sweep_alloc(omx_context *c, int nb, bool f64, bool sh) {
   }
   w.basis.ensure(sizeof(cplx) * Np * (m + 1) * nb, T);
   w.basisZ.ensure(sizeof(cplx) * Np * (m + 1) * nb, T);
-  w.gpart.ensure(sizeof(cplx) * Np * omx::kGemvSplitMax * nb, T);
+  w.gpart.ensure(sizeof(cplx) * Np * omx::gemv_part_rows(nb), T);
   w.kz.ensure(sizeof(cplx) * 2 * nb, T);
   w.omz.ensure(sizeof(double) * nb, T);
 }
@@ -2354,7 +2354,7 @@ void group_alloc(omx_context *L, int nb, bool f64, bool sh) {
   for(DBuf *b : {&w.status, &w.status2}) b->ensure(sizeof(int) * 4 * nb, T);
   w.basis.ensure(sizeof(cplx) * Np * (m + 1) * nb, T);
   w.basisZ.ensure(sizeof(cplx) * Np * (m + 1) * nb, T);
-  w.gpart.ensure(sizeof(cplx) * Np * omx::kGemvSplitMax * nb, T);
+  w.gpart.ensure(sizeof(cplx) * Np * omx::gemv_part_rows(nb), T);
   L->d_status.ensure(64, T);
 }
 
@@ -2766,7 +2766,7 @@ int omx_dense_solve(omx_context *c, int N, const double *A, const double *b, dou
     ctx.d_r.ensure(sizeof(cplx) * Np, &ctx.total);
     ctx.d_w1.ensure(sizeof(cplx) * Np, &ctx.total);
     ctx.d_w2.ensure(sizeof(cplx) * Np, &ctx.total);
-    ctx.d_gpart.ensure(sizeof(cplx) * Np * omx::kGemvSplitMax, &ctx.total);
+    ctx.d_gpart.ensure(sizeof(cplx) * Np * omx::gemv_part_rows(1), &ctx.total);
     ctx.d_nrm.ensure(sizeof(double) * 256, &ctx.total);
     alloc_matrices(&ctx);
     HIPCHK(hipMemsetAsync(ctx.d_Q.p, 0, sizeof(cplx) * Np, ctx.st));

@@ -2,6 +2,9 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
+
 #include "omx_math.hpp"
 
 namespace omx {
@@ -254,7 +257,8 @@ int gemv_partial(const cplx *A, size_t lda, int N, const cplx *x, cplx *part, hi
                  size_t sA = 0, size_t sv = 0, const int *flag = nullptr, int live = 1);
 int gemv_partial(const float2 *A, size_t lda, int N, const cplx *x, cplx *part, hipStream_t st,
                  const int *flag = nullptr);
-constexpr int kGemvSplitMax = 32;
+constexpr int kGemvSplit = 32, kGemvSplitMax = 96;  // column parts: most of a batch's product, of a single one's
+inline size_t gemv_part_rows(int nb) { return std::max(kGemvSplitMax, kGemvSplit * nb); }  // vectors of partial sums
 
 // GMRES with its small algebra on the device (omx_krylov.hip), nb systems in
 // lockstep: the state of each, and the vectors they share.

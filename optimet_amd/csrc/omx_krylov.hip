@@ -150,6 +150,7 @@ __global__ __launch_bounds__(kRows) void kry_dots(KryState s, const cplx *gpart,
   if(r < s.n) {
     if(ns > 0) {
       const cplx *g = gpart + z * sg + r;
+#pragma unroll 8
       for(int k = 0; k < ns; ++k) w = w + g[(size_t)k * s.n];
       W[r] = w;
     } else {
@@ -338,6 +339,7 @@ __global__ __launch_bounds__(kRows) void kry_resid(KryState s, const cplx *b, co
     if(ns > 0) {
       const cplx *g = gpart + z * sg + r;
       cplx a = mk(0.0);
+#pragma unroll 8
       for(int k = 0; k < ns; ++k) a = a + g[(size_t)k * s.n];
       v = bv - a;
     } else if(ns < 0) {  // the product is in w

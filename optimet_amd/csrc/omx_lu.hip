@@ -154,6 +154,16 @@ __device__ inline float2 ld_stream(const float2 *p) {
   r.y = v.y;
   return r;
 }
+// 16 bytes
+__device__ inline void ld_stream16(const cplx *p, cplx (&e)[1]) { e[0] = ld_stream(p); }
+__device__ inline void ld_stream16(const float2 *p, float2 (&e)[2]) {
+  typedef float f4 __attribute__((ext_vector_type(4)));
+  const f4 v = __builtin_nontemporal_load(reinterpret_cast<const f4 *>(p));
+  e[0].x = v.x;
+  e[0].y = v.y;
+  e[1].x = v.z;
+  e[1].y = v.w;
+}
 __device__ inline void st_stream(float2 *p, float2 c) {
   typedef float f2 __attribute__((ext_vector_type(2)));
   const f2 v = {c.x, c.y};
@@ -1844,64 +1854,82 @@ template void lu_solve<float2>(const float2 *, int, size_t, LuWork &, const cplx
 
 // ------------------------------------------------------------------ gemv
 // y = A x for the FP64 matrix (residuals and GMRES) or its complex-FP32 copy
-// (entries widened to FP64, FP64 vectors and sums), two-stage column split.
-constexpr int kGemvSplit = 32;
+// (entries widened to FP64, FP64 vectors and sums), two-stage column split: 256
+// rows by a run of columns per workgroup, 16 bytes of a column per thread and
+// load (two FP32 rows, one FP64).
+//
+// Bound: HBM, once enough loads are in flight.  FP32, N = 49152: 3171 us with one
+// row per thread and 32 parts (6.1 TB/s), 2772 with two and 16 (6.97); N = 10240:
+// 191 and 128 us (6.5 TB/s).
 template <typename T>
-__global__ __launch_bounds__(256) void gemv_part_kernel(const T *__restrict__ A, size_t lda, int N,
-                                                        const cplx *__restrict__ x, cplx *part, int chunk, size_t sA,
-                                                        size_t sv, const int *flag) {
+__global__ __launch_bounds__(sizeof(T) == 8 ? 128 : 256) void gemv_part_kernel(const T *__restrict__ A, size_t lda,
+                                                                              int N, const cplx *__restrict__ x,
+                                                                              cplx *part, int chunk, size_t sA,
+                                                                              size_t sv, const int *flag) {
+  constexpr int RPT = 16 / sizeof(T), TPB = 256 / RPT;
   const size_t zs = blockIdx.z;
   if(flag && !flag[zs * KF_COUNT]) return;
   A += zs * sA;
   x += zs * sv;
   part += (size_t)blockIdx.z * gridDim.y * N;
   __shared__ cplx xs[512];
-  const int r = blockIdx.x * 256 + threadIdx.x;
+  const int r = blockIdx.x * 256 + threadIdx.x * RPT;
   const int c0 = blockIdx.y * chunk, c1 = min(N, c0 + chunk);
-  cplx acc = mk(0.0);
+  cplx acc[RPT];
+#pragma unroll
+  for(int i = 0; i < RPT; ++i) acc[i] = mk(0.0);
   for(int cb = c0; cb < c1; cb += 512) {
     int ce = min(c1, cb + 512);
     __syncthreads();
-    for(int i = threadIdx.x; i < ce - cb; i += 256) xs[i] = x[cb + i];
+    for(int i = threadIdx.x; i < ce - cb; i += TPB) xs[i] = x[cb + i];
     __syncthreads();
     if(r < N) {
       const T *a = A + (size_t)cb * lda + r;
       int n = ce - cb;
 #pragma unroll 8
       for(int c = 0; c < n; ++c) {
-        const T e = ld_stream(a + (size_t)c * lda);
-        const double vx = e.x, vy = e.y;
-        acc.x += vx * xs[c].x - vy * xs[c].y;
-        acc.y += vx * xs[c].y + vy * xs[c].x;
+        T e[RPT];
+        ld_stream16(a + (size_t)c * lda, e);
+#pragma unroll
+        for(int i = 0; i < RPT; ++i) {
+          const double vx = e[i].x, vy = e[i].y;
+          acc[i].x += vx * xs[c].x - vy * xs[c].y;
+          acc[i].y += vx * xs[c].y + vy * xs[c].x;
+        }
       }
     }
   }
-  if(r < N) part[(size_t)blockIdx.y * N + r] = acc;
+  if(r < N)
+#pragma unroll
+    for(int i = 0; i < RPT; ++i) part[(size_t)blockIdx.y * N + r + i] = acc[i];
 }
-// Column parts of a batched product: the fewest (the longest runs of
-// columns, the fewest partial vectors) that still give 1280 workgroups, about
-// five per CU.  Measured on 3840 x 3840 systems: 6.75 TB/s with 8 parts for 64
-// systems against 5.94 with 32, 6.20 with 24 parts for 4 systems; one system of
-// 10240 is fastest with kGemvSplit parts.
-inline int gemv_parts(int N, int nz) {
-  if(nz <= 1) return kGemvSplit;
+// Column parts of a product: the fewest (the longest runs of columns, the fewest
+// partial vectors) that still give `want` workgroups.  FP64: 1280, about five per
+// CU.  Measured on 3840 x 3840 systems: 6.75 TB/s with 8 parts for 64 systems
+// against 5.94 with 32, 6.20 with 24 parts for 4 systems; one system with 32 / 64 /
+// 96 parts: N = 2176 32.4 / 21.5 / 16.8 us, 2752 44 / 28 / 22, 5120 100 / 62 / 65,
+// 10240 254 / 296 / 264.  FP32: 2560 of half the threads.  Few rows (N < 1280)
+// keep 32 parts: the product is 4 us with either, and the next kernel adds them up.
+inline int gemv_parts(int N, int nz, int most, int want) {
   const long rb = (N + 255) / 256;
-  for(int s : {8, 12, 16, 24})
-    if(rb * nz * s >= 1280) return s;
-  return kGemvSplit;
+  if(nz <= 1 && rb <= 5) return kGemvSplit;
+  for(int s : {8, 12, 16, 24, 32, 48, 64, 96})
+    if(s >= most || rb * nz * s >= want) return std::min(s, most);
+  return most;
 }
 int gemv_partial(const cplx *A, size_t lda, int N, const cplx *x, cplx *part, hipStream_t st, int nb, size_t sA,
                  size_t sv, const int *flag, int live) {
-  const int ns = gemv_parts(N, live), chunk = (N + ns - 1) / ns;  // ns <= kGemvSplitMax
+  const int ns = gemv_parts(N, live, nb == 1 ? kGemvSplitMax : kGemvSplit, 1280), chunk = (N + ns - 1) / ns;
   hipLaunchKernelGGL(gemv_part_kernel<cplx>, dim3((N + 255) / 256, ns, nb), dim3(256), 0, st, A, lda, N, x, part,
                      chunk, sA, sv, flag);
   return ns;
 }
 int gemv_partial(const float2 *A, size_t lda, int N, const cplx *x, cplx *part, hipStream_t st, const int *flag) {
-  const int chunk = (N + kGemvSplit - 1) / kGemvSplit;
-  hipLaunchKernelGGL(gemv_part_kernel<float2>, dim3((N + 255) / 256, kGemvSplit, 1), dim3(256), 0, st, A, lda, N, x,
-                     part, chunk, (size_t)0, (size_t)0, flag);
-  return kGemvSplit;
+  // N even, A's columns on 16 bytes: the padded order is a multiple of 64
+  const int ns = gemv_parts(N, 1, kGemvSplitMax, 2560), chunk = (N + ns - 1) / ns;
+  hipLaunchKernelGGL(gemv_part_kernel<float2>, dim3((N + 255) / 256, ns, 1), dim3(128), 0, st, A, lda, N, x, part,
+                     chunk, (size_t)0, (size_t)0, flag);
+  return ns;
 }
 
 }  // namespace omx
