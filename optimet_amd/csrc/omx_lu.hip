@@ -357,46 +357,52 @@ __device__ inline unsigned order_key(double m) { return (unsigned)__double2hiint
 // 64), their inverses, the gather map that brings the rows to the top
 // (mdst <- msrc, at most 128 entries) and the permutation.
 //
-// As diag_lu: a wave holds 8 columns, here of RPL rows per lane; a panel of 8
-// columns' owner runs its pivot steps without barriers (the largest
-// max(|re|, |im|) of the rows left, to 20 bits of mantissa, the first row on
-// ties) and publishes the multipliers; after one barrier the later columns'
-// waves apply its 8 rank-1 updates.  A pivot row sits in one of RPL register
-// slots: the step branches on the slot, uniform in the wave.
+// As diag_lu, which stands below: a wave holds 8 columns, here of RPL rows per
+// lane; the owner of a column takes the largest max(|re|, |im|) of the rows left
+// (to 20 bits of mantissa, the first row on ties), and the waves of later columns
+// follow by the published steps.  A pivot row sits in one of RPL register slots:
+// the step branches on the slot, uniform in the wave.  The multipliers of four
+// panels of 8 columns are kept; the owner of a fifth waits until the waves behind
+// it have read the first.
 //
 // Bound: the chain of 64 pivot steps, per level of the tree.  With 128 rows per
 // workgroup in 256 threads, three barriers a column and a tree of fan-in two,
 // plus the inverses by one thread a column in a kernel of its own, the panels of
-// an FP64 system of 1500 took 1.0 ms each; now 0.25 ms (100 us a level), and the
-// solve 7.75 ms against 26.5.
+// an FP64 system of 1500 took 1.0 ms each and the solve 26.5 ms; with a barrier
+// every 8 columns instead of the published steps 96 us a level and 7.3 ms; now 54 us
+// and 4.8 ms.
 template <typename T, int RPL>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(1, 2))) void tslu_panel(
     const T *A, size_t lda, int Np, int j0, int gin, const int *cin, int *cout, T *wlu, T *dinv, int *mdst, int *msrc,
     int *mcnt, int *perm, int *status) {
   using C = CxOf<T>;
-  constexpr int ROWS = 64 * RPL, LM = 2 * 8 * ROWS, FB = 64 * 65;
-  // the multipliers of two panels of 8 columns ([parity][step][row]), and after
-  // the last of them the factored block
+  constexpr int ROWS = 64 * RPL, RING = 4, LM = RING * 8 * ROWS, FB = 64 * 65;
+  // the multipliers of RING panels of 8 columns ([step][row]), and after the last
+  // of them the factored block
   __shared__ C buf[LM > FB ? LM : FB];
-  __shared__ int rid[ROWS], pidx[64], pb[2][8], outpos[64], wtop[64];
-  __shared__ C rinv[64];
-  const int t = threadIdx.x, lane = t & 63, q = t >> 6, g = blockIdx.x;
+  // step c, once published: 1 + its row's place, + 1024 for a zero pivot; the
+  // reciprocals (64 more slots in both take the other lanes' stores); the panels
+  // that wave q has read; the step of each place
+  __shared__ int step[128], seen[8], pos[ROWS];
+  __shared__ C rinv[128];
+  __shared__ int rid[ROWS], outpos[64], wtop[64];
+  const int t = threadIdx.x, lane = t & 63, q = __builtin_amdgcn_readfirstlane(t >> 6), g = blockIdx.x;
   const bool root = gridDim.x == 1;
   const C zero{};
   const int r0 = j0 + g * ROWS;
   const int R = cin ? 64 * min(RPL, gin - RPL * g) : min(ROWS, Np - r0);
   if(t < R) rid[t] = cin ? cin[g * ROWS + t] : r0 + t;
+  if(t < 64) step[t] = 0;
+  if(t < 8) seen[t] = 0;
+  if(t < ROWS) pos[t] = -1;
   __syncthreads();
-  const int pq = 2 * (q & 3) + (q >> 2);  // as diag_lu
   C v[RPL][8];
   bool used[RPL];
-  int mypos[RPL];
 #pragma unroll
   for(int s = 0; s < RPL; ++s) {
     const int idx = lane + 64 * s;
     used[s] = idx >= R;
-    mypos[s] = -1;
-    const T *row = A + (size_t)(j0 + 8 * pq) * lda + (idx < R ? rid[idx] : j0);
+    const T *row = A + (size_t)(j0 + 8 * q) * lda + (idx < R ? rid[idx] : j0);
 #pragma unroll
     for(int j = 0; j < 8; ++j) {
       const T a = row[(size_t)j * lda];
@@ -413,93 +419,110 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
           if(j >= from) pr[j] = rdl(v[s][j], b);
       }
   };
+  // the steps of the earlier owners
 #pragma unroll 1
-  for(int pc = 0; pc < 8; ++pc) {
-    const int par = pc & 1;
-    C *lm = buf + par * 8 * ROWS;
-    if(pq == pc) {
+  for(int c = 0; c < 8 * q; ++c) {
+    int e;
+    do
+      e = __builtin_amdgcn_readfirstlane(__hip_atomic_load(&step[c], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP));
+    while(e == 0);
+    e = (e & 1023) - 1;
+    const int sl = e >> 6, b = e & 63;
+    const C *lm = buf + (c & (8 * RING - 1)) * ROWS + lane;
+    C pr[8], l[RPL];
 #pragma unroll
-      for(int jj = 0; jj < 8; ++jj) {
-        const int c = 8 * pc + jj;
-        unsigned key[RPL], kx = 0;
-#pragma unroll
-        for(int s = 0; s < RPL; ++s) {
-          const auto ax = fabs(v[s][jj].x), ay = fabs(v[s][jj].y);  // -0 orders as 0
-          key[s] = used[s] ? 0u : order_key(ax > ay ? ax : ay);
-          kx = max(kx, key[s]);
-        }
-        const unsigned M = wave_max_u32(kx);
-        int sl = 0, b = 0;
-#pragma unroll
-        for(int s = RPL - 1; s >= 0; --s) {
-          const unsigned long long m = __ballot(!used[s] && key[s] == M);
-          if(m) {
-            sl = s;
-            b = __ffsll((long long)m) - 1;
-          }
-        }
-        sl = __builtin_amdgcn_readfirstlane(sl);
-        b = __builtin_amdgcn_readfirstlane(b);
-        C pr[8];
-        pivot_row(sl, b, pr, jj);
-        const bool sing = !(mag2(pr[jj]) > 0.0);
-        if(root && sing && lane == b) atomicCAS(&status[0], 0, j0 + c + 1);
-        const C ip = csel(sing, zero, crecip(pr[jj]));
-        if(lane == 0) {
-          pb[par][jj] = 64 * sl + b;
-          pidx[c] = 64 * sl + b;
-          rinv[c] = ip;
-        }
-#pragma unroll
-        for(int s = 0; s < RPL; ++s) {
-          if(s == sl && lane == b) {
-            used[s] = true;
-            mypos[s] = c;
-          }
-          const C l = csel(used[s], zero, cm(v[s][jj], ip));
-          v[s][jj] = csel(used[s], v[s][jj], l);
-          lm[jj * ROWS + 64 * s + lane] = l;
-#pragma unroll
-          for(int j = jj + 1; j < 8; ++j) v[s][j] = cfms(v[s][j], l, pr[j]);
-        }
-      }
+    for(int s = 0; s < RPL; ++s) {
+      l[s] = lm[64 * s];
+      used[s] = used[s] || (s == sl && lane == b);
     }
-    __syncthreads();  // one barrier per panel: the buffers alternate
-    if(pq != pc) {
-#pragma unroll 1
-      for(int jj = 0; jj < 8; ++jj) {
-        const int e = __builtin_amdgcn_readfirstlane(pb[par][jj]), sl = e >> 6, b = e & 63;
+    pivot_row(sl, b, pr, 0);
 #pragma unroll
-        for(int s = 0; s < RPL; ++s)
-          if(s == sl && lane == b) {
-            used[s] = true;
-            mypos[s] = 8 * pc + jj;
-          }
-        if(pq > pc) {
-          C pr[8];
-          pivot_row(sl, b, pr, 0);
+    for(int s = 0; s < RPL; ++s)
 #pragma unroll
-          for(int s = 0; s < RPL; ++s) {
-            const C l = lm[jj * ROWS + 64 * s + lane];
-#pragma unroll
-            for(int j = 0; j < 8; ++j) v[s][j] = cfms(v[s][j], l, pr[j]);
-          }
-        }
-      }
-    }
+      for(int j = 0; j < 8; ++j) v[s][j] = cfms(v[s][j], l[s], pr[j]);
+    if((c & 7) == 7 && lane == 0)
+      __hip_atomic_store(&seen[q], c / 8 + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
   }
-  __syncthreads();
+  // its own: the ring's slots are free once every later wave has read panel q -
+  // RING (they wait for earlier panels only, so this ends)
+  if(q >= RING)
+    for(int o = q + 1; o < 8; ++o)
+      while(__builtin_amdgcn_readfirstlane(
+                __hip_atomic_load(&seen[o], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP)) < q - RING + 1) {
+      }
+  __builtin_amdgcn_s_setprio(3);
+#pragma unroll
+  for(int jj = 0; jj < 8; ++jj) {
+    const int c = 8 * q + jj;
+    unsigned key[RPL], kx = 0;
+    C best = v[0][jj];  // this lane's candidate: its largest row left, the first on ties
+    bool have = false;
+#pragma unroll
+    for(int s = 0; s < RPL; ++s) {
+      const auto ax = fabs(v[s][jj].x), ay = fabs(v[s][jj].y);  // -0 orders as 0
+      key[s] = used[s] ? 0u : order_key(ax > ay ? ax : ay);
+      best = csel(!used[s] && (!have || key[s] > kx), v[s][jj], best);
+      have = have || !used[s];
+      kx = max(kx, key[s]);
+    }
+    // every lane the reciprocal of its own candidate while the maximum is found
+    const bool sing = !nonzero(best);
+    const C ir = csel(sing, zero, crecip(best));
+    const unsigned M = wave_max_u32(kx);
+    int sl = 0, b = 0;
+#pragma unroll
+    for(int s = RPL - 1; s >= 0; --s) {
+      const unsigned long long m = __ballot(!used[s] && key[s] == M);
+      if(m) {
+        sl = s;
+        b = __ffsll((long long)m) - 1;
+      }
+    }
+    sl = __builtin_amdgcn_readfirstlane(sl);
+    b = __builtin_amdgcn_readfirstlane(b);
+    C pr[8];
+    pivot_row(sl, b, pr, jj);
+    const C ip = rdl(ir, b);
+    C *lm = buf + (c & (8 * RING - 1)) * ROWS + lane;
+#pragma unroll
+    for(int s = 0; s < RPL; ++s) {
+      used[s] = used[s] || (s == sl && lane == b);
+      const C l = csel(used[s], zero, cm(v[s][jj], ip));
+      v[s][jj] = csel(used[s], v[s][jj], l);
+      lm[64 * s] = l;
+#pragma unroll
+      for(int j = jj + 1; j < 8; ++j) v[s][j] = cfms(v[s][j], l, pr[j]);
+    }
+    // published after the multipliers: a wave's LDS stores are done in order
+    const int slot = lane == b ? c : 64 + lane;
+    rinv[slot] = ir;
+    asm volatile("" ::: "memory");
+    __hip_atomic_store(&step[slot], (sing ? 1025 : 1) + 64 * sl + lane, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_WORKGROUP);
+  }
+  __builtin_amdgcn_s_setprio(0);
+  __syncthreads();  // all steps published and all multipliers read
+  const int own = step[lane], mine = (own & 1023) - 1;  // the place of step `lane`
   if(!root) {
-    if(t < 64) cout[g * 64 + t] = rid[pidx[t]];
+    if(q == 0) cout[g * 64 + lane] = rid[mine];
     return;
   }
+  if(q == 0) {
+    pos[mine] = lane;
+    const unsigned long long zm = __ballot(own > 1024);
+    if(zm && lane == 0) atomicCAS(&status[0], 0, j0 + __ffsll((long long)zm));
+  }
+  __syncthreads();
+  int mypos[RPL];
+#pragma unroll
+  for(int s = 0; s < RPL; ++s) mypos[s] = pos[lane + 64 * s];
   // the selected rows' factors in pivoted order
 #pragma unroll
   for(int s = 0; s < RPL; ++s)
     if(mypos[s] >= 0) {
 #pragma unroll
       for(int j = 0; j < 8; ++j) {
-        const int col = 8 * pq + j;
+        const int col = 8 * q + j;
         buf[col * 65 + mypos[s]] = v[s][j];
         T o;
         o.x = v[s][j].x;
@@ -512,7 +535,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
   if(q == 0) {
     // winner lane goes to row j0 + lane; the top rows that did not win take the
     // places of the winners from further down, in order
-    const int X = rid[pidx[lane]];
+    const int X = rid[mine];
     const bool in_top = X < j0 + 64;
     if(in_top) wtop[X - j0] = 1;
     const unsigned long long below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
