@@ -838,9 +838,15 @@ __global__ __launch_bounds__(PairCfg<NMAX>::NT) void origin_kernel(OriginArgs a)
 }
 
 // ------------------------------------------------------------------ cross sections
-// Block j: partial sums [Cext, Csca, Cabs, Csca_SH] of object j.
+// Block (j, z): partial sums [Cext, Csca, Cabs, Csca_SH] of object j, system z.
 __global__ void cross_kernel(CrossArgs a) {
-  const int j = blockIdx.x, t = threadIdx.x;
+  const int j = blockIdx.x, z = blockIdx.z, t = threadIdx.x;
+  a.x += z * a.zvec;
+  if(a.xsh) a.xsh += z * a.zvec;
+  a.incloc += z * a.zvec;
+  a.w += z * a.zw;
+  a.ov += z * a.zov;
+  a.out += (size_t)z * 4 * a.P;
   const int nf = a.nmax * (a.nmax + 2), S = a.nmax + 1;
   __shared__ double red[4][256];
   double c[4] = {0, 0, 0, 0};
@@ -923,7 +929,7 @@ void run_objects(const ObjArgs &a, hipStream_t st, int nb) {
 void run_pairs(const PairArgs &a, hipStream_t st, int nb) { OMX_NMAX_SWITCH(a.nmax, launch_pair, a, st, nb); }
 void run_origin(const OriginArgs &a, hipStream_t st, int nb) { OMX_NMAX_SWITCH(a.nmax, launch_origin, a, st, nb); }
 void run_cross(const CrossArgs &a, hipStream_t st) {
-  hipLaunchKernelGGL(cross_kernel, dim3(a.P), dim3(256), 0, st, a);
+  hipLaunchKernelGGL(cross_kernel, dim3(a.P, 1, a.nb), dim3(256), 0, st, a);
 }
 void run_pad64(cplx *A, int N, int Np, size_t lda, hipStream_t st, int nb, size_t zs) {
   if(Np == N) return;

@@ -1712,9 +1712,7 @@ void sweep_chunk(omx_context *c, int nb, const double *lam, const cplx *eps, con
   } else {
     refine(false, lwS, FS, w.Q.as<cplx>(), w.x.as<cplx>());
   }
-  for(int z = 0; z < nb; ++z)
-    omx::vmul_ov(w.xint.as<cplx>() + z * lda, w.x.as<cplx>() + z * lda, w.ov.as<cplx>() + z * ovs, omx::OV_IAUX, P,
-                 nmax, nullptr, N, st);
+  omx::vmul_ov(w.xint.as<cplx>(), w.x.as<cplx>(), w.ov.as<cplx>(), omx::OV_IAUX, P, nmax, nullptr, N, st, nb, lda, ovs);
   if(sh) {
     if(c->cg_nmax != nmax) {
       size_t nf = (size_t)c->nf, sz = nf * nf * nf;
@@ -1723,28 +1721,28 @@ void sweep_chunk(omx_context *c, int nb, const double *lam, const cplx *eps, con
       c->cg_nmax = nmax;
     }
     HIPCHK(hipMemsetAsync(w.K.p, 0, w.K.bytes, st));
-    for(int z = 0; z < nb; ++z) {
-      const double omega = omx::kC0 * (2.0 * omx::kPi / lam[z]);
-      omx::ShArgs sa{P, nmax, omega, bge, bgm, c->d_radius.as<double>(), w.eps.as<cplx>() + (size_t)z * P,
-                     c->d_mu.as<cplx>(), w.eps_sh.as<cplx>() + (size_t)z * P, c->d_kppp.as<cplx>(),
-                     c->d_kpar.as<cplx>(), c->d_gam.as<cplx>(), w.ov.as<cplx>() + z * ovs, c->d_cg.as<double>(),
-                     w.xint.as<cplx>() + z * lda, w.K.as<cplx>() + z * lda, w.K1.as<cplx>() + z * lda};
-      omx::run_shsrc(sa, st);
-    }
+    omx::ShArgs sa{P, nmax, hom[0], bge, bgm, c->d_radius.as<double>(), w.eps.as<cplx>(), c->d_mu.as<cplx>(),
+                   w.eps_sh.as<cplx>(), c->d_kppp.as<cplx>(), c->d_kpar.as<cplx>(), c->d_gam.as<cplx>(),
+                   w.ov.as<cplx>(), c->d_cg.as<double>(), w.xint.as<cplx>(), w.K.as<cplx>(), w.K1.as<cplx>()};
+    sa.nb = nb;
+    sa.omz = w.omz.as<double>();
+    sa.zvec = lda;
+    sa.zov = ovs;
+    omx::run_shsrc(sa, st);
     vq.join();  // V's factorisation enqueued (and its event recorded) before the wait below
     HIPCHK(hipStreamWaitEvent(st, c->xev[1], 0));  // V's factorisation
     refine(true, lwV, FV, w.K.as<cplx>(), w.xsh.as<cplx>());
-    for(int z = 0; z < nb; ++z)
-      omx::vmul_ov(w.xintsh.as<cplx>() + z * lda, w.xsh.as<cplx>() + z * lda, w.ov.as<cplx>() + z * ovs,
-                   omx::OV_IAUXSH1, P, nmax, w.K1.as<cplx>() + z * lda, N, st);
+    omx::vmul_ov(w.xintsh.as<cplx>(), w.xsh.as<cplx>(), w.ov.as<cplx>(), omx::OV_IAUXSH1, P, nmax, w.K1.as<cplx>(), N,
+                 st, nb, lda, ovs);
   }
   // cross sections (Result.cpp:557-761)
-  for(int z = 0; z < nb; ++z) {
-    omx::CrossArgs ca{P, nmax, w.x.as<cplx>() + z * lda, sh ? w.xsh.as<cplx>() + z * lda : nullptr,
-                      w.incloc.as<cplx>() + z * lda, w.w.as<double>() + z * ws, w.ov.as<cplx>() + z * ovs,
-                      w.cross.as<double>() + (size_t)z * 4 * P};
-    omx::run_cross(ca, st);
-  }
+  omx::CrossArgs ca{P, nmax, w.x.as<cplx>(), sh ? w.xsh.as<cplx>() : nullptr, w.incloc.as<cplx>(), w.w.as<double>(),
+                    w.ov.as<cplx>(), w.cross.as<double>()};
+  ca.nb = nb;
+  ca.zvec = lda;
+  ca.zw = ws;
+  ca.zov = ovs;
+  omx::run_cross(ca, st);
   // SH absorption (Result.cpp:763-794), every system in one batch
   if(sh) {
     omx::AbsShArgs aa{P, nmax, hom[0], bge, bgm, c->d_radius.as<double>(), w.eps.as<cplx>(), c->d_mu.as<cplx>(),

@@ -7,8 +7,13 @@
 namespace omx {
 
 // y[i] = x[i] * ov[kind][obj][pol][deg(i)] - sub[i], over the N = 2 nf P unknowns
+// of system blockIdx.z
 __global__ void vmul_ov_k(cplx *y, const cplx *x, const cplx *ov, int kind, int P, int nmax, const cplx *sub,
-                          int n) {
+                          int n, size_t zvec, size_t zov) {
+  y += blockIdx.z * zvec;
+  x += blockIdx.z * zvec;
+  ov += blockIdx.z * zov;
+  if(sub) sub += blockIdx.z * zvec;
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if(i >= n) return;
   const int nf = nmax * (nmax + 2);
@@ -91,8 +96,9 @@ void pad_vector(cplx *dst, int Nd, const cplx *src, int Ns, hipStream_t st) {
   hipLaunchKernelGGL(pad_vector_k, g1(Nd), dim3(256), 0, st, dst, Nd, src, Ns);
 }
 void vmul_ov(cplx *y, const cplx *x, const cplx *ov, int kind, int P, int nmax, const cplx *sub, int n,
-             hipStream_t st) {
-  hipLaunchKernelGGL(vmul_ov_k, g1(n), dim3(256), 0, st, y, x, ov, kind, P, nmax, sub, n);
+             hipStream_t st, int nb, size_t zvec, size_t zov) {
+  hipLaunchKernelGGL(vmul_ov_k, dim3((n + 255) / 256, 1, nb), dim3(256), 0, st, y, x, ov, kind, P, nmax, sub, n, zvec,
+                     zov);
 }
 void nrm2sq(const cplx *x, int n, double *part, double *out, hipStream_t st) {
   int nb = std::min(kRedBlocks, (n + 255) / 256);

@@ -111,7 +111,10 @@ struct CrossArgs {
   const cplx *x, *xsh, *incloc;
   const double *w;
   const cplx *ov;
-  double *out;                       // [P][4]
+  double *out;                       // [nb][P][4]
+  // nb systems: the vectors zvec, w zw and ov zov apart
+  int nb = 1;
+  size_t zvec = 0, zw = 0, zov = 0;
 };
 
 // Result::getEHFields / setFields (Result.cpp:74-301, 797-933): E and H at
@@ -303,7 +306,7 @@ void pad_matrix64(cplx *dst, int Nd, const cplx *src, int Ns, hipStream_t st);
 void pad_matrix32(float2 *dst, int Nd, const cplx *src, int Ns, hipStream_t st);
 void pad_vector(cplx *dst, int Nd, const cplx *src, int Ns, hipStream_t st);
 void vmul_ov(cplx *y, const cplx *x, const cplx *ov, int kind, int P, int nmax, const cplx *sub, int n,
-             hipStream_t st);                                                  // y = x (.) ov[kind] - sub
+             hipStream_t st, int nb = 1, size_t zvec = 0, size_t zov = 0);     // y = x (.) ov[kind] - sub
 void nrm2sq(const cplx *x, int n, double *part, double *out, hipStream_t st);
 
 }  // namespace omx

@@ -132,28 +132,40 @@ __global__ void cg_kernel(int nf, double *out) {
   out[8 * sz + idx] = b2 * Wf(J1, J1, M1, J2 - 1, J2, M2, J, M) + a2 * Wf(J1, J1, M1, J2 + 1, J2, M2, J, M);
 }
 
-// Block (object j, output harmonic kk).
-__global__ __launch_bounds__(256) void shsrc_kernel(ShArgs a) {
-  const int j = blockIdx.x, kk = blockIdx.y, t = threadIdx.x;
+// Block (PB objects of the batch, output harmonic kk): the tables' entries serve
+// all PB objects.
+//
+// Bound: the tables, whose entries of one kk lie 8 bytes in every cache line or
+// two: 0.7 MB of them for every (object, kk) at nmax 10.  With one object a block
+// and a launch per system, 64 systems of 16 objects took 14.4 ms; with four
+// objects a block, in one launch, 4.4 ms.
+template <int PB> __global__ __launch_bounds__(256, PB > 1 ? 2 : 4) void shsrc_kernel(ShArgs a) {
+  const int pr0 = blockIdx.x * PB, np = min(PB, a.P * a.nb - pr0), kk = blockIdx.y, t = threadIdx.x;
   const int nmax = a.nmax, nf = nmax * (nmax + 2), S = nmax + 1, P = a.P;
   const size_t sz = (size_t)nf * nf * nf;
-  __shared__ cplx A0[kMaxNmax * (kMaxNmax + 2)], A1[kMaxNmax * (kMaxNmax + 2)], Am1[kMaxNmax * (kMaxNmax + 2)];
-  __shared__ cplx red[4][256];
-  const double R = a.radius[j];
-  const cplx kj = a.omega * csqrt_(a.eps[j] * a.mu[j]);
+  constexpr int NF = kMaxNmax * (kMaxNmax + 2);
+  __shared__ cplx A0[PB][NF], A1[PB][NF], Am1[PB][NF];
+  __shared__ cplx red[4][256], tot[PB][4];
   const cplx I = mk(0.0, 1.0);
-  for(int p = t; p < nf; p += blockDim.x) {
+  auto omega = [&](int z) { return a.omz ? a.omz[z] : a.omega; };
+  for(int e = t; e < np * nf; e += blockDim.x) {
+    const int o = e / nf, p = e % nf, z = (pr0 + o) / P, j = (pr0 + o) % P;
     int n, m;
     unflat(p, n, m);
-    cplx c = conj(a.xint[(size_t)j * 2 * nf + p]), d = conj(a.xint[(size_t)j * 2 * nf + nf + p]);
-    cplx jn = a.ov[(((size_t)OV_SHRAD * P + j) * 2 + 0) * S + n];
-    cplx rd = a.ov[(((size_t)OV_SHRAD * P + j) * 2 + 1) * S + n];
-    A0[p] = jn * c;                                                   // Symbol.cpp:52-58
-    A1[p] = I * (mk(1.0) / kj) * rd * d;                              // :61-67
-    Am1[p] = I * sqrt(n * (n + 1.0)) * ((mk(1.0) / kj) / R) * jn * d;  // :70-78
+    const cplx *xint = a.xint + z * a.zvec, *ov = a.ov + z * a.zov;
+    const double R = a.radius[j];
+    const cplx kj = omega(z) * csqrt_(a.eps[(size_t)z * P + j] * a.mu[j]);
+    cplx c = conj(xint[(size_t)j * 2 * nf + p]), d = conj(xint[(size_t)j * 2 * nf + nf + p]);
+    cplx jn = ov[(((size_t)OV_SHRAD * P + j) * 2 + 0) * S + n];
+    cplx rd = ov[(((size_t)OV_SHRAD * P + j) * 2 + 1) * S + n];
+    A0[o][p] = jn * c;                                                   // Symbol.cpp:52-58
+    A1[o][p] = I * (mk(1.0) / kj) * rd * d;                              // :61-67
+    Am1[o][p] = I * sqrt(n * (n + 1.0)) * ((mk(1.0) / kj) / R) * jn * d;  // :70-78
   }
   __syncthreads();
-  cplx sv = mk(0.0), su = mk(0.0), g = mk(0.0), f = mk(0.0);
+  cplx sv[PB], su[PB], g[PB], f[PB];
+#pragma unroll
+  for(int o = 0; o < PB; ++o) sv[o] = su[o] = g[o] = f[o] = mk(0.0);
   const double *tb = a.tab + (size_t)kk * nf * nf;
   // every table entry carries the Clebsch-Gordan factor <J M | J1 M1 J2 M2>,
   // zero unless M1 + M2 = M: only q = (J2, M - M1) is visited for each p
@@ -168,41 +180,57 @@ __global__ __launch_bounds__(256) void shsrc_kernel(ShArgs a) {
     const int q = flat(n2, m2), e = p * nf + q;
     double c10 = tb[e], c11 = tb[sz + e], c00 = tb[2 * sz + e], c01 = tb[3 * sz + e];
     double wm = tb[4 * sz + e], w11 = tb[5 * sz + e], w00 = tb[6 * sz + e], w10 = tb[7 * sz + e], w01 = tb[8 * sz + e];
-    cplx a1p = A1[p], a0p = A0[p], amq = Am1[q];
-    sv = sv + (a1p * amq) * c00 + (a0p * amq) * c01;
-    su = su + (a1p * amq) * c10 + (a0p * amq) * c11;
-    g = g + (Am1[p] * amq) * wm;
-    f = f + (a1p * A1[q]) * w11 + (a0p * A0[q]) * w00 + (a1p * A0[q]) * w10 + (a0p * A1[q]) * w01;
+#pragma unroll
+    for(int o = 0; o < PB; ++o) {
+      if(PB > 1 && o >= np) break;
+      cplx a1p = A1[o][p], a0p = A0[o][p], amq = Am1[o][q];
+      sv[o] = sv[o] + (a1p * amq) * c00 + (a0p * amq) * c01;
+      su[o] = su[o] + (a1p * amq) * c10 + (a0p * amq) * c11;
+      g[o] = g[o] + (Am1[o][p] * amq) * wm;
+      f[o] = f[o] + (a1p * A1[o][q]) * w11 + (a0p * A0[o][q]) * w00 + (a1p * A0[o][q]) * w10 + (a0p * A1[o][q]) * w01;
+    }
   }
-  red[0][t] = sv;
-  red[1][t] = su;
-  red[2][t] = g;
-  red[3][t] = f;
-  __syncthreads();
-  for(int st = 128; st > 0; st >>= 1) {
-    if(t < st)
-      for(int e = 0; e < 4; ++e) red[e][t] = red[e][t] + red[e][t + st];
+  // each sum by halves of the 256 threads; wave w takes the w-th of the four
+  const int w = t >> 6, l = t & 63;
+#pragma unroll
+  for(int o = 0; o < PB; ++o) {
+    if(o >= np) break;
+    red[0][t] = sv[o];
+    red[1][t] = su[o];
+    red[2][t] = g[o];
+    red[3][t] = f[o];
+    __syncthreads();
+    cplx s = (red[w][l] + red[w][l + 128]) + (red[w][l + 64] + red[w][l + 192]);
+#pragma unroll
+    for(int h = 32; h > 0; h >>= 1) {
+      s.x += __shfl_xor(s.x, h, 64);
+      s.y += __shfl_xor(s.y, h, 64);
+    }
+    if(l == 0) tot[o][w] = s;
     __syncthreads();
   }
-  if(t == 0) {
+  if(t < np) {
+    const int z = (pr0 + t) / P, j = (pr0 + t) % P;
+    const cplx *ov = a.ov + z * a.zov;
+    const double R = a.radius[j];
     int n, m;
     unflat(kk, n, m);
     const cplx mu0 = mk(4.0 * kPi * 1e-7);
     const cplx eps0 = mk(1.0 / (4.0 * kPi * 1e-7 * kC0 * kC0));
     const cplx eta = csqrt_(a.bg_mu / a.bg_eps) / csqrt_(mu0 / eps0);
-    const cplx k01 = a.omega * csqrt_(eps0 * mu0);
-    const cplx kpar = a.ksiparppar[j], kppp = a.ksippp[j], gam = a.gamma[j], epsj2 = a.eps_sh[j];
-    cplx vp = red[0][0] * mk(2.0) * kpar * eta;                                   // Symbol.cpp:274-275
-    cplx up = red[1][0] * mk(2.0) * I * kpar * eta;                               // :212-213
+    const cplx k01 = omega(z) * csqrt_(eps0 * mu0);
+    const cplx kpar = a.ksiparppar[j], kppp = a.ksippp[j], gam = a.gamma[j], epsj2 = a.eps_sh[(size_t)z * P + j];
+    cplx vp = tot[t][0] * mk(2.0) * kpar * eta;                                   // Symbol.cpp:274-275
+    cplx up = tot[t][1] * mk(2.0) * I * kpar * eta;                               // :212-213
     double snn = sqrt((double)(n * (n + 1)));
-    cplx upp = I * kppp * snn * red[2][0] / k01 / R +                              // :347-351
-               I * gam * (eps0 / epsj2) * snn * (red[2][0] + red[3][0]) / k01 / R;
-    auto ovv = [&](int kind, int pol) { return a.ov[(((size_t)kind * P + j) * 2 + pol) * S + n]; };
-    size_t b = (size_t)j * 2 * nf;
-    a.K[b + kk] = ovv(OV_TSH1O, 0) * vp + ovv(OV_TSH2O, 0) * mk(0.0);
-    a.K[b + nf + kk] = ovv(OV_TSH1O, 1) * up + ovv(OV_TSH2O, 1) * upp;
-    a.K1[b + kk] = ovv(OV_IAUXSH2, 0) * mk(0.0);
-    a.K1[b + nf + kk] = ovv(OV_IAUXSH2, 1) * upp;
+    cplx upp = I * kppp * snn * tot[t][2] / k01 / R +                              // :347-351
+               I * gam * (eps0 / epsj2) * snn * (tot[t][2] + tot[t][3]) / k01 / R;
+    auto ovv = [&](int kind, int pol) { return ov[(((size_t)kind * P + j) * 2 + pol) * S + n]; };
+    cplx *K = a.K + z * a.zvec + (size_t)j * 2 * nf, *K1 = a.K1 + z * a.zvec + (size_t)j * 2 * nf;
+    K[kk] = ovv(OV_TSH1O, 0) * vp + ovv(OV_TSH2O, 0) * mk(0.0);
+    K[nf + kk] = ovv(OV_TSH1O, 1) * up + ovv(OV_TSH2O, 1) * upp;
+    K1[kk] = ovv(OV_IAUXSH2, 0) * mk(0.0);
+    K1[nf + kk] = ovv(OV_IAUXSH2, 1) * upp;
   }
 }
 
@@ -381,9 +409,14 @@ void run_abssh(const AbsShArgs &a, hipStream_t st) {
   hipLaunchKernelGGL(abssh_sum_kernel, dim3((a.P + 63) / 64, 1, a.nb), dim3(64), 0, st, a);
 }
 
+// Four objects a block once that leaves two blocks for every CU (nmax 10, 64
+// systems of 16: above; one system of 17 objects, nmax 7: 24 us with one).
 void run_shsrc(const ShArgs &a, hipStream_t st) {
-  int nf = a.nmax * (a.nmax + 2);
-  hipLaunchKernelGGL(shsrc_kernel, dim3(a.P, nf), dim3(256), 0, st, a);
+  const int nf = a.nmax * (a.nmax + 2), np = a.P * a.nb;
+  if((long)np * nf >= 4 * 512)
+    hipLaunchKernelGGL(shsrc_kernel<4>, dim3((np + 3) / 4, nf), dim3(256), 0, st, a);
+  else
+    hipLaunchKernelGGL(shsrc_kernel<1>, dim3(np, nf), dim3(256), 0, st, a);
 }
 
 }  // namespace omx

@@ -15,6 +15,10 @@ struct ShArgs {
   const double *tab;             // nine tables [9][nf][nf][nf]
   const cplx *xint;              // x_int (N); the source uses conj(x_int)
   cplx *K, *K1;                  // out: N each
+  // nb systems: omega at omz, eps and eps_sh P apart, the vectors zvec, ov zov
+  int nb = 1;
+  const double *omz = nullptr;
+  size_t zvec = 0, zov = 0;
 };
 
 // Result::getAbsorptionCrossSection_SH (Result.cpp:763-794): per object the
