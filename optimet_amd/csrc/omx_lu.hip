@@ -1326,17 +1326,19 @@ struct SplitTile {
   static constexpr int TM = 128, TN = 128, WGM = 2, WGN = 2, BK = 16, GM = 8;
 };
 
-constexpr long kThinRows = 16384;  // columns that fill the chip with split tiles of 128 rows, half of it busy
 // The bulk update with K = KD (2 NB or 4 NB): split-bf16 for FP32 factors when
 // `split`, gemm_tile otherwise.  M and N are multiples of 64.
+constexpr int kThinTiles = 512;  // two split tiles for every CU
 template <typename T, int KD = 2 * kNB>
 void bulk_update(T *A, size_t lda, int row0, int col0, int k0, int M, int N, hipStream_t st, int nb, size_t sA,
                  bool split) {
   if(M <= 0 || N <= 0) return;
-  if(N <= 2 * kNB || (M <= 2 * kNB && (long)N * nb <= kThinRows)) {
+  const long tiles = (long)((M + 127) / 128) * ((N + 127) / 128) * nb;
+  if((M <= 2 * kNB || N <= 2 * kNB) && (!split || tiles < kThinTiles)) {
     // the next pair's columns or a second pair's block rows (on the panel chain's
     // critical path): small tiles over many workgroups finish sooner than a few
-    // large split tiles (128 rows by 1800 columns: 9 us against 29)
+    // large split tiles (128 rows by 1800 columns: 9 us against 29); a batch's
+    // fill the chip with split tiles as well
     trailing_update<T, KD, ThinTile>(A, lda, row0, col0, k0, M, N, st, nb, sA);
     return;
   }
