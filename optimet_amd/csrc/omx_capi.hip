@@ -352,6 +352,7 @@ void alloc_lu(omx_context *c, omx::LuWork &w, DBuf &perm, DBuf &dinv, bool secon
   w.status = status.as<int>();
   w.wlu = c->d_wlu.as<cplx>() + (size_t)half * 3 * omx::kNB * omx::kNB;
   w.dinv = dinv.p;
+  w.links = true;
   w.pivot = c->pivot;
   hipEvent_t *ev = second ? c->lu_ev2 : c->lu_ev;
   w.aux = second ? c->aux2 : c->aux;
@@ -1282,6 +1283,7 @@ omx::LuWork sweep_lu(omx_context *c, int nb, bool second) {
   omx::LuWork lw{};
   lw.perm = (second ? w.perm2 : w.perm).as<int>();
   lw.dinv = (second ? w.dinv2 : w.dinv).p;
+  lw.links = true;
   const int ms = Np + 2 * omx::kNB;
   int *map = (second ? w.map2 : w.map).as<int>();
   lw.mdst = map;

@@ -1354,6 +1354,46 @@ void bulk_update(T *A, size_t lda, int row0, int col0, int k0, int M, int N, hip
   trailing_update<T, KD>(A, lda, row0, col0, k0, M, N, st, nb, sA);
 }
 
+// ------------------------------------------------------------------ links
+// The triangular solves' links Linv_k L[k, k-1] (blockIdx.y = 0, k = blockIdx.x +
+// 1) and Uinv_k U[k, k+1] (1, k = blockIdx.x), beside the inverses they are formed
+// with: 64 x 64, column-major.  Wave w takes 16 rows.
+template <typename T>
+__global__ __launch_bounds__(256) void link_kernel(const T *A, size_t lda, const T *dinv, T *links, BatchStrides bs) {
+  using C = CxOf<T>;
+  using V4 = typename CT<T>::V4;
+  const bool up = blockIdx.y;
+  const int k = blockIdx.x + (up ? 0 : 1), kc = up ? k + 1 : k - 1;
+  const size_t at = blockIdx.z * bs.inv + (size_t)k * 2 * kNB * kNB + (up ? kNB * kNB : 0);
+  const T *M = dinv + at, *B = A + blockIdx.z * bs.a + (size_t)kc * kNB * lda + (size_t)k * kNB;
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6, li = lane & 15, g = lane >> 4;
+  C m[16];
+#pragma unroll
+  for(int s = 0; s < 16; ++s) {
+    const T v = M[(4 * s + g) * kNB + 16 * w + li];
+    m[s] = C{v.x, v.y};
+  }
+#pragma unroll
+  for(int n = 0; n < 4; ++n) {
+    V4 xr = {0, 0, 0, 0}, xi = {0, 0, 0, 0};
+#pragma unroll
+    for(int s = 0; s < 16; ++s) {
+      const T v = B[(size_t)(16 * n + li) * lda + 4 * s + g];
+      xr = CT<T>::mfma(v.x, m[s].x, xr);
+      xi = CT<T>::mfma(v.x, m[s].y, xi);
+      xr = CT<T>::mfma(-v.y, m[s].y, xr);
+      xi = CT<T>::mfma(v.y, m[s].x, xi);
+    }
+#pragma unroll
+    for(int v = 0; v < 4; ++v) {
+      T o;
+      o.x = xr[v];
+      o.y = xi[v];
+      links[at + (16 * n + CT<T>::row(lane, v)) * kNB + 16 * w + li] = o;
+    }
+  }
+}
+
 // ------------------------------------------------------------------ driver
 // Panels of NB columns are taken in pairs (p0 = J, p1 = J + NB), and pairs in
 // groups of one or two, so that the bulk of the trailing update runs with K = 2 NB
@@ -1398,6 +1438,11 @@ int lu_factor(T *A, int Np, size_t lda, LuWork &w, hipStream_t st, LuProf *prof)
     prof->gemm_flop = 0.0;
     prof->gemm_launches = 0;
   }
+  auto links = [&] {
+    if(w.links && Np > kNB)
+      hipLaunchKernelGGL((link_kernel<T>), dim3(Np / kNB - 1, 2, nb), dim3(256), 0, st, A, lda, dinv,
+                         dinv + links_at(Np), bs);
+  };
   if(block) {
     // G panels a group: quads (two pairs), whose bulk update has K = 4 NB, where
     // that update is the split-bf16 one, which C's traffic holds back at K = 2 NB;
@@ -1496,6 +1541,7 @@ int lu_factor(T *A, int Np, size_t lda, LuWork &w, hipStream_t st, LuProf *prof)
     if(Np > kNB)
       hipLaunchKernelGGL((laswp_left<T>), dim3((Np - kNB) / 8, Np / kNB - 1, nb), dim3(256), 0, st, A, lda,
                          w.msrc, bs);
+    links();
     return 0;
   }
 
@@ -1566,6 +1612,7 @@ int lu_factor(T *A, int Np, size_t lda, LuWork &w, hipStream_t st, LuProf *prof)
     if(w.ev_mark && p1 + kNB >= w.mark_col && p0 < w.mark_col) mark(w, st);
   }
   if(w.ev_mark && Np < w.mark_col) mark(w, st);
+  links();
   return 0;
 }
 
@@ -1601,7 +1648,12 @@ __global__ void gather_kernel(const cplx *b, const int *perm, cplx *y, int Np, B
 // super-block's own blocks are solved in sequence inside the workgroup -- the
 // contributions of the blocks just solved, then the stored inverse of the
 // diagonal block -- so only every SB-th link of the chain crosses
-// workgroups.  With PRE the near phase's tiles (diagonal-block inverses and
+// workgroups.  SB = 1 with links: the neighbour's contribution comes last, by one
+// product with the stored Dinv_k L[k, k-1]: what waits on the chain's last link
+// is that product alone, the rest and the inverse having been applied before (a
+// solve of N = 2208: 95 -> 70 us FP64, N = 2176: 71 -> 62 us FP32, 10240: 360 ->
+// 330; forming the links takes 12 us, 46 us at 10240).
+// With PRE the near phase's tiles (diagonal-block inverses and
 // the intra-super-block L tiles) are loaded into registers at kernel start
 // (PRE = 1) or after the far phase (PRE = 2).  Thread t handles row
 // r = t % 64 and columns 16 (t / 64) .. 16 (t / 64) + 15 of every tile.
@@ -1617,7 +1669,8 @@ __global__ void gather_kernel(const cplx *b, const int *perm, cplx *y, int Np, B
 template <typename T, bool LOWER, int SB, int PRE>
 __global__ __launch_bounds__(256) void trsv_kernel(const T *__restrict__ A, size_t lda, int Np,
                                                    const T *__restrict__ dinv, cplx *x,
-                                                   int *status, BatchStrides bs, const int *live) {
+                                                   int *status, BatchStrides bs, const int *live,
+                                                   const T *__restrict__ links) {
   constexpr int NB = kNB;
   constexpr int NI = SB * (SB - 1) / 2;
   const size_t zs = blockIdx.z;
@@ -1670,8 +1723,51 @@ __global__ __launch_bounds__(256) void trsv_kernel(const T *__restrict__ A, size
       }
   };
   if(PRE == 1) preload();
-  const int nfar = LOWER ? kb0 : nblk - (kb0 + nb);
+  const int nfar_all = LOWER ? kb0 : nblk - (kb0 + nb);
+  const bool lk = SB == 1 && links != nullptr && nfar_all > 0;
+  const int nfar = nfar_all - (lk ? 1 : 0);
+  T wl[SB == 1 ? 16 : 1];
+  if constexpr(SB == 1)
+    if(lk) tile(links + zs * bs.inv + (size_t)kb0 * 2 * NB * NB + (LOWER ? 0 : NB * NB), NB, wl);
   auto fblk = [&](int j) { return LOWER ? j : nblk - 1 - j; };  // j-th far block in order of publication
+  // wave 0, one entry per lane: the far blocks from j0 on, as far as they are
+  // published (at least one, at most CH, none past end), into xs: each poll reads
+  // a whole block and keeps it when every word carries the tag; the blocks after
+  // a published one are tried at once
+  auto poll = [&](int j0, int end) {
+    unsigned spins = 0;
+    int nr = 0;
+    bool drain = false;
+    while(nr < CH && j0 + nr < end) {
+      const unsigned long long *src =
+          reinterpret_cast<const unsigned long long *>(x + (size_t)fblk(j0 + nr) * NB + t);
+      const unsigned long long re = __hip_atomic_load(src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const unsigned long long im = __hip_atomic_load(src + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const bool ok = (re & kTagMask) == tg && (im & kTagMask) == tg;
+      if(__ballot(ok) == ~0ull) {
+        xs[nr * NB + t] = mk(__longlong_as_double((long long)re), __longlong_as_double((long long)im));
+        ++nr;
+        continue;
+      }
+      if(nr > 0) break;
+      if(__builtin_amdgcn_readfirstlane(
+             __hip_atomic_load(&status[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0) {
+        drain = true;
+        break;
+      }
+      if(++spins > (1u << 24)) {
+        if(t == 0) __hip_atomic_store(&status[1], 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        drain = true;
+        break;
+      }
+      __builtin_amdgcn_s_sleep(1);
+    }
+    if(drain) {  // a timed-out wait: finish with zeros (the host reports the error)
+      nr = min(CH, end - j0);
+      for(int c = 0; c < nr; ++c) xs[c * NB + t] = mk(0.0);
+    }
+    if(t == 0) nready_s = nr;
+  };
   // ---- far phase
   cplx acc[SB];
 #pragma unroll
@@ -1679,43 +1775,7 @@ __global__ __launch_bounds__(256) void trsv_kernel(const T *__restrict__ A, size
   T cur[16], nxt[16];
   if(nfar > 0) tile(a_base(kb0, fblk(0)), lda, cur);
   for(int j0 = 0; j0 < nfar;) {
-    // the next far blocks, as far as they are published (wave 0, one entry
-    // per lane): each poll reads a whole block and keeps it when every word
-    // carries the tag; the blocks after a published one are tried at once
-    if(t < 64) {
-      unsigned spins = 0;
-      int nr = 0;
-      bool drain = false;
-      while(nr < CH && j0 + nr < nfar) {
-        const unsigned long long *src =
-            reinterpret_cast<const unsigned long long *>(x + (size_t)fblk(j0 + nr) * NB + t);
-        const unsigned long long re = __hip_atomic_load(src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const unsigned long long im = __hip_atomic_load(src + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const bool ok = (re & kTagMask) == tg && (im & kTagMask) == tg;
-        if(__ballot(ok) == ~0ull) {
-          xs[nr * NB + t] = mk(__longlong_as_double((long long)re), __longlong_as_double((long long)im));
-          ++nr;
-          continue;
-        }
-        if(nr > 0) break;
-        if(__builtin_amdgcn_readfirstlane(
-               __hip_atomic_load(&status[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0) {
-          drain = true;
-          break;
-        }
-        if(++spins > (1u << 24)) {
-          if(t == 0) __hip_atomic_store(&status[1], 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          drain = true;
-          break;
-        }
-        __builtin_amdgcn_s_sleep(1);
-      }
-      if(drain) {  // a timed-out wait: finish with zeros (the host reports the error)
-        nr = min(CH, nfar - j0);
-        for(int c = 0; c < nr; ++c) xs[c * NB + t] = mk(0.0);
-      }
-      if(t == 0) nready_s = nr;
-    }
+    if(t < 64) poll(j0, nfar);
     __syncthreads();
     const int nr = nready_s;
     for(int c = 0; c < nr; ++c) {
@@ -1811,8 +1871,24 @@ __global__ __launch_bounds__(256) void trsv_kernel(const T *__restrict__ A, size
       }
       part[cq][r] = y;
       __syncthreads();
+      cplx sum = mk(0.0);
+      if(t < NB) sum = part[0][t] + part[1][t] + part[2][t] + part[3][t];
+      if constexpr(SB == 1)
+        if(lk) {
+          if(t < 64) poll(nfar, nfar_all);
+          __syncthreads();
+          cplx l = mk(0.0);
+#pragma unroll
+          for(int cc = 0; cc < 16; ++cc) {
+            const cplx xv = xs[cq * 16 + cc];
+            l.x += (double)wl[cc].x * xv.x - (double)wl[cc].y * xv.y;
+            l.y += (double)wl[cc].x * xv.y + (double)wl[cc].y * xv.x;
+          }
+          part[cq][r] = l;
+          __syncthreads();
+          if(t < NB) sum = sum - (part[0][t] + part[1][t] + part[2][t] + part[3][t]);
+        }
       if(t < NB) {
-        const cplx sum = part[0][t] + part[1][t] + part[2][t] + part[3][t];
         const cplx xk = mk(with_tag(sum.x, tg), with_tag(sum.y, tg));
         xsb[s][t] = xk;
         unsigned long long *dst = reinterpret_cast<unsigned long long *>(x + (size_t)k * NB + t);
@@ -1845,12 +1921,12 @@ template <typename T, int V>
 static void trsv_pair(const T *A, int Np, size_t lda, LuWork &w, cplx *x, int nz, hipStream_t st) {
   constexpr int SB = TrsvCfg<T>::SB[V];
   constexpr int PRE = TrsvCfg<T>::PRE[V];
-  const T *dinv = reinterpret_cast<const T *>(w.dinv);
+  const T *dinv = reinterpret_cast<const T *>(w.dinv), *links = w.links ? dinv + links_at(Np) : nullptr;
   const int nblk = Np / kNB, nsb = (nblk + SB - 1) / SB;
   hipLaunchKernelGGL((trsv_kernel<T, true, SB, PRE>), dim3(nsb, 1, nz), dim3(256), 0, st, A, lda, Np, dinv, x,
-                     w.status, w.bs, w.live);
+                     w.status, w.bs, w.live, links);
   hipLaunchKernelGGL((trsv_kernel<T, false, SB, PRE>), dim3(nsb, 1, nz), dim3(256), 0, st, A, lda, Np, dinv, x,
-                     w.status, w.bs, w.live);
+                     w.status, w.bs, w.live, links);
 }
 
 template <typename T>
