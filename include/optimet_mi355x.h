@@ -217,7 +217,10 @@ int omx_set_cg_tables(omx_context *ctx, int nmax, const double *const *tables);
 int omx_build_cg_tables(omx_context *ctx, int nmax);
 
 /* AbstractSolver::update(): plane-wave coefficients, T-matrices, source
- * vector Q, scattering matrix S and, with SH_cond, V on the device. */
+ * vector Q, scattering matrix S and, with SH_cond, V on the device.  Returns
+ * once its kernels are enqueued on the context's streams; every later call on
+ * the context (or on a group's leader) is ordered behind them, and
+ * omx_get_stats waits for their times. */
 int omx_update(omx_context *ctx);
 
 /* AbstractSolver::solve(): writes N complex values into each non-NULL output

@@ -325,7 +325,7 @@ bool is_lu(int kind) { return kind == OMX_SOLVER_LU64 || kind == OMX_SOLVER_LU32
 void alloc_lu(omx_context *c, omx::LuWork &w, DBuf &perm, DBuf &dinv, bool second) {
   const int Np = c->Np;
   const int gmax = (Np + omx::kPanelRows - 1) / omx::kPanelRows + 1;
-  dinv.ensure(sizeof(cplx) * omx::dinv_elems(Np), &c->total);
+  dinv.ensure(sizeof(cplx) * omx::dinv_elems(Np, c->kind == OMX_SOLVER_LU64), &c->total);
   perm.ensure(sizeof(int) * Np, &c->total);
   // tournament scratch: one half per system, as S and V may be factored
   // at the same time
@@ -352,7 +352,7 @@ void alloc_lu(omx_context *c, omx::LuWork &w, DBuf &perm, DBuf &dinv, bool secon
   w.status = status.as<int>();
   w.wlu = c->d_wlu.as<cplx>() + (size_t)half * 3 * omx::kNB * omx::kNB;
   w.dinv = dinv.p;
-  w.links = true;
+  w.links = c->kind == OMX_SOLVER_LU64;
   w.pivot = c->pivot;
   hipEvent_t *ev = second ? c->lu_ev2 : c->lu_ev;
   w.aux = second ? c->aux2 : c->aux;
@@ -1263,7 +1263,7 @@ void sweep_alloc(omx_context *c, int nb, bool f64, bool sh) {
   w.abssh.ensure(sizeof(double) * P * nb, T);
   w.absbes.ensure(sizeof(cplx) * P * omx::kAbsBes * nb, T);
   for(DBuf *b : {&w.perm, &w.perm2}) b->ensure(sizeof(int) * Np * nb, T);
-  for(DBuf *b : {&w.dinv, &w.dinv2}) b->ensure(sizeof(cplx) * omx::dinv_elems(Np) * nb, T);
+  for(DBuf *b : {&w.dinv, &w.dinv2}) b->ensure(sizeof(cplx) * omx::dinv_elems(Np, f64) * nb, T);
   w.map.ensure(sizeof(int) * 3 * (Np + 2 * omx::kNB) * nb, T);
   w.status.ensure(sizeof(int) * 4 * nb, T);
   if(sh) {  // V's factorisation runs beside S's: maps and status words of its own
@@ -1283,7 +1283,7 @@ omx::LuWork sweep_lu(omx_context *c, int nb, bool second) {
   omx::LuWork lw{};
   lw.perm = (second ? w.perm2 : w.perm).as<int>();
   lw.dinv = (second ? w.dinv2 : w.dinv).p;
-  lw.links = true;
+  lw.links = c->kind == OMX_SOLVER_LU64;
   const int ms = Np + 2 * omx::kNB;
   int *map = (second ? w.map2 : w.map).as<int>();
   lw.mdst = map;
@@ -1303,7 +1303,7 @@ omx::LuWork sweep_lu(omx_context *c, int nb, bool second) {
   lw.split = c->lu32_gemm == OMX_GEMM_BF16X3;
   lw.nb = nb;
   lw.bs.a = (size_t)Np * Np;
-  lw.bs.inv = omx::dinv_elems(Np);
+  lw.bs.inv = omx::dinv_elems(Np, c->kind == OMX_SOLVER_LU64);
   lw.bs.vec = (size_t)Np;
   lw.bs.perm = Np;
   lw.bs.map = ms;
@@ -2353,7 +2353,7 @@ void group_alloc(omx_context *L, int nb, bool f64, bool sh) {
   }
   for(DBuf *b : {&w.Q, &w.x, &w.xsh, &w.K, &w.r, &w.w1, &w.w2}) b->ensure(sizeof(cplx) * Np * nb, T);
   for(DBuf *b : {&w.perm, &w.perm2}) b->ensure(sizeof(int) * Np * nb, T);
-  for(DBuf *b : {&w.dinv, &w.dinv2}) b->ensure(sizeof(cplx) * omx::dinv_elems(Np) * nb, T);
+  for(DBuf *b : {&w.dinv, &w.dinv2}) b->ensure(sizeof(cplx) * omx::dinv_elems(Np, f64) * nb, T);
   for(DBuf *b : {&w.map, &w.map2}) b->ensure(sizeof(int) * 3 * (Np + 2 * omx::kNB) * nb, T);
   for(DBuf *b : {&w.status, &w.status2}) b->ensure(sizeof(int) * 4 * nb, T);
   w.basis.ensure(sizeof(cplx) * Np * (m + 1) * nb, T);

@@ -203,7 +203,7 @@ struct LuWork {
   int *status;          // [0]: singular pivot column+1, [1]: wait timeout
   void *wlu;            // NB x NB complex: the tournament's selected-block factors
   void *dinv;           // per panel [L11^{-1} | U11^{-1}], 2 NB^2 elements of T, column-major
-  bool links = false;   // the triangular solves' links follow in dinv
+  bool links = false;   // FP64 factors: the triangular solves' links follow in dinv
   hipStream_t aux;      // look-ahead stream of the panel pivoting
   hipEvent_t ev_next, ev_piv, ev_bulk, ev_pan;
   int gmax;
@@ -218,10 +218,10 @@ struct LuWork {
   void (*on_mark)(void *) = nullptr;  // then on_mark(mark_arg) is called (on the host,
   void *mark_arg = nullptr;           // in the middle of the enqueueing)
 };
-// Elements of T in a factorisation's dinv: 2 NB^2 per panel, and as many of the
-// triangular solves' links, from links_at on.
+// Elements of T in a factorisation's dinv: 2 NB^2 per panel, and (FP64 factors) as
+// many of the triangular solves' links, from links_at on.
 inline size_t links_at(int Np) { return 2 * (size_t)64 * Np; }
-inline size_t dinv_elems(int Np) { return 2 * links_at(Np); }
+inline size_t dinv_elems(int Np, bool f64) { return (f64 ? 2 : 1) * links_at(Np); }
 
 // Pivot search of a panel: among the rows of its diagonal block only
 // (followed by iterative refinement), or over the whole column (tournament).

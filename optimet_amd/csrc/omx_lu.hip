@@ -1355,7 +1355,7 @@ void bulk_update(T *A, size_t lda, int row0, int col0, int k0, int M, int N, hip
 }
 
 // ------------------------------------------------------------------ links
-// The triangular solves' links Linv_k L[k, k-1] (blockIdx.y = 0, k = blockIdx.x +
+// The triangular solves' links (FP64 factors) Linv_k L[k, k-1] (blockIdx.y = 0, k = blockIdx.x +
 // 1) and Uinv_k U[k, k+1] (1, k = blockIdx.x), beside the inverses they are formed
 // with: 64 x 64, column-major.  Wave w takes 16 rows.
 template <typename T>
@@ -1439,9 +1439,10 @@ int lu_factor(T *A, int Np, size_t lda, LuWork &w, hipStream_t st, LuProf *prof)
     prof->gemm_launches = 0;
   }
   auto links = [&] {
-    if(w.links && Np > kNB)
-      hipLaunchKernelGGL((link_kernel<T>), dim3(Np / kNB - 1, 2, nb), dim3(256), 0, st, A, lda, dinv,
-                         dinv + links_at(Np), bs);
+    if constexpr(std::is_same<T, double2>::value)
+      if(w.links && Np > kNB)
+        hipLaunchKernelGGL((link_kernel<T>), dim3(Np / kNB - 1, 2, nb), dim3(256), 0, st, A, lda, dinv,
+                           dinv + links_at(Np), bs);
   };
   if(block) {
     // G panels a group: quads (two pairs), whose bulk update has K = 4 NB, where
@@ -1651,8 +1652,9 @@ __global__ void gather_kernel(const cplx *b, const int *perm, cplx *y, int Np, B
 // workgroups.  SB = 1 with links: the neighbour's contribution comes last, by one
 // product with the stored Dinv_k L[k, k-1]: what waits on the chain's last link
 // is that product alone, the rest and the inverse having been applied before (a
-// solve of N = 2208: 95 -> 70 us FP64, N = 2176: 71 -> 62 us FP32, 10240: 360 ->
-// 330; forming the links takes 12 us, 46 us at 10240).
+// solve of N = 2208: 95 -> 70 us; forming the links takes 12 us).  FP64 factors
+// only: a product of FP32 factors would have to be rounded to 32 bits between the
+// FP64 sums of the two products it replaces (and gave 71 -> 62 us at N = 2176).
 // With PRE the near phase's tiles (diagonal-block inverses and
 // the intra-super-block L tiles) are loaded into registers at kernel start
 // (PRE = 1) or after the far phase (PRE = 2).  Thread t handles row
@@ -1921,7 +1923,8 @@ template <typename T, int V>
 static void trsv_pair(const T *A, int Np, size_t lda, LuWork &w, cplx *x, int nz, hipStream_t st) {
   constexpr int SB = TrsvCfg<T>::SB[V];
   constexpr int PRE = TrsvCfg<T>::PRE[V];
-  const T *dinv = reinterpret_cast<const T *>(w.dinv), *links = w.links ? dinv + links_at(Np) : nullptr;
+  const T *dinv = reinterpret_cast<const T *>(w.dinv), *links = nullptr;
+  if(std::is_same<T, double2>::value && w.links) links = dinv + links_at(Np);
   const int nblk = Np / kNB, nsb = (nblk + SB - 1) / SB;
   hipLaunchKernelGGL((trsv_kernel<T, true, SB, PRE>), dim3(nsb, 1, nz), dim3(256), 0, st, A, lda, Np, dinv, x,
                      w.status, w.bs, w.live, links);
