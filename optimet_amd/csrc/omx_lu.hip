@@ -1494,7 +1494,11 @@ int lu_factor(T *A, int Np, size_t lda, LuWork &w, hipStream_t st, LuProf *prof)
       // for a bulk update that it can run beside
       const int last = far - 2 * kNB;  // the group's last pair
       const bool apart = restf > 0 && (long)restf / 16 * nb > kWideStrips;
-      if(apart) through(last, true, 0, far);
+      if(apart) {
+        // by the kernel of a single panel, whose workgroups fit beside the update's
+        const int pl = last + kNB;
+        panel_products<T, false>(A, lda, pl, 0, restf, far, 0, far, dk(pl), nullptr, nullptr, nullptr, sb, nb, bs);
+      }
       if(rec) (void)hipEventRecord(pe[1], sb);
       if(restf > 0) {
         (void)hipStreamWaitEvent(sb, w.ev_bulk, 0);
