@@ -33,7 +33,7 @@ BF16_MFMA_TFLOPS = 2500.0  # MI355X dense bf16 matrix peak
 SPLIT_TFLOPS = BF16_MFMA_TFLOPS / 6
 FP64_MFMA_TFLOPS = 78.6    # MI355X dense FP64 matrix peak
 HBM_GBS = 8000.0
-GEMM_KERNEL = {"lu32ir": "gemm_split<128,128,128,4,2,16,8,true,true> (bf16x3 split, complex FP32, double-buffered split planes, nontemporal C; next-pair 128 columns on gemm_tile<float2,32,32>)",
+GEMM_KERNEL = {"lu32ir": "gemm_split<128,128,256,2,2,16,8> (bf16x3 split, complex FP32, K = 256, nontemporal C; the next 256 columns on gemm_tile<float2,32,32>)",
                "lu64": "gemm_tile<double2,128,64,128,4,2,16> (next-pair 128 columns on gemm_tile<double2,32,32>)"}
 TRAFFIC_FILE = os.path.join(os.path.dirname(os.path.abspath(__file__)), "profiles",
                             "traffic_gemm_split_config2.txt")
@@ -84,7 +84,7 @@ def stage_rooflines(c, st, mixed_copy):
         out["assembly"] = {"bound": "hbm", "kernel": "pair_kernel (S and V) with objects, incident and origin kernels",
                            "achieved": gbs, "peak": HBM_GBS, "unit": "GB/s", "frac": gbs / HBM_GBS,
                            "bytes": store, "ms": st["t_assemble_ms"]}
-    mv = matvec_roofline(st, "gemv_part_kernel (FP64 matvec of the refinement) + gemv_reduce_kernel")
+    mv = matvec_roofline(st, "gemv_part_kernel (FP64 matvec of GMRES and of the refinement)")
     if mv is not None:
         out["refinement_matvec"] = mv
     return out
@@ -159,7 +159,7 @@ def run_sweep(cluster, lams, kind, steps, warmup, batch, graphs=False):
     return {"lat": lat, "total": total, "out": out, "stats": st, "prof": prof}
 
 
-def matvec_roofline(st, kernel="gemv_part_kernel (batched FP64 matvec of the refinement) + gemv_reduce_kernel"):
+def matvec_roofline(st, kernel="gemv_part_kernel (batched FP64 matvec of the refinement)"):
     """The Krylov or refinement matvecs: their algorithmic bytes (16 Np^2 per
     FP64 product, 8 Np^2 per FP32-matrix product, per system) over the
     HIP-event time of their launches on the stream they run on."""
@@ -303,7 +303,7 @@ def config4_main(args):
                    "rule": "N >= 16384: the mixed Krylov within a budget of the mixed LU's cost (0.0143 N FP32 "
                            "products), else or when it does not converge there, the mixed LU + GMRES-IR"},
         "roofline": matvec_roofline(au["stats"], "gemv_part_kernel<float2> (inner products on the FP32 copy) and "
-                                    "gemv_part_kernel<cplx> (outer FP64 products), with gemv_reduce_kernel")
+                                    "gemv_part_kernel<cplx> (outer FP64 products)")
         if picked == "gmres32ir" else res["lu32ir"].get("roofline"),
         "speedup_vs_fp64": total["lu64"] / total["auto"],
         "speedup_mixed_lu_vs_fp64_lu": total["lu64"] / total["lu32ir"],
@@ -650,7 +650,7 @@ def main():
         tr = traffic_per_launch()
         roof["traffic"] = tr["bytes_per_split_launch"] if tr else None
         if tr:
-            roof["traffic_note"] = ("HBM bytes per gemm_split launch (the wide part of a pair's bulk update; "
+            roof["traffic_note"] = ("HBM bytes per gemm_split launch (the wide part of a group's bulk update; "
                                     f"algorithmic {tr['algorithmic_bytes_per_split_launch']:.3g} B), rocprofv3 "
                                     "FETCH_SIZE + WRITE_SIZE, copy-calibrated")
     line = {
