@@ -123,6 +123,7 @@ constexpr int kInnerSteps = 30;
 constexpr double kInnerTol = 1e-6;
 
 constexpr int kMarkN = 9216;  // see omx_solve
+constexpr int kSymN = 8192;   // see sym_args
 // OMX_SOLVER_AUTO: systems of order N >= kAutoKrylovN start with the mixed
 // Krylov, within a budget of outer steps whose matvecs cost what the mixed LU
 // would (8/3 N^3 flop at about 140 TFLOP/s against an 8 N^2-byte product at
@@ -206,7 +207,7 @@ struct omx_context {
   DBuf d_status2, d_map2;
   std::vector<hipEvent_t> pev2;
   omx::LuProf prof2{};
-  DBuf d_basis, d_basisZ, d_w1, d_w2, d_r, d_nrm, d_gpart;
+  DBuf d_basis, d_basisZ, d_w1, d_w2, d_r, d_nrm, d_gpart, d_sym;
   KryWs kry;
   // pinned host staging of the geometry, and the event after its last copy
   double *geo_pin = nullptr;
@@ -678,6 +679,9 @@ struct Krylov {
   const float2 *A32 = nullptr;
   std::function<void(const cplx *, cplx *)> op = nullptr;
   double op_bytes = 0.0;
+  // with scratch: the Arnoldi steps' products from half the blocks (the residuals
+  // come from the whole matrix)
+  omx::SymArgs sym{};
   // out = M^{-1} in for the systems whose flag is set (identity when null)
   std::function<void(const cplx *in, cplx *out, const int *live)> prec = nullptr;
   bool x_zero = false;     // x starts at 0: no product before the first cycle
@@ -690,12 +694,20 @@ struct Krylov {
   int bits = 0;            // binary digits between the residual and its goal, as last known
 
   // Enqueues A x into gpart (returns the column parts) or w (returns 0).
-  int product(const cplx *x, const int *flag, int live) {
+  int product(const cplx *x, const int *flag, int live, bool step) {
     const bool prof = c->profile;
     if(prof) HIPCHK(hipEventRecord(c->ev[6], s));
     int ns = 0;
     if(op)
       op(x, w);
+    else if(step && sym.scratch) {
+      omx::SymArgs a = sym;
+      a.flag = flag;
+      if(A32)
+        omx::sym_product(a, A32, x, w, s);
+      else
+        omx::sym_product(a, A, x, w, s);
+    }
     else if(A32)
       ns = omx::gemv_partial(A32, (size_t)c->Np, n, x, gpart, s, flag);
     else
@@ -709,10 +721,11 @@ struct Krylov {
     }
     return ns;
   }
-  void count(int live) {
+  void count(int live, bool step) {
     if(live < 1) return;
     ++c->mv_calls;
-    c->mv_bytes += (op ? op_bytes : (A32 ? 8.0 : 16.0) * n * (double)n) * live;
+    const double half = step && sym.scratch ? 0.5 : 1.0;
+    c->mv_bytes += (op ? op_bytes : half * (A32 ? 8.0 : 16.0) * n * (double)n) * live;
   }
   // Solves A x = b; x holds the initial guesses.  res: the final relative
   // residuals, its: the iterations.  (A one-cycle solve leaves both unread.)
@@ -765,13 +778,13 @@ struct Krylov {
       const int gain = last_bits - bits;
       left = known != restart && gain > 0 ? (double)bits / gain : 0.0;
       last_bits = bits;
-      if(known != restart) count(before);
+      if(known != restart) count(before, true);
     };
     int ns = 0;
     if(!x_zero && !one_cycle) {
-      ns = product(x, nullptr, nb);
+      ns = product(x, nullptr, nb, false);
       if(op) ns = -1;
-      count(nb);
+      count(nb, false);
     }
     omx::kry_restart(st, b, x, gpart, ns, (size_t)std::max(0, ns) * n, true, batch, slot(tick + 1), s);
     mark();
@@ -786,7 +799,7 @@ struct Krylov {
           prec(vj, zj, live);
           pj = zj;
         }
-        ns = product(pj, live, nlive);
+        ns = product(pj, live, nlive, true);
         omx::kry_step(st, gpart, ns, (size_t)ns * n, slot(tick + 1), s);
         mark();
         // Go on at once when the steps enqueued since the last known one are
@@ -802,9 +815,9 @@ struct Krylov {
       while(known < tick) wait();
       omx::kry_end_cycle(st, x, !one_cycle, batch, s);
       if(one_cycle) return;
-      ns = product(x, active, nb);
+      ns = product(x, active, nb, false);
       if(op) ns = -1;
-      count(nb);
+      count(nb, false);
       omx::kry_restart(st, b, x, gpart, ns, (size_t)std::max(0, ns) * n, false, batch, slot(tick + 1), s);
       mark();
       restart = tick;
@@ -1066,6 +1079,17 @@ bool backward_stable(omx_context *c, const cplx *A64, const cplx *rhs, const cpl
   return eta <= kBackwardErrorBound;
 }
 
+// Products of the assembled S (V) from half its blocks, from N = kSymN on (below,
+// the caches hold much of the matrix: N = 2142 20 us whole, 28 from its half; 10240
+// 244 and 193); without scratch otherwise.
+omx::SymArgs sym_args(omx_context *c, bool shf) {
+  omx::SymArgs a{c->P, c->nmax, c->Np, (size_t)c->Np, c->d_ov.as<cplx>(), shf ? omx::OV_TSH : omx::OV_T, nullptr};
+  if(c->kind == OMX_SOLVER_ACA_GMRES || !c->updated || c->P < 2 || c->N < kSymN) return a;
+  c->d_sym.ensure(sizeof(cplx) * omx::sym_scratch(c->P, c->nmax), &c->total);
+  a.scratch = c->d_sym.as<cplx>();
+  return a;
+}
+
 // Solves (S or V) x = rhs with the context's solver kind, on the system's
 // stream (a factorisation already enqueued by factor_enqueue is used).
 void solve_system(omx_context *c, bool shf, const cplx *rhs, cplx *x, int *iters, double *res) {
@@ -1087,6 +1111,8 @@ void solve_system(omx_context *c, bool shf, const cplx *rhs, cplx *x, int *iters
     *iters = gm.its[0];
     *res = gm.res[0];
   };
+  const omx::SymArgs sym = sym_args(c, shf);
+  if(!is_lu(c->kind) && !shf) gm.sym = sym;
   if(c->kind == OMX_SOLVER_ACA_GMRES) {  // Gmres_Zcomp on the compressed operator
     gm.op = [c, shf, st](const cplx *in, cplx *out) { aca_apply(c, shf, in, out, st); };
     gm.op_bytes = c->aca[shf ? 1 : 0].bytes;
@@ -1104,6 +1130,7 @@ void solve_system(omx_context *c, bool shf, const cplx *rhs, cplx *x, int *iters
     if(dirty) omx::demote(A32w, A64, (size_t)Np * lda, st);  // an earlier factorisation overwrote it
     dirty = false;
     inner.A32 = A32w;
+    inner.sym = sym;
     inner.one_cycle = true;
     gm.lazy = true;  // its preconditioner is a solve of its own
     gm.prec = [&inner, &gm, Np, st](const cplx *in, cplx *out, const int *) {
@@ -1140,9 +1167,11 @@ void solve_system(omx_context *c, bool shf, const cplx *rhs, cplx *x, int *iters
     omx::zero_ints(status.as<int>(), 4, st);
     HIPCHK(hipMemsetAsync(x, 0, sizeof(cplx) * Np, st));
     const int maxit = std::min(c->maxit, c->auto_budget > 0 ? c->auto_budget : auto_gmres64_steps(c->N));
+    gm.sym = sym;
     gm.x_zero = true;
     run(x, maxit);
     gm.x_zero = false;
+    gm.sym = omx::SymArgs{};
     if(*res <= 1e3 * c->tol || backward_stable(c, A64, rhs, x, *res, st)) return;
     ++c->fallbacks;
   }
@@ -1693,6 +1722,11 @@ void sweep_chunk(omx_context *c, int nb, const double *lam, const cplx *eps, con
     // system short of the target is left to the one-at-a-time path
     status_scan(bad, false);
     Krylov gm = sweep_krylov(c, nb, cS64);
+    if((double)N * N * nb >= (double)kSymN * kSymN) {  // as sym_args
+      c->d_sym.ensure(sizeof(cplx) * omx::sym_scratch(P, nmax) * nb, &c->total);
+      gm.sym = omx::SymArgs{P,  nmax, (int)Np, lda, w.ov.as<cplx>(), omx::OV_T, c->d_sym.as<cplx>(), nb,
+                            (size_t)Np * Np, lda, ovs};
+    }
     cplx *Sx = w.x.as<cplx>();
     gm.x_zero = true;
     HIPCHK(hipMemsetAsync(Sx, 0, sizeof(cplx) * lda * nb, st));
@@ -1892,7 +1926,7 @@ void omx_destroy(omx_context *c) {
                   &c->d_S32, &c->d_V64, &c->d_V32, &c->d_x, &c->d_xsh, &c->d_xint, &c->d_xintsh, &c->d_K,
                   &c->d_K1, &c->d_cross, &c->d_cg, &c->d_perm, &c->d_cand, &c->d_map,
                   &c->d_wlu, &c->d_status, &c->d_basis, &c->d_basisZ, &c->d_w1, &c->d_w2, &c->d_r,
-                  &c->d_nrm, &c->d_gpart, &c->d_perm2,
+                  &c->d_nrm, &c->d_gpart, &c->d_sym, &c->d_perm2,
                   &c->d_dinv, &c->d_dinv2, &c->d_F64, &c->d_F64sh, &c->d_abscoef, &c->d_abssh, &c->d_absbes,
                   &c->d_fpts, &c->d_fout, &c->d_fown, &c->d_fpart};
   for(DBuf *b : bufs) b->release(&c->total);
@@ -2946,7 +2980,7 @@ int omx_trim(omx_context *c) {
     auto &w = c->sw;
     DBuf *big[] = {&c->d_S64, &c->d_S32, &c->d_V64, &c->d_V32, &c->d_F64, &c->d_F64sh, &w.S64, &w.S32, &w.V64,
                    &w.V32, &w.F64, &w.F64sh, &w.basis, &w.basisZ, &w.gpart, &c->d_basis, &c->d_basisZ,
-                   &c->d_gpart};
+                   &c->d_gpart,  &c->d_sym};
     for(DBuf *b : big) b->release(&c->total);
     aca_release(c);
     c->ws_in.release(&c->total);

@@ -266,6 +266,24 @@ int gemv_partial(const float2 *A, size_t lda, int N, const cplx *x, cplx *part, 
 constexpr int kGemvSplit = 32, kGemvSplitMax = 96;  // column parts: most of a batch's product, of a single one's
 inline size_t gemv_part_rows(int nb) { return std::max(kGemvSplitMax, kGemvSplit * nb); }  // vectors of partial sums
 
+// y = S x for nb assembled scattering matrices from half their blocks: S_ji[p][q]
+// is S_ij[p][q] times (T_j / T_i)[p] and the parity sign of (p, q), so a pair's two
+// products read one block, for each row p the one of the larger |T[p]|.
+// Scratch: sym_scratch(P, nmax) complex values per system.
+struct SymArgs {
+  int P, nmax, Np;
+  size_t lda;
+  const cplx *ov;  // the rows' factors T, of kind tkind (OV_T: S, OV_TSH: V)
+  int tkind;
+  cplx *scratch;
+  int nb = 1;
+  size_t sA = 0, sv = 0, zov = 0;  // matrices, vectors and ov of the systems apart
+  const int *flag = nullptr;       // systems whose flag (KF_COUNT ints apart) is 0 are left out
+};
+size_t sym_scratch(int P, int nmax);
+void sym_product(const SymArgs &a, const cplx *A, const cplx *x, cplx *y, hipStream_t st);
+void sym_product(const SymArgs &a, const float2 *A, const cplx *x, cplx *y, hipStream_t st);
+
 // GMRES with its small algebra on the device (omx_krylov.hip), nb systems in
 // lockstep: the state of each, and the vectors they share.
 enum { KF_LIVE = 0, KF_ACTIVE, KF_J, KF_ITS, KF_STALL, KF_TINY, KF_COUNT = 8 };  // flags, ints

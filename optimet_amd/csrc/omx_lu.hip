@@ -2040,4 +2040,169 @@ int gemv_partial(const float2 *A, size_t lda, int N, const cplx *x, cplx *part, 
   return ns;
 }
 
+// ------------------------------------------------------------------ products of half the blocks
+// Objects j of a workgroup: one while the pairs are few, eight from 64 objects on
+// (their sum over j then leaves the workgroup once).
+inline int sym_chunk(int P) { return P > 64 ? 8 : 1; }
+size_t sym_scratch(int P, int nmax) {
+  const size_t n = 2 * (size_t)nmax * (nmax + 2), nc = (P + sym_chunk(P) - 1) / sym_chunk(P);
+  return (nc * P + (size_t)P * (P - 1) / 2) * n;
+}
+__device__ inline cplx sym_T(const SymArgs &a, const cplx *ov, int j, int pol, int n) {
+  return ov[(((size_t)a.tkind * a.P + j) * 2 + pol) * (a.nmax + 1) + n];
+}
+// Row p's degree and polarisation, and its parity factor: (-1)^n, times -1 for TM.
+__device__ inline double sym_sign(int p, int nf, int &n, int &pol) {
+  int m;
+  pol = p >= nf;
+  unflat(p % nf, n, m);
+  return ((n & 1) != 0) != (pol != 0) ? -1.0 : 1.0;
+}
+__device__ inline cplx sym_widen(cplx v) { return v; }
+__device__ inline cplx sym_widen(float2 v) { return cplx{(double)v.x, (double)v.y}; }
+
+// Block (chunk c of objects j, object i < j): thread t is row p = t % n, the
+// columns u, u + G, .. of u = t / n.  The sums over j of y_i go to part[c][i], each
+// y_j's to z[pair].
+//
+// Bound: HBM, at half the bytes of the plain product, and the barriers between
+// objects.  N = 49152: FP32 2.78 -> 2.29 ms, FP64 5.45 -> 4.06; N = 10240, FP64: 244 ->
+// 193 us; N = 2142: 20 -> 28, so single systems take it from kSymN on.
+template <typename T>
+__global__ __launch_bounds__(512) void sym_pairs(SymArgs a, const T *__restrict__ A, const cplx *__restrict__ x, int CH,
+                                                int G) {
+  const int c = blockIdx.x, i = blockIdx.y, zs = blockIdx.z, P = a.P, nf = a.nmax * (a.nmax + 2), n = 2 * nf;
+  if(a.flag && !a.flag[(size_t)zs * KF_COUNT]) return;
+  const int j1 = min(P, (c + 1) * CH);
+  if(j1 <= i + 1) return;  // no object of the chunk past i
+  A += zs * a.sA;
+  x += zs * a.sv;
+  const cplx *ov = a.ov + zs * a.zov;
+  const int nc = (P + CH - 1) / CH;
+  cplx *part = a.scratch + zs * (((size_t)nc * P + (size_t)P * (P - 1) / 2) * n), *z = part + (size_t)nc * P * n;
+  extern __shared__ cplx sh[];
+  // the objects' vectors, with and without the signs; the column groups' sums
+  cplx *xi = sh, *si = sh + n, *xj = sh + 2 * n, *sj = sh + 3 * n, *red = sh + 4 * n;
+  const int t = threadIdx.x, u = t / n, p = t % n;
+  const bool in = u < G;
+  auto load = [&](int o, cplx *v, cplx *sv) {
+    for(int q = t; q < n; q += blockDim.x) {
+      int d, pl;
+      const cplx e = x[(size_t)o * n + q];
+      v[q] = e;
+      sv[q] = sym_sign(q, nf, d, pl) * e;
+    }
+  };
+  load(i, xi, si);
+  int deg, pol;
+  const double sp = sym_sign(p, nf, deg, pol);
+  const cplx Ti = sym_T(a, ov, i, pol, deg);
+  cplx acc = mk(0.0);
+  // Columns in eights, the next eight (of the next object after the last) on their
+  // way while these are summed: the barriers between objects then wait for no load
+  constexpr int E = 8;
+  const int j0 = max(i + 1, c * CH), cnt = n / G, steps = (cnt + E - 1) / E;
+  cplx Tn = sym_T(a, ov, j0, pol, deg);
+  T cur[E], nxt[E];
+  // the block whose row is the larger: S_ij times x_j, and with the signs x_i for
+  // y_j; or S_ji times x_i, and with the signs x_j for y_i
+  auto base = [&](int j, bool own) {
+    return A + (size_t)((own ? j : i) * n + u) * a.lda + (size_t)(own ? i : j) * n + p;
+  };
+  auto fetch = [&](const T *e, int b, T(&d)[E]) {
+#pragma unroll
+    for(int k = 0; k < E; ++k) d[k] = ld_stream(e + (size_t)(G * min(E * b + k, cnt - 1)) * a.lda);
+  };
+  bool own = norm2(Ti) >= norm2(Tn);
+  const T *e = base(j0, own);
+  if(in) fetch(e, 0, cur);
+  for(int j = j0; j < j1; ++j) {
+    const cplx Tj = Tn;
+    if(j + 1 < j1) Tn = sym_T(a, ov, j + 1, pol, deg);
+    __syncthreads();
+    load(j, xj, sj);
+    __syncthreads();
+    cplx f = mk(0.0), h = mk(0.0);
+    const bool ownj = own;
+    if(in) {
+      const cplx *v = ownj ? xj : xi, *w = ownj ? si : sj;
+      for(int b = 0; b < steps; ++b) {
+        if(b + 1 < steps) {
+          fetch(e, b + 1, nxt);
+        } else if(j + 1 < j1) {
+          own = norm2(Ti) >= norm2(Tn);
+          e = base(j + 1, own);
+          fetch(e, 0, nxt);
+        }
+#pragma unroll
+        for(int k = 0; k < E; ++k) {
+          const int q = u + G * (E * b + k);
+          if(E * b + k < cnt) {
+            const cplx m = sym_widen(cur[k]);
+            f = f + m * v[q];
+            h = h + m * w[q];
+          }
+        }
+#pragma unroll
+        for(int k = 0; k < E; ++k) cur[k] = nxt[k];
+      }
+      const cplx big = ownj ? Ti : Tj, small = ownj ? Tj : Ti;
+      h = sp * ((norm2(big) > 0.0 ? small / big : mk(0.0)) * h);
+    }
+    const cplx yi = ownj ? f : h;
+    cplx yj = ownj ? h : f;
+    acc = acc + yi;
+    if(G > 1) {
+      if(in && u > 0) red[(u - 1) * n + p] = yj;
+      __syncthreads();
+      if(u == 0)
+        for(int g = 1; g < G; ++g) yj = yj + red[(g - 1) * n + p];
+    }
+    if(u == 0) z[((size_t)j * (j - 1) / 2 + i) * n + p] = yj;
+  }
+  if(G > 1) {
+    __syncthreads();
+    if(in && u > 0) red[(u - 1) * n + p] = acc;
+    __syncthreads();
+    if(u == 0)
+      for(int g = 1; g < G; ++g) acc = acc + red[(g - 1) * n + p];
+  }
+  if(u == 0) part[((size_t)c * P + i) * n + p] = acc;
+}
+// y of object i: x (the unit blocks), the parts of its row and the pairs (k, i), k < i.
+__global__ __launch_bounds__(256) void sym_sum(SymArgs a, const cplx *__restrict__ x, cplx *y, int CH) {
+  const int r = blockIdx.x * 64 + (threadIdx.x & 63), w = threadIdx.x >> 6, zs = blockIdx.z, P = a.P;
+  if(a.flag && !a.flag[(size_t)zs * KF_COUNT]) return;
+  const int n = 2 * a.nmax * (a.nmax + 2), nc = (P + CH - 1) / CH;
+  const cplx *part = a.scratch + zs * (((size_t)nc * P + (size_t)P * (P - 1) / 2) * n), *z = part + (size_t)nc * P * n;
+  __shared__ cplx red[3][64];
+  cplx s = mk(0.0);
+  if(r < P * n) {  // the waves share the terms
+    const int i = r / n, p = r % n, c0 = (i + 1) / CH;
+    if(i + 1 < P)
+#pragma unroll 4
+      for(int c = c0 + w; c < nc; c += 4) s = s + part[((size_t)c * P + i) * n + p];
+#pragma unroll 4
+    for(int k = w; k < i; k += 4) s = s + z[((size_t)i * (i - 1) / 2 + k) * n + p];
+  }
+  if(w > 0) red[w - 1][threadIdx.x & 63] = s;
+  __syncthreads();
+  if(w > 0 || r >= a.Np) return;
+  const int l = threadIdx.x & 63;
+  y[zs * a.sv + r] = x[zs * a.sv + r] + ((s + red[0][l]) + (red[1][l] + red[2][l]));
+}
+template <typename T> void sym_run(const SymArgs &a, const T *A, const cplx *x, cplx *y, hipStream_t st) {
+  const int n = 2 * a.nmax * (a.nmax + 2), CH = sym_chunk(a.P), nc = (a.P + CH - 1) / CH;
+  // column groups (of one size) that fill the waves best, 512 threads at most
+  int G = 1;
+  auto fill = [&](int g) { return (double)(n * g) / ((n * g + 63) / 64 * 64); };
+  for(int g = 2; n * g <= 512; ++g)
+    if(n % g == 0 && fill(g) > fill(G) + 0.03) G = g;
+  hipLaunchKernelGGL((sym_pairs<T>), dim3(nc, a.P - 1, a.nb), dim3((n * G + 63) / 64 * 64),
+                     sizeof(cplx) * (4 + G - 1) * n, st, a, A, x, CH, G);
+  hipLaunchKernelGGL(sym_sum, dim3((a.Np + 63) / 64, 1, a.nb), dim3(256), 0, st, a, x, y, CH);
+}
+void sym_product(const SymArgs &a, const cplx *A, const cplx *x, cplx *y, hipStream_t st) { sym_run(a, A, x, y, st); }
+void sym_product(const SymArgs &a, const float2 *A, const cplx *x, cplx *y, hipStream_t st) { sym_run(a, A, x, y, st); }
+
 }  // namespace omx
