@@ -1081,7 +1081,7 @@ bool backward_stable(omx_context *c, const cplx *A64, const cplx *rhs, const cpl
 
 // Products of the assembled S (V) from half its blocks, from N = kSymN on (below,
 // the caches hold much of the matrix: N = 2142 20 us whole, 28 from its half; 10240
-// 244 and 193); without scratch otherwise.
+// 244 and 181); without scratch otherwise.
 omx::SymArgs sym_args(omx_context *c, bool shf) {
   omx::SymArgs a{c->P, c->nmax, c->Np, (size_t)c->Np, c->d_ov.as<cplx>(), shf ? omx::OV_TSH : omx::OV_T, nullptr};
   if(c->kind == OMX_SOLVER_ACA_GMRES || !c->updated || c->P < 2 || c->N < kSymN) return a;

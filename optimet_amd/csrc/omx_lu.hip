@@ -2066,8 +2066,8 @@ __device__ inline cplx sym_widen(float2 v) { return cplx{(double)v.x, (double)v.
 // y_j's to z[pair].
 //
 // Bound: HBM, at half the bytes of the plain product, and the barriers between
-// objects.  N = 49152: FP32 2.78 -> 2.29 ms, FP64 5.45 -> 4.06; N = 10240, FP64: 244 ->
-// 193 us; N = 2142: 20 -> 28, so single systems take it from kSymN on.
+// objects.  N = 49152: FP32 2.78 -> 2.24 ms, FP64 5.45 -> 3.70; N = 10240, FP64: 244 ->
+// 181 us; N = 2142: 20 -> 28, so single systems take it from kSymN on.
 template <typename T>
 __global__ __launch_bounds__(512) void sym_pairs(SymArgs a, const T *__restrict__ A, const cplx *__restrict__ x, int CH,
                                                 int G) {
@@ -2098,9 +2098,11 @@ __global__ __launch_bounds__(512) void sym_pairs(SymArgs a, const T *__restrict_
   const double sp = sym_sign(p, nf, deg, pol);
   const cplx Ti = sym_T(a, ov, i, pol, deg);
   cplx acc = mk(0.0);
-  // Columns in eights, the next eight (of the next object after the last) on their
-  // way while these are summed: the barriers between objects then wait for no load
-  constexpr int E = 8;
+  // Columns by E, the next E (of the next object after the last) on their way while
+  // these are summed: the barriers between objects then wait for no load.  E: four
+  // waves a SIMD in either type (FP64 with 4 / 6 / 8: N = 49152 3.67 / 3.69 / 4.03
+  // ms, 10240 176 / 205 / 193 us; FP32: 2.31 / 2.20 / 2.26 ms)
+  constexpr int E = sizeof(T) == 8 ? 6 : 4;
   const int j0 = max(i + 1, c * CH), cnt = n / G, steps = (cnt + E - 1) / E;
   cplx Tn = sym_T(a, ov, j0, pol, deg);
   T cur[E], nxt[E];
