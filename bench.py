@@ -84,7 +84,7 @@ def stage_rooflines(c, st, mixed_copy):
         out["assembly"] = {"bound": "hbm", "kernel": "pair_kernel (S and V) with objects, incident and origin kernels",
                            "achieved": gbs, "peak": HBM_GBS, "unit": "GB/s", "frac": gbs / HBM_GBS,
                            "bytes": store, "ms": st["t_assemble_ms"]}
-    mv = matvec_roofline(st, "gemv_part_kernel (FP64 matvec of GMRES and of the refinement)")
+    mv = matvec_roofline(st, "sym_pairs (FP64 GMRES steps, half of S) and gemv_part_kernel (residuals, refinement)")
     if mv is not None:
         out["refinement_matvec"] = mv
     return out
@@ -302,8 +302,8 @@ def config4_main(args):
                    "solver": "auto", "picked": picked,
                    "rule": "N >= 16384: the mixed Krylov within a budget of the mixed LU's cost (0.0143 N FP32 "
                            "products), else or when it does not converge there, the mixed LU + GMRES-IR"},
-        "roofline": matvec_roofline(au["stats"], "gemv_part_kernel<float2> (inner products on the FP32 copy) and "
-                                    "gemv_part_kernel<cplx> (outer FP64 products)")
+        "roofline": matvec_roofline(au["stats"], "sym_pairs<float2> (inner products, half of the FP32 copy), sym_pairs<cplx> and "
+                                    "gemv_part_kernel<cplx> (outer FP64 products, residuals)")
         if picked == "gmres32ir" else res["lu32ir"].get("roofline"),
         "speedup_vs_fp64": total["lu64"] / total["auto"],
         "speedup_mixed_lu_vs_fp64_lu": total["lu64"] / total["lu32ir"],
