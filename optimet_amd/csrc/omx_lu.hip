@@ -2058,6 +2058,9 @@ __device__ inline double sym_sign(int p, int nf, int &n, int &pol) {
   unflat(p % nf, n, m);
   return ((n & 1) != 0) != (pol != 0) ? -1.0 : 1.0;
 }
+// The size by which a row's factors are compared: |T| falls like x^(2n+1) of the
+// size parameter x, and its square underflows from degree 8 on at x = 2e-10
+__device__ inline double sym_mag(cplx v) { return fmax(fabs(v.x), fabs(v.y)); }
 __device__ inline cplx sym_widen(cplx v) { return v; }
 __device__ inline cplx sym_widen(float2 v) { return cplx{(double)v.x, (double)v.y}; }
 
@@ -2115,7 +2118,7 @@ __global__ __launch_bounds__(512) void sym_pairs(SymArgs a, const T *__restrict_
 #pragma unroll
     for(int k = 0; k < E; ++k) d[k] = ld_stream(e + (size_t)(G * min(E * b + k, cnt - 1)) * a.lda);
   };
-  bool own = norm2(Ti) >= norm2(Tn);
+  bool own = sym_mag(Ti) >= sym_mag(Tn);
   const T *e = base(j0, own);
   if(in) fetch(e, 0, cur);
   for(int j = j0; j < j1; ++j) {
@@ -2132,7 +2135,7 @@ __global__ __launch_bounds__(512) void sym_pairs(SymArgs a, const T *__restrict_
         if(b + 1 < steps) {
           fetch(e, b + 1, nxt);
         } else if(j + 1 < j1) {
-          own = norm2(Ti) >= norm2(Tn);
+          own = sym_mag(Ti) >= sym_mag(Tn);
           e = base(j + 1, own);
           fetch(e, 0, nxt);
         }
@@ -2149,7 +2152,7 @@ __global__ __launch_bounds__(512) void sym_pairs(SymArgs a, const T *__restrict_
         for(int k = 0; k < E; ++k) cur[k] = nxt[k];
       }
       const cplx big = ownj ? Ti : Tj, small = ownj ? Tj : Ti;
-      h = sp * ((norm2(big) > 0.0 ? small / big : mk(0.0)) * h);
+      h = sp * ((sym_mag(big) > 0.0 ? small / big : mk(0.0)) * h);
     }
     const cplx yi = ownj ? f : h;
     cplx yj = ownj ? h : f;

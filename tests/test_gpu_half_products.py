@@ -44,3 +44,35 @@ def test_matches_the_factorisation(P, nmax, kind):
     st = s.stats()
     assert st["residual"] <= 1e-12 and 0 < st["iterations"] < 60
     assert rel(got, want) < 1e-10
+
+
+def test_tiny_size_parameters():
+    """Size parameters of 2e-10, where the factors of degree 8 are about 1e-179 and
+    their squares 0: every degree's coefficients, against the fixed point of x = Q
+    - (S - 1) x on the host (the spheres couple weakly: a hundredth a step).  The
+    high degrees come from their neighbours' fields alone, so a product that loses
+    a row's blocks is wrong by its own size there; 1e-6 is far from that and from
+    the rounding of a few Krylov steps."""
+    from optimet_amd import solver
+    P, nmax = 52, 8
+    rng = np.random.default_rng(0)
+    xyz = 400 * NM * np.array([(i, j, k) for i in range(4) for j in range(4) for k in range(4)][:P], float)
+    eps = np.full(P, 2.25 + 0j)
+    c = Cluster(xyz=xyz + 60 * NM * rng.random((P, 3)), radius=60 * NM * (0.8 + 0.2 * rng.random(P)), eps_r=eps,
+                eps_r_sh=eps, nmax=nmax, wavelength=2 * np.pi * 60 * NM / 2e-10, sh=False)
+    assert c.N >= 8192
+    s = solver.Solver(c, kind="gmres64", tol=1e-14)
+    s.update()
+    S, Q = s.matrix(), s.vector("Q")
+    want = Q
+    for _ in range(12):
+        want = Q - (S @ want - want)
+    got = s.solve()["x_sca"]
+    p = np.arange(2 * c.nf)
+    deg = np.tile(np.sqrt(p % c.nf + 1.0).astype(int), P)
+    pol = np.tile(p // c.nf, P)
+    for n in range(1, nmax + 1):
+        for q in (0, 1):
+            k = (deg == n) & (pol == q)
+            d = got[k] / np.abs(want[k]).max() - want[k] / np.abs(want[k]).max()
+            assert np.abs(d).max() < 1e-6, (n, q, np.abs(d).max())
