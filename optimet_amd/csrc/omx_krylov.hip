@@ -311,7 +311,8 @@ __global__ __launch_bounds__(kRows) void kry_update(KryState s, cplx *x) {
 }
 
 // A correction below the FP64 resolution of x ends the refinement: a batch's
-// system at once, a single one after its residual has been formed.
+// system at once (its cycle may have ended with steps to go: neither flag stays),
+// a single one after its residual has been formed.
 __global__ __launch_bounds__(kRows) void kry_tiny(KryState s, int nblk, int nb, int at_once) {
   const int z = blockIdx.x;
   const Sys q(s, z);
@@ -321,7 +322,7 @@ __global__ __launch_bounds__(kRows) void kry_tiny(KryState s, int nblk, int nb, 
   const double x = sqrt(sum_norms(s.pnrm + ((size_t)nb + z) * nblk, nblk, lds));
   if(threadIdx.x == 0 && d <= 1e-16 * x) {
     q.fl[KF_TINY] = 1;
-    if(at_once) q.fl[KF_ACTIVE] = 0;
+    if(at_once) q.fl[KF_ACTIVE] = q.fl[KF_LIVE] = 0;
   }
 }
 

@@ -4,7 +4,7 @@ step, of a few and longer than the solve; budgets that end inside a cycle."""
 import numpy as np
 import pytest
 
-from optimet_amd.problem import Cluster, random_cluster
+from optimet_amd.problem import Cluster, drude_cluster, random_cluster
 
 pytestmark = pytest.mark.gpu
 
@@ -55,3 +55,25 @@ def test_budget(maxit):
         except solver.OmxError as e:
             assert "converge" in str(e)
         assert s.stats()["iterations"] <= maxit
+
+
+def test_a_batch_counts_its_systems_steps_alone():
+    """Systems that leave a batch at the FP64 floor, by a correction too small to
+    change them, take no further steps while the others go on: each one's count is
+    that of the same system alone, to a few cycles of two steps that rounding at
+    the floor shifts (8; those that went on took the slowest one's 56 instead of
+    about 30)."""
+    from optimet_amd import solver
+    c = drude_cluster(14, 8, 700 * NM, 40, 80, 1000, 10, seed=91)
+    lams = np.linspace(450, 850, 8) * NM
+
+    def its(l):
+        s = solver.Solver(c, kind="auto", tol=1e-18, restart=2, maxit=2000)
+        s.ctx.set_autotune(False)
+        s.ctx.set_auto_budget(1000)
+        out = s.sweep(l, batch=len(l), outputs=("x_sca",))["iterations"][:, 0]
+        s.ctx.close()
+        return out
+
+    together, alone = its(lams), np.concatenate([its([l]) for l in lams])
+    assert (np.abs(together - alone) <= 8).all(), (together, alone)
