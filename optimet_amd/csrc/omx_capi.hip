@@ -216,6 +216,7 @@ struct omx_context {
   char *out_pin = nullptr;
   size_t out_pin_bytes = 0;
   hipEvent_t geo_ev = nullptr;
+  hipEvent_t mv_ev[2] = {nullptr, nullptr};  // around a product, with profiling on
   // omx_update's times (start, objects done, assembly done) and its joins
   bool upd_timed = false;
   hipEvent_t uev[3] = {nullptr, nullptr, nullptr}, ujoin[2] = {nullptr, nullptr};
@@ -696,7 +697,7 @@ struct Krylov {
   // Enqueues A x into gpart (returns the column parts) or w (returns 0).
   int product(const cplx *x, const int *flag, int live, bool step) {
     const bool prof = c->profile;
-    if(prof) HIPCHK(hipEventRecord(c->ev[6], s));
+    if(prof) HIPCHK(hipEventRecord(c->mv_ev[0], s));
     int ns = 0;
     if(op)
       op(x, w);
@@ -713,10 +714,10 @@ struct Krylov {
     else
       ns = omx::gemv_partial(A, (size_t)c->Np, n, x, gpart, s, nb, sA, (size_t)n, flag, std::max(1, live));
     if(prof) {
-      HIPCHK(hipEventRecord(c->ev[7], s));
-      HIPCHK(hipEventSynchronize(c->ev[7]));
+      HIPCHK(hipEventRecord(c->mv_ev[1], s));
+      HIPCHK(hipEventSynchronize(c->mv_ev[1]));
       float ms = 0;
-      HIPCHK(hipEventElapsedTime(&ms, c->ev[6], c->ev[7]));
+      HIPCHK(hipEventElapsedTime(&ms, c->mv_ev[0], c->mv_ev[1]));
       c->mv_ms += ms;
     }
     return ns;
@@ -1901,6 +1902,7 @@ int omx_create(omx_context **out, int device) {
       for(auto &e : c->xev) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
       for(auto &e : c->ev) HIPCHK(hipEventCreate(&e));
       for(auto &e : c->uev) HIPCHK(hipEventCreate(&e));
+      for(auto &e : c->mv_ev) HIPCHK(hipEventCreate(&e));
       for(hipEvent_t *e : {&c->geo_ev, &c->ujoin[0], &c->ujoin[1]})
         HIPCHK(hipEventCreateWithFlags(e, hipEventDisableTiming));
       omx::upload_factorials();
@@ -1953,7 +1955,7 @@ void omx_destroy(omx_context *c) {
     if(e) (void)hipEventDestroy(e);
   for(auto e : c->xev)
     if(e) (void)hipEventDestroy(e);
-  for(hipEvent_t e : {c->geo_ev, c->uev[0], c->uev[1], c->uev[2], c->ujoin[0], c->ujoin[1]})
+  for(hipEvent_t e : {c->mv_ev[0], c->mv_ev[1], c->geo_ev, c->uev[0], c->uev[1], c->uev[2], c->ujoin[0], c->ujoin[1]})
     if(e) (void)hipEventDestroy(e);
   for(auto e : c->pev2)
     if(e) (void)hipEventDestroy(e);

@@ -77,3 +77,22 @@ def test_a_batch_counts_its_systems_steps_alone():
 
     together, alone = its(lams), np.concatenate([its([l]) for l in lams])
     assert (np.abs(together - alone) <= 8).all(), (together, alone)
+
+
+def test_a_profiled_sweep_times_itself():
+    """The sweep's time holds its products, and is not shorter than half of the same
+    sweep's without the products' events."""
+    from optimet_amd import solver
+    c = drude_cluster(6, 5, 700 * NM, 40, 80, 700, 10, seed=3)
+    s = solver.Solver(c, kind="lu32ir")
+    s.ctx.set_profile(True)
+    s.sweep(np.linspace(450, 850, 8) * NM, batch=4)
+    st = s.stats()
+    s.ctx.close()
+    assert st["matvec_calls"] > 4 and st["t_matvec_ms"] > 0
+    wall = st["t_solve_ms"]
+    s = solver.Solver(c, kind="lu32ir")
+    s.sweep(np.linspace(450, 850, 8) * NM, batch=4)  # the same sweep without the events
+    plain = s.stats()["t_solve_ms"]
+    s.ctx.close()
+    assert wall > st["t_matvec_ms"] and wall > 0.5 * plain
