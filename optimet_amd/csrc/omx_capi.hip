@@ -10,6 +10,7 @@
 #include <functional>
 #include <cstdlib>
 #include <cstring>
+#include <exception>
 #include <map>
 #include <mutex>
 #include <thread>
@@ -318,6 +319,19 @@ template <typename F> int guard(F &&f) {
     return OMX_ERR_ARG;
   }
 }
+
+// A call that fails leaves none of its work in flight.  The status words of a
+// factorisation are looked at with the first steps of its refinement enqueued, and V's
+// factorisation runs on the second stream while S's solve may fail; the next call
+// starts on the first stream, in the same workspaces.
+struct DrainOnError {
+  omx_context *c;
+  int before = std::uncaught_exceptions();
+  ~DrainOnError() {
+    if(std::uncaught_exceptions() <= before) return;
+    for(hipStream_t s : {c->st, c->aux, c->st2, c->aux2}) (void)hipStreamSynchronize(s);
+  }
+};
 
 cplx C(const double *p, int i) { return omx::mk(p[2 * i], p[2 * i + 1]); }
 
@@ -2261,6 +2275,7 @@ int omx_solve(omx_context *c, double *x_sca, double *x_int, double *x_sca_sh, do
   return guard([&] {
     if(!c || !c->updated) throw OmxError(OMX_ERR_STATE, "omx_update must precede omx_solve");
     HIPCHK(hipSetDevice(c->device));
+    DrainOnError drain{c};
     const int N = c->N, P = c->P, nmax = c->nmax;
     double tf = 0, ts = 0, tsh = 0;
     HIPCHK(hipEventRecord(c->ev[0], c->st));
@@ -2413,6 +2428,7 @@ int omx_solve_group(omx_context *L, int n, omx_context *const *mem) {
         if(mem[j] == m) throw OmxError(OMX_ERR_ARG, "omx_solve_group: a member appears twice");
     }
     HIPCHK(hipSetDevice(L->device));
+    DrainOnError drain{L};
     const bool f64 = mem[0]->kind == OMX_SOLVER_LU64, sh = mem[0]->sh != 0;
     int Np = 0;
     for(int i = 0; i < n; ++i) Np = std::max(Np, mem[i]->Np);
@@ -2777,6 +2793,7 @@ int omx_dense_solve(omx_context *c, int N, const double *A, const double *b, dou
     if(!c || N < 1 || !A || !b || !x || (kind != OMX_SOLVER_LU64 && kind != OMX_SOLVER_LU32_IR))
       throw OmxError(OMX_ERR_ARG, "invalid dense solve");
     HIPCHK(hipSetDevice(c->device));
+    DrainOnError drain{c};
     // reuse the context machinery with a synthetic "geometry" of the right
     // size; the geometry's sizes, solver kind and SH flag come back on every
     // exit (a failed solve must not leave the dense sizes behind: the next
@@ -2848,6 +2865,7 @@ int omx_solve_sweep(omx_context *c, int nl, const double *lambdas, const double 
     for(int l = 0; l < nl; ++l)
       if(!(lambdas[l] > 0.0)) throw OmxError(OMX_ERR_ARG, "non-positive wavelength");
     HIPCHK(hipSetDevice(c->device));
+    DrainOnError drain{c};
     alloc_all(c);
     c->d_status.ensure(64, &c->total);
     const int P = c->P, N = c->N;

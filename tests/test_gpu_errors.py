@@ -70,3 +70,28 @@ def test_loose_tolerance_does_not_accept_fp32_quality():
         assert ctx.stats()["pivot_fallbacks"] == before + 1
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("kind", ["lu32ir", "lu64", "auto"])
+def test_solve_after_a_failed_one(kind):
+    """A solve that fails in S, with V's factorisation on its way on the second
+    stream, leaves nothing behind that runs into the next assembly and solve: the
+    same coefficients, bit for bit, as on a context that never failed."""
+    from optimet_amd import solver
+    c = drude_cluster(20, 7, 700e-9, 40, 80, 1000, 10, seed=8, sh=True)
+    want = solver.Solver(c, kind=kind)
+    want.update()
+    ref = want.solve()
+    s = solver.Solver(c, kind=kind, tol=1e-30, maxit=1)
+    s.update()
+    try:
+        s.solve()
+    except solver.OmxError as e:
+        assert e.code == -6
+    s.ctx.set_solver(kind)
+    s.update()
+    got = s.solve()
+    for k in ref:
+        assert np.array_equal(got[k], ref[k]), k
+    want.ctx.close()
+    s.ctx.close()
