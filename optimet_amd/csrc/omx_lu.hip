@@ -344,11 +344,6 @@ template <typename T> __device__ __forceinline__ void invert_block(CxOf<T> *F, c
   }
 }
 
-// The unsigned word that orders non-negative values: all of a float, the
-// upper half of a double (11 bits of exponent, 20 of mantissa).
-__device__ inline unsigned order_key(float m) { return __float_as_uint(m); }
-__device__ inline unsigned order_key(double m) { return (unsigned)__double2hiint(m); }
-
 // Tournament pivoting (TSLU, Grigori, Demmel and Xiang 2011): the panel's pivot
 // rows are chosen by a tree of local partial-pivoting LUs of up to 64 RPL rows,
 // each in one workgroup of 8 waves: the leaves nominate 64 rows of their chunk,
@@ -358,9 +353,9 @@ __device__ inline unsigned order_key(double m) { return (unsigned)__double2hiint
 // (mdst <- msrc, at most 128 entries) and the permutation.
 //
 // As diag_lu, which stands below: a wave holds 8 columns, here of RPL rows per
-// lane; the owner of a column takes the largest max(|re|, |im|) of the rows left
-// (to 20 bits of mantissa, the first row on ties), and the waves of later columns
-// follow by the published steps.  A pivot row sits in one of RPL register slots:
+// lane; the owner of a column takes the largest |.|^2 of the rows left, in FP64 (the
+// upper words are compared first, the lower ones when lanes tie; the first row on
+// ties), and the waves of later columns follow by the published steps.  A pivot row sits in one of RPL register slots:
 // the step branches on the slot, uniform in the wave.  The multipliers of four
 // panels of 8 columns are kept; the owner of a fifth waits until the waves behind
 // it have read the first.
@@ -454,25 +449,36 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
 #pragma unroll
   for(int jj = 0; jj < 8; ++jj) {
     const int c = 8 * q + jj;
-    unsigned key[RPL], kx = 0;
-    C best = v[0][jj];  // this lane's candidate: its largest row left, the first on ties
+    // this lane's candidate: its largest row left, the first on ties (NaN counts as
+    // large: every step finds a row of its own)
+    C best = v[0][jj];
+    double kx = -1.0;
+    int slot_of = 0;
     bool have = false;
 #pragma unroll
     for(int s = 0; s < RPL; ++s) {
-      const auto ax = fabs(v[s][jj].x), ay = fabs(v[s][jj].y);  // -0 orders as 0
-      key[s] = used[s] ? 0u : order_key(ax > ay ? ax : ay);
-      best = csel(!used[s] && (!have || key[s] > kx), v[s][jj], best);
-      have = have || !used[s];
-      kx = max(kx, key[s]);
+      const double m = mag2(v[s][jj]);
+      const bool take = !used[s] && !(m <= kx);
+      best = csel(take, v[s][jj], best);
+      kx = take ? m : kx;
+      slot_of = take ? s : slot_of;
+      have = have || take;
     }
     // every lane the reciprocal of its own candidate while the maximum is found
-    const bool sing = !nonzero(best);
+    const bool sing = !(kx > 0.0);
     const C ir = csel(sing, zero, crecip(best));
-    const unsigned M = wave_max_u32(kx);
+    const unsigned hi = have ? (unsigned)__double2hiint(kx) : 0u;
+    const unsigned M = wave_max_u32(hi);
+    unsigned long long tied = __ballot(have && hi == M);
+    if(tied & (tied - 1)) {  // the lower words among the lanes that tie in the upper one
+      const unsigned lo = have && hi == M ? (unsigned)__double2loint(kx) : 0u;
+      const unsigned L = wave_max_u32(lo);
+      tied = __ballot(have && hi == M && lo == L);
+    }
     int sl = 0, b = 0;
 #pragma unroll
     for(int s = RPL - 1; s >= 0; --s) {
-      const unsigned long long m = __ballot(!used[s] && key[s] == M);
+      const unsigned long long m = tied & __ballot(slot_of == s);
       if(m) {
         sl = s;
         b = __ffsll((long long)m) - 1;

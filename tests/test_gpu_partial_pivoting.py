@@ -85,3 +85,31 @@ def test_negative_zeros_do_not_order_first(ctx, kind):
     finally:
         ctx.set_pivoting("block")
     assert rel(x, np.linalg.solve(A, b)) < 1e-11
+
+
+@pytest.mark.parametrize("N", [64, 130, 192])
+def test_pivots_are_the_largest_of_their_columns(ctx, N):
+    """Up to 192 rows the panel's rows meet in one workgroup, so every pivot is the
+    column's largest in modulus: no multiplier above 1, to the rounding of the
+    panel's products with the inverse of its triangle (u times a condition number
+    of 1e4: 1e-11).  The moduli of the first column differ by 1e-8 at most."""
+    from tests.test_zz_no_alloc import _Dev, _hip
+    hip = _hip()
+    rng = np.random.default_rng(N)
+    Np = -(-N // 64) * 64
+    A = np.exp(2j * np.pi * rng.random((N, N))) * (1 + 1e-8 * rng.random((N, N)))
+    b = rng.standard_normal(N) + 1j * rng.standard_normal(N)
+    cols = np.zeros((Np, Np), complex)  # row c is column c of A
+    cols[:N, :N] = A.T
+    dA, db, dx = _Dev(hip, cols.nbytes), _Dev(hip, b.nbytes), _Dev(hip, b.nbytes)
+    try:
+        dA.put(cols)
+        db.put(b)
+        ctx.dense_solve_noalloc(N, dA.p.value, Np, db.p.value, dx.p.value)
+        L = np.tril(dA.get((Np, Np), np.complex128).T, -1)
+        x = dx.get(N, np.complex128)
+    finally:
+        for d in (dA, db, dx):
+            d.free()
+    assert np.abs(L).max() <= 1 + 1e-11, np.abs(L).max() - 1
+    assert rel(x, np.linalg.solve(A, b)) < 1e-11
