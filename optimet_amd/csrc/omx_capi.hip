@@ -1096,11 +1096,12 @@ bool backward_stable(omx_context *c, const cplx *A64, const cplx *rhs, const cpl
 
 // Products of the assembled S (V) from half its blocks, from N = kSymN on (below,
 // the caches hold much of the matrix: N = 2142 20 us whole, 28 from its half; 10240
-// 244 and 181); without scratch otherwise.
-omx::SymArgs sym_args(omx_context *c, bool shf) {
+// 244 and 181) and for the block orders that gain by it; without scratch otherwise.
+omx::SymArgs sym_args(omx_context *c, bool shf, bool f32) {
   omx::SymArgs a{c->P, c->nmax, c->Np, (size_t)c->Np, c->d_ov.as<cplx>(), shf ? omx::OV_TSH : omx::OV_T, nullptr};
-  if(c->kind == OMX_SOLVER_ACA_GMRES || !c->updated || c->P < 2 || c->N < kSymN) return a;
-  c->d_sym.ensure(sizeof(cplx) * omx::sym_scratch(c->P, c->nmax), &c->total);
+  if(c->kind == OMX_SOLVER_ACA_GMRES || !c->updated || c->P < 2 || c->N < kSymN || !omx::sym_pays(c->nmax, f32))
+    return a;
+  c->d_sym.ensure(sizeof(cplx) * omx::sym_scratch(c->P, c->nmax, 1), &c->total);
   a.scratch = c->d_sym.as<cplx>();
   return a;
 }
@@ -1126,8 +1127,8 @@ void solve_system(omx_context *c, bool shf, const cplx *rhs, cplx *x, int *iters
     *iters = gm.its[0];
     *res = gm.res[0];
   };
-  const omx::SymArgs sym = sym_args(c, shf);
-  if(!is_lu(c->kind) && !shf) gm.sym = sym;
+  // (V's few outer products read the whole matrix)
+  if(!is_lu(c->kind) && !shf) gm.sym = sym_args(c, shf, false);
   if(c->kind == OMX_SOLVER_ACA_GMRES) {  // Gmres_Zcomp on the compressed operator
     gm.op = [c, shf, st](const cplx *in, cplx *out) { aca_apply(c, shf, in, out, st); };
     gm.op_bytes = c->aca[shf ? 1 : 0].bytes;
@@ -1145,7 +1146,7 @@ void solve_system(omx_context *c, bool shf, const cplx *rhs, cplx *x, int *iters
     if(dirty) omx::demote(A32w, A64, (size_t)Np * lda, st);  // an earlier factorisation overwrote it
     dirty = false;
     inner.A32 = A32w;
-    inner.sym = sym;
+    inner.sym = sym_args(c, shf, true);
     inner.one_cycle = true;
     gm.lazy = true;  // its preconditioner is a solve of its own
     gm.prec = [&inner, &gm, Np, st](const cplx *in, cplx *out, const int *) {
@@ -1182,7 +1183,7 @@ void solve_system(omx_context *c, bool shf, const cplx *rhs, cplx *x, int *iters
     omx::zero_ints(status.as<int>(), 4, st);
     HIPCHK(hipMemsetAsync(x, 0, sizeof(cplx) * Np, st));
     const int maxit = std::min(c->maxit, c->auto_budget > 0 ? c->auto_budget : auto_gmres64_steps(c->N));
-    gm.sym = sym;
+    gm.sym = sym_args(c, shf, false);
     gm.x_zero = true;
     run(x, maxit);
     gm.x_zero = false;
@@ -1737,8 +1738,8 @@ void sweep_chunk(omx_context *c, int nb, const double *lam, const cplx *eps, con
     // system short of the target is left to the one-at-a-time path
     status_scan(bad, false);
     Krylov gm = sweep_krylov(c, nb, cS64);
-    if((double)N * N * nb >= (double)kSymN * kSymN) {  // as sym_args
-      c->d_sym.ensure(sizeof(cplx) * omx::sym_scratch(P, nmax) * nb, &c->total);
+    if((double)N * N * nb >= (double)kSymN * kSymN && omx::sym_pays(nmax, false)) {  // as sym_args
+      c->d_sym.ensure(sizeof(cplx) * omx::sym_scratch(P, nmax, nb), &c->total);
       gm.sym = omx::SymArgs{P,  nmax, (int)Np, lda, w.ov.as<cplx>(), omx::OV_T, c->d_sym.as<cplx>(), nb,
                             (size_t)Np * Np, lda, ovs};
     }

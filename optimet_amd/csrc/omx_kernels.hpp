@@ -269,7 +269,7 @@ inline size_t gemv_part_rows(int nb) { return std::max(kGemvSplitMax, kGemvSplit
 // y = S x for nb assembled scattering matrices from half their blocks: S_ji[p][q]
 // is S_ij[p][q] times (T_j / T_i)[p] and the parity sign of (p, q), so a pair's two
 // products read one block, for each row p the one of the larger |T[p]|.
-// Scratch: sym_scratch(P, nmax) complex values per system.
+// Scratch: sym_scratch(P, nmax, nb) complex values for nb systems.
 struct SymArgs {
   int P, nmax, Np;
   size_t lda;
@@ -280,7 +280,8 @@ struct SymArgs {
   size_t sA = 0, sv = 0, zov = 0;  // matrices, vectors and ov of the systems apart
   const int *flag = nullptr;       // systems whose flag (KF_COUNT ints apart) is 0 are left out
 };
-size_t sym_scratch(int P, int nmax);
+size_t sym_scratch(int P, int nmax, int nb);
+bool sym_pays(int nmax, bool f32);  // whether such a product is the faster one at this block order
 void sym_product(const SymArgs &a, const cplx *A, const cplx *x, cplx *y, hipStream_t st);
 void sym_product(const SymArgs &a, const float2 *A, const cplx *x, cplx *y, hipStream_t st);
 

@@ -2047,13 +2047,27 @@ int gemv_partial(const float2 *A, size_t lda, int N, const cplx *x, cplx *part, 
 }
 
 // ------------------------------------------------------------------ products of half the blocks
-// Objects j of a workgroup: one while the pairs are few, eight from 64 objects on
-// (their sum over j then leaves the workgroup once).
-inline int sym_chunk(int P) { return P > 64 ? 8 : 1; }
-size_t sym_scratch(int P, int nmax) {
-  const size_t n = 2 * (size_t)nmax * (nmax + 2), nc = (P + sym_chunk(P) - 1) / sym_chunk(P);
-  return (nc * P + (size_t)P * (P - 1) / 2) * n;
+// Objects j of a workgroup (their sum over j leaves it once): as many as leave 1536
+// workgroups, at most 8 and an eighth of the objects.  Not a number of chunks that 8
+// divides: workgroups go to the 8 XCDs in turn, and a chunk's work grows with its
+// index.  Times in us with 1, 2, 4, 8 objects: FP64, 66 objects of n = 126 (n = 2 nmax
+// (nmax + 2)) 120, 110, 136, 206; 171 of 48 123, 112, 105, 111; 513 of 96 3220, 3160,
+// 3137, 3135; 251 of 96 770, 767, 763, 999 (32 chunks of 8).
+inline int sym_chunk(int P, int nb) {
+  int ch = (int)std::max(1L, std::min({8L, (long)P / 8, (long)nb * P * P / 3072}));
+  while(ch > 1 && (P + ch - 1) / ch % 8 == 0) ++ch;
+  return ch;
 }
+size_t sym_scratch(int P, int nmax, int nb) {
+  const size_t n = 2 * (size_t)nmax * (nmax + 2), ch = sym_chunk(P, nb), nc = (P + ch - 1) / ch;
+  return nb * (nc * P + (size_t)P * (P - 1) / 2) * n;
+}
+// Small blocks leave a thread few columns between the barriers of its objects.
+// Whole / half products, us: FP64 n = 6, N = 8202 167 / 628; n = 16, N = 8208 165 / 150,
+// 24016 1387 / 1125; n = 30, N = 8220 165 / 142.  FP32 n = 16, N = 24016 706 / 843; n =
+// 30, N = 8220 88 / 96, 49230 3017 / 3073; n = 48, N = 8208 86 / 74; n = 70 (rows of 560
+// bytes), N = 8260 89 / 93, 24010 692 / 684; n = 96, N = 8256 87 / 65.
+bool sym_pays(int nmax, bool f32) { return f32 ? nmax == 4 || nmax >= 6 : nmax >= 2; }
 __device__ inline cplx sym_T(const SymArgs &a, const cplx *ov, int j, int pol, int n) {
   return ov[(((size_t)a.tkind * a.P + j) * 2 + pol) * (a.nmax + 1) + n];
 }
@@ -2076,7 +2090,7 @@ __device__ inline cplx sym_widen(float2 v) { return cplx{(double)v.x, (double)v.
 //
 // Bound: HBM, at half the bytes of the plain product, and the barriers between
 // objects.  N = 49152: FP32 2.78 -> 2.24 ms, FP64 5.45 -> 3.70; N = 10240, FP64: 244 ->
-// 181 us; N = 2142: 20 -> 28, so single systems take it from kSymN on.
+// 181 us; N = 2142: 20 -> 28, so single systems take it from kSymN on, where sym_pays.
 template <typename T>
 __global__ __launch_bounds__(512) void sym_pairs(SymArgs a, const T *__restrict__ A, const cplx *__restrict__ x, int CH,
                                                 int G) {
@@ -2203,7 +2217,7 @@ __global__ __launch_bounds__(256) void sym_sum(SymArgs a, const cplx *__restrict
   y[zs * a.sv + r] = x[zs * a.sv + r] + ((s + red[0][l]) + (red[1][l] + red[2][l]));
 }
 template <typename T> void sym_run(const SymArgs &a, const T *A, const cplx *x, cplx *y, hipStream_t st) {
-  const int n = 2 * a.nmax * (a.nmax + 2), CH = sym_chunk(a.P), nc = (a.P + CH - 1) / CH;
+  const int n = 2 * a.nmax * (a.nmax + 2), CH = sym_chunk(a.P, a.nb), nc = (a.P + CH - 1) / CH;
   // column groups (of one size) that fill the waves best, 512 threads at most
   int G = 1;
   auto fill = [&](int g) { return (double)(n * g) / ((n * g + 63) / 64 * 64); };

@@ -76,3 +76,21 @@ def test_tiny_size_parameters():
             k = (deg == n) & (pol == q)
             d = got[k] / np.abs(want[k]).max() - want[k] / np.abs(want[k]).max()
             assert np.abs(d).max() < 1e-6, (n, q, np.abs(d).max())
+
+
+@pytest.mark.parametrize("P,nmax,kind,half", [(1366, 1, "gmres64", False), (512, 2, "gmres64", True),
+                                              (275, 3, "gmres64", True), (66, 7, "gmres64", True)])
+def test_orders_that_gain(P, nmax, kind, half):
+    """Blocks of order 6 are read whole (their half takes four times as long), the
+    others from half of them: by the bytes that the products count, 16 N^2 each or
+    half of it in the Arnoldi steps.  The cycle's residuals are whole products: two
+    of them beside 5 or more steps."""
+    from optimet_amd import solver
+    s = solver.Solver(lattice(P, nmax), kind=kind, tol=1e-12)
+    s.update()
+    s.ctx.set_profile(True)
+    s.solve()
+    st = s.stats()
+    per = st["matvec_bytes"] / (16.0 * st["Np"] ** 2 * st["matvec_calls"])
+    assert st["matvec_calls"] >= 7
+    assert abs(per - 1.0) < 1e-12 if not half else 0.5 <= per < 0.7
