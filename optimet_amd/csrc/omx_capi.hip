@@ -1094,6 +1094,19 @@ bool backward_stable(omx_context *c, const cplx *A64, const cplx *rhs, const cpl
   return eta <= kBackwardErrorBound;
 }
 
+// The scratch of such products, or none when memory is short (the products then read
+// the whole matrix).
+cplx *sym_ensure(omx_context *c, size_t elems) {
+  try {
+    c->d_sym.ensure(sizeof(cplx) * elems, &c->total);
+  } catch(OmxError &e) {
+    if(e.code != OMX_ERR_MEMORY) throw;
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  return c->d_sym.as<cplx>();
+}
+
 // Products of the assembled S (V) from half its blocks, from N = kSymN on (below,
 // the caches hold much of the matrix: N = 2142 20 us whole, 28 from its half; 10240
 // 244 and 181) and for the block orders that gain by it; without scratch otherwise.
@@ -1101,8 +1114,7 @@ omx::SymArgs sym_args(omx_context *c, bool shf, bool f32) {
   omx::SymArgs a{c->P, c->nmax, c->Np, (size_t)c->Np, c->d_ov.as<cplx>(), shf ? omx::OV_TSH : omx::OV_T, nullptr};
   if(c->kind == OMX_SOLVER_ACA_GMRES || !c->updated || c->P < 2 || c->N < kSymN || !omx::sym_pays(c->nmax, f32))
     return a;
-  c->d_sym.ensure(sizeof(cplx) * omx::sym_scratch(c->P, c->nmax, 1), &c->total);
-  a.scratch = c->d_sym.as<cplx>();
+  a.scratch = sym_ensure(c, omx::sym_scratch(c->P, c->nmax, 1));
   return a;
 }
 
@@ -1739,9 +1751,8 @@ void sweep_chunk(omx_context *c, int nb, const double *lam, const cplx *eps, con
     status_scan(bad, false);
     Krylov gm = sweep_krylov(c, nb, cS64);
     if((double)N * N * nb >= (double)kSymN * kSymN && omx::sym_pays(nmax, false)) {  // as sym_args
-      c->d_sym.ensure(sizeof(cplx) * omx::sym_scratch(P, nmax, nb), &c->total);
-      gm.sym = omx::SymArgs{P,  nmax, (int)Np, lda, w.ov.as<cplx>(), omx::OV_T, c->d_sym.as<cplx>(), nb,
-                            (size_t)Np * Np, lda, ovs};
+      gm.sym = omx::SymArgs{P,  nmax, (int)Np, lda, w.ov.as<cplx>(), omx::OV_T, sym_ensure(c, omx::sym_scratch(P, nmax, nb)),
+                            nb, (size_t)Np * Np, lda, ovs};
     }
     cplx *Sx = w.x.as<cplx>();
     gm.x_zero = true;

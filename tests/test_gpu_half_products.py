@@ -94,3 +94,33 @@ def test_orders_that_gain(P, nmax, kind, half):
     per = st["matvec_bytes"] / (16.0 * st["Np"] ** 2 * st["matvec_calls"])
     assert st["matvec_calls"] >= 7
     assert abs(per - 1.0) < 1e-12 if not half else 0.5 <= per < 0.7
+
+
+def test_without_memory_for_the_scratch():
+    """With the device's memory taken, all but 64 to 128 MB, the scratch of these
+    products (300 MB) does not fit and they read the whole matrix: the solve goes
+    through, with the solution of one that had the memory (1e-10, as above)."""
+    from optimet_amd import solver
+    from tests.test_zz_no_alloc import _Dev, _hip
+    hip = _hip()
+    c = lattice(1366, 2)
+    a, b = solver.Solver(c, kind="gmres64", tol=1e-12), solver.Solver(c, kind="gmres64", tol=1e-12)
+    a.update()
+    want = a.solve()["x_sca"]
+    b.update()
+    b.vector("Q")
+    held, size = [], 16 << 30
+    try:
+        while size >= 64 << 20:
+            try:
+                held.append(_Dev(hip, size))
+            except AssertionError:
+                size //= 2
+        held.pop().free()
+        got = b.solve()["x_sca"]
+    finally:
+        for d in held:
+            d.free()
+    assert rel(got, want) < 1e-10
+    a.ctx.close()
+    b.ctx.close()
