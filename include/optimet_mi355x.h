@@ -303,7 +303,10 @@ int omx_solve_sweep(omx_context *ctx, int nl, const double *lambdas, const doubl
  * context holds (the footprint a scheduler admits requests against). */
 int omx_mem_info(omx_context *ctx, size_t *free_bytes, size_t *total_bytes, size_t *held_bytes);
 /* Releases the context's matrix-sized buffers (matrices, factors, Krylov
- * bases); the next update or sweep allocates them again. */
+ * bases, compressed operators); the next update or sweep allocates them again.
+ * Between updates of clusters of one shape (number of objects and nmax)
+ * OMX_SOLVER_ACA_GMRES keeps its operators' memory, with an eighth to spare,
+ * and the compression's staging, at most 1.5 GB. */
 int omx_trim(omx_context *ctx);
 
 /* Stand-alone dense complex solve A x = b on the device (A column-major,

@@ -242,11 +242,11 @@ struct omx_context {
     double rsum = 0, bytes = 0, ref_mb = 0;
     std::vector<int> rank;           // [i P + j]: r, -1 dense, 0 diagonal
     std::vector<const cplx *> where;  // [i P + j]: U (compressed) or the block (dense)
-    std::vector<DBuf> pools;          // factor pools, one per compression chunk (kept between builds)
+    std::vector<DBuf> pools;          // factor pools, one per compression chunk (kept for the next build)
     DBuf dense, desc, rowptr, acalist, t, part;
     bool built = false;
-    // forgets the operator; its device buffers stay for the next one (a scan
-    // rebuilds it at every wavelength; freeing and mapping gigabytes again took
+    // forgets the operator; its device buffers stay for the next one of its shape (a
+    // scan rebuilds it at every wavelength; freeing and mapping gigabytes again took
     // 6 of 28 ms per solve of 300 spheres at nmax 5, and 140 of 173 ms in a
     // process that had solved larger systems before)
     void reset() {
@@ -442,9 +442,15 @@ void alloc_all(omx_context *c) {
   c->d_nrm.ensure(sizeof(double) * 256, T);
 }
 
+// Gives back the compression's staging (not needed by the operators).
+void aca_release_staging(omx_context *c) {
+  for(DBuf *x : {&c->d_acaA, &c->d_acaU, &c->d_acaV}) x->release(&c->total);
+}
+
 void alloc_matrices(omx_context *c) {
   const size_t n2 = (size_t)c->Np * c->Np;
   size_t *T = &c->total;
+  if(c->kind != OMX_SOLVER_ACA_GMRES) aca_release_staging(c);
   // FP64 matrix: factorised (LU64), streamed (GMRES) or the residual operator
   // (IR); the compressed operators of ACA replace it
   bool need64 = c->kind != OMX_SOLVER_ACA_GMRES;
@@ -504,15 +510,33 @@ constexpr double kAcaStagingBytes = 1.5e9;  // assembly + factor staging of one 
 void aca_release(omx_context *c) {
   c->aca[0].release(&c->total);
   c->aca[1].release(&c->total);
-  DBuf *b[] = {&c->d_acaA, &c->d_acaU, &c->d_acaV};
-  for(DBuf *x : b) x->release(&c->total);
+  aca_release_staging(c);
+}
+
+// A buffer kept from the operator before: allocated again when it is too small or
+// more than twice what is wanted, with spare (want) where memory allows.
+void fit(DBuf &b, size_t need, size_t want, size_t *T) {
+  if(b.p && b.bytes >= need && b.bytes <= 2 * want) return;
+  b.release(T);
+  try {
+    b.ensure(want, T);
+  } catch(OmxError &e) {
+    if(e.code != OMX_ERR_MEMORY || want == need) throw;
+    (void)hipGetLastError();
+    b.ensure(need, T);
+  }
 }
 
 void aca_build(omx_context *c, bool shf) {
   omx_context::AcaMat &m = c->aca[shf ? 1 : 0];
   size_t *T = &c->total;
-  m.reset();
   const int P = c->P, nmax = c->nmax, n = 2 * c->nf;
+  // kept between updates of one cluster's shape (a scan, an optimiser's loop) only
+  if(m.P && (m.P != P || m.n != n)) {
+    m.release(T);
+    aca_release_staging(c);
+  }
+  m.reset();
   const size_t n2 = (size_t)n * n;
   hipStream_t st = c->st;
   m.n = n;
@@ -555,8 +579,10 @@ void aca_build(omx_context *c, bool shf) {
                      c->d_coef.as<double>(), (size_t)n, nullptr, nullptr};
   base.zblk = n2;  // S_ij of pair b at 2 b n2, S_ji behind it
   const size_t listn = std::max(dl.size(), (size_t)1);
+  size_t used = 0;  // pools
+  if(!m.ndense) m.dense.release(T);
   if(m.ndense) {
-    m.dense.ensure(sizeof(cplx) * n2 * m.ndense, T);
+    fit(m.dense, sizeof(cplx) * n2 * m.ndense, sizeof(cplx) * n2 * m.ndense, T);
     c->d_plist.ensure(sizeof(int) * listn, T);
     HIPCHK(hipMemcpyAsync(c->d_plist.p, dl.data(), sizeof(int) * dl.size(), hipMemcpyHostToDevice, st));
     omx::PairArgs pa = base;
@@ -570,9 +596,7 @@ void aca_build(omx_context *c, bool shf) {
   if(m.naca) {
     // blocks of a chunk: whole pairs
     const int C = 2 * (int)std::max<double>(1.0, std::min<double>(m.naca / 2, kAcaStagingBytes / (96.0 * n2)));
-    c->d_acaA.ensure(sizeof(cplx) * n2 * C, T);
-    c->d_acaU.ensure(sizeof(cplx) * n2 * C, T);
-    c->d_acaV.ensure(sizeof(cplx) * n2 * C, T);
+    for(DBuf *b : {&c->d_acaA, &c->d_acaU, &c->d_acaV}) fit(*b, sizeof(cplx) * n2 * C, sizeof(cplx) * n2 * C, T);
     c->d_acaR.ensure(sizeof(int) * C, T);
     c->d_acaOff.ensure(sizeof(size_t) * C, T);
     c->d_plist.ensure(sizeof(int) * std::max((size_t)C, listn), T);
@@ -602,7 +626,7 @@ void aca_build(omx_context *c, bool shf) {
       DBuf &pool = m.pools[chunk];
       // an eighth to spare when it has to grow: ranks vary a little from one
       // wavelength to the next
-      if(pool.bytes < sizeof(cplx) * tot) pool.ensure(sizeof(cplx) * (tot + tot / 8), T);
+      fit(pool, sizeof(cplx) * tot, sizeof(cplx) * (tot + tot / 8), T);
       HIPCHK(hipMemcpyAsync(c->d_acaOff.p, off.data(), sizeof(size_t) * nb, hipMemcpyHostToDevice, st));
       omx::run_aca_pack(c->d_acaU.as<cplx>(), c->d_acaV.as<cplx>(), n, nb, c->d_acaR.as<int>(), pool.as<cplx>(),
                         c->d_acaOff.as<size_t>(), st);
@@ -612,7 +636,9 @@ void aca_build(omx_context *c, bool shf) {
       }
       HIPCHK(hipStreamSynchronize(st));  // off, rk and the list buffer are reused
     }
+    used = chunk;
   }
+  for(; m.pools.size() > used; m.pools.pop_back()) m.pools.back().release(T);
   // descriptors, block row by block row
   std::vector<omx::AcaDesc> desc;
   std::vector<int> rowptr(P + 1, 0), acalist;
@@ -1297,6 +1323,7 @@ void sweep_alloc(omx_context *c, int nb, bool f64, bool sh) {
   size_t *T = &c->total;
   const size_t Np = c->Np, n2 = Np * Np, P = c->P, S = c->nmax + 1;
   const int m = c->restart;
+  aca_release_staging(c);
   w.S64.ensure(sizeof(cplx) * n2 * nb, T);
   if(f64) {
     w.F64.ensure(sizeof(cplx) * n2 * nb, T);
@@ -2171,6 +2198,7 @@ int omx_update(omx_context *c) {
     if(c->kind_req == OMX_SOLVER_AUTO)
       c->kind = c->N >= kAutoKrylovN ? OMX_SOLVER_GMRES32_IR : OMX_SOLVER_LU32_IR;
     c->krylov_s = c->kind_req == OMX_SOLVER_AUTO && c->kind == OMX_SOLVER_LU32_IR && c->sh;
+    if(c->kind != OMX_SOLVER_ACA_GMRES) aca_release(c);
     alloc_all(c);
     alloc_matrices(c);
     c->tuned = false;
@@ -2207,10 +2235,20 @@ int omx_update(omx_context *c) {
     HIPCHK(hipEventRecord(c->ujoin[1], st2));
     const size_t lda = (size_t)c->Np;
     if(c->kind == OMX_SOLVER_ACA_GMRES) {
-      aca_build(c, false);
-      if(c->sh) aca_build(c, true); else c->aca[1].release(&c->total);
+      if(!c->sh) c->aca[1].release(&c->total);
+      auto build = [&] {
+        aca_build(c, false);
+        if(c->sh) aca_build(c, true);
+      };
+      try {
+        build();
+      } catch(OmxError &e) {  // without what is kept from the operators before
+        if(e.code != OMX_ERR_MEMORY) throw;
+        (void)hipGetLastError();
+        aca_release(c);
+        build();
+      }
     } else {
-      aca_release(c);
       omx::PairArgs pa{P, nmax, omx::OV_T, c->waveK(), c->d_sph.as<double>(), c->d_ov.as<cplx>(),
                        c->d_coef.as<double>(), lda, c->d_S64.as<cplx>(), c->d_S32.as<float2>()};
       if(c->sh) {  // V in the same launch
@@ -2408,6 +2446,7 @@ void group_alloc(omx_context *L, int nb, bool f64, bool sh) {
   size_t *T = &L->total;
   const size_t Np = L->Np, n2 = Np * Np;
   const int m = L->restart;
+  aca_release_staging(L);
   w.S64.ensure(sizeof(cplx) * n2 * nb, T);
   if(f64) w.F64.ensure(sizeof(cplx) * n2 * nb, T); else w.S32.ensure(sizeof(float2) * n2 * nb, T);
   if(sh) {

@@ -3,7 +3,7 @@
 import numpy as np
 import pytest
 
-from optimet_amd.problem import Cluster, random_cluster
+from optimet_amd.problem import Cluster, drude_cluster, random_cluster
 
 pytestmark = pytest.mark.gpu
 
@@ -47,3 +47,36 @@ def test_orders(nmax):
             assert (E.max(axis=1) <= small).sum() >= r and (E.max(axis=0) <= small).sum() >= r, (i, j, r)
     x = s.solve()["x_sca"]
     assert rel(x, np.linalg.solve(A, s.vector("Q"))) < 1e-11
+
+
+def test_memory_follows_the_cluster():
+    """A context that compressed a large cluster holds no more for a small one than
+    a fresh context, except the vectors of the larger order (basis of 240 steps and
+    partial sums, about 440 of them): the pools and the staging are kept for
+    clusters of the same shape only.  Another kind of solver gives them back."""
+    from optimet_amd import solver
+
+    def cluster(P):
+        return drude_cluster(P, 5, 800 * NM, 30, 60, 2500, 10, seed=1, sh=False)
+
+    small, large = cluster(60), cluster(200)
+    fresh = solver.Solver(small, kind="aca")
+    fresh.update()
+    want = fresh.solve()["x_sca"]
+    bound = fresh.ctx.mem_info()[2] + 16 * large.N * 441
+    fresh.ctx.close()
+    s = solver.Solver(large, kind="aca")
+    s.update()
+    s.solve()
+    s.set_cluster(small)
+    for _ in range(2):
+        s.update()
+        assert np.array_equal(s.solve()["x_sca"], want)
+        assert s.ctx.mem_info()[2] <= bound
+    s.ctx.set_solver("lu64")
+    s.update()
+    d = solver.Solver(small, kind="lu64")
+    d.update()
+    assert s.ctx.mem_info()[2] <= d.ctx.mem_info()[2] + 16 * large.N * 441
+    s.ctx.close()
+    d.ctx.close()
