@@ -235,6 +235,13 @@ struct omx_context {
         abssh, absbes;
     DBuf perm, perm2, dinv, dinv2, map, status, basis, basisZ, r, w1, w2, gpart, kz, omz, map2, status2;
     KryWs kry;
+    void release(size_t *T) {
+      DBuf *b[] = {&S64, &S32, &V64, &V32, &F64, &F64sh, &eps, &eps_sh, &ov, &incloc, &Q, &w, &x, &xint, &xsh, &xintsh,
+                   &K, &K1, &cross, &abscoef, &abssh, &absbes, &perm, &perm2, &dinv, &dinv2, &map, &status, &basis,
+                   &basisZ, &r, &w1, &w2, &gpart, &kz, &omz, &map2, &status2};
+      for(DBuf *p : b) p->release(T);
+      kry.release(T);
+    }
   } sw;
   // ACA-compressed operators S (0) and V (1) of OMX_SOLVER_ACA_GMRES
   struct AcaMat {
@@ -1361,6 +1368,16 @@ void sweep_alloc(omx_context *c, int nb, bool f64, bool sh) {
   w.omz.ensure(sizeof(double) * nb, T);
 }
 
+// Bytes of one system of a large batch (sweep_alloc, and the scratch of the half
+// products with S by GMRES).
+double sweep_bytes(const omx_context *c, bool krylov_s) {
+  const bool f64 = c->kind == OMX_SOLVER_LU64;
+  const double Np = c->Np, nm = c->sh ? 2.0 : 1.0;
+  const double vectors = 12.0 + 2.0 * (c->restart + 1) + omx::kGemvSplit;
+  return nm * Np * Np * (f64 ? 32.0 : 24.0) + 16.0 * Np * vectors + 32.0 * omx::dinv_elems(c->Np, f64) +
+         (krylov_s ? 16.0 * omx::sym_scratch(c->P, c->nmax, 1) : 0.0);
+}
+
 omx::LuWork sweep_lu(omx_context *c, int nb, bool second) {
   auto &w = c->sw;
   const int Np = c->Np;
@@ -1985,17 +2002,11 @@ void omx_destroy(omx_context *c) {
                   &c->d_dinv, &c->d_dinv2, &c->d_F64, &c->d_F64sh, &c->d_abscoef, &c->d_abssh, &c->d_absbes,
                   &c->d_fpts, &c->d_fout, &c->d_fown, &c->d_fpart};
   for(DBuf *b : bufs) b->release(&c->total);
-  auto &w = c->sw;
-  DBuf *sbufs[] = {&w.S64, &w.S32, &w.V64, &w.V32, &w.F64, &w.F64sh, &w.eps, &w.eps_sh, &w.ov, &w.incloc, &w.Q,
-                   &w.w, &w.x, &w.xint, &w.xsh, &w.xintsh, &w.K, &w.K1, &w.cross, &w.perm, &w.perm2,
-                   &w.dinv, &w.dinv2, &w.map, &w.status, &w.basis, &w.basisZ, &w.r, &w.w1, &w.w2, &w.gpart,
-                   &w.abscoef, &w.abssh, &w.absbes, &w.kz, &w.omz};
-  for(DBuf *b : sbufs) b->release(&c->total);
+  c->sw.release(&c->total);
   c->aca[0].release(&c->total);
   c->aca[1].release(&c->total);
   c->ws_in.release(&c->total);
   c->kry.release(&c->total);
-  w.kry.release(&c->total);
   DBuf *abufs[] = {&c->d_acaA, &c->d_acaU, &c->d_acaV, &c->d_acaR, &c->d_acaOff, &c->d_plist};
   for(DBuf *b : abufs) b->release(&c->total);
   for(auto &e : c->ev)
@@ -2923,8 +2934,7 @@ int omx_solve_sweep(omx_context *c, int nl, const double *lambdas, const double 
     // geometry and material constants on the device (as omx_update)
     upload_geometry(c);
     // batch size: at most 64 systems and half of the free device memory
-    const bool f64 = c->kind == OMX_SOLVER_LU64;
-    const double per = (double)c->Np * c->Np * ((c->sh ? 2 : 1) * (f64 ? 32.0 : 24.0));
+    const double per = sweep_bytes(c, krylov_s);
     size_t fr = 0, tot = 0;
     HIPCHK(hipMemGetInfo(&fr, &tot));
     int nb = batch > 0 ? batch : 64;
@@ -2964,15 +2974,12 @@ int omx_solve_sweep(omx_context *c, int nl, const double *lambdas, const double 
     const float t_batch = elapsed(c, 6, 7);
     // systems the batch could not solve: one at a time with partial pivoting
     if(!redo.empty()) {
-      // the batch's matrix-sized buffers are released first, so the
-      // one-at-a-time solves (which allocate a single system's matrices,
+      // the batch's buffers are released first (its results are on the host), so
+      // the one-at-a-time solves (which allocate a single system's matrices,
       // copies and bases) never hold memory beside a whole batch: the
       // context's peak stays the batch footprint a scheduler admitted
-      {
-        auto &w = c->sw;
-        DBuf *big[] = {&w.S64, &w.S32, &w.V64, &w.V32, &w.F64, &w.F64sh, &w.basis, &w.basisZ, &w.gpart};
-        for(DBuf *b : big) b->release(&c->total);
-      }
+      c->sw.release(&c->total);
+      c->d_sym.release(&c->total);
       const double lam0 = c->lambda;
       const std::vector<cplx> e0 = c->eps, es0 = c->eps_sh;
       const int piv0 = c->pivot;

@@ -65,20 +65,32 @@ GROUP_RATIO = 1.5  # with orders within this factor of the oldest one's (padding
 
 
 def footprint(cluster, batch, kind):
-    """Device bytes of a batch of `batch` systems of this cluster: the FP64
-    matrix (16 N^2) and, per solver kind, its FP32 copy (8 N^2) or FP64
-    factors (16 N^2), for S and (with the second harmonic) V, plus the
-    per-system vectors, panel inverses and the two Krylov bases (restart 40);
-    "auto" is the mixed LU's footprint (the Krylov path holds the same
-    matrices plus a 31-vector inner basis)."""
-    Np = -(-cluster.N // 64) * 64
-    per_matrix = Np * Np * (32 if kind == "lu64" else 24)
-    if kind == "auto" and cluster.N >= KRYLOV_N:
+    """Device bytes of a batch of `batch` systems of this cluster, in a context
+    of its own: the FP64 matrix (16 N^2) and, per solver kind, its FP32 copy
+    (8 N^2) or FP64 factors (16 N^2), for S and (with the second harmonic) V;
+    the per-system vectors, panel inverses (with FP64 factors as many products
+    for the triangular solves), partial sums, the two Krylov bases (restart 40)
+    and the iteration's state; and the context's own vectors.  "auto" is the
+    mixed LU's footprint and the scratch of products from half the blocks (the
+    Krylov path, one system at a time, also has an inner basis of 31 vectors
+    and partial sums of its own).  The second harmonic's tables (72 nf^3
+    bytes), which a context keeps for good, are not counted."""
+    Np, P, nmax = -(-cluster.N // 64) * 64, cluster.nobj, cluster.nmax
+    krylov = kind == "auto" and cluster.N >= KRYLOV_N
+    if krylov:
         batch = 1
-        per_matrix += Np * 16 * 32 // (2 if cluster.sh else 1)
-    mats = 2 if cluster.sh else 1
-    vectors = Np * (16 * 16 + 2 * 16 * 2 * 64 + 2 * 16 * 41 + 16 * 32)
-    return batch * (mats * per_matrix + vectors)
+    matrices = (2 if cluster.sh else 1) * Np * Np * (32 if kind == "lu64" else 24)
+    objects = P * (16 * 9 * 2 * (nmax + 1) + 1024)  # T-matrix vectors and radial functions
+    inverses = Np * 4096 * (2 if kind == "lu64" else 1)
+    blocks = -(-Np // 256)
+    steps = 30000 + blocks * 1400  # Hessenberg columns and the dots' partial sums
+    system = matrices + inverses + 16 * Np * (12 + 2 * 41) + 40 * (Np + 128) + objects + steps
+    if kind == "auto":
+        system += 24 * P * cluster.N
+    own = 16 * Np * (12 + 96 * (2 if krylov else 1)) + objects + (1 << 19)
+    if krylov:
+        own += 16 * Np * 33 + steps
+    return batch * system + 16 * Np * max(96, 32 * batch) + own
 
 
 class Request:

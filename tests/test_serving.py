@@ -246,3 +246,41 @@ def test_grouped_requests_match_their_sweeps():
             d = np.linalg.norm(res.out[key] - a[key]) / np.linalg.norm(a[key])
             assert d < 1e-10, (res.id, key, d)
         assert np.allclose(res.out["xs"], a["xs"], rtol=1e-10, atol=0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,P,nmax,nl,sh", [("lu64", 5, 5, 6, True), ("lu64", 5, 5, 1, True), ("lu64", 3, 1, 3, False),
+                                               ("lu32ir", 16, 1, 2, True), ("lu32ir", 5, 5, 40, True),
+                                               ("auto", 17, 7, 15, True), ("lu64", 2, 10, 4, True)])
+def test_footprint_covers_what_a_context_holds(kind, P, nmax, nl, sh):
+    """A sweep, and a single solve in a context of its own, hold no more than the
+    bytes they are admitted with (and the second harmonic's tables)."""
+    from optimet_amd import solver
+    c = drude_cluster(P, nmax, 700e-9, 40, 80, 1000, 10, seed=3, sh=sh)
+    tables = 72 * c.nf ** 3 if sh else 0
+    s = solver.Solver(c, kind=kind)
+    s.sweep(np.linspace(450e-9, 850e-9, nl), batch=nl, outputs=("x_sca",))
+    assert s.stats()["sweep_batch"] == nl
+    assert s.ctx.mem_info()[2] <= footprint(c, nl, kind) + tables
+    s.ctx.close()
+    s = solver.Solver(c, kind=kind)
+    s.update()
+    s.solve()
+    assert s.ctx.mem_info()[2] <= footprint(c, 1, kind) + tables
+    s.ctx.close()
+
+
+@pytest.mark.gpu
+def test_systems_redone_alone_hold_one_system():
+    """A sweep whose refinements may take one step only redoes every system alone;
+    afterwards the context holds a single system's bytes, none of the batch's (the
+    scratch of its products from half the blocks among them)."""
+    from optimet_amd import solver
+    c = drude_cluster(24, 6, 700e-9, 40, 80, 1000, 10, seed=3)
+    c.meta.pop("drude")
+    c.eps_r = c.eps_r_sh = np.full(24, 2.25 + 0j)
+    s = solver.Solver(c, kind="auto", maxit=1)
+    s.sweep(np.linspace(600e-9, 850e-9, 13), batch=13, outputs=("x_sca",))
+    assert s.stats()["pivot_fallbacks"] >= 13
+    assert s.ctx.mem_info()[2] <= footprint(c, 1, "auto") + 72 * c.nf ** 3
+    s.ctx.close()
