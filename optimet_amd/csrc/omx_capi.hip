@@ -1430,7 +1430,8 @@ Krylov sweep_krylov(omx_context *c, int nb, const cplx *A) {
 
 // ------------------------------------------------------------------ autotuner
 // Per shape (device, padded order, batch, factor type) the batched sweeps
-// pick the bulk-update product of FP32 factors (split-bf16 or FP32 MFMA) and
+// pick the bulk-update product of FP32 factors (split-bf16 with K = 256 or FP32
+// MFMA with K = 128, timed on the same 256 columns' worth of update) and
 // the triangular-solve variant by timing every candidate on the batch's own
 // buffers before its first chunk (zeroed matrices, identity permutations:
 // the kernels have no value-dependent branches, so the times are those of the
@@ -1495,10 +1496,10 @@ TuneChoice sweep_tune(omx_context *c, int nb, bool f64) {
   void *F = f64 ? w.F64.p : w.S32.p;
   const size_t fbytes = (f64 ? sizeof(double2) : sizeof(float2)) * n2 * nb;
   HIPCHK(hipMemsetAsync(F, 0, fbytes, st));
-  if(!f64) {
+  if(!f64 && Np > 4 * omx::kNB) {  // a smaller factorisation has no bulk update
     float2 *A = static_cast<float2 *>(F);
-    ch.t_prod[0] = time_median(st, [&] { omx::bulk_update_probe<float2>(A, Np, lda, nb, n2, true, st); });
-    ch.t_prod[1] = time_median(st, [&] { omx::bulk_update_probe<float2>(A, Np, lda, nb, n2, false, st); });
+    ch.t_prod[0] = time_median(st, [&] { omx::bulk_update_probe(A, Np, lda, nb, n2, true, st); });
+    ch.t_prod[1] = time_median(st, [&] { omx::bulk_update_probe(A, Np, lda, nb, n2, false, st); });
     const int dflt = ch.split ? 0 : 1, other = 1 - dflt;
     if(ch.t_prod[other] < kTuneMargin * ch.t_prod[dflt]) ch.split = other == 0;
     HIPCHK(hipMemsetAsync(F, 0, fbytes, st));
@@ -1548,10 +1549,10 @@ TuneChoice single_tune(omx_context *c, bool f64) {
   void *F = f64 ? c->d_F64.p : c->d_S32.p;
   const size_t fbytes = (f64 ? sizeof(double2) : sizeof(float2)) * n2;
   HIPCHK(hipMemsetAsync(F, 0, fbytes, st));
-  if(!f64) {
+  if(!f64 && Np > 4 * omx::kNB) {  // a smaller factorisation has no bulk update
     float2 *A = static_cast<float2 *>(F);
-    ch.t_prod[0] = time_median(st, [&] { omx::bulk_update_probe<float2>(A, Np, lda, 1, 0, true, st); });
-    ch.t_prod[1] = time_median(st, [&] { omx::bulk_update_probe<float2>(A, Np, lda, 1, 0, false, st); });
+    ch.t_prod[0] = time_median(st, [&] { omx::bulk_update_probe(A, Np, lda, 1, 0, true, st); });
+    ch.t_prod[1] = time_median(st, [&] { omx::bulk_update_probe(A, Np, lda, 1, 0, false, st); });
     const int dflt = ch.split ? 0 : 1, other = 1 - dflt;
     if(ch.t_prod[other] < kTuneMargin * ch.t_prod[dflt]) ch.split = other == 0;
     HIPCHK(hipMemsetAsync(F, 0, fbytes, st));

@@ -245,11 +245,11 @@ int lu_factor(T *A, int Np, size_t lda, LuWork &w, hipStream_t st, LuProf *prof 
 // and when the near-phase tiles are loaded (0: as used, 1: at kernel start,
 // 2: after the far phase).  Variant 0 is the default of each type.
 constexpr int kTrsvVariants = 3;
-// One bulk update of the shape the factorisation's first panel pair makes
-// (M = N = Np - 128, K = 128) on nb matrices sA apart: a timing probe for the
-// autotuner (A's contents are overwritten).
-template <typename T>
-void bulk_update_probe(T *A, int Np, size_t lda, int nb, size_t sA, bool split, hipStream_t st);
+// The bulk updates of an FP32 factorisation's first four panels on the columns
+// behind them (M = N = Np - 256) as it runs them with either product: one with K =
+// 256 (split) or two with K = 128, on nb matrices sA apart.  A timing probe for the
+// autotuner; nothing to do up to Np = 256.  (A's contents are overwritten.)
+void bulk_update_probe(float2 *A, int Np, size_t lda, int nb, size_t sA, bool split, hipStream_t st);
 // Solve with the factors: x = A^{-1} b, vectors always complex FP64.
 template <typename T>
 void lu_solve(const T *A, int Np, size_t lda, LuWork &w, const cplx *b, cplx *x, hipStream_t st);

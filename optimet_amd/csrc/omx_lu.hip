@@ -1953,13 +1953,15 @@ void lu_solve(const T *A, int Np, size_t lda, LuWork &w, const cplx *b, cplx *x,
   }
 }
 
-template <typename T>
-void bulk_update_probe(T *A, int Np, size_t lda, int nb, size_t sA, bool split, hipStream_t st) {
-  if(Np <= 2 * kNB) return;
-  bulk_update<T>(A, lda, 2 * kNB, 2 * kNB, 0, Np - 2 * kNB, Np - 2 * kNB, st, nb, sA, split);
+void bulk_update_probe(float2 *A, int Np, size_t lda, int nb, size_t sA, bool split, hipStream_t st) {
+  const int m = Np - 4 * kNB;
+  if(m <= 0) return;
+  if(split) {
+    bulk_update<float2, 4 * kNB>(A, lda, 4 * kNB, 4 * kNB, 0, m, m, st, nb, sA, true);
+    return;
+  }
+  for(int k0 : {0, 2 * kNB}) bulk_update<float2>(A, lda, 4 * kNB, 4 * kNB, k0, m, m, st, nb, sA, false);
 }
-template void bulk_update_probe<double2>(double2 *, int, size_t, int, size_t, bool, hipStream_t);
-template void bulk_update_probe<float2>(float2 *, int, size_t, int, size_t, bool, hipStream_t);
 
 template int lu_factor<double2>(double2 *, int, size_t, LuWork &, hipStream_t, LuProf *);
 template int lu_factor<float2>(float2 *, int, size_t, LuWork &, hipStream_t, LuProf *);

@@ -51,3 +51,27 @@ def test_tuning_is_cached_and_reproducible():
     for k in ("x_sca", "x_sca_sh"):
         assert rel(on[k], off[k]) < 1e-10, k
         assert rel(again[k], on[k]) < 1e-12, k
+
+
+def test_the_split_product_is_timed_as_it_runs():
+    """The probe's time is that of the factorisation's update behind its first four
+    panels (K = 256, M = N = Np - 256): the rate it implies is that of the
+    factorisation's own bulk updates, which include smaller ones and their thin
+    first columns (half as fast again at the most; timed with K = 128 the probe
+    seemed more than twice as fast)."""
+    from optimet_amd import solver
+    c = drude_cluster(64, 8, 800e-9, 40, 80, 1000, 10, seed=2000, sh=False)
+    s = solver.Solver(c, kind="lu32ir")
+    s.update()
+    s.solve()
+    s.ctx.set_profile(True)
+    s.update()
+    s.solve()
+    st = s.stats()
+    Np = st["Np"]
+    q = solver.tune_query(Np, 1)
+    assert q["split"]
+    own = st["lu_gemm_flop"] / st["t_lu_gemm_ms"]
+    implied = 8.0 * (Np - 256) ** 2 * 256 / q["times_ms"][0]
+    s.ctx.close()
+    assert 0.8 < implied / own < 1.75, implied / own
