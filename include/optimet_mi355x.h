@@ -164,7 +164,8 @@ int omx_set_autotune(omx_context *ctx, int on);
 /* The tuned choice of a shape: *split (1 split-bf16, 0 FP32 MFMA), *trsv (the
  * triangular-solve variant, 0 = default), times[5] (ms: the two products'
  * probes, the bulk update behind the first 256 columns by either, FP32 factors
- * of Np > 256 only, then the three triangular-solve variants).
+ * of Np > 256 only, then the three triangular-solve variants; with FP64 factors
+ * the second's holds a third of the time that forming its links takes).
  * OMX_ERR_STATE when the shape has not been tuned in this process. */
 int omx_tune_query(int device, int Np, int nb, int fp64, int *split, int *trsv, double *times);
 

@@ -222,6 +222,7 @@ struct omx_context {
   bool upd_timed = false;
   hipEvent_t uev[3] = {nullptr, nullptr, nullptr}, ujoin[2] = {nullptr, nullptr};
   omx::LuWork lu{}, lu_sh{};
+  bool links_room = false;  // alloc_lu leaves room for links
   bool profile = false;
   std::vector<hipEvent_t> pev;
   omx::LuProf prof{};
@@ -348,7 +349,7 @@ bool is_lu(int kind) { return kind == OMX_SOLVER_LU64 || kind == OMX_SOLVER_LU32
 void alloc_lu(omx_context *c, omx::LuWork &w, DBuf &perm, DBuf &dinv, bool second) {
   const int Np = c->Np;
   const int gmax = (Np + omx::kPanelRows - 1) / omx::kPanelRows + 1;
-  dinv.ensure(sizeof(cplx) * omx::dinv_elems(Np, c->kind == OMX_SOLVER_LU64), &c->total);
+  dinv.ensure(sizeof(cplx) * omx::dinv_elems(Np, c->links_room), &c->total);
   perm.ensure(sizeof(int) * Np, &c->total);
   // tournament scratch: one half per system, as S and V may be factored
   // at the same time
@@ -375,7 +376,6 @@ void alloc_lu(omx_context *c, omx::LuWork &w, DBuf &perm, DBuf &dinv, bool secon
   w.status = status.as<int>();
   w.wlu = c->d_wlu.as<cplx>() + (size_t)half * 3 * omx::kNB * omx::kNB;
   w.dinv = dinv.p;
-  w.links = c->kind == OMX_SOLVER_LU64;
   w.pivot = c->pivot;
   hipEvent_t *ev = second ? c->lu_ev2 : c->lu_ev;
   w.aux = second ? c->aux2 : c->aux;
@@ -384,6 +384,15 @@ void alloc_lu(omx_context *c, omx::LuWork &w, DBuf &perm, DBuf &dinv, bool secon
   w.ev_bulk = ev[2];
   w.ev_pan = ev[3];
   w.gmax = gmax;
+}
+
+// The triangular-solve variant of a system's factors; FP64 ones solved by variant 1
+// take links.
+void set_trsv(omx_context *c, omx::LuWork &w, DBuf &dinv, int trsv) {
+  w.trsv = trsv;
+  w.links = c->kind == OMX_SOLVER_LU64 && trsv == 1;
+  dinv.ensure(sizeof(cplx) * omx::dinv_elems(c->Np, w.links), &c->total);
+  w.dinv = dinv.p;
 }
 
 // The geometry's arrays on the device in one copy: mu, eps, eps_sh and the
@@ -1000,6 +1009,7 @@ std::vector<uintptr_t> single_key(omx_context *c, bool with_v, int mark) {
   for(const omx::LuWork *w : lw) {
     const void *p[] = {w->perm, w->mdst, w->msrc, w->mcnt, w->status, w->dinv, w->aux};
     for(const void *x : p) k.push_back((uintptr_t)x);
+    k.push_back((uintptr_t)w->links);
   }
   const void *b[] = {c->d_S64.p, c->d_S32.p, c->d_V64.p, c->d_V32.p, c->d_F64.p, c->d_F64sh.p, c->d_status.p,
                      c->d_status2.p};
@@ -1354,7 +1364,6 @@ void sweep_alloc(omx_context *c, int nb, bool f64, bool sh) {
   w.abssh.ensure(sizeof(double) * P * nb, T);
   w.absbes.ensure(sizeof(cplx) * P * omx::kAbsBes * nb, T);
   for(DBuf *b : {&w.perm, &w.perm2}) b->ensure(sizeof(int) * Np * nb, T);
-  for(DBuf *b : {&w.dinv, &w.dinv2}) b->ensure(sizeof(cplx) * omx::dinv_elems(Np, f64) * nb, T);
   w.map.ensure(sizeof(int) * 3 * (Np + 2 * omx::kNB) * nb, T);
   w.status.ensure(sizeof(int) * 4 * nb, T);
   if(sh) {  // V's factorisation runs beside S's: maps and status words of its own
@@ -1378,13 +1387,14 @@ double sweep_bytes(const omx_context *c, bool krylov_s) {
          (krylov_s ? 16.0 * omx::sym_scratch(c->P, c->nmax, 1) : 0.0);
 }
 
-omx::LuWork sweep_lu(omx_context *c, int nb, bool second) {
+// One system's or a batch's triangular-solve variant: see set_trsv.
+omx::LuWork sweep_lu(omx_context *c, int nb, bool second, int trsv) {
   auto &w = c->sw;
   const int Np = c->Np;
   omx::LuWork lw{};
   lw.perm = (second ? w.perm2 : w.perm).as<int>();
-  lw.dinv = (second ? w.dinv2 : w.dinv).p;
-  lw.links = c->kind == OMX_SOLVER_LU64;
+  lw.links = c->kind == OMX_SOLVER_LU64 && trsv == 1;
+  lw.trsv = trsv;
   const int ms = Np + 2 * omx::kNB;
   int *map = (second ? w.map2 : w.map).as<int>();
   lw.mdst = map;
@@ -1404,7 +1414,10 @@ omx::LuWork sweep_lu(omx_context *c, int nb, bool second) {
   lw.split = c->lu32_gemm == OMX_GEMM_BF16X3;
   lw.nb = nb;
   lw.bs.a = (size_t)Np * Np;
-  lw.bs.inv = omx::dinv_elems(Np, c->kind == OMX_SOLVER_LU64);
+  lw.bs.inv = omx::dinv_elems(Np, lw.links);
+  DBuf &dinv = second ? w.dinv2 : w.dinv;
+  dinv.ensure(sizeof(cplx) * lw.bs.inv * nb, &c->total);
+  lw.dinv = dinv.p;
   lw.bs.vec = (size_t)Np;
   lw.bs.perm = Np;
   lw.bs.map = ms;
@@ -1449,6 +1462,13 @@ std::mutex g_tune_mu;
 std::map<std::tuple<int, int, int, int>, TuneChoice> g_tune;  // (device, Np, nb, fp64)
 constexpr double kTuneMargin = 0.95;
 
+bool tune_lookup(const omx_context *c, int nb, bool f64, TuneChoice *out) {
+  std::lock_guard<std::mutex> g(g_tune_mu);
+  auto it = g_tune.find(std::make_tuple(c->device, c->Np, nb, f64 ? 1 : 0));
+  if(it != g_tune.end()) *out = it->second;
+  return it != g_tune.end();
+}
+
 double time_median(hipStream_t st, const std::function<void()> &f, int reps = 5) {
   hipEvent_t a, b;
   HIPCHK(hipEventCreate(&a));
@@ -1476,22 +1496,21 @@ double time_median(hipStream_t st, const std::function<void()> &f, int reps = 5)
   return ts[ts.size() / 2];
 }
 
-omx::LuWork sweep_lu(omx_context *c, int nb, bool second);
+// A solve's share of forming the links: a factorisation is applied about three times,
+// to the right-hand side and in two refinement steps.
+double links_share(const double2 *F, int Np, const omx::LuWork &lw, hipStream_t st) {
+  return time_median(st, [&] { omx::lu_links(F, Np, (size_t)Np, lw, st); }) / 3.0;
+}
 
 // The tuned choice for this batch (tuning it first if needed); runs on the
 // chunk's buffers before the chunk fills them.
 TuneChoice sweep_tune(omx_context *c, int nb, bool f64) {
-  const auto key = std::make_tuple(c->device, c->Np, nb, f64 ? 1 : 0);
-  {
-    std::lock_guard<std::mutex> g(g_tune_mu);
-    auto it = g_tune.find(key);
-    if(it != g_tune.end()) return it->second;
-  }
+  TuneChoice ch;
+  if(tune_lookup(c, nb, f64, &ch)) return ch;
   auto &w = c->sw;
   const int Np = c->Np;
   const size_t n2 = (size_t)Np * Np, lda = (size_t)Np;
   hipStream_t st = c->st;
-  TuneChoice ch;
   ch.split = c->lu32_gemm == OMX_GEMM_BF16X3;
   void *F = f64 ? w.F64.p : w.S32.p;
   const size_t fbytes = (f64 ? sizeof(double2) : sizeof(float2)) * n2 * nb;
@@ -1509,25 +1528,28 @@ TuneChoice sweep_tune(omx_context *c, int nb, bool f64) {
   for(int z = 0; z < nb; ++z)
     for(int i = 0; i < Np; ++i) ident[(size_t)z * Np + i] = i;
   HIPCHK(hipMemcpyAsync(w.perm.p, ident.data(), sizeof(int) * ident.size(), hipMemcpyHostToDevice, st));
+  const size_t before = w.dinv.bytes;
+  (void)sweep_lu(c, nb, false, 1);  // room for the links
   HIPCHK(hipMemsetAsync(w.dinv.p, 0, w.dinv.bytes, st));
   HIPCHK(hipMemsetAsync(w.r.p, 0, w.r.bytes, st));
-  omx::LuWork lw = sweep_lu(c, nb, false);
   for(int v = 0; v < omx::kTrsvVariants; ++v) {
-    lw.trsv = v;
+    omx::LuWork lw = sweep_lu(c, nb, false, v);
     ch.t_trsv[v] = time_median(st, [&] {
       if(f64)
         omx::lu_solve<double2>(static_cast<const double2 *>(F), Np, lda, lw, w.r.as<cplx>(), w.w2.as<cplx>(), st);
       else
         omx::lu_solve<float2>(static_cast<const float2 *>(F), Np, lda, lw, w.r.as<cplx>(), w.w2.as<cplx>(), st);
     });
+    if(lw.links) ch.t_trsv[v] += links_share(static_cast<const double2 *>(F), Np, lw, st);
   }
   int best = 0;
   for(int v = 1; v < omx::kTrsvVariants; ++v)
     if(ch.t_trsv[v] < ch.t_trsv[best]) best = v;
   ch.trsv = ch.t_trsv[best] < kTuneMargin * ch.t_trsv[0] ? best : 0;
+  if(ch.trsv != 1 && w.dinv.bytes > before) w.dinv.release(&c->total);
   HIPCHK(hipStreamSynchronize(st));  // ident ends here
   std::lock_guard<std::mutex> g(g_tune_mu);
-  g_tune[key] = ch;
+  g_tune[std::make_tuple(c->device, Np, nb, f64 ? 1 : 0)] = ch;
   return ch;
 }
 
@@ -1535,16 +1557,10 @@ TuneChoice sweep_tune(omx_context *c, int nb, bool f64) {
 // with batch 1 and the context's own buffers (before the assembly fills
 // them).
 TuneChoice single_tune(omx_context *c, bool f64) {
-  const auto key = std::make_tuple(c->device, c->Np, 1, f64 ? 1 : 0);
-  {
-    std::lock_guard<std::mutex> g(g_tune_mu);
-    auto it = g_tune.find(key);
-    if(it != g_tune.end()) return it->second;
-  }
+  TuneChoice ch;
   const int Np = c->Np;
   const size_t n2 = (size_t)Np * Np, lda = (size_t)Np;
   hipStream_t st = c->st;
-  TuneChoice ch;
   ch.split = c->lu32_gemm == OMX_GEMM_BF16X3;
   void *F = f64 ? c->d_F64.p : c->d_S32.p;
   const size_t fbytes = (f64 ? sizeof(double2) : sizeof(float2)) * n2;
@@ -1560,11 +1576,13 @@ TuneChoice single_tune(omx_context *c, bool f64) {
   std::vector<int> ident(Np);
   for(int i = 0; i < Np; ++i) ident[i] = i;
   HIPCHK(hipMemcpyAsync(c->d_perm.p, ident.data(), sizeof(int) * Np, hipMemcpyHostToDevice, st));
+  omx::LuWork &lw = c->lu;
+  set_trsv(c, lw, c->d_dinv, 1);  // room for the links
   HIPCHK(hipMemsetAsync(c->d_dinv.p, 0, c->d_dinv.bytes, st));
   HIPCHK(hipMemsetAsync(c->d_r.p, 0, c->d_r.bytes, st));
-  omx::LuWork &lw = c->lu;
   for(int v = 0; v < omx::kTrsvVariants; ++v) {
     lw.trsv = v;
+    lw.links = f64 && v == 1;
     ch.t_trsv[v] = time_median(st, [&] {
       if(f64)
         omx::lu_solve<double2>(static_cast<const double2 *>(F), Np, lda, lw, c->d_r.as<cplx>(), c->d_w2.as<cplx>(),
@@ -1572,15 +1590,15 @@ TuneChoice single_tune(omx_context *c, bool f64) {
       else
         omx::lu_solve<float2>(static_cast<const float2 *>(F), Np, lda, lw, c->d_r.as<cplx>(), c->d_w2.as<cplx>(), st);
     });
+    if(lw.links) ch.t_trsv[v] += links_share(static_cast<const double2 *>(F), Np, lw, st);
   }
-  lw.trsv = 0;
   int best = 0;
   for(int v = 1; v < omx::kTrsvVariants; ++v)
     if(ch.t_trsv[v] < ch.t_trsv[best]) best = v;
   ch.trsv = ch.t_trsv[best] < kTuneMargin * ch.t_trsv[0] ? best : 0;
   HIPCHK(hipStreamSynchronize(st));  // ident ends here
   std::lock_guard<std::mutex> g(g_tune_mu);
-  g_tune[key] = ch;
+  g_tune[std::make_tuple(c->device, Np, 1, f64 ? 1 : 0)] = ch;
   return ch;
 }
 
@@ -1693,13 +1711,11 @@ void sweep_chunk(omx_context *c, int nb, const double *lam, const cplx *eps, con
   // V does not depend on the fundamental solution: its factorisation starts
   // on the second stream pair right after the assembly and runs beside S's
   // factorisation and refinement; V's refinement waits for it
-  omx::LuWork lwS = sweep_lu(c, nb, false), lwV{};
+  omx::LuWork lwS = sweep_lu(c, nb, false, tune.trsv), lwV{};
   lwS.split = tune.split;
-  lwS.trsv = tune.trsv;
   if(sh) {
-    lwV = sweep_lu(c, nb, true);
+    lwV = sweep_lu(c, nb, true, tune.trsv);
     lwV.split = tune.split;
-    lwV.trsv = tune.trsv;
   }
   void *FS = f64 ? w.F64.p : w.S32.p, *FV = sh ? (f64 ? w.F64sh.p : w.V32.p) : nullptr;
   SideEnqueue vq;
@@ -1715,7 +1731,8 @@ void sweep_chunk(omx_context *c, int nb, const double *lam, const cplx *eps, con
   } else if(c->graphs) {
     // captured once per batch shape and buffers, then replayed chunk after chunk
     auto &g = c->fg_sweep;
-    std::vector<uintptr_t> key{2, (uintptr_t)nb, (uintptr_t)Np, (uintptr_t)f64, (uintptr_t)sh, (uintptr_t)tune.split};
+    std::vector<uintptr_t> key{2, (uintptr_t)nb, (uintptr_t)Np, (uintptr_t)f64, (uintptr_t)sh, (uintptr_t)tune.split,
+                               (uintptr_t)lwS.links};
     const void *p[] = {w.S64.p, w.S32.p, w.V64.p, w.V32.p, w.F64.p, w.F64sh.p, w.perm.p, w.perm2.p, w.map.p,
                        w.map2.p, w.status.p, w.status2.p, w.dinv.p, w.dinv2.p};
     for(const void *x : p) key.push_back((uintptr_t)x);
@@ -1973,7 +1990,6 @@ int omx_create(omx_context **out, int device) {
       for(auto &e : c->xev) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
       for(auto &e : c->ev) HIPCHK(hipEventCreate(&e));
       for(auto &e : c->uev) HIPCHK(hipEventCreate(&e));
-      for(auto &e : c->mv_ev) HIPCHK(hipEventCreate(&e));
       for(hipEvent_t *e : {&c->geo_ev, &c->ujoin[0], &c->ujoin[1]})
         HIPCHK(hipEventCreateWithFlags(e, hipEventDisableTiming));
       omx::upload_factorials();
@@ -2212,13 +2228,23 @@ int omx_update(omx_context *c) {
     c->krylov_s = c->kind_req == OMX_SOLVER_AUTO && c->kind == OMX_SOLVER_LU32_IR && c->sh;
     if(c->kind != OMX_SOLVER_ACA_GMRES) aca_release(c);
     alloc_all(c);
+    const bool tune = c->autotune && is_lu(c->kind), f64 = c->kind == OMX_SOLVER_LU64;
+    TuneChoice t;
+    const bool known = tune && tune_lookup(c, 1, f64, &t);
+    c->links_room = tune && f64 && (!known || t.trsv == 1);
     alloc_matrices(c);
     c->tuned = false;
-    if(c->autotune && is_lu(c->kind)) {
-      const TuneChoice t = single_tune(c, c->kind == OMX_SOLVER_LU64);
-      c->lu.trsv = t.trsv;
-      if(c->sh) c->lu_sh.trsv = t.trsv;
-      c->tuned = true;
+    if(tune && !known) {
+      t = single_tune(c, f64);
+      if(c->links_room && t.trsv != 1) {  // no links after all
+        c->d_dinv.release(&c->total);
+        c->d_dinv2.release(&c->total);
+      }
+    }
+    c->tuned = tune;
+    if(tune) {
+      set_trsv(c, c->lu, c->d_dinv, t.trsv);
+      if(c->sh) set_trsv(c, c->lu_sh, c->d_dinv2, t.trsv);
       c->tuned_split = t.split;
     }
     const int P = c->P, nmax = c->nmax;
@@ -2467,7 +2493,6 @@ void group_alloc(omx_context *L, int nb, bool f64, bool sh) {
   }
   for(DBuf *b : {&w.Q, &w.x, &w.xsh, &w.K, &w.r, &w.w1, &w.w2}) b->ensure(sizeof(cplx) * Np * nb, T);
   for(DBuf *b : {&w.perm, &w.perm2}) b->ensure(sizeof(int) * Np * nb, T);
-  for(DBuf *b : {&w.dinv, &w.dinv2}) b->ensure(sizeof(cplx) * omx::dinv_elems(Np, f64) * nb, T);
   for(DBuf *b : {&w.map, &w.map2}) b->ensure(sizeof(int) * 3 * (Np + 2 * omx::kNB) * nb, T);
   for(DBuf *b : {&w.status, &w.status2}) b->ensure(sizeof(int) * 4 * nb, T);
   w.basis.ensure(sizeof(cplx) * Np * (m + 1) * nb, T);
@@ -2551,13 +2576,11 @@ int omx_solve_group(omx_context *L, int n, omx_context *const *mem) {
                          : omx::lu_factor<float2>(static_cast<float2 *>(F), Np, lda, lw, fst, nullptr);
       if(rc) throw OmxError(OMX_ERR_DEVICE, "batched lu_factor launch failed (" + std::to_string(rc) + ")");
     };
-    omx::LuWork lwS = sweep_lu(L, nb, false), lwV{};
+    omx::LuWork lwS = sweep_lu(L, nb, false, tune.trsv), lwV{};
     lwS.split = tune.split;
-    lwS.trsv = tune.trsv;
     if(sh) {
-      lwV = sweep_lu(L, nb, true);
+      lwV = sweep_lu(L, nb, true, tune.trsv);
       lwV.split = tune.split;
-      lwV.trsv = tune.trsv;
       HIPCHK(hipEventRecord(L->xev[0], st));
       HIPCHK(hipStreamWaitEvent(L->st2, L->xev[0], 0));
       factor(FV, lwV, L->st2);
@@ -2767,6 +2790,9 @@ int omx_get_stats(const omx_context *c, omx_stats *out) {
 int omx_set_profile(omx_context *c, int on) {
   return guard([&] {
     if(!c) throw OmxError(OMX_ERR_ARG, "null context");
+    HIPCHK(hipSetDevice(c->device));
+    for(auto &e : c->mv_ev)
+      if(on && !e) HIPCHK(hipEventCreate(&e));
     c->profile = on != 0;
     c->prof_gemm_ms = c->prof_panel_ms = c->prof_flop = c->prof_total_ms = 0;
     c->prof_launches = 0;
@@ -2880,6 +2906,7 @@ int omx_dense_solve(omx_context *c, int N, const double *A, const double *b, dou
     ctx.kind = kind;
     ctx.sh = 0;
     ctx.updated = false;
+    ctx.links_room = false;
     const size_t Np = ctx.Np;
     ctx.d_x.ensure(sizeof(cplx) * Np, &ctx.total);
     ctx.d_Q.ensure(sizeof(cplx) * Np, &ctx.total);

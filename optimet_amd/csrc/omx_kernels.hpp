@@ -203,7 +203,7 @@ struct LuWork {
   int *status;          // [0]: singular pivot column+1, [1]: wait timeout
   void *wlu;            // NB x NB complex: the tournament's selected-block factors
   void *dinv;           // per panel [L11^{-1} | U11^{-1}], 2 NB^2 elements of T, column-major
-  bool links = false;   // FP64 factors: the triangular solves' links follow in dinv
+  bool links = false;   // FP64 factors solved by variant 1: the triangular solves' links follow in dinv
   hipStream_t aux;      // look-ahead stream of the panel pivoting
   hipEvent_t ev_next, ev_piv, ev_bulk, ev_pan;
   int gmax;
@@ -218,10 +218,10 @@ struct LuWork {
   void (*on_mark)(void *) = nullptr;  // then on_mark(mark_arg) is called (on the host,
   void *mark_arg = nullptr;           // in the middle of the enqueueing)
 };
-// Elements of T in a factorisation's dinv: 2 NB^2 per panel, and (FP64 factors) as
-// many of the triangular solves' links, from links_at on.
+// Elements of T in a factorisation's dinv: 2 NB^2 per panel, and with links as many
+// of them, from links_at on.
 inline size_t links_at(int Np) { return 2 * (size_t)64 * Np; }
-inline size_t dinv_elems(int Np, bool f64) { return (f64 ? 2 : 1) * links_at(Np); }
+inline size_t dinv_elems(int Np, bool links) { return (links ? 2 : 1) * links_at(Np); }
 
 // Pivot search of a panel: among the rows of its diagonal block only
 // (followed by iterative refinement), or over the whole column (tournament).
@@ -250,6 +250,9 @@ constexpr int kTrsvVariants = 3;
 // 256 (split) or two with K = 128, on nb matrices sA apart.  A timing probe for the
 // autotuner; nothing to do up to Np = 256.  (A's contents are overwritten.)
 void bulk_update_probe(float2 *A, int Np, size_t lda, int nb, size_t sA, bool split, hipStream_t st);
+// The triangular solves' links of factored FP64 matrices (with w.links; lu_factor ends
+// with them).
+void lu_links(const double2 *A, int Np, size_t lda, const LuWork &w, hipStream_t st);
 // Solve with the factors: x = A^{-1} b, vectors always complex FP64.
 template <typename T>
 void lu_solve(const T *A, int Np, size_t lda, LuWork &w, const cplx *b, cplx *x, hipStream_t st);

@@ -1361,7 +1361,7 @@ void bulk_update(T *A, size_t lda, int row0, int col0, int k0, int M, int N, hip
 }
 
 // ------------------------------------------------------------------ links
-// The triangular solves' links (FP64 factors) Linv_k L[k, k-1] (blockIdx.y = 0, k = blockIdx.x +
+// The triangular solves' links (FP64 factors, variant 1) Linv_k L[k, k-1] (blockIdx.y = 0, k = blockIdx.x +
 // 1) and Uinv_k U[k, k+1] (1, k = blockIdx.x), beside the inverses they are formed
 // with: 64 x 64, column-major.  Wave w takes 16 rows.
 template <typename T>
@@ -1398,6 +1398,13 @@ __global__ __launch_bounds__(256) void link_kernel(const T *A, size_t lda, const
       links[at + (16 * n + CT<T>::row(lane, v)) * kNB + 16 * w + li] = o;
     }
   }
+}
+
+void lu_links(const double2 *A, int Np, size_t lda, const LuWork &w, hipStream_t st) {
+  double2 *dinv = reinterpret_cast<double2 *>(w.dinv);
+  if(w.links && Np > kNB)
+    hipLaunchKernelGGL((link_kernel<double2>), dim3(Np / kNB - 1, 2, w.nb), dim3(256), 0, st, A, lda, dinv,
+                       dinv + links_at(Np), w.bs);
 }
 
 // ------------------------------------------------------------------ driver
@@ -1445,10 +1452,7 @@ int lu_factor(T *A, int Np, size_t lda, LuWork &w, hipStream_t st, LuProf *prof)
     prof->gemm_launches = 0;
   }
   auto links = [&] {
-    if constexpr(std::is_same<T, double2>::value)
-      if(w.links && Np > kNB)
-        hipLaunchKernelGGL((link_kernel<T>), dim3(Np / kNB - 1, 2, nb), dim3(256), 0, st, A, lda, dinv,
-                           dinv + links_at(Np), bs);
+    if constexpr(std::is_same<T, double2>::value) lu_links(A, Np, lda, w, st);
   };
   if(block) {
     // G panels a group: quads (two pairs), whose bulk update has K = 4 NB, where

@@ -75,3 +75,42 @@ def test_the_split_product_is_timed_as_it_runs():
     implied = 8.0 * (Np - 256) ** 2 * 256 / q["times_ms"][0]
     s.ctx.close()
     assert 0.8 < implied / own < 1.75, implied / own
+
+
+def test_links_only_where_they_are_read():
+    """The one-block triangular solves of FP64 factors read links, 128 complex values
+    a row; a context that solves by another variant neither forms nor holds them,
+    and the solutions agree to the refinement's residual (1e-10)."""
+    from optimet_amd import solver
+    c = drude_cluster(12, 6, 700e-9, 40, 80, 900, 10, seed=3, sh=False)
+    out, held = {}, {}
+    for on in (False, True):
+        s = solver.Solver(c, kind="lu64")
+        s.ctx.set_autotune(on)
+        s.update()
+        out[on] = s.solve()["x_sca"]
+        held[on] = s.ctx.mem_info()[2]
+        Np = s.stats()["Np"]
+        s.ctx.close()
+    q = solver.tune_query(Np, 1, fp64=True)
+    assert held[True] - held[False] == (2048 * Np if q["trsv"] == 1 else 0), (held, q)
+    assert rel(out[True], out[False]) < 1e-10
+
+
+@pytest.mark.parametrize("graphs", [False, True])
+def test_fp64_sweep_with_the_tuner_on_and_off(graphs):
+    """Batches of FP64 factors by either variant, eager and captured, one captured
+    state after the other in one context."""
+    from optimet_amd import solver
+    c = drude_cluster(9, 6, 700e-9, 40, 80, 900, 10, seed=22)
+    lams = np.linspace(480e-9, 860e-9, 6)
+    s = solver.Solver(c, kind="lu64")
+    s.ctx.set_graphs(graphs)
+    outs = []
+    for on in (False, True, False):
+        s.ctx.set_autotune(on)
+        outs.append(s.sweep(lams, batch=3, outputs=("x_sca", "x_sca_sh")))
+    s.ctx.close()
+    for k in ("x_sca", "x_sca_sh"):
+        assert np.array_equal(outs[0][k], outs[2][k])
+        assert rel(outs[1][k], outs[0][k]) < 1e-10
