@@ -2069,11 +2069,11 @@ size_t sym_scratch(int P, int nmax, int nb) {
   return nb * (nc * P + (size_t)P * (P - 1) / 2) * n;
 }
 // Small blocks leave a thread few columns between the barriers of its objects.
-// Whole / half products, us: FP64 n = 6, N = 8202 167 / 628; n = 16, N = 8208 165 / 150,
-// 24016 1387 / 1125; n = 30, N = 8220 165 / 142.  FP32 n = 16, N = 24016 706 / 843; n =
-// 30, N = 8220 88 / 96, 49230 3017 / 3073; n = 48, N = 8208 86 / 74; n = 70 (rows of 560
-// bytes), N = 8260 89 / 93, 24010 692 / 684; n = 96, N = 8256 87 / 65.
-bool sym_pays(int nmax, bool f32) { return f32 ? nmax == 4 || nmax >= 6 : nmax >= 2; }
+// Whole / half products, us: FP64 n = 6, N = 8202 167 / 628; n = 16, N = 8208 161 / 149,
+// 24016 1377 / 1130; n = 30, N = 8220 164 / 140.  FP32 n = 16, N = 24016 709 / 849; n =
+// 30, N = 8220 89 / 105, 24030 694 / 745; n = 48, N = 8208 89 / 78; n = 70 (rows of 560
+// bytes), N = 8260 93 / 96, 24010 725 / 677, 49210 3006 / 2558; n = 96, N = 8256 86 / 66.
+bool sym_pays(int nmax, bool f32) { return nmax >= (f32 ? 4 : 2); }
 __device__ inline cplx sym_T(const SymArgs &a, const cplx *ov, int j, int pol, int n) {
   return ov[(((size_t)a.tkind * a.P + j) * 2 + pol) * (a.nmax + 1) + n];
 }
