@@ -380,7 +380,9 @@ __global__ __launch_bounds__(kRows) void kry_begin(KryState s, cplx *x, int firs
     s.V[z * s.sz + r] = (1.0 / beta) * s.r[z * s.sv + r];
   }
   if(!lead) return;
-  const double prev = first ? 0.0 : q.sc[KS_PREV], res = bn > 0.0 ? beta / bn : 0.0;
+  // (a single system's NaN right-hand side: a NaN residual, which no caller accepts;
+  // a batch's is left as it is)
+  const double prev = first ? 0.0 : q.sc[KS_PREV], res = bn == 0.0 || (batch && !(bn > 0.0)) ? 0.0 : beta / bn;
   int stall = first ? 0 : q.fl[KF_STALL];
   const int its = first ? 0 : q.fl[KF_ITS];
   bool go = !(first && bn == 0.0) && !(res <= s.tol) && its < s.maxit && res == res;

@@ -95,3 +95,21 @@ def test_solve_after_a_failed_one(kind):
         assert np.array_equal(got[k], ref[k]), k
     want.ctx.close()
     s.ctx.close()
+
+
+@pytest.mark.parametrize("kind", ["lu32ir", "gmres64", "gmres32ir", "auto"])
+def test_no_solution_from_a_source_that_is_not_a_number(kind):
+    """A sphere of the background's material has no scattered wave and an internal
+    one that the coefficients cannot give (0 times infinity): the second harmonic's
+    source is not a number, and the solve reports that it did not converge.  (The
+    FP64 LU ends with the plain partial-pivoting answer, which is returned as it is.)"""
+    from optimet_amd import solver
+    c = drude_cluster(3, 3, 700e-9, 40, 80, 500, 10, seed=4, sh=True)
+    c.meta.pop("drude")
+    c.eps_r = np.array([2.25, 1.0, 2.25], complex)
+    s = solver.Solver(c, kind=kind, maxit=40)
+    s.update()
+    with pytest.raises(solver.OmxError) as e:
+        s.solve()
+    assert e.value.code == -6
+    s.ctx.close()
