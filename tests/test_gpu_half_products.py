@@ -124,3 +124,28 @@ def test_without_memory_for_the_scratch():
     assert rel(got, want) < 1e-10
     a.ctx.close()
     b.ctx.close()
+
+
+def test_second_harmonic_operator():
+    """V's inner products by the mixed Krylov read half of V's blocks, with the factors
+    of the second harmonic: an outer step gains the six digits of an inner solve with
+    the right operator, two to three steps to 1e-12, and one to two digits with the
+    factors of S or another sign, five steps or more."""
+    from optimet_amd import solver
+    c = lattice(66, 7)
+    c.sh = True
+    c.eps_r, c.eps_r_sh = np.full(66, 2.25 + 0j), np.full(66, 3.0 + 0j)
+    c.ksippp, c.ksiparppar, c.gamma = np.full(66, 1e-18 + 0j), np.full(66, 3e-19 + 0j), np.full(66, 1e-19 + 0j)
+    assert c.N >= 8192
+    ref = solver.Solver(c, kind="lu64")
+    ref.update()
+    want = ref.solve()
+    s = solver.Solver(c, kind="gmres32ir", tol=1e-12)
+    s.update()
+    got = s.solve()
+    st = s.stats()
+    assert st["residual_sh"] <= 1e-12 and 0 < st["iterations_sh"] <= 3
+    for k in ("x_sca", "x_sca_sh"):
+        assert rel(got[k], want[k]) < 1e-10, k
+    ref.ctx.close()
+    s.ctx.close()
