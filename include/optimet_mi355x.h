@@ -326,7 +326,7 @@ int omx_dense_solve(omx_context *ctx, int N, const double *A, const double *b, d
  * identity-padded matrix's LU factors.  b and x hold N complex128 values.
  * Every work array (pivots, permutations, status words, diagonal-block inverses,
  * staged right-hand side) lives in one library-held scratch array per device
- * (about 8.6 MiB, held until the process ends), so N is limited to
+ * (about 8.3 MiB, held until the process ends), so N is limited to
  * 1 <= N <= 4096 (OMX_ERR_ARG beyond).  Calls that overlap on one device share
  * that array and race: issue them from one host thread at a time.  The call
  * runs on the context's stream and returns after x is written. */

@@ -354,7 +354,7 @@ void alloc_lu(omx_context *c, omx::LuWork &w, DBuf &perm, DBuf &dinv, bool secon
   // tournament scratch: one half per system, as S and V may be factored
   // at the same time
   c->d_cand.ensure(sizeof(int) * 4 * gmax * omx::kNB, &c->total);
-  c->d_wlu.ensure(sizeof(cplx) * 6 * omx::kNB * omx::kNB, &c->total);
+  c->d_wlu.ensure(sizeof(cplx) * 2 * omx::kNB * omx::kNB, &c->total);
   if(!second) {
     c->d_map.ensure(sizeof(int) * (3 * ((size_t)Np + 2 * omx::kNB)), &c->total);
     c->d_status.ensure(64, &c->total);
@@ -374,7 +374,7 @@ void alloc_lu(omx_context *c, omx::LuWork &w, DBuf &perm, DBuf &dinv, bool secon
   w.msrc = map.as<int>() + (Np + 2 * omx::kNB);
   w.mcnt = map.as<int>() + 2 * (Np + 2 * omx::kNB);
   w.status = status.as<int>();
-  w.wlu = c->d_wlu.as<cplx>() + (size_t)half * 3 * omx::kNB * omx::kNB;
+  w.wlu = c->d_wlu.as<cplx>() + (size_t)half * omx::kNB * omx::kNB;
   w.dinv = dinv.p;
   w.pivot = c->pivot;
   hipEvent_t *ev = second ? c->lu_ev2 : c->lu_ev;
@@ -1364,10 +1364,10 @@ void sweep_alloc(omx_context *c, int nb, bool f64, bool sh) {
   w.abssh.ensure(sizeof(double) * P * nb, T);
   w.absbes.ensure(sizeof(cplx) * P * omx::kAbsBes * nb, T);
   for(DBuf *b : {&w.perm, &w.perm2}) b->ensure(sizeof(int) * Np * nb, T);
-  w.map.ensure(sizeof(int) * 3 * (Np + 2 * omx::kNB) * nb, T);
+  w.map.ensure(sizeof(int) * Np * nb, T);
   w.status.ensure(sizeof(int) * 4 * nb, T);
   if(sh) {  // V's factorisation runs beside S's: maps and status words of its own
-    w.map2.ensure(sizeof(int) * 3 * (Np + 2 * omx::kNB) * nb, T);
+    w.map2.ensure(sizeof(int) * Np * nb, T);
     w.status2.ensure(sizeof(int) * 4 * nb, T);
   }
   w.basis.ensure(sizeof(cplx) * Np * (m + 1) * nb, T);
@@ -1395,13 +1395,8 @@ omx::LuWork sweep_lu(omx_context *c, int nb, bool second, int trsv) {
   lw.perm = (second ? w.perm2 : w.perm).as<int>();
   lw.links = c->kind == OMX_SOLVER_LU64 && trsv == 1;
   lw.trsv = trsv;
-  const int ms = Np + 2 * omx::kNB;
-  int *map = (second ? w.map2 : w.map).as<int>();
-  lw.mdst = map;
-  lw.msrc = map + (size_t)ms * nb;
-  lw.mcnt = map + 2 * (size_t)ms * nb;
+  lw.msrc = (second ? w.map2 : w.map).as<int>();
   lw.status = (second ? w.status2 : w.status).as<int>();
-  lw.wlu = c->d_wlu.p ? c->d_wlu.as<cplx>() + (second ? 3 * omx::kNB * omx::kNB : 0) : nullptr;
   // V's factorisation runs on the second stream pair, beside S's work
   lw.aux = second ? c->aux2 : c->aux;
   const hipEvent_t *ev = second ? c->lu_ev2 : c->lu_ev;
@@ -1420,8 +1415,7 @@ omx::LuWork sweep_lu(omx_context *c, int nb, bool second, int trsv) {
   lw.dinv = dinv.p;
   lw.bs.vec = (size_t)Np;
   lw.bs.perm = Np;
-  lw.bs.map = ms;
-  lw.bs.cnt = ms;
+  lw.bs.map = Np;
   lw.bs.status = 4;
   return lw;
 }
@@ -1926,8 +1920,8 @@ struct NoAllocLayout {
   static constexpr size_t perm = status + align256(16 * sizeof(int));  // Np ints
   static constexpr size_t cand = perm + align256(Np * sizeof(int));  // 2 x gmax x 64 ints
   static constexpr size_t map = cand + align256(2 * gmax * omx::kNB * sizeof(int));  // 3 x (Np + 128) ints
-  static constexpr size_t wlu = map + align256(3 * (Np + 2 * omx::kNB) * sizeof(int));  // 3 x 64 x 64 complex
-  static constexpr size_t dinv = wlu + align256(3 * omx::kNB * omx::kNB * sizeof(cplx));  // 2 x 64 x Np complex
+  static constexpr size_t wlu = map + align256(3 * (Np + 2 * omx::kNB) * sizeof(int));  // 64 x 64 complex
+  static constexpr size_t dinv = wlu + align256(omx::kNB * omx::kNB * sizeof(cplx));  // 2 x 64 x Np complex
   static constexpr size_t rhs = dinv + align256(2 * omx::kNB * (size_t)Np * sizeof(cplx));  // Np complex
   static constexpr size_t x = rhs + align256(Np * sizeof(cplx));  // Np complex
   static constexpr size_t bytes = x + align256(Np * sizeof(cplx));
@@ -2493,7 +2487,7 @@ void group_alloc(omx_context *L, int nb, bool f64, bool sh) {
   }
   for(DBuf *b : {&w.Q, &w.x, &w.xsh, &w.K, &w.r, &w.w1, &w.w2}) b->ensure(sizeof(cplx) * Np * nb, T);
   for(DBuf *b : {&w.perm, &w.perm2}) b->ensure(sizeof(int) * Np * nb, T);
-  for(DBuf *b : {&w.map, &w.map2}) b->ensure(sizeof(int) * 3 * (Np + 2 * omx::kNB) * nb, T);
+  for(DBuf *b : {&w.map, &w.map2}) b->ensure(sizeof(int) * Np * nb, T);
   for(DBuf *b : {&w.status, &w.status2}) b->ensure(sizeof(int) * 4 * nb, T);
   w.basis.ensure(sizeof(cplx) * Np * (m + 1) * nb, T);
   w.basisZ.ensure(sizeof(cplx) * Np * (m + 1) * nb, T);

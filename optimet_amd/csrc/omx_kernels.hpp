@@ -189,8 +189,7 @@ struct BatchStrides {
   size_t inv = 0;  // per-panel inverse sets (elements of T)
   size_t vec = 0;  // right-hand sides and solutions (complex FP64 elements)
   int perm = 0;    // permutations
-  int map = 0;     // gather maps (mdst, msrc)
-  int cnt = 0;     // map counts
+  int map = 0;     // row maps (msrc)
   int status = 0;  // status words
 };
 

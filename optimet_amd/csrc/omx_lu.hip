@@ -21,10 +21,11 @@
 //                  v_mfma_f64_16x16x4f64 (FP64) or v_mfma_f32_16x16x4f32
 //                  (FP32), four real MFMAs per complex tile product, planar
 //                  re/im operands staged through LDS; panels are taken in
-//                  pairs so that the bulk update runs with K = 2 NB
-//   gemm_split     the FP32 bulk update (K = 2 NB) on the bf16 matrix cores:
-//                  operands split in three bf16 terms, six products per
-//                  real product, FP32 accumulation (FP32-accurate)
+//                  pairs so that the bulk update runs with K = 2 NB (groups of
+//                  four, K = 4 NB, with gemm_split)
+//   gemm_split     the FP32 bulk update (groups of four panels, K = 4 NB) on the
+//                  bf16 matrix cores: operands split in three bf16 terms, six
+//                  products per real product, FP32 accumulation (FP32-accurate)
 //   trsv_kernel    sync-free blocked triangular solves: workgroup k owns
 //                  block row k, consumes earlier blocks as they are
 //                  published (tagged words) and applies its stored
@@ -877,26 +878,19 @@ void panel_products(T *A, size_t lda, int p0, int p1, int rows, int first_r, int
 }
 
 // ------------------------------------------------------------------ swaps
-// Applies a gather map (rows mdst[i] <- msrc[i], i < *mcnt <= 128) to the
-// columns c0 .. cend-1, leaving out skip0 .. skip0 + NB - 1 when skip0 >= 0:
-// each workgroup handles 8 columns, reads all moved entries into registers,
-// then writes them back.  With wlu (the tournament), the columns j0 .. j0 + NB -
-// 1 then take the factored block from it.
+// Tournament pivoting: applies the gather map (rows mdst[i] <- msrc[i], i < *mcnt <=
+// 128) to every column: each workgroup handles 8 columns, reads all moved entries
+// into registers, then writes them back.  The columns j0 .. j0 + NB - 1 then take
+// the factored block from wlu.
 template <typename T>
-__global__ __launch_bounds__(256) void laswp_map(T *A, size_t lda, int c0, int cend, const int *__restrict__ mdst,
+__global__ __launch_bounds__(256) void laswp_map(T *A, size_t lda, int Np, const int *__restrict__ mdst,
                                                  const int *__restrict__ msrc, const int *__restrict__ mcnt,
-                                                 int skip0, BatchStrides bs, const T *__restrict__ wlu, int j0) {
-  A += blockIdx.z * bs.a;
-  mdst += (size_t)blockIdx.z * bs.map;
-  msrc += (size_t)blockIdx.z * bs.map;
-  mcnt += (size_t)blockIdx.z * bs.cnt;
+                                                 const T *__restrict__ wlu, int j0) {
   const int m = *mcnt;
-  const int cl = threadIdx.x / 32, li = threadIdx.x % 32;
-  int col = c0 + blockIdx.x * 8 + cl;
-  if(skip0 >= 0 && col >= skip0) col += kNB;
+  const int cl = threadIdx.x / 32, li = threadIdx.x % 32, col = blockIdx.x * 8 + cl;
   T v[4];
   int d[4];
-  if(col < cend) {
+  if(col < Np) {
     T *a = A + (size_t)col * lda;
 #pragma unroll
     for(int k = 0; k < 4; ++k) {
@@ -906,13 +900,13 @@ __global__ __launch_bounds__(256) void laswp_map(T *A, size_t lda, int c0, int c
     }
   }
   __syncthreads();
-  if(col < cend) {
+  if(col < Np) {
     T *a = A + (size_t)col * lda;
 #pragma unroll
     for(int k = 0; k < 4; ++k)
       if(d[k] >= 0) a[d[k]] = v[k];
   }
-  if(wlu && col >= j0 && col < j0 + kNB) {
+  if(col >= j0 && col < j0 + kNB) {
     // the moves into the block's rows came from this column's 32 lanes, half a
     // wave: in order before these stores
     T *a = A + (size_t)col * lda + j0;
@@ -921,14 +915,6 @@ __global__ __launch_bounds__(256) void laswp_map(T *A, size_t lda, int c0, int c
     a[li] = w[li];
     a[li + 32] = w[li + 32];
   }
-}
-template <typename T>
-void laswp(T *A, size_t lda, int c0, int cend, const int *mdst, const int *msrc, const int *mcnt, int skip0,
-           hipStream_t st, int nb = 1, BatchStrides bs = BatchStrides{}, const T *wlu = nullptr, int j0 = 0) {
-  const int n = cend - c0 - (skip0 >= 0 ? kNB : 0);
-  if(n > 0)
-    hipLaunchKernelGGL((laswp_map<T>), dim3((n + 7) / 8, 1, nb), dim3(256), 0, st, A, lda, c0, cend, mdst, msrc, mcnt,
-                       skip0, bs, wlu, j0);
 }
 
 // Deferred interchanges of block pivoting: panel k = blockIdx.y (>= 1)
@@ -1580,7 +1566,7 @@ int lu_factor(T *A, int Np, size_t lda, LuWork &w, hipStream_t st, LuProf *prof)
   // interchanges on every column, and the factored block
   auto swaps = [&](int j0) {
     (void)hipStreamWaitEvent(st, w.ev_piv, 0);
-    laswp<T>(A, lda, 0, Np, w.mdst, w.msrc, w.mcnt, -1, st, 1, BatchStrides{}, wlu, j0);
+    hipLaunchKernelGGL((laswp_map<T>), dim3(Np / 8), dim3(256), 0, st, A, lda, Np, w.mdst, w.msrc, w.mcnt, wlu, j0);
   };
   // L21 and U12 of panel j0
   auto solves = [&](int j0) {
