@@ -28,59 +28,6 @@
 namespace omx {
 
 // ------------------------------------------------------------------ objects
-// sph_bessel's values and derivatives into memory (LDS): f[0 .. nmax+1] and
-// d[0 .. nmax], the same operations in the same order.
-__device__ inline void sph_bessel_to(int kind, cplx z, int nmax, cplx *f, cplx *d) {
-  const int top = nmax + 1;
-  const double az = hypot(z.x, z.y);
-  if(az <= kErrEps) {
-    for(int i = 0; i <= top; ++i) f[i] = mk(0.0);
-    for(int i = 0; i <= nmax; ++i) d[i] = mk(0.0);
-    if(kind == 0) f[0] = mk(1.0);
-    return;
-  }
-  if(kind == 1) {
-    cplx eiz = cexp_(mk(-z.y, z.x));
-    f[0] = mk(0.0, -1.0) * eiz / z;
-    f[1] = -(eiz * (z + mk(0.0, 1.0))) / (z * z);
-    for(int n = 1; n < top; ++n) f[n + 1] = ((2.0 * n + 1.0) * f[n]) / z - f[n - 1];
-  } else {
-    int start = (top > (int)ceil(az) ? top : (int)ceil(az)) + 30 + (int)ceil(4.0 * cbrt(az)) + (int)ceil(0.5 * az);
-    cplx fp1 = mk(0.0), fn = mk(1e-300);
-    for(int n = start; n > top; --n) {
-      cplx fm1 = ((2.0 * n + 1.0) * fn) / z - fp1;
-      fp1 = fn;
-      fn = fm1;
-      if(fabs(fn.x) + fabs(fn.y) > 1e200) {
-        fn = 1e-200 * fn;
-        fp1 = 1e-200 * fp1;
-      }
-    }
-    f[top] = fn;
-    cplx nxt = fp1;
-    for(int n = top; n >= 1; --n) {
-      cplx up = (n == top) ? nxt : f[n + 1];
-      f[n - 1] = ((2.0 * n + 1.0) * f[n]) / z - up;
-      if(fabs(f[n - 1].x) + fabs(f[n - 1].y) > 1e200) {
-        for(int k = n - 1; k <= top; ++k) f[k] = 1e-200 * f[k];
-        nxt = 1e-200 * nxt;
-      }
-    }
-    double mx = fmax(cabs(f[0]), cabs(f[1]));
-    for(int n = 0; n <= top; ++n) f[n] = f[n] / mx;
-    cplx s = csin_(z), c = ccos_(z);
-    cplx j0 = s / z, j1 = s / (z * z) - c / z;
-    double w = norm2(f[0]) + norm2(f[1]);
-    cplx sc = (j0 * conj(f[0]) + j1 * conj(f[1])) / w;
-    for(int n = 0; n <= top; ++n) f[n] = sc * f[n];
-  }
-  for(int i = 0; i <= nmax; ++i) d[i] = -f[i + 1] + (((double)i) * f[i]) / z;
-  if(kind == 0 && z.y == 0.0) {
-    for(int i = 0; i <= top; ++i) f[i].y = 0.0;
-    for(int i = 0; i <= nmax; ++i) d[i].y = 0.0;
-  }
-}
-
 // One workgroup of two waves per object.  Output ov[kind][obj][2][nmax+1] (TE
 // at [0], TM at [1]).  Bound: the latency of a Miller recurrence (about 60
 // complex divisions in a row); the seven Bessel sets of an object run side by
@@ -132,7 +79,7 @@ __global__ __launch_bounds__(128) void objects_kernel(ObjArgs a) {
       cplx kj = a.omega * csqrt_(eps * mu);
       z = R * kj;
     }
-    sph_bessel_to(set >= 5, z, nmax, bf[set], bd[set]);
+    sph_bessel(set >= 5, z, nmax, bf[set], bd[set]);
   }
   __syncthreads();
   if(t < 2 * nmax) {
@@ -249,71 +196,6 @@ struct DivBy {
   }
 };
 
-// Values j_l(z) (kind 0) or h_l^(1)(z) (kind 1), l < nv, into memory: the
-// steps of sph_values_to with the recurrences' divisions by z as above.
-__device__ inline void radial_to(int kind, cplx z, int nv, cplx *out) {
-  double az = hypot(z.x, z.y);
-  if(az <= kErrEps) {
-    for(int i = 0; i < nv; ++i) out[i] = mk(0.0);
-    if(kind == 0) out[0] = mk(1.0);
-    return;
-  }
-  const DivBy by(z);
-  if(kind == 1) {
-    cplx eiz = cexp_(mk(-z.y, z.x));
-    cplx h0 = mk(0.0, -1.0) * eiz / z;
-    cplx h1 = -(eiz * (z + mk(0.0, 1.0))) / (z * z);
-    out[0] = h0;
-    if(nv > 1) out[1] = h1;
-    for(int n = 1; n + 1 < nv; ++n) {
-      cplx h2 = by((2.0 * n + 1.0) * h1) - h0;
-      out[n + 1] = h2;
-      h0 = h1;
-      h1 = h2;
-    }
-    return;
-  }
-  const int top = nv - 1;
-  int start = ((top + 1) > (int)ceil(az) ? (top + 1) : (int)ceil(az)) + 30 + (int)ceil(4.0 * cbrt(az)) +
-              (int)ceil(0.5 * az);
-  cplx fp1 = mk(0.0), fn = mk(1e-300);
-  for(int n = start; n > top; --n) {
-    cplx fm1 = by((2.0 * n + 1.0) * fn) - fp1;
-    fp1 = fn;
-    fn = fm1;
-    if(fabs(fn.x) + fabs(fn.y) > 1e200) {
-      fn = 1e-200 * fn;
-      fp1 = 1e-200 * fp1;
-    }
-  }
-  out[top] = fn;
-  cplx up = fp1, cur = fn;
-  for(int n = top; n >= 1; --n) {
-    cplx lo = by((2.0 * n + 1.0) * cur) - up;
-    out[n - 1] = lo;
-    up = cur;
-    cur = lo;
-    if(fabs(lo.x) + fabs(lo.y) > 1e200) {
-      for(int k = n - 1; k <= top; ++k) out[k] = 1e-200 * out[k];
-      up = 1e-200 * up;
-      cur = 1e-200 * cur;
-    }
-  }
-  cplx f0 = out[0], f1 = nv > 1 ? out[1] : mk(0.0);
-  double mx = fmax(cabs(f0), cabs(f1));
-  f0 = f0 / mx;
-  f1 = f1 / mx;
-  cplx s = csin_(z), c = ccos_(z);
-  cplx j0 = s / z, j1 = s / (z * z) - c / z;
-  double w = norm2(f0) + norm2(f1);
-  cplx sc = ((j0 * conj(f0) + j1 * conj(f1)) / w) / mx;
-  for(int n = 0; n <= top; ++n) {
-    cplx v = sc * out[n];
-    if(z.y == 0.0) v.y = 0.0;
-    out[n] = v;
-  }
-}
-
 // Computes z_l and Y_l^k for pair vector R (r, theta, phi) and wavenumber k.
 template <int NMAX>
 __device__ void pair_setup(PairLDS<NMAX> &s, double Rr, double Rt, double Rp, cplx k, bool hankel,
@@ -324,7 +206,7 @@ __device__ void pair_setup(PairLDS<NMAX> &s, double Rr, double Rt, double Rp, cp
     // +m instance: k; -m instance: conj(k) (regular) or -conj(k) (irregular)
     // (TranslationAdditionCoefficients.h:72-74)
     cplx kk = (t == 0) ? k : (hankel ? -conj(k) : conj(k));
-    radial_to(hankel ? 1 : 0, Rr * kk, L + 1, s.h[t]);
+    sph_values_to<DivBy>(hankel ? 1 : 0, Rr * kk, L + 1, s.h[t]);
   } else if(t >= 64 && t < 64 + L) {
     // normalised associated Legendre, column |k| = am, rows l = am .. L-1; all
     // coefficients are loaded before the recurrence starts

@@ -67,11 +67,11 @@ __host__ __device__ inline cplx csqrt_(cplx a) {
 // Spherical Bessel (kind 0) or Hankel h^(1) (kind 1) values f[0..nmax+1]
 // and derivatives d[0..nmax] with the conventions of Bessel.h:58-143:
 // |z| <= 1e-10 gives zeros (j_0 = 1); real z gives real j_n.
-template <int CAP>
-__host__ __device__ inline void sph_bessel(int kind, cplx z, int nmax, cplx (&f)[CAP], cplx (&d)[CAP]) {
-  for(int i = 0; i < CAP; ++i) f[i] = d[i] = mk(0.0);
+__host__ __device__ inline void sph_bessel(int kind, cplx z, int nmax, cplx *f, cplx *d) {
   double az = hypot(z.x, z.y);
   if(az <= kErrEps) {
+    for(int i = 0; i <= nmax + 1; ++i) f[i] = mk(0.0);
+    for(int i = 0; i <= nmax; ++i) d[i] = mk(0.0);
     if(kind == 0) f[0] = mk(1.0);
     return;
   }
@@ -119,16 +119,24 @@ __host__ __device__ inline void sph_bessel(int kind, cplx z, int nmax, cplx (&f)
   }
 }
 
+// Division by a fixed z, the plain way (sph_values_to's default).
+struct PlainDiv {
+  cplx z;
+  __device__ PlainDiv(cplx v) : z(v) {}
+  __device__ cplx operator()(cplx a) const { return a / z; }
+};
+
 // Values only, written straight to memory (LDS) by one thread, without local
 // arrays: out[0..nv) = j_l(z) (kind 0) or h_l^(1)(z) (kind 1), same
-// algorithms and edge rules as sph_bessel.
-__device__ inline void sph_values_to(int kind, cplx z, int nv, cplx *out) {
+// algorithms and edge rules as sph_bessel; the recurrences divide by z with Div.
+template <class Div = PlainDiv> __device__ inline void sph_values_to(int kind, cplx z, int nv, cplx *out) {
   double az = hypot(z.x, z.y);
   if(az <= kErrEps) {
     for(int i = 0; i < nv; ++i) out[i] = mk(0.0);
     if(kind == 0) out[0] = mk(1.0);
     return;
   }
+  const Div by(z);
   if(kind == 1) {
     cplx eiz = cexp_(mk(-z.y, z.x));
     cplx h0 = mk(0.0, -1.0) * eiz / z;
@@ -136,7 +144,7 @@ __device__ inline void sph_values_to(int kind, cplx z, int nv, cplx *out) {
     out[0] = h0;
     if(nv > 1) out[1] = h1;
     for(int n = 1; n + 1 < nv; ++n) {
-      cplx h2 = ((2.0 * n + 1.0) * h1) / z - h0;
+      cplx h2 = by((2.0 * n + 1.0) * h1) - h0;
       out[n + 1] = h2;
       h0 = h1;
       h1 = h2;
@@ -148,7 +156,7 @@ __device__ inline void sph_values_to(int kind, cplx z, int nv, cplx *out) {
               (int)ceil(0.5 * az);
   cplx fp1 = mk(0.0), fn = mk(1e-300);
   for(int n = start; n > top; --n) {
-    cplx fm1 = ((2.0 * n + 1.0) * fn) / z - fp1;
+    cplx fm1 = by((2.0 * n + 1.0) * fn) - fp1;
     fp1 = fn;
     fn = fm1;
     if(fabs(fn.x) + fabs(fn.y) > 1e200) {
@@ -159,7 +167,7 @@ __device__ inline void sph_values_to(int kind, cplx z, int nv, cplx *out) {
   out[top] = fn;
   cplx up = fp1, cur = fn;
   for(int n = top; n >= 1; --n) {
-    cplx lo = ((2.0 * n + 1.0) * cur) / z - up;
+    cplx lo = by((2.0 * n + 1.0) * cur) - up;
     out[n - 1] = lo;
     up = cur;
     cur = lo;
