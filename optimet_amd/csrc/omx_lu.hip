@@ -859,9 +859,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
     store(p1);
   }
 }
-constexpr long kWideStrips = 512;
 // Strip width: 16 while that fills the chip no more than twice, else 32 (the
-// 64 x 64 operands are then read half as often).
+// 64 x 64 operands are then read half as often).  The line is not sharp: with 256 /
+// 512 / 1024 / 4096 strips FP64 solves of 2208 take 3.67 / 3.68 / 3.66 / 3.67 ms, mixed
+// ones of 10240 31.6 / 31.6 / 31.7 / 31.7.
+constexpr long kWideStrips = 512;
 template <typename T, bool PAIR>
 void panel_products(T *A, size_t lda, int p0, int p1, int rows, int first_r, int cols, int first_c, const T *d0,
                     const T *d1, const int *ms0, const int *ms1, hipStream_t st, int nb, BatchStrides bs) {
@@ -1486,15 +1488,7 @@ int lu_factor(T *A, int Np, size_t lda, LuWork &w, hipStream_t st, LuProf *prof)
         bulk_update<T>(A, lda, q, q, J, Np - q, (np - 2) * kNB, sb, nb, bs.a, w.split);
         pair(q, np > 3);
       }
-      // L21 of the last panel goes with the far columns' strips, unless they wait
-      // for a bulk update that it can run beside
       const int last = far - 2 * kNB;  // the group's last pair
-      const bool apart = restf > 0 && (long)restf / 16 * nb > kWideStrips;
-      if(apart) {
-        // by the kernel of a single panel, whose workgroups fit beside the update's
-        const int pl = last + kNB;
-        panel_products<T, false>(A, lda, pl, 0, restf, far, 0, far, dk(pl), nullptr, nullptr, nullptr, sb, nb, bs);
-      }
       if(rec) (void)hipEventRecord(pe[1], sb);
       if(restf > 0) {
         (void)hipStreamWaitEvent(sb, w.ev_bulk, 0);
@@ -1502,7 +1496,7 @@ int lu_factor(T *A, int Np, size_t lda, LuWork &w, hipStream_t st, LuProf *prof)
           through(J, false, restf, far);
           bulk_update<T>(A, lda, q, far, J, 2 * kNB, restf, sb, nb, bs.a, w.split);
         }
-        through(last, !apart, restf, far);
+        through(last, true, restf, far);  // and L21 of the last panel
       }
       (void)hipEventRecord(w.ev_pan, sb);
       (void)hipStreamWaitEvent(st, w.ev_pan, 0);
