@@ -159,10 +159,13 @@ def run_sweep(cluster, lams, kind, steps, warmup, batch, graphs=False):
     return {"lat": lat, "total": total, "out": out, "stats": st, "prof": prof}
 
 
-def matvec_roofline(st, kernel="gemv_part_kernel (batched FP64 matvec of the refinement)"):
+MATVEC = "gemv_part_kernel (batched FP64 matvec of the refinement)"
+
+
+def matvec_roofline(st, kernel=MATVEC):
     """The Krylov or refinement matvecs: their algorithmic bytes (16 Np^2 per
-    FP64 product, 8 Np^2 per FP32-matrix product, per system) over the
-    HIP-event time of their launches on the stream they run on."""
+    FP64 product, 8 Np^2 per FP32-matrix product, per system; half of them where half of
+    the blocks are read) over the HIP-event time of their launches on the stream they run on."""
     if st["t_matvec_ms"] <= 0 or st["matvec_calls"] <= 0:
         return None
     gbs = st["matvec_bytes"] / (st["t_matvec_ms"] * 1e-3) / 1e9
@@ -209,7 +212,8 @@ def sweep_main(args):
         "step": "one sweep of all wavelengths (a solve = one wavelength at omega and 2 omega)",
         "p50_ms_per_sweep": 1e3 * pct(mixed["lat"], 50), "p99_ms_per_sweep": 1e3 * pct(mixed["lat"], 99),
         "max_iterations": [ms["iterations"], ms["iterations_sh"]], "max_residual": [ms["residual"], ms["residual_sh"]],
-        "roofline": matvec_roofline(mixed["prof"]),
+        "roofline": matvec_roofline(mixed["prof"], "sym_pairs (FP64 GMRES steps, half of S) and gemv_part_kernel "
+                                    "(residuals, refinement), batched" if args.sweep_kind == "auto" else MATVEC),
         "autotune": {"lu32ir": tuned(ms["Np"], ms["sweep_batch"], False),
                      "lu64": tuned(ms["Np"], ms["sweep_batch"], True) if fp64 is not None else None},
         "systems_redone_alone": ms["pivot_fallbacks"],
@@ -466,8 +470,8 @@ def config5_main(args):
                 "launches": sum(st["lu_gemm_launches"] for st in log)}
     elif mv_ms > 0:
         a = mv_bytes / (mv_ms * 1e-3) / 1e9
-        roof = {"bound": "hbm", "kernel": "gemv_part_kernel (refinement and Krylov products)", "achieved": a,
-                "peak": HBM_GBS, "unit": "GB/s", "frac": a / HBM_GBS, "traffic": None}
+        roof = {"bound": "hbm", "kernel": "sym_pairs (Krylov steps) and gemv_part_kernel (residuals, refinement)",
+                "achieved": a, "peak": HBM_GBS, "unit": "GB/s", "frac": a / HBM_GBS, "traffic": None}
     else:
         roof = None
     if roof is not None:

@@ -68,10 +68,11 @@ extern "C" {
                                   OMX_SOLVER_LU32_IR on the same matrices; smaller systems use
                                   OMX_SOLVER_LU32_IR, except that with the second harmonic S
                                   is first tried with FP64 GMRES (within N / 125 products)
-                                  while V's mixed LU factorises (from half of V's columns
-                                  on); batched sweeps from N = 2048 with the second harmonic
-                                  try S by lockstep FP64 GMRES (within 2 N / 125 steps)
-                                  beside V's batched mixed LU */
+                                  while V's mixed LU factorises (together below N = 9216,
+                                  from a quarter of V's columns on above); batched sweeps
+                                  from N = 2048 with the second harmonic try S by lockstep
+                                  FP64 GMRES (within 2 N / 125 steps) beside V's batched
+                                  mixed LU */
 
 /* Pivot search of the LU factorisations (omx_set_pivoting). */
 #define OMX_PIVOT_BLOCK 0     /* among the rows of each 64 x 64 diagonal block, then
@@ -79,7 +80,8 @@ extern "C" {
                                  zero pivot or a refinement that does not converge */
 #define OMX_PIVOT_PARTIAL 1   /* partial pivoting over the whole column (tournament) */
 
-/* Products of the complex-FP32 factorisation's bulk updates (omx_set_lu32_gemm). */
+/* Products of the complex-FP32 factorisation's bulk updates (omx_set_lu32_gemm);
+ * in large batches (from 512 tiles of 128 x 128 on) its panels' updates take them too. */
 #define OMX_GEMM_BF16X3 0     /* each FP32 operand split in three bf16 terms, six
                                  bf16 MFMA products per real product, FP32
                                  accumulation: FP32 accuracy at the bf16 rate */
@@ -102,7 +104,7 @@ typedef struct {
   size_t device_bytes;   /* device memory held by the context */
   /* with omx_set_profile(ctx, 1), accumulated over the factorisations since:
    * HIP-event times on the streams the kernels run on */
-  double t_lu_gemm_ms;   /* bulk trailing updates (K = 128) */
+  double t_lu_gemm_ms;   /* bulk trailing updates (K = 256 with split products, else 128) */
   double lu_gemm_flop;   /* their algorithmic flop, 8 m n k per launch */
   int lu_gemm_launches;  /* their kernel launches */
   double t_lu_panel_ms;  /* panel work of each pair up to its far-column step */
@@ -111,7 +113,8 @@ typedef struct {
   int sweep_batch;       /* systems per batch of the last omx_solve_sweep */
   int matvec_calls;      /* FP64 matrix-vector products of the iterative solvers (since omx_set_profile) */
   double t_matvec_ms;    /* their HIP-event time (profiling on) */
-  double matvec_bytes;   /* their algorithmic bytes, 16 Np^2 per system and product */
+  double matvec_bytes;   /* their algorithmic bytes, 16 Np^2 per system and product (half of it
+                            where a product reads half of the blocks) */
   int graph_captures;    /* factorisation graphs captured (omx_set_graphs) since creation */
   int graph_launches;    /* factorisations run as graph launches since creation */
 } omx_stats;

@@ -1152,7 +1152,7 @@ cplx *sym_ensure(omx_context *c, size_t elems) {
 
 // Products of the assembled S (V) from half its blocks, from N = kSymN on (below,
 // the caches hold much of the matrix: N = 2142 20 us whole, 28 from its half; 10240
-// 244 and 181) and for the block orders that gain by it; without scratch otherwise.
+// 249 and 171) and for the block orders that gain by it; without scratch otherwise.
 omx::SymArgs sym_args(omx_context *c, bool shf, bool f32) {
   omx::SymArgs a{c->P, c->nmax, c->Np, (size_t)c->Np, c->d_ov.as<cplx>(), shf ? omx::OV_TSH : omx::OV_T, nullptr};
   if(c->kind == OMX_SOLVER_ACA_GMRES || !c->updated || c->P < 2 || c->N < kSymN || !omx::sym_pays(c->nmax, f32))

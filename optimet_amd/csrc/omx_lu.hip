@@ -366,7 +366,7 @@ template <typename T> __device__ __forceinline__ void invert_block(CxOf<T> *F, c
 // plus the inverses by one thread a column in a kernel of its own, the panels of
 // an FP64 system of 1500 took 1.0 ms each and the solve 26.5 ms; with a barrier
 // every 8 columns instead of the published steps 96 us a level and 7.3 ms; now 54 us
-// and 4.8 ms.
+// and 4.76 ms.
 template <typename T, int RPL>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(1, 2))) void tslu_panel(
     const T *A, size_t lda, int Np, int j0, int gin, const int *cin, int *cout, T *wlu, T *dinv, int *mdst, int *msrc,
@@ -2075,8 +2075,9 @@ __device__ inline cplx sym_widen(float2 v) { return cplx{(double)v.x, (double)v.
 // y_j's to z[pair].
 //
 // Bound: HBM, at half the bytes of the plain product, and the barriers between
-// objects.  N = 49152: FP32 2.78 -> 2.24 ms, FP64 5.45 -> 3.70; N = 10240, FP64: 244 ->
-// 181 us; N = 2142: 20 -> 28, so single systems take it from kSymN on, where sym_pays.
+// objects.  N = 49152 (n = 96): FP32 2.78 -> 1.86 ms, 5.2 TB/s of the half, FP64 5.50 ->
+// 3.38, 5.7 TB/s; N = 10240 (n = 160), FP64: 249 -> 171 us, 4.9 TB/s; N = 2142: 20 -> 28,
+// so single systems take it from kSymN on, where sym_pays.
 template <typename T>
 __global__ __launch_bounds__(512) void sym_pairs(SymArgs a, const T *__restrict__ A, const cplx *__restrict__ x, int CH,
                                                 int G) {
@@ -2109,8 +2110,8 @@ __global__ __launch_bounds__(512) void sym_pairs(SymArgs a, const T *__restrict_
   cplx acc = mk(0.0);
   // Columns by E, the next E (of the next object after the last) on their way while
   // these are summed: the barriers between objects then wait for no load.  E: four
-  // waves a SIMD in either type (FP64 with 4 / 6 / 8: N = 49152 3.67 / 3.69 / 4.03
-  // ms, 10240 176 / 205 / 193 us; FP32: 2.31 / 2.20 / 2.26 ms)
+  // waves a SIMD in either type (by 8 objects, FP64 with 4 / 6 / 8: N = 49152 3.67 /
+  // 3.69 / 4.03 ms, 10240 176 / 205 / 193 us; FP32: 2.31 / 2.20 / 2.26 ms)
   constexpr int E = sizeof(T) == 8 ? 6 : 4;
   const int j0 = max(i + 1, c * CH), cnt = n / G, steps = (cnt + E - 1) / E;
   cplx Tn = sym_T(a, ov, j0, pol, deg);
