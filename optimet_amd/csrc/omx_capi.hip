@@ -1182,7 +1182,8 @@ void solve_system(omx_context *c, bool shf, const cplx *rhs, cplx *x, int *iters
     *iters = gm.its[0];
     *res = gm.res[0];
   };
-  // (V's few outer products read the whole matrix)
+  // (V's FP64 products read the whole matrix: those of S were measured, and of the
+  // choices that a size makes only the mixed Krylov has any of V's, about five a solve)
   if(!is_lu(c->kind) && !shf) gm.sym = sym_args(c, shf, false);
   if(c->kind == OMX_SOLVER_ACA_GMRES) {  // Gmres_Zcomp on the compressed operator
     gm.op = [c, shf, st](const cplx *in, cplx *out) { aca_apply(c, shf, in, out, st); };
